@@ -1317,6 +1317,15 @@ extern "C" void dvmh_loop_cuda_red_finish_C(DvmType curLoop, DvmType redIndex) {
     gpuRedFinish(sl, r);
 }
 
+extern "C" void dvmh_amd_loop_red_in_kernel_C(DvmType curLoop, DvmType items, DvmhAmdRedFinish *out) {
+    gpuRedInKernel(asSpec(curLoop, "dvmh_amd_loop_red_in_kernel_C"), items, out);
+}
+
+extern "C" void dvmh_amd_loop_red_result_C(DvmType curLoop, DvmType redIndex, void **outVal, void **outLoc) {
+    SpecLoop *sl = asSpec(curLoop, "dvmh_amd_loop_red_result_C");
+    gpuRedResult(redOf(sl->loop, redIndex, "dvmh_amd_loop_red_result_C").get(), outVal, outLoc);
+}
+
 extern "C" void dvmh_loop_red_post_C(DvmType curLoop, DvmType redIndex, const void *arrayAddr, const void *locAddr) {   // :4386
     Loop *l = loopOf(curLoop, "dvmh_loop_red_post_C");
     redOf(l, redIndex, "dvmh_loop_red_post_C")->postValues(arrayAddr, locAddr);

@@ -103,6 +103,9 @@ void Gpu::init() {
     // launch leaves them zero again
     HIP_CHECK(hipMalloc((void **)&finishCounters, 64 * sizeof(unsigned)));
     HIP_CHECK(hipMemset(finishCounters, 0, 64 * sizeof(unsigned)));
+    const size_t redBytes = sizeof(unsigned) * DVMH_AMD_RED_STRIDE * (1 + DVMH_AMD_RED_GROUPS);
+    HIP_CHECK(hipMalloc((void **)&redCounters, redBytes));
+    HIP_CHECK(hipMemset(redCounters, 0, redBytes));
     void *done = nullptr;
     HIP_CHECK(hipHostMalloc(&done, 64, hipHostMallocMapped));
     doneHost = (volatile unsigned long long *)done;

@@ -192,10 +192,12 @@ void gpuRedPrepare(SpecLoop *sl, Reduction *r, long count, bool fill) {
     DVMH_CHECK(count > 0, "Reduction partial count must be positive");
     DVMH_CHECK(r->gpuArr == nullptr, "dvmh_loop_cuda_red_prepare_C called twice for one reduction");
     r->items = count;
-    r->gpuArr = gpu.alloc((size_t)(r->elemCount * r->elemSize * count));
+    // a scalar's partials may be folded by the loop's own launch, group by group
+    const long slots = r->elemCount == 1 ? count + redGroups(count) : r->elemCount * count;
+    r->gpuArr = gpu.alloc((size_t)(r->elemSize * slots));
     if (r->gpuArrPtr) *r->gpuArrPtr = r->gpuArr;
     if (r->isLoc()) {
-        r->gpuLoc = gpu.alloc((size_t)(r->elemCount * r->locSize * count));
+        r->gpuLoc = gpu.alloc((size_t)(r->locSize * slots));
         if (r->gpuLocPtr) *r->gpuLocPtr = r->gpuLoc;
     }
     if (fill) {
@@ -207,6 +209,50 @@ void gpuRedPrepare(SpecLoop *sl, Reduction *r, long count, bool fill) {
                         sl->stream);
         }
     }
+}
+
+// One group up to 256 partials (four per lane of the folding wave); beyond, a
+// power of two near the square root, so that the two folds are about equally
+// long, and at most DVMH_AMD_RED_GROUPS groups.
+unsigned redGroupSize(long items) {
+    if (items <= 256) return 256;
+    unsigned g = 64;
+    while ((long)g * g < items || (items + g - 1) / g > DVMH_AMD_RED_GROUPS) g *= 2;
+    return g;
+}
+
+// The loop's launch finishes its reductions: counters, group shape and the
+// completion word it publishes (none while capturing: a graph's replays would
+// all publish the same value).
+void gpuRedInKernel(SpecLoop *sl, long items, DvmhAmdRedFinish *out) {
+    DVMH_CHECK(items > 0 && items < (1L << 32), "In-kernel finish of %ld partials", items);
+    sl->redInKernel = true;
+    sl->redSeq = graphCapturing() ? 0 : ++gpu.doneSeq;
+    out->counters = gpu.redCounters;
+    out->done = sl->redSeq ? gpu.doneDev : nullptr;
+    out->doneSeq = sl->redSeq;
+    out->items = (unsigned)items;
+    out->groupSize = redGroupSize(items);
+    out->groups = (unsigned)redGroups(items);
+}
+
+// One folded record of a reduction in pinned host memory: its L values, then
+// (16-byte aligned) its L loc records.  A captured finish writes into a slot
+// owned by the graph.
+static void takeRecord(const Reduction *r, char **val, char **loc) {
+    const long L = r->elemCount;
+    const size_t locOff = ((size_t)(L * r->elemSize) + 15) & ~(size_t)15;
+    const size_t recBytes = r->isLoc() ? locOff + (size_t)(L * r->locSize) : (size_t)(L * r->elemSize);
+    *val = graphCapturing() ? graphPinnedSlot(recBytes) : pinnedPool.take(recBytes);
+    *loc = r->isLoc() ? *val + locOff : nullptr;
+}
+
+void gpuRedResult(Reduction *r, void **outVal, void **outLoc) {
+    DVMH_CHECK(r->gpuArr != nullptr && r->elemCount == 1, "dvmh_amd_loop_red_result_C without dvmh_loop_cuda_red_prepare_C");
+    takeRecord(r, &r->resVal, &r->resLoc);
+    char *dev = mappedDevicePtr(r->resVal);
+    *outVal = dev;
+    if (outLoc) *outLoc = r->resLoc ? dev + (r->resLoc - r->resVal) : nullptr;
 }
 
 // DvmhReductionCuda::finish (rts/dvmh/loop.cpp:301-408): fold the partials on
@@ -235,9 +281,27 @@ void gpuRedFinish(SpecLoop *sl, const std::shared_ptr<Reduction> &r) {
 void gpuRedFinishFlush(SpecLoop *sl) {
     auto &q = sl->finishQueue;
     if (q.empty()) return;
-    // One folded record per reduction, posted in the order the handler asked
-    // for the finishes (a captured graph's replays re-post them in that order):
-    // its L values, then (16-byte aligned) its L loc records.
+    auto releasePartials = [&q]() {
+        for (auto &r : q) {
+            gpu.release(r->gpuArr);
+            r->gpuArr = nullptr;
+            if (r->gpuLoc) { gpu.release(r->gpuLoc); r->gpuLoc = nullptr; }
+        }
+        q.clear();
+    };
+    // Records are posted in the order the handler asked for the finishes (a
+    // captured graph's replays re-post them in that order).
+    if (sl->redInKernel) {
+        for (auto &r : q) {
+            DVMH_CHECK(r->resVal != nullptr, "dvmh_amd_loop_red_result_C was not called for a reduction finished in the kernel");
+            if (graphCapturing()) graphNotePost(r, r->resVal, r->resLoc);
+            addPendingPost(r, r->resVal, r->resLoc);
+            r->resVal = r->resLoc = nullptr;
+        }
+        pendingDone = sl->redSeq;
+        releasePartials();
+        return;
+    }
     struct Entry {
         Reduction *r;
         long e;
@@ -245,16 +309,12 @@ void gpuRedFinishFlush(SpecLoop *sl) {
     };
     std::vector<Entry> entries;
     for (auto &r : q) {
-        const long L = r->elemCount;
-        const size_t locOff = ((size_t)(L * r->elemSize) + 15) & ~(size_t)15;
-        const size_t recBytes = r->isLoc() ? locOff + (size_t)(L * r->locSize) : (size_t)(L * r->elemSize);
-        // a captured finish writes into a slot owned by the graph
-        char *host = graphCapturing() ? graphPinnedSlot(recBytes) : pinnedPool.take(recBytes);
-        char *hostLoc = r->isLoc() ? host + locOff : nullptr;
+        char *host, *hostLoc;
+        takeRecord(r.get(), &host, &hostLoc);
         if (graphCapturing()) graphNotePost(r, host, hostLoc);
         char *dev = mappedDevicePtr(host);
-        for (long e = 0; e < L; e++)
-            entries.push_back(Entry{r.get(), e, dev + e * r->elemSize, r->isLoc() ? dev + locOff + e * r->locSize : nullptr});
+        for (long e = 0; e < r->elemCount; e++)
+            entries.push_back(Entry{r.get(), e, dev + e * r->elemSize, hostLoc ? dev + (hostLoc - host) + e * r->locSize : nullptr});
         addPendingPost(r, host, hostLoc);
     }
     // every element of every reduction is folded by one multi-finish entry;
@@ -299,12 +359,7 @@ void gpuRedFinishFlush(SpecLoop *sl) {
         if (signal) pendingDone = seq;
         for (void *p : slots) gpu.release(p);
     }
-    for (auto &r : q) {
-        gpu.release(r->gpuArr);
-        r->gpuArr = nullptr;
-        if (r->gpuLoc) { gpu.release(r->gpuLoc); r->gpuLoc = nullptr; }
-    }
-    q.clear();
+    releasePartials();
 }
 
 // ------------------------------------------------------------ layout policy

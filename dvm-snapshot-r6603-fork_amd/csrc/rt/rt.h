@@ -81,6 +81,7 @@ public:
     DeviceProps props;
     hipStream_t stream = nullptr;
     unsigned *finishCounters = nullptr;   // arrival counters of the multi-reduction finish (kept zero between launches)
+    unsigned *redCounters = nullptr;      // arrival counters of in-kernel finishes (one launch at a time on the stream; kept zero)
     // completion word in mapped pinned host memory: a reduction finish sets it
     // to its sequence number once its results are written
     volatile unsigned long long *doneHost = nullptr;
@@ -232,6 +233,7 @@ struct Reduction {
     void **gpuArrPtr = nullptr, **gpuLocPtr = nullptr;
     void *gpuArr = nullptr, *gpuLoc = nullptr;
     long items = 0;
+    char *resVal = nullptr, *resLoc = nullptr;   // where an in-kernel finish leaves the folded record (pinned host memory)
     std::vector<char> localArr, localLoc;
     void initValues(void *arr, void *loc) const;                               // :37-91
     // lowerLocOnTie: equal values take the lower scalar-integer loc (the merge
@@ -268,6 +270,8 @@ struct SpecLoop : Object {
     bool explore = false;           // the tuner times this execution (candidate still lacks repeats)
     hipEvent_t tuneStart = nullptr; // recorded at the pick when exploring
     std::vector<std::shared_ptr<Reduction>> finishQueue;   // red_finish requests, run when the handler returns
+    bool redInKernel = false;       // the loop's launch folds its reductions itself (dvmh_amd_loop_red_in_kernel_C)
+    unsigned long long redSeq = 0;  // and publishes this completion word (0: none)
     std::vector<void *> toFree;
     SpecLoop(Loop *l, int dev): Object(Kind::SpecLoop), loop(l), device(dev) {}
 };
@@ -334,6 +338,11 @@ void performLoop(Loop *loop);
 // reductions on the GPU (kernels in csrc/kernels/reduce.hip)
 void gpuRedPrepare(SpecLoop *sl, Reduction *r, long count, bool fill);
 void gpuRedFinish(SpecLoop *sl, const std::shared_ptr<Reduction> &r);
+// Groups of consecutive partials an in-kernel finish of `items` folds them in.
+unsigned redGroupSize(long items);
+inline long redGroups(long items) { return (items + redGroupSize(items) - 1) / redGroupSize(items); }
+void gpuRedInKernel(SpecLoop *sl, long items, DvmhAmdRedFinish *out);
+void gpuRedResult(Reduction *r, void **outVal, void **outLoc);
 void gpuRedFinishFlush(SpecLoop *sl);
 void flushDeferredPosts();
 void flushPostsFor(const void *addr);   // when a pending post targets addr

@@ -97,6 +97,14 @@ class Loop:
         """Elements of a reduction variable (1 for a scalar)."""
         return int(self.red_lengths.get(red[1], 1))
 
+    def finish_in_kernel(self):
+        """The loop's reductions can be folded by its own (single) launch:
+        scalars of plain types, loc records that are plain integers."""
+        plain = {'char', 'signed char', 'unsigned char', 'int', 'unsigned', 'unsigned int', 'long', 'unsigned long', 'long long',
+                 'unsigned long long', 'float', 'double'}
+        return bool(self.reds) and all(
+            self.rlen(red) == 1 and red[2] in plain and (len(red) <= 3 or red[4] in plain - {'float', 'double'}) for red in self.reds)
+
     def _is_stencil(self, name):
         """True when the body only reads `name` and every access is
         name[v0 +- 0/1][v1 +- 0/1]... with the loop variables in order."""
@@ -445,6 +453,95 @@ def red_kernel_params(L):
     return fp
 
 
+def red_finish_params(L):
+    """Kernel parameters of the in-kernel finish (after red_kernel_params)."""
+    if not L.finish_in_kernel():
+        return []
+    fp = ['DvmhAmdRedFinish dvmh_fin']
+    for red in L.reds:
+        fp.append(f'{red[2]} *{red[1]}_out')
+        if len(red) > 3:
+            fp.append(f'{red[4]} *{red[3]}_out')
+    return fp
+
+
+def red_finish_args(L):
+    if not L.finish_in_kernel():
+        return []
+    a = ['dvmh_fin']
+    for red in L.reds:
+        a.append(f'{red[1]}_out')
+        if len(red) > 3:
+            a.append(f'{red[3]}_out')
+    return a
+
+
+def red_finish_query(L, count_expr):
+    """Handler lines after handler_reds_prepare: where the launch leaves its results."""
+    if not L.finish_in_kernel():
+        return []
+    h = ['DvmhAmdRedFinish dvmh_fin;', f'dvmh_amd_loop_red_in_kernel_C(loop_ref, {count_expr}, &dvmh_fin);']
+    for i, red in enumerate(L.reds):
+        h.append(f'{red[2]} *{red[1]}_out;')
+        loc = '0'
+        if len(red) > 3:
+            h.append(f'{red[4]} *{red[3]}_out;')
+            loc = f'(void **)&{red[3]}_out'
+        h.append(f'dvmh_amd_loop_red_result_C(loop_ref, {i + 1}, (void **)&{red[1]}_out, {loc});')
+    return h
+
+
+def red_kernel_finish(L, slot):
+    """Workgroup reduction, then the fold of every workgroup's partials by the
+    last to arrive; loops that can't (finish_in_kernel) store their partials."""
+    if not L.finish_in_kernel():
+        return red_kernel_tail(L, slot, accumulate=False)
+    s = []
+
+    def each(value, record):
+        for red in L.reds:
+            s.extend(IND + ln for ln in (record if len(red) > 3 else value)(red))
+
+    for red in L.reds:
+        f, v, ct = red[0], red[1], red[2]
+        if len(red) > 3:
+            s.append(f'dvmh_dev::blockReduceLoc<{ct}, {red[4]}, {"true" if f == "maxloc" else "false"}>({v}, {red[3]});')
+        else:
+            s.append(f'{v} = dvmh_dev::blockReduce({v}, dvmh_dev::{RED_OP[f]}());')
+    store = lambda at: each(  # noqa: E731
+        lambda r: [f'if (dvmh_dev::linearTid() == 0) dvmh_dev::agentStore(&{r[1]}_grid[{at}], {r[1]});'],
+        lambda r: [f'if (dvmh_dev::linearTid() == 0) {{ dvmh_dev::agentStore(&{r[1]}_grid[{at}], {r[1]}); '
+                   f'dvmh_dev::agentStore(&{r[3]}_grid[{at}], {r[3]}); }}'])
+    fold = lambda at, n: each(  # noqa: E731
+        lambda r: [f'{r[1]} = dvmh_dev::foldSlots({r[1]}_grid + {at}, {n}, dvmh_dev::{RED_OP[r[0]]}());'],
+        lambda r: [f'dvmh_dev::foldSlotsLoc<{r[2]}, {r[4]}, {"true" if r[0] == "maxloc" else "false"}>({r[1]}_grid + {at}, '
+                   f'{r[3]}_grid + {at}, {n}, {r[1]}, {r[3]});'])
+    s.append('if (dvmh_dev::linearTid() < 64) {')
+    s.append(IND + f'const unsigned dvmh_slot = (unsigned)({slot}), dvmh_g = dvmh_slot / dvmh_fin.groupSize;')
+    s.append(IND + 'const unsigned dvmh_first = dvmh_g * dvmh_fin.groupSize;')
+    s.append(IND + 'const unsigned dvmh_left = dvmh_fin.items - dvmh_first;')
+    s.append(IND + 'const unsigned dvmh_n = dvmh_left < dvmh_fin.groupSize ? dvmh_left : dvmh_fin.groupSize;')
+    store('dvmh_slot')
+    s.append(IND + 'if (!dvmh_dev::lastArrival(dvmh_fin.counters + DVMH_AMD_RED_STRIDE * (1 + dvmh_g), dvmh_n)) return;')
+    fold('dvmh_first', '(int)dvmh_n')
+    s.append(IND + 'if (dvmh_fin.groups > 1) {')
+    at = len(s)
+    store('dvmh_fin.items + dvmh_g')
+    s.append(IND + 'if (!dvmh_dev::lastArrival(dvmh_fin.counters, dvmh_fin.groups)) return;')
+    fold('dvmh_fin.items', '(int)dvmh_fin.groups')
+    s[at:] = [IND + ln for ln in s[at:]]
+    s.append(IND + '}')
+    s.append(IND + 'if (dvmh_dev::linearTid() == 0) {')
+    at = len(s)
+    each(lambda r: [f'dvmh_dev::hostStore({r[1]}_out, {r[1]});'],
+         lambda r: [f'dvmh_dev::hostStore({r[1]}_out, {r[1]});', f'dvmh_dev::hostStore({r[3]}_out, {r[3]});'])
+    s.append(IND + 'dvmh_dev::publishDone(dvmh_fin);')
+    s[at:] = [IND + ln for ln in s[at:]]
+    s.append(IND + '}')
+    s.append('}')
+    return s
+
+
 def red_kernel_locals(L):
     s = []
     for red in L.reds:
@@ -616,7 +713,7 @@ def parallel_kernel(L):
     for i in range(r):
         fp += [f'IndexT lo{i}', f'IndexT cnt{i}', f'IndexT st{i}']
     fp += ['IndexT nbx', 'IndexT nby', 'IndexT nbz', 'long nblocks', 'int xcd']
-    fp += red_kernel_params(L)
+    fp += red_kernel_params(L) + red_finish_params(L)
     k = []
     k.append(f'template <typename IndexT, int DEPTH>')
     k.append(f'__global__ __launch_bounds__(1024) void {L.name}_kernel({", ".join(fp)}) {{')
@@ -687,7 +784,7 @@ def parallel_kernel(L):
         b.append('}')
     else:
         b += inner
-    b += red_kernel_tail(L, 'blockIdx.x', accumulate=False)
+    b += red_kernel_finish(L, 'blockIdx.x')
     k.append(indent('\n'.join(b) + '\n', 1).rstrip('\n'))
     k.append('}')
     return '\n'.join(k) + '\n'
@@ -891,7 +988,7 @@ def march_kernel(L, tail=None):
         return '\n'.join(k) + '\n'
     # the per-loop kernel: one tile per workgroup
     names = [p_[1] for p_ in L.params]
-    kp = list(fp[:-4]) + ['IndexT nbx', 'IndexT nby', 'IndexT nbz', 'long nblocks', 'int xcd', 'IndexT march', 'IndexT xshift'] + red_kernel_params(L)
+    kp = list(fp[:-4]) + ['IndexT nbx', 'IndexT nby', 'IndexT nbz', 'long nblocks', 'int xcd', 'IndexT march', 'IndexT xshift'] + red_kernel_params(L) + red_finish_params(L)
     call = []
     for p_ in L.arrays:
         _, nm, ct, ar = p_
@@ -909,7 +1006,7 @@ def march_kernel(L, tail=None):
          f'__global__ __launch_bounds__(1024) void {L.name}_march_kernel({", ".join(kp)}) {{']
     gb = red_kernel_locals(L)
     gb.append(f'{L.name}_march_tile<IndexT, COLS, NPF>({", ".join(call)});')
-    gb += red_kernel_tail(L, 'blockIdx.x', accumulate=False)
+    gb += red_kernel_finish(L, 'blockIdx.x')
     g.append(indent('\n'.join(gb) + '\n', 1).rstrip('\n'))
     g.append('}')
     return '\n'.join(k) + '\n\n' + '\n'.join(g) + '\n'
@@ -987,7 +1084,7 @@ def parallel_handler(L):
         b.append('}')
     nb = 'nbx * nby * nbz' + ''.join(f' * cnt{a}' for a in range(0, r - 3))
     b.append(f'DvmType nblocks = {nb};')
-    b += handler_reds_prepare(L, 'nblocks', 0)
+    b += handler_reds_prepare(L, 'nblocks', 0) + red_finish_query(L, 'nblocks')
     kernels = []
     for it in ['int', 'long long']:
         for dp in [1, 2, 4, 8]:
@@ -1002,7 +1099,7 @@ def parallel_handler(L):
         for i in range(r):
             args += [f'({it})boundsLow[{i}]', f'({it})cnt{i}', f'({it})loopSteps[{i}]']
         args += [f'({it})nbx', f'({it})nby', f'({it})nbz', 'nblocks', '(int)tune[DVMH_AMD_T_XCD]', f'({it})march', f'({it})xshift']
-        args += red_fact_args(L)
+        args += red_fact_args(L) + red_finish_args(L)
         for cols, sets in MARCH_NPF.items():
             for v in sets:
                 b.append(IND * 2 + f'if (mcols == {cols} && npf == {v}) hipLaunchKernelGGL(({L.name}_march_kernel<{it}, {cols}, {v}>), '
@@ -1016,7 +1113,7 @@ def parallel_handler(L):
         for i in range(r):
             args += [f'({it})boundsLow[{i}]', f'({it})cnt{i}', f'({it})loopSteps[{i}]']
         args += [f'({it})nbx', f'({it})nby', f'({it})nbz', 'nblocks', '(int)tune[DVMH_AMD_T_XCD]']
-        args += red_fact_args(L)
+        args += red_fact_args(L) + red_finish_args(L)
         ks = [(c, k) for c, k in kernels if (('rt_INT' in c) == (it == 'int'))]
         b += [ind2 + s for s in launch_dispatch(ks, args, 'dim3((unsigned)nblocks)')]
     if L.stencil:
@@ -2015,7 +2112,7 @@ def line_kernel(L, dep):
     for i in range(r):
         fp += [f'IndexT lo{i}', f'IndexT cnt{i}', f'IndexT st{i}']
     fp += ['IndexT nbx', 'IndexT nby', 'long nblocks', 'int xcd', 'int chunk']
-    fp += red_kernel_params(L)
+    fp += red_kernel_params(L) + red_finish_params(L)
     k = [f'template <typename IndexT>',
          f'__global__ __launch_bounds__(1024) void {L.name}_line{dep}_kernel({", ".join(fp)}) {{']
     b = list(setup)
@@ -2049,7 +2146,7 @@ def line_kernel(L, dep):
     inner.append('}')
     b += [IND + ln for ln in '\n'.join(inner).split('\n')]
     b.append('}')
-    b += red_kernel_tail(L, 'blockIdx.x', accumulate=False)
+    b += red_kernel_finish(L, 'blockIdx.x')
     k.append(indent('\n'.join(b) + '\n', 1).rstrip('\n'))
     k.append('}')
     return '\n'.join(k) + '\n'
@@ -2077,7 +2174,7 @@ def line_reg_kernel(L, dep):
     for i in range(r):
         fp += [f'IndexT lo{i}', f'IndexT cnt{i}', f'IndexT st{i}']
     fp += ['IndexT nbx', 'IndexT nby', 'long nblocks', 'int xcd']
-    fp += red_kernel_params(L)
+    fp += red_kernel_params(L) + red_finish_params(L)
     k = ['template <typename IndexT, int CK, int DIR>',
          f'__global__ __launch_bounds__(256) void {L.name}_lreg{dep}_kernel({", ".join(fp)}) {{']
     b = list(setup)
@@ -2132,7 +2229,7 @@ def line_reg_kernel(L, dep):
     inner.append('}')
     b += [IND + ln for ln in '\n'.join(inner).split('\n')]
     b.append('}')
-    b += red_kernel_tail(L, 'blockIdx.x', accumulate=False)
+    b += red_kernel_finish(L, 'blockIdx.x')
     k.append(indent('\n'.join(b) + '\n', 1).rstrip('\n'))
     k.append('}')
     return '\n'.join(k) + '\n'
@@ -2146,14 +2243,14 @@ def line_reg_launch(L, dep):
     b = [f'DvmType nbx = (cnt{ax_x} + threads.x - 1) / threads.x;',
          f'DvmType nby = {"(cnt%d + threads.y - 1) / threads.y" % ax_y if ax_y is not None else "1"};',
          'DvmType nblocks = nbx * nby;']
-    b += handler_reds_prepare(L, 'nblocks', 0)
+    b += handler_reds_prepare(L, 'nblocks', 0) + red_finish_query(L, 'nblocks')
     b.append('if (nblocks > 0) {')
     b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 0);')
     args = array_fact_args(L, 'int')
     for i in range(r):
         args += [f'(int)boundsLow[{i}]', f'(int)cnt{i}', f'(int)loopSteps[{i}]']
     args += ['(int)nbx', '(int)nby', 'nblocks', '(int)tune[DVMH_AMD_T_XCD]']
-    args += red_fact_args(L)
+    args += red_fact_args(L) + red_finish_args(L)
     for ck in LINE_REG_CK:
         for d in (1, -1):
             b.append(IND + f'if (CK == {ck} && loopSteps[{dep}] == {d}) hipLaunchKernelGGL(({L.name}_lreg{dep}_kernel<int, {ck}, {d}>), '
@@ -2174,7 +2271,7 @@ def line_launch(L, dep):
     b.append(f'DvmType nby = {"(cnt%d + threads.y - 1) / threads.y" % ax_y if ax_y is not None else "1"};')
     nb = 'nbx * nby' + ''.join(f' * cnt{a}' for a in ind[:-2])
     b.append(f'DvmType nblocks = {nb};')
-    b += handler_reds_prepare(L, 'nblocks', 0)
+    b += handler_reds_prepare(L, 'nblocks', 0) + red_finish_query(L, 'nblocks')
     b.append('if (nblocks > 0) {')
     b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 0);')
     for it in ['int', 'long long']:
@@ -2182,7 +2279,7 @@ def line_launch(L, dep):
         for i in range(r):
             args += [f'({it})boundsLow[{i}]', f'({it})cnt{i}', f'({it})loopSteps[{i}]']
         args += [f'({it})nbx', f'({it})nby', 'nblocks', '(int)tune[DVMH_AMD_T_XCD]', '(int)tune[DVMH_AMD_T_CHUNK]']
-        args += red_fact_args(L)
+        args += red_fact_args(L) + red_finish_args(L)
         cond = f'kernelIndexT == {"rt_INT" if it == "int" else "rt_LLONG"}'
         b += [IND + s for s in launch_dispatch([(cond, f'{L.name}_line{dep}_kernel<{it}>')], args, 'dim3((unsigned)nblocks)')]
     b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 1);')
@@ -2542,7 +2639,7 @@ def line_tile_kernel(L):
     for i in range(r):
         fp += [f'IndexT lo{i}', f'IndexT cnt{i}', f'IndexT st{i}']
     fp += ['IndexT dl_nlines']
-    fp += red_kernel_params(L)
+    fp += red_kernel_params(L) + red_finish_params(L)
     kx = r - 1
     # at most 256 threads (the handler checks): lines are few, so registers
     # for deep prefetch matter more than occupancy
@@ -2650,7 +2747,7 @@ def line_tile_kernel(L):
           IND + '}',
           IND + '__syncthreads();',
           '}']
-    b += red_kernel_tail(L, 'blockIdx.x', accumulate=False)
+    b += red_kernel_finish(L, 'blockIdx.x')
     k.append(indent('\n'.join(b) + '\n', 1).rstrip('\n'))
     k.append('}')
     return '\n'.join(k) + '\n'
@@ -2660,7 +2757,7 @@ def line_tile_launch(L):
     r = L.rank
     b = ['DvmType nlines = 1' + ''.join(f' * cnt{a}' for a in range(r - 1)) + ';',
          'DvmType nblocks = (nlines + threads.x - 1) / threads.x;']
-    b += handler_reds_prepare(L, 'nblocks', 0)
+    b += handler_reds_prepare(L, 'nblocks', 0) + red_finish_query(L, 'nblocks')
     b.append('if (nblocks > 0) {')
     b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 0);')
     for it in ['int', 'long long']:
@@ -2668,7 +2765,7 @@ def line_tile_launch(L):
         for i in range(r):
             args += [f'({it})boundsLow[{i}]', f'({it})cnt{i}', f'({it})loopSteps[{i}]']
         args += [f'({it})nlines']
-        args += red_fact_args(L)
+        args += red_fact_args(L) + red_finish_args(L)
         for ck in LINE_TILE_CK:
             for d in (1, -1):
                 for reg in ((0, 1) if it == 'int' else (0,)):
@@ -2708,7 +2805,7 @@ def line_vec_kernel(L):
     for i in range(r):
         fp += [f'IndexT lo{i}', f'IndexT cnt{i}', f'IndexT st{i}']
     fp += ['IndexT nlines']
-    fp += red_kernel_params(L)
+    fp += red_kernel_params(L) + red_finish_params(L)
     k = ['template <typename IndexT, int DIR>',
          '// a thread per line leaves one or two waves per SIMD: registers go to chunks in flight',
          f'__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void {L.name}_lvec_kernel({", ".join(fp)}) {{']
@@ -2934,7 +3031,7 @@ def line_vec_kernel(L):
     inner += [IND * 2 + ln for ln in partial('lv_c')]
     b += [IND + ln for ln in '\n'.join(inner).split('\n')]
     b.append('}')
-    b += red_kernel_tail(L, 'blockIdx.x', accumulate=False)
+    b += red_kernel_finish(L, 'blockIdx.x')
     k.append(indent('\n'.join(b) + '\n', 1).rstrip('\n'))
     k.append('}')
     return '\n'.join(k) + '\n'
@@ -2944,14 +3041,14 @@ def line_vec_launch(L):
     r = L.rank
     b = ['DvmType nlines = 1' + ''.join(f' * cnt{a}' for a in range(r - 1)) + ';',
          'DvmType nblocks = (nlines + threads.x - 1) / threads.x;']
-    b += handler_reds_prepare(L, 'nblocks', 0)
+    b += handler_reds_prepare(L, 'nblocks', 0) + red_finish_query(L, 'nblocks')
     b.append('if (nblocks > 0) {')
     b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 0);')
     args = array_fact_args(L, 'int')
     for i in range(r):
         args += [f'(int)boundsLow[{i}]', f'(int)cnt{i}', f'(int)loopSteps[{i}]']
     args += ['(int)nlines']
-    args += red_fact_args(L)
+    args += red_fact_args(L) + red_finish_args(L)
     for d in (1, -1):
         b.append(IND + f'if (loopSteps[{r - 1}] == {d}) hipLaunchKernelGGL(({L.name}_lvec_kernel<int, {d}>), '
                  f'dim3((unsigned)nblocks), threads, 0, stream, {", ".join(args)});')

@@ -49,6 +49,25 @@ extern "C" {
                                   PAIR: 1 = the pair handler picks its march shape from the pairs' sizes */
 void dvmh_amd_loop_get_tuning_C(DvmType curLoop, DvmType kind, DvmType tune[]);
 
+/* ---- in-kernel reduction finish --------------------------------------------------
+ * A handler whose loop is one launch may let the launch fold its scalar
+ * reductions itself (see dvmh_hip_device.h): after dvmh_loop_cuda_red_prepare_C
+ * of each reduction it asks for the launch's finish record, passes it and each
+ * reduction's result addresses (mapped host memory) to the kernel, and still
+ * calls dvmh_loop_cuda_red_finish_C, which then launches nothing.  `items`
+ * partials are folded in `groups` groups of groupSize consecutive ones (the
+ * last may be smaller); slots [items, items + groups) hold the groups' results. */
+typedef struct {
+    unsigned *counters;          /* word 0: groups arrived; word DVMH_AMD_RED_STRIDE * (1 + g): arrivals of group g */
+    unsigned long long *done;    /* 0, or the word to set to doneSeq once the results are written */
+    unsigned long long doneSeq;
+    unsigned items, groupSize, groups;
+} DvmhAmdRedFinish;
+#define DVMH_AMD_RED_STRIDE 16   /* counters lie 64 bytes apart */
+#define DVMH_AMD_RED_GROUPS 1024 /* groups at most */
+void dvmh_amd_loop_red_in_kernel_C(DvmType curLoop, DvmType items, DvmhAmdRedFinish *out);
+void dvmh_amd_loop_red_result_C(DvmType curLoop, DvmType redIndex, void **outVal, void **outLoc);
+
 /* ---- kernel timing -----------------------------------------------------------
  * Emitted handlers bracket their main kernel launches with phase 0 / phase 1
  * marks.  With timing enabled the runtime records HIP events on the loop's
