@@ -1317,6 +1317,11 @@ extern "C" void dvmh_loop_cuda_red_finish_C(DvmType curLoop, DvmType redIndex) {
     gpuRedFinish(sl, r);
 }
 
+extern "C" DvmType dvmh_amd_flow_workspace_C(DvmType tiles, DvmType cellWords, DvmhAmdFlow *out) {
+    DVMH_CHECK(tiles > 0 && cellWords >= 0 && out, "dvmh_amd_flow_workspace_C: %ld tiles, %ld words", tiles, cellWords);
+    return gpu.flowWorkspace(tiles, cellWords, out) ? 1 : 0;
+}
+
 extern "C" void dvmh_amd_loop_red_in_kernel_C(DvmType curLoop, DvmType items, DvmhAmdRedFinish *out) {
     gpuRedInKernel(asSpec(curLoop, "dvmh_amd_loop_red_in_kernel_C"), items, out);
 }

@@ -58,6 +58,7 @@ void Settings::load() {
     syncMode = (int)envLong("DVMH_AMD_SYNC", 0);
     allowAsync = envLong("DVMH_ALLOW_ASYNC", 0) != 0;   // rts/dvmh/settings.cpp:361
     pollDone = envLong("DVMH_AMD_POLL", 1) != 0;
+    flowTag = envLong("DVMH_AMD_FLOW_TAG", 0);
     graph = envLong("DVMH_AMD_GRAPH", 0) != 0;
     graphMinNodes = envLong("DVMH_AMD_GRAPH_MIN_NODES", 6);
     tuneRepeats = (int)envLong("DVMH_AMD_TUNE_REPEATS", 1);
@@ -173,6 +174,74 @@ void Gpu::trimCache() {
     for (auto &kv : freeBlocks)
         for (void *p : kv.second) HIP_CHECK(hipFree(p));
     freeBlocks.clear();
+    if (!graphsExist() && !graphCapturing()) flowRetire(true);
+}
+
+// Zeroes a dataflow workspace outside the runtime's stream (which may be
+// capturing); the caller sees to it that no launch uses it.
+void Gpu::flowZero(const FlowSpace &w) {
+    static hipStream_t side = nullptr;
+    if (!side) HIP_CHECK(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
+    const long zero = 0;
+    dvmh_hip_fill(w.p, &zero, sizeof(zero), (long)(w.bytes / sizeof(zero)), side);
+    // DVMH_AMD_FLOW_TAG: the last tag already used when the process starts
+    if (!flowStarted && settings.flowTag) {
+        const long control = (long)((unsigned long)settings.flowTag << 32);
+        dvmh_hip_fill(w.p, &control, sizeof(control), 1, side);
+    }
+    flowStarted = true;
+    HIP_CHECK(hipStreamSynchronize(side));
+}
+
+bool Gpu::flowWorkspace(long tiles, long cellWords, DvmhAmdFlow *out) {
+    const size_t head = 256, flags = ((size_t)tiles * 8 + 255) & ~(size_t)255, need = head + flags + (size_t)cellWords * 8;
+    if (!flowWrapped) {
+        void *h = nullptr;
+        HIP_CHECK(hipHostMalloc(&h, 64, hipHostMallocMapped));
+        flowWrapped = (volatile unsigned *)h;
+        *flowWrapped = 0;
+        HIP_CHECK(hipHostGetDevicePointer((void **)&flowWrappedDev, h, 0));
+    }
+    if (flowSpaces.empty() || flowSpaces.back().bytes < need) {
+        // earlier launches (and graphs) may still use the smaller one: it stays
+        // until no graph does
+        void *p = nullptr;
+        if (hipMalloc(&p, need) != hipSuccess) {
+            (void)hipGetLastError();
+            if (graphCapturing()) return false;
+            trimCache();
+            if (hipMalloc(&p, need) != hipSuccess) {
+                (void)hipGetLastError();
+                return false;
+            }
+        }
+        flowSpaces.push_back(FlowSpace{(char *)p, need});
+        flowZero(flowSpaces.back());
+        if (!graphCapturing() && !graphsExist()) flowRetire(false);
+    }
+    if (!graphCapturing()) flowCheckWrap();
+    char *p = flowSpaces.back().p;
+    out->control = (unsigned long long *)p;
+    out->flags = (unsigned long long *)(p + head);
+    out->cells = (unsigned long long *)(p + head + flags);
+    out->wrapped = flowWrappedDev;
+    return true;
+}
+
+void Gpu::flowCheckWrap() {
+    if (!flowWrapped || !*flowWrapped) return;
+    HIP_CHECK(hipStreamSynchronize(stream));
+    for (auto &w : flowSpaces) flowZero(w);
+    *flowWrapped = 0;
+}
+
+void Gpu::flowRetire(bool all) {
+    HIP_CHECK(hipStreamSynchronize(stream));
+    const size_t keep = all || flowSpaces.empty() ? 0 : 1;
+    while (flowSpaces.size() > keep) {
+        HIP_CHECK(hipFree(flowSpaces.front().p));
+        flowSpaces.erase(flowSpaces.begin());
+    }
 }
 
 void *Gpu::pinnedStaging(size_t bytes) {

@@ -145,6 +145,7 @@ void graphRunRegion(Region *region) {
     std::string key = rt.curFile + "#" + signature(region);
     GraphEntry &g = graphs[key];
     if (g.exec && !g.noCapture) {
+        gpu.flowCheckWrap();
         HIP_CHECK(hipGraphLaunch(g.exec, gpu.stream));
         graphReplays++;
         rt.loopsOnGpu += (long)region->deferred.size();
@@ -358,6 +359,7 @@ bool batchGraphRun(const std::vector<Loop *> &loops, bool eligible, const std::f
     BatchGraph &bg = *found;
     GraphEntry &g = bg.g;
     if (g.exec) {
+        gpu.flowCheckWrap();
         HIP_CHECK(hipGraphLaunch(g.exec, gpu.stream));
         graphReplays++;
         rt.loopsOnGpu += (long)loops.size();
@@ -412,6 +414,14 @@ bool batchGraphRun(const std::vector<Loop *> &loops, bool eligible, const std::f
     return false;
 }
 
+bool graphsExist() {
+    for (auto &kv : graphs)
+        if (kv.second.exec) return true;
+    for (auto &kv : batchGraphs)
+        if (kv.second.g.exec) return true;
+    return false;
+}
+
 void graphReleaseAll() {
     gpu.sync();
     for (auto &kv : graphs) destroyEntry(kv.second);
@@ -419,6 +429,7 @@ void graphReleaseAll() {
     for (auto &kv : batchGraphs) destroyEntry(kv.second.g);
     batchGraphs.clear();
     lastBatchGraph = nullptr;
+    gpu.flowRetire(false);
 }
 
 }  // namespace dvmh

@@ -60,6 +60,7 @@ struct Settings {
     bool tuneTransforms = true;    // DVMH_AMD_TUNE_TRANSFORMS (default 1): candidates may re-lay out arrays of ACROSS loops
     bool fuse = true;              // DVMH_AMD_FUSE (default 1): registered loop pairs held back together run fused
     bool index64 = false;          // DVMH_AMD_INDEX64: every loop's kernels take 64-bit index arithmetic
+    long flowTag = 0;              // DVMH_AMD_FLOW_TAG: launch tag dataflow workspaces start from
     std::string tuneDb;         // DVMH_AMD_TUNEDB: file of recorded timings
     std::string modelFile;      // DVMH_AMD_MODEL: trained cost-model weights
     void load();
@@ -88,6 +89,11 @@ public:
     unsigned long long *doneDev = nullptr;
     unsigned long long doneSeq = 0;
     long h2dBytes = 0, d2hBytes = 0;   // array and variable bytes moved by h2d / d2h
+    // workspace of dataflow launches (one at a time on the stream): the current
+    // one and, while graphs that use them exist, smaller earlier ones
+    bool flowWorkspace(long tiles, long cellWords, DvmhAmdFlow *out);
+    void flowCheckWrap();                    // starts the tags over when a launch has said they run out
+    void flowRetire(bool all);               // frees the earlier ones (all: the current one too)
     void waitDone(unsigned long long seq);   // until the word reaches seq (or the stream drains)
     void init();
     void *alloc(size_t bytes);          // size-keyed cache in front of hipMalloc
@@ -102,6 +108,12 @@ private:
     std::map<void *, size_t> liveBlocks;
     void *staging = nullptr;
     size_t stagingBytes = 0;
+    struct FlowSpace { char *p; size_t bytes; };
+    std::vector<FlowSpace> flowSpaces;       // the last is the current one
+    volatile unsigned *flowWrapped = nullptr;
+    unsigned *flowWrappedDev = nullptr;
+    bool flowStarted = false;
+    void flowZero(const FlowSpace &w);
 };
 extern Gpu gpu;
 
@@ -378,6 +390,7 @@ long layoutChanges();
 
 // lazy regions and graphs (graph.cpp)
 bool regionIsLazy(const Region *r);
+bool graphsExist();                 // some captured graph may be replayed
 bool graphCapturing();
 void graphNoteAlloc(void *p);
 char *graphPinnedSlot(size_t bytes);

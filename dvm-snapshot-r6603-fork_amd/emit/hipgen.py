@@ -172,6 +172,53 @@ class Loop:
                 return False
         return True
 
+    def flow_eligible(self):
+        """Rank 2 or 3, every loop axis in the ACROSS clause with widths <= 1;
+        the body reads the ACROSS array at X[i + d0][j + d1].. with at most one
+        offset, |offset| <= 1, writes it at the loop point only, and writes
+        nothing else but its own variables and reductions: the sweep can then
+        run as one dataflow launch (other arrays and scalars are not passed
+        between the workgroups)."""
+        if not self.across or self.rank not in (2, 3):
+            return False
+        w = self.across['widths']
+        if len(w) != self.rank or any(lo > 1 or hi > 1 or (lo == 0 and hi == 0) for lo, hi in w):
+            return False
+        X = self.across['array']
+        arr = [p for p in self.arrays if p[1] == X]
+        if not arr or arr[0][3] != self.rank or arr[0][2] not in ('float', 'double', 'int', 'long'):
+            return False
+        if re.search(r'\b' + X + r'\b(?!\s*\[)', self.body) or re.search(r'(\+\+|--|&)\s*' + X + r'\b', self.body):
+            return False
+        written = False
+        assign = r'(?:=(?!=)|\+=|-=|\*=|/=|%=|&=|\|=|\^=|<<=|>>=|\+\+|--)'
+        for m in re.finditer(r'\b' + X + r'\s*((?:\[[^\[\]]*\]\s*)+)(' + assign + ')?', self.body):
+            idx = re.findall(r'\[([^\[\]]*)\]', m.group(1))
+            if len(idx) != self.rank:
+                return False
+            moved = 0
+            for (v, _), e in zip(self.vars, idx):
+                mm = re.fullmatch(r'\s*' + v + r'\s*(?:([+-])\s*([01])\s*)?', e)
+                if not mm:
+                    return False
+                moved += mm.group(2) == '1'
+            if moved > (0 if m.group(2) else 1):
+                return False
+            written = written or bool(m.group(2))
+        if not written:
+            return False
+        for p in self.params:
+            if p[1] == X:
+                continue
+            if p[0] not in ('array', 'scalar') or re.search(r'(\+\+|--|&)\s*' + p[1] + r'\b', self.body):
+                return False
+            if re.search(r'(?<![\w.>])' + p[1] + r'\s*(?:\[[^\]]*\]\s*)*' + assign, self.body):
+                return False
+            # an array whose name appears other than subscripted may be passed on and written
+            if p[0] == 'array' and re.search(r'\b' + p[1] + r'\b(?!\s*\[)', self.body):
+                return False
+        return all(self.rlen(red) == 1 for red in self.reds)
+
     def chain_eligible(self):
         """Consecutive executions (sweeps) of the loop may run pipelined by a
         chain handler: a tiled-wavefront ACROSS loop marked for batching that
@@ -2600,6 +2647,108 @@ def tile_kernel(L):
     return out
 
 
+def flow_kernel(L):
+    """The whole sweep of an ACROSS loop whose axes all depend as one launch
+    (dvmh_hip_device.h, dataflow wavefront), and for loops with a chain handler
+    several consecutive sweeps of it."""
+    X = L.across['array']
+    r = L.rank
+    xct = [p for p in L.arrays if p[1] == X][0][2]
+    fp, setup = [f'dvmh_dev::FlowArgs<{xct}, int, {r}> dvmh_f'], []
+    for p in L.arrays:
+        _, nm, ct, ar = p
+        if nm == X:
+            continue
+        fp.append(f'{ct} *__restrict__ {nm}_base')
+        fp += [f'int {nm}_s{k}' for k in range(ar)]
+        strides = ', '.join(f'{nm}_s{k}' for k in range(ar))
+        setup.append(f'const int {nm}_str[{ar}] = {{{strides}}};')
+        setup.append(f'const auto {nm} = dvmh_dev::makeView<{ct}, int, {ar}, false>({nm}_base, {nm}_str);')
+    for p in L.scalars:
+        fp.append(f'{p[2]} *__restrict__ {p[1]}_ptr')
+        setup.append(scalar_bind(L.body, p))
+    body = []
+    for v, ct in L.vars:
+        body.append(f'{ct} {v};')
+    for pr in L.privates:
+        body.append(pr + ';')
+    for i in range(r):
+        body.append(var_assign(L, i, f'dvmh_t{i}', f'dvmh_f.lo[{i}]', '1'))
+    at = ', '.join(f'(int){v}' for v, _ in L.vars)
+    body.append(f'const dvmh_dev::StarView<{xct}, int, {r}> {X}{{dvmh_v, {{{at}}}, 0}};')
+    body.append('{\n' + indent(L.body + '\n', 1) + '}')
+
+    def kernel(name, chain, params, init, tail):
+        k = [f'__global__ __launch_bounds__(64) void {name}({", ".join(params)}) {{']
+        b = [f'__shared__ {xct} dvmh_ring[dvmh_dev::FlowShape<{r}>::LDS];'] + setup
+        b.append('const dvmh_dev::FlowTask dvmh_task = dvmh_dev::flowTake(dvmh_f.ntA, dvmh_f.ntB, dvmh_f.sweeps, dvmh_f.ws);')
+        b += init
+        b.append(f'dvmh_dev::flowTile<{xct}, int, {r}, {"true" if chain else "false"}>(dvmh_f, dvmh_task, dvmh_ring, '
+                 f'[&]({xct} *dvmh_v, int dvmh_t0, int dvmh_t1, int dvmh_t2) {{')
+        b += [IND + '(void)dvmh_t2;'] + [IND + ln for ln in '\n'.join(body).split('\n')]
+        b.append('});')
+        b += tail
+        k.append(indent('\n'.join(b) + '\n', 1).rstrip('\n'))
+        k.append('}')
+        return '\n'.join(k) + '\n'
+
+    tile = '(long)dvmh_task.ta * dvmh_f.ntB + dvmh_task.tb'
+    out = kernel(f'{L.name}_flow_kernel', False, fp + red_kernel_params(L) + red_finish_params(L), red_kernel_locals(L),
+                 red_kernel_finish(L, tile))
+    return out
+
+
+def flow_args(L):
+    """Handler lines that set up dvmh_f, and the kernel arguments before the reductions."""
+    X = L.across['array']
+    r = L.rank
+    xct = [p for p in L.arrays if p[1] == X][0][2]
+    rng = L.stencil_range(X)
+    b = [f'dvmh_dev::FlowArgs<{xct}, int, {r}> dvmh_f;', f'dvmh_f.base = {X};']
+    for a in range(r):
+        b.append(f'dvmh_f.s[{a}] = (int){X}_devHdr[{a + 1}]; dvmh_f.lo[{a}] = (int)boundsLow[{a}]; dvmh_f.cnt[{a}] = (int)cnt{a};')
+        b.append(f'dvmh_f.rlo[{a}] = (int)boundsLow[{a}] + ({rng[a][0]}); dvmh_f.rhi[{a}] = (int)(boundsLow[{a}] + cnt{a} - 1) + ({rng[a][1]});')
+    sh = f'dvmh_dev::FlowShape<{r}>'
+    b.append(f'dvmh_f.ntA = (int)((cnt0 + {sh}::PA - 1) / {sh}::PA);')
+    b.append(f'dvmh_f.ntB = {f"(int)((cnt1 + {sh}::PB - 1) / {sh}::PB)" if r == 3 else "1"};')
+    b.append('DvmType tiles = (DvmType)dvmh_f.ntA * dvmh_f.ntB;')
+    rows = f'({sh}::PA + {sh}::PB)' if r == 3 else f'{sh}::PB'
+    words = f'tiles * {rows} * cnt{r - 1} * dvmh_dev::FlowCell<{xct}>::WORDS'
+    args = ['dvmh_f']
+    for p in L.arrays:
+        if p[1] != X:
+            args += [p[1]] + [f'(int){p[1]}_devHdr[{k + 1}]' for k in range(p[3])]
+    args += [p[1] for p in L.scalars]
+    return b, args, words
+
+
+def flow_launch(L, otherwise):
+    """The dataflow launch where it applies -- unit forward steps, natural
+    layouts, 32-bit indices, room for its workspace -- else `otherwise`.  No
+    size is left to the other kernels: they pay a launch (4-14 us) per
+    hyperplane or tile-plane, this one about 5 us per tile of a diagonal and
+    0.12-0.16 us per step.  One sweep: 2-D 998^2 0.38 against 9.2 ms, 64^2 11
+    against 500 us; 3-D 128^3 0.154 against 0.43 ms, 318^3 0.76 against 1.84."""
+    r = L.rank
+    cond = ['tune[DVMH_AMD_T_VARIANT] == 0', 'kernelIndexT == rt_INT'] + [f'loopSteps[{i}] == 1' for i in range(r)]
+    cond += [f'{p[1]}_tfm == 0' for p in L.arrays] + [f'{L.across["array"]}_devHdr[{r}] == 1']
+    setup, args, words = flow_args(L)
+    b = ['bool flow = ' + ' && '.join(cond) + ';'] + setup
+    b.append(f'if (flow) flow = dvmh_amd_flow_workspace_C(tiles, {words}, &dvmh_f.ws) != 0;')
+    b.append('if (flow) {')
+    b.append(IND + 'dvmh_f.sweeps = 1;')
+    b += [IND + ln for ln in handler_reds_prepare(L, 'tiles', 0) + red_finish_query(L, 'tiles')]
+    b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 0);')
+    b.append(IND + f'hipLaunchKernelGGL({L.name}_flow_kernel, dim3((unsigned)tiles), dim3(64), 0, stream, '
+             f'{", ".join(args + red_fact_args(L) + red_finish_args(L))});')
+    b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 1);')
+    b += [IND + ln for ln in handler_reds_finish(L)]
+    b.append('} else {')
+    b += [IND + ln for ln in otherwise]
+    b.append('}')
+    return b
+
+
 # Chunk lengths (iterations per staged chunk) the tiled line sweep is
 # instantiated for; a thread keeps its share of the next chunk, CK + 1
 # elements, in registers while the current one is computed.
@@ -3285,6 +3434,9 @@ def across_handler(L):
         for deps in itertools.combinations(range(r), m):
             mask = sum(1 << (r - 1 - a) for a in deps)
             b.append(f'}} else if (dependency_mask == {mask}) {{')
+            rest = wave_launch(L, list(deps))
+            if m == r and L.flow_eligible():
+                rest = flow_launch(L, rest)
             if m == 3 and L.tile_eligible():
                 X = L.across['array']
                 xct = [p for p in L.arrays if p[1] == X][0][2]
@@ -3296,10 +3448,10 @@ def across_handler(L):
                 b.append(IND + 'if (tiled) {')
                 b += [IND * 2 + s for s in tile_launch(L)]
                 b.append(IND + '} else {')
-                b += [IND * 2 + s for s in wave_launch(L, list(deps))]
+                b += [IND * 2 + s for s in rest]
                 b.append(IND + '}')
             else:
-                b += [IND + s for s in wave_launch(L, list(deps))]
+                b += [IND + s for s in rest]
     b.append('} else {')
     b.append(IND + f'fprintf(stderr, "{L.name}: unsupported dependency mask %ld\\n", (long)dependency_mask);')
     b.append(IND + 'abort();')
@@ -3358,6 +3510,8 @@ def gpu_loop(L):
         for m in range(2, r + 1):
             for deps in itertools.combinations(range(r), m):
                 text.append(wave_kernel(L, list(deps)))
+        if L.flow_eligible():
+            text.append(flow_kernel(L))
         if L.tile_eligible():
             text.append(tile_kernel(L))
         if L.line_tile_eligible():

@@ -68,6 +68,19 @@ typedef struct {
 void dvmh_amd_loop_red_in_kernel_C(DvmType curLoop, DvmType items, DvmhAmdRedFinish *out);
 void dvmh_amd_loop_red_result_C(DvmType curLoop, DvmType redIndex, void **outVal, void **outLoc);
 
+/* ---- dataflow wavefront ------------------------------------------------------------
+ * Workspace of a loop run as one dataflow launch (see dvmh_hip_device.h): a
+ * control word (tag of the last sweep, next ticket), a flag per tile and the
+ * cells tiles hand their upper faces on in.  The runtime keeps one workspace,
+ * as large as the largest request, zeroed once: tags never repeat. */
+typedef struct {
+    unsigned long long *control, *flags, *cells;
+    unsigned *wrapped;           /* mapped host memory: set when tags run out (the runtime then starts over) */
+} DvmhAmdFlow;
+/* 1 with *out filled, or 0 when there is no memory for it (the handler then
+ * runs another kernel). */
+DvmType dvmh_amd_flow_workspace_C(DvmType tiles, DvmType cellWords, DvmhAmdFlow *out);
+
 /* ---- kernel timing -----------------------------------------------------------
  * Emitted handlers bracket their main kernel launches with phase 0 / phase 1
  * marks.  With timing enabled the runtime records HIP events on the loop's

@@ -28,6 +28,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "dvmhlib_types.h"
 #include "dvmhlib_const.h"
 #include "dvmh_amd.h"
@@ -537,6 +539,457 @@ __device__ __forceinline__ void publishDone(const DvmhAmdRedFinish &f) {
     if (!f.done) return;
     storesDone();
     __hip_atomic_store(f.done, f.doneSeq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// ------------------------------------------------------------------ dataflow wavefront
+// ACROSS loops whose axes all depend (rank 2 or 3) in one launch.  A wave owns
+// a tile of the leading axes -- 8 x 8 points for rank 3, 64 for rank 2, one
+// lane per point -- and walks the innermost axis; lane (p, q) runs one step
+// behind lanes (p - 1, q) and (p, q - 1), so at every step each lane's lower
+// neighbours are the previous step's results and its upper ones are still old:
+// the order of the sequential sweep.  Tiles are taken in the order of their
+// diagonal from a ticket counter, so a tile only ever waits for tiles that are
+// running or done, whatever the launch's residency.
+//
+// The rows of a tile pass through LDS in blocks of eight steps, three of them
+// at a time.  A row is held at the step its elements are walked at (element r
+// of row (p, q) in slot r + p + q), so in every step all lanes use the same
+// slots, at offsets known to the compiler, and a finished block of steps is
+// stored at once.  A block's loads and stores move 64 bytes of eight rows per
+// instruction; two blocks' loads are in flight while one is walked.  Rows a
+// tile needs from its lower neighbours come through cells in device memory: a
+// value in halves, each in an 8-byte word with a 32-bit tag that no earlier
+// launch used, so one load tells whether it is there.
+//
+// Bound by the chain of dependent steps: 0.12 us a step for rank 2 (eight
+// dependent FP64 operations and a lane shift), 0.155 for rank 3 (one neighbour
+// through LDS), and along a diagonal of tiles, per tile, the lanes' skew plus
+// about 4 us until a finished block is seen by the next tile.  Measured, one
+// sweep with reductions: 2-D 998^2 0.38 ms (a launch per hyperplane: 9.2), 3-D
+// 128^3 0.154 ms (a launch per tile-plane: 0.43), 318^3 0.76 ms (1.84).
+template <int RANK> struct FlowShape;
+template <> struct FlowShape<3> {
+    // row (p, q), -1 <= p, q <= 8, at (p + 1) * BP + (q + 1) * QP: the 32 lanes
+    // of an LDS cycle in 32 different bank pairs
+    static constexpr int PA = 8, PB = 8, BP = 264, QP = 25, LDS = 9 * 264 + 9 * 25 + 24;
+};
+template <> struct FlowShape<2> {
+    static constexpr int PA = 64, PB = 1, BP = 25, QP = 0, LDS = 65 * 25 + 24;
+};
+
+// The element at the loop point (slot 0) and its neighbours along axis a, one
+// below (slot 1 + 2 a) and one above (slot 2 + 2 a), as X[i][j][k].
+template <typename T, typename I, int R, int AX = 0>
+struct StarView {
+    T *v;
+    I at[R];
+    int slot;
+    __device__ __forceinline__ decltype(auto) operator[](I x) const {
+        const I d = x - at[AX];
+        const int s = d < 0 ? 1 + 2 * AX : (d > 0 ? 2 + 2 * AX : slot);
+        if constexpr (AX + 1 == R) {
+            return (v[s]);
+        } else {
+            StarView<T, I, R, AX + 1> n;
+            n.v = v;
+#pragma unroll
+            for (int a = 0; a < R; a++) n.at[a] = at[a];
+            n.slot = s;
+            return n;
+        }
+    }
+};
+
+template <typename T, typename I, int RANK>
+struct FlowArgs {
+    T *base;
+    I s[RANK];              // element strides (the innermost is 1)
+    I lo[RANK], cnt[RANK];  // the loop
+    I rlo[RANK], rhi[RANK]; // array indices the body may read: loads are clamped into them
+    int ntA, ntB, sweeps;
+    DvmhAmdFlow ws;
+};
+
+struct FlowTask {
+    int sweep, ta, tb;
+    unsigned tag;           // of the task's sweep
+};
+
+// Tiles on diagonal d of an ntA x ntB grid.
+__device__ __forceinline__ int flowDiagonal(int d, int ntA, int ntB) {
+    const int hi = d < ntA - 1 ? d : ntA - 1, lo = d - ntB + 1 > 0 ? d - ntB + 1 : 0;
+    return d < 0 || hi < lo ? 0 : hi - lo + 1;
+}
+
+// The wave's task: tickets in the order of ta + tb + 2 * sweep, which every
+// task a task waits for precedes.  The control word holds the tag of the last
+// sweep so far (high half) and the next ticket; the taker of the last ticket
+// sets it up for the next launch.
+__device__ __forceinline__ FlowTask flowTake(int ntA, int ntB, int sweeps, const DvmhAmdFlow &ws) {
+    unsigned ticket = 0, epoch = 0;
+    if (threadIdx.x == 0) {
+        const unsigned long long c = __hip_atomic_fetch_add(ws.control, 1ULL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        ticket = (unsigned)c;
+        epoch = (unsigned)(c >> 32);
+        if (ticket == (unsigned)ntA * (unsigned)ntB * (unsigned)sweeps - 1) {
+            const unsigned long long next = epoch + (unsigned)sweeps;
+            __hip_atomic_store(ws.control, next << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (next >> 31) __hip_atomic_store(ws.wrapped, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+    ticket = __builtin_amdgcn_readfirstlane(ticket);
+    epoch = __builtin_amdgcn_readfirstlane(epoch);
+    const int lane = threadIdx.x;
+    int t = (int)ticket, key = 0;
+    for (int k0 = 0;; k0 += 64) {
+        int n = 0;
+        for (int s = 0; s < sweeps; s++) n += flowDiagonal(k0 + lane - 2 * s, ntA, ntB);
+        int upTo = n;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int below = __shfl_up(upTo, o, 64);
+            if (lane >= o) upTo += below;
+        }
+        const unsigned long long past = __ballot(upTo > t);
+        if (past) {
+            const int at = __builtin_ctzll(past);
+            t -= __shfl(upTo - n, at, 64);
+            key = k0 + at;
+            break;
+        }
+        t -= __shfl(upTo, 63, 64);
+    }
+    int s = 0;
+    for (;; s++) {
+        const int n = flowDiagonal(key - 2 * s, ntA, ntB);
+        if (t < n) break;
+        t -= n;
+    }
+    const int d = key - 2 * s;
+    const int a = (d - ntB + 1 > 0 ? d - ntB + 1 : 0) + t;
+    return FlowTask{__builtin_amdgcn_readfirstlane(s), __builtin_amdgcn_readfirstlane(a), __builtin_amdgcn_readfirstlane(d - a),
+                    epoch + (unsigned)s + 1};
+}
+
+// A cell: the value's bytes in 32-bit parts, each beside the tag.
+template <typename T>
+struct FlowCell {
+    static constexpr int WORDS = sizeof(T) > 4 ? 2 : 1;
+    unsigned long long w[WORDS];
+    __device__ __forceinline__ void load(const unsigned long long *p) {
+#pragma unroll
+        for (int i = 0; i < WORDS; i++) w[i] = __hip_atomic_load(p + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ bool holds(unsigned tag) const {
+        bool h = true;
+#pragma unroll
+        for (int i = 0; i < WORDS; i++) h &= (unsigned)(w[i] >> 32) == tag;
+        return h;
+    }
+    __device__ __forceinline__ T value() const {
+        unsigned x[2] = {(unsigned)w[0], (unsigned)w[WORDS - 1]};
+        T v;
+        __builtin_memcpy(&v, x, sizeof(T));
+        return v;
+    }
+    static __device__ __forceinline__ void store(unsigned long long *p, T v, unsigned tag) {
+        unsigned x[2] = {0, 0};
+        __builtin_memcpy(x, &v, sizeof(T));
+#pragma unroll
+        for (int i = 0; i < WORDS; i++)
+            __hip_atomic_store(p + i, (unsigned long long)tag << 32 | x[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+};
+
+// Lane l gets lane l - 1's x, lane 0 gets `first` (whole wave active).
+template <typename T>
+__device__ __forceinline__ T laneBelow(T x, T first) {
+    int w[2] = {0, 0}, o[2] = {0, 0};
+    __builtin_memcpy(w, &x, sizeof(T));
+    __builtin_memcpy(o, &first, sizeof(T));
+    constexpr int WAVE_SHR1 = 0x138;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) + 3) / 4; i++) w[i] = __builtin_amdgcn_update_dpp(o[i], w[i], WAVE_SHR1, 0xf, 0xf, false);
+    T r;
+    __builtin_memcpy(&r, w, sizeof(T));
+    return r;
+}
+
+// x is in its register here (its load is issued before, not sunk to its use).
+template <typename T>
+__device__ __forceinline__ void readHere(T &x) { asm volatile("" : "+v"(x)); }
+
+// Walks the task's tile.  body(v, t0, t1, t2) runs the loop body at position
+// (t0, t1, t2) of the loop (t2 unused for rank 2) with v the star around it.
+// CHAIN: several sweeps of the array in one launch; its elements then pass
+// between workgroups, so they are loaded and stored at agent scope, and a
+// tile's flag says how many blocks of which sweep are in memory.
+template <typename T, typename I, int RANK, bool CHAIN, typename Body>
+__device__ __forceinline__ void flowTile(const FlowArgs<T, I, RANK> &f, const FlowTask &task, T *ring, Body &&body) {
+    using S = FlowShape<RANK>;
+    constexpr int K = RANK - 1, SKEW = S::PA + S::PB - 2, SLOTS = 24;
+    const int lane = threadIdx.x, g = lane >> 3, e = lane & 7;   // block transfers: eight rows of eight elements
+    const int p = RANK == 3 ? g : lane, q = RANK == 3 ? e : 0;   // the lane's own row
+    const int ta = task.ta, tb = task.tb;
+    const I a0 = (I)ta * S::PA, b0 = (I)tb * S::PB;
+    const int na = f.cnt[0] - a0 < S::PA ? (int)(f.cnt[0] - a0) : S::PA;
+    const int nb = RANK == 2 ? 1 : (f.cnt[1] - b0 < S::PB ? (int)(f.cnt[1] - b0) : S::PB);
+    const int n = (int)f.cnt[K];
+    const int blocks = (n + na + nb - 2 + 7) >> 3;   // blocks of steps
+    auto clampTo = [](I x, I lo, I hi) { return x < lo ? lo : (x > hi ? hi : x); };
+    auto rowOff = [&](int pp, int qq) -> I {
+        I o = clampTo(f.lo[0] + a0 + pp, f.rlo[0], f.rhi[0]) * f.s[0];
+        if constexpr (RANK == 3) o += clampTo(f.lo[1] + b0 + qq, f.rlo[1], f.rhi[1]) * f.s[1];
+        return o;
+    };
+    auto rowAt = [](int pp, int qq) { return (pp + 1) * S::BP + (qq + 1) * S::QP; };
+    // the row a lane moves in transfer `it` of a block
+    auto rowP = [&](int it) { return RANK == 3 ? it : it * 8 + g; };
+    auto rowQ = [&](int) { return RANK == 3 ? g : 0; };
+    // rows moved block by block: the tile's 64, the ones above it and, at the
+    // array's lower edges, the ones below it (elsewhere those come in cells)
+    const bool edgeA = ta == 0, edgeB = RANK == 3 && tb == 0;
+    I off[8];
+#pragma unroll
+    for (int it = 0; it < 8; it++) off[it] = rowOff(rowP(it), rowQ(it));
+    const I offA = rowOff(S::PA, g), offB = RANK == 3 ? rowOff(g, S::PB) : 0;
+    const I offLA = rowOff(-1, g), offLB = RANK == 3 ? rowOff(g, -1) : 0;
+    const int gq = RANK == 3 ? g : 0;   // second coordinate of a face row of the first axis
+    // two blocks' loads are in flight while a block is walked (a block of steps
+    // takes less than a round trip to memory), in two sets of registers
+    struct Ahead {
+        T own[8], vA, vB, vLA, vLB;
+    } even{}, odd{};
+    // (issued on every path, past the row's end from its last element, so that
+    // the waits know how many younger loads may stay in flight)
+    auto issue = [&](Ahead &h, int b) {
+        const I k = f.lo[K] + 8 * b + e;
+        auto ld = [&](I o, int skew) -> T {
+            const T *x = f.base + (o + clampTo(k - skew, f.rlo[K], f.rhi[K]));
+            return CHAIN ? agentLoad(x) : *x;
+        };
+#pragma unroll
+        for (int it = 0; it < 8; it++) h.own[it] = ld(off[it], rowP(it) + rowQ(it));
+        h.vA = ld(offA, S::PA + gq);
+        if constexpr (RANK == 3) h.vB = ld(offB, g + S::PB);
+        if (edgeA) h.vLA = ld(offLA, gq - 1);
+        if constexpr (RANK == 3) if (edgeB) h.vLB = ld(offLB, g - 1);
+    };
+    auto commit = [&](const Ahead &h, int b) {
+        T *to = ring + (b % 3) * 8 + e;
+#pragma unroll
+        for (int it = 0; it < 8; it++) to[rowAt(rowP(it), rowQ(it))] = h.own[it];
+        if constexpr (RANK == 3) {
+            to[rowAt(S::PA, g)] = h.vA;
+            to[rowAt(g, S::PB)] = h.vB;
+            if (edgeA) to[rowAt(-1, g)] = h.vLA;
+            if (edgeB) to[rowAt(g, -1)] = h.vLB;
+        } else if (g == 0) {
+            to[rowAt(S::PA, 0)] = h.vA;
+            if (edgeA) to[rowAt(-1, 0)] = h.vLA;
+        }
+    };
+    // cells of a tile's upper faces: PB rows of n towards ta + 1, PA rows towards tb + 1
+    constexpr int W = FlowCell<T>::WORDS;
+    const long tiles = (long)f.ntA * f.ntB, tile = (long)ta * f.ntB + tb;
+    unsigned long long *const cellsA = f.ws.cells, *const cellsB = f.ws.cells + tiles * S::PB * n * W;
+    const bool fromA = ta > 0, fromB = RANK == 3 && tb > 0;
+    const bool toA = ta + 1 < f.ntA, toB = RANK == 3 && tb + 1 < f.ntB;
+    // lane (g, e) fetches element 8 m + e - g of face row g: what lane (0, g)
+    // (or (g, 0)) needs at step e of block m
+    const bool rowA = fromA && g < nb, rowB = fromB && g < na;
+    auto inRow = [&](int r) { return (unsigned)r < (unsigned)n; };
+    auto cellOf = [&](unsigned long long *c, long t, int rows, int r) { return c + ((t * rows + g) * n + r) * W; };
+    unsigned long long *const inA = cellOf(cellsA, tile - f.ntB, S::PB, 0), *const inB = cellOf(cellsB, tile - 1, S::PA, 0);
+    unsigned long long *const outA = cellOf(cellsA, tile, S::PB, 0), *const outB = cellOf(cellsB, tile, S::PA, 0);
+    // (every lane loads something, some the first cell in vain: a load in a
+    // branch would have to be waited for at the branch's end)
+    FlowCell<T> cA{}, cB{};
+    auto fetch = [&](int m) {
+        const int r = 8 * m + e - g;
+        cA.load(rowA & inRow(r) ? inA + r * W : cellsA);
+        if constexpr (RANK == 3) cB.load(rowB & inRow(r) ? inB + r * W : cellsA);
+    };
+    auto missing = [&](int m) {
+        const bool in = inRow(8 * m + e - g);
+        bool miss = in & rowA & !cA.holds(task.tag);
+        if constexpr (RANK == 3) miss |= in & rowB & !cB.holds(task.tag);
+        return __any(miss);
+    };
+    // chain: the flags of the tiles whose previous sweep this one reads (itself
+    // and the two above); each sweep has its own, as several sweeps of a tile
+    // run at a time
+    unsigned long long *const flag = f.ws.flags;
+    const long flagged = task.sweep * tiles + tile;
+    long watch = -1;
+    if constexpr (CHAIN) {
+        const long before = flagged - tiles;
+        if (task.sweep > 0) watch = lane == 0 ? before : lane == 1 && ta + 1 < f.ntA ? before + f.ntB : lane == 2 && tb + 1 < f.ntB ? before + 1 : -1;
+    }
+    unsigned long long seen = 0;
+    auto await = [&](int b) {
+        if constexpr (CHAIN) {
+            if (task.sweep == 0) return;
+            const int most = (n + SKEW + 7) >> 3;
+            const unsigned long long need = (unsigned long long)(task.tag - 1) << 32 | (unsigned)(b + 1 < most ? b + 1 : most);
+            while (__any(watch >= 0 && seen < need)) {
+                if (watch >= 0 && seen < need) seen = __hip_atomic_load(flag + watch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            asm volatile("" ::: "memory");   // no element is loaded before its flag
+        }
+    };
+    auto publish = [&](int count) {
+        if (lane == 0) __hip_atomic_store(flag + flagged, (unsigned long long)task.tag << 32 | (unsigned)count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+
+    await(0);
+    issue(even, 0);
+    commit(even, 0);
+    await(1);
+    issue(odd, 1);
+    await(2);
+    issue(even, 2);
+    // the lower edge rows' elements before the first block's
+    if (lane == 0) {
+        if (edgeA) ring[rowAt(-1, 0) + SLOTS - 1] = f.base[rowOff(-1, 0) + f.lo[K]];
+        if (edgeB) ring[rowAt(0, -1) + SLOTS - 1] = f.base[rowOff(0, -1) + f.lo[K]];
+    }
+    fetch(0);
+    const bool mine = p < na && q < nb, whole = na == S::PA && nb == S::PB;
+    T *const row = ring + rowAt(p, q);
+    T prev = f.base[rowOff(p, q) + clampTo(f.lo[K] - 1, f.rlo[K], f.rhi[K])];   // the element before the first point
+    readHere(prev);   // (waited for here, not by every block of steps)
+    asm volatile("" ::: "memory");
+    // upper neighbours are read two steps ahead (an LDS read takes longer than
+    // what is left of a step once its operands are there)
+    T c = row[0], kp = row[1], ip = row[S::BP + 1], jp{}, kp2 = row[2], ip2 = row[S::BP + 2], jp2{};
+    if constexpr (RANK == 3) {
+        jp = row[S::QP + 1];
+        jp2 = row[S::QP + 2];
+    }
+    // eight steps; GUARD: some lanes are outside the loop in some of them
+    auto walk = [&](int m, auto guard) {
+        const T *before = row + (m + 2) % 3 * 8, *after = row + (m + 1) % 3 * 8;
+        T *now = row + m % 3 * 8;
+        // lower neighbours: what the lanes before did a step ago (their prev),
+        // at the tile's edge the row below (there since the block began: read
+        // ahead too); along the first axis of a rank 3 tile they are eight
+        // lanes away: through LDS
+        constexpr int EDGE = RANK == 3 ? S::QP : S::BP;
+        T edge = before[7 - EDGE], edge1 = now[-EDGE], edge2{};
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            T low{};
+            if constexpr (RANK == 3) low = (u == 0 ? before + 7 : now + u - 1)[-S::BP];
+            const T *up = u < 5 ? now + u + 3 : after + u - 5;
+            const T kp3 = up[0], ip3 = up[S::BP];
+            T jp3{};
+            if constexpr (RANK == 3) jp3 = up[S::QP];
+            if (u < 6) edge2 = now[u + 1 - EDGE];
+            T v[1 + 2 * RANK];
+            v[0] = c;
+            if constexpr (RANK == 3) {
+                readHere(low);
+                const T beside = laneBelow(prev, prev);
+                v[1] = low;
+                v[3] = q == 0 ? edge : beside;
+                v[4] = jp;
+            } else {
+                v[1] = laneBelow(prev, edge);
+            }
+            v[2] = ip;
+            v[1 + 2 * K] = prev;
+            v[2 + 2 * K] = kp;
+            const int r = 8 * m + u - p - q;
+            if (!decltype(guard)::value || (mine && r >= 0 && r < n)) {
+                body(v, a0 + p, RANK == 3 ? b0 + q : (I)r, (I)r);
+                now[u] = v[0];
+                prev = v[0];
+            }
+            asm volatile("" ::: "memory");   // the next step's lanes read what this one wrote
+            c = kp;
+            kp = kp2;
+            kp2 = kp3;
+            ip = ip2;
+            ip2 = ip3;
+            jp = jp2;
+            jp2 = jp3;
+            edge = edge1;
+            edge1 = edge2;
+        }
+    };
+    // every lane inside the loop at every step of block m
+    auto inner = [&](int m) { return whole && 8 * m >= SKEW && 8 * m + 7 < n; };
+    // next: the set that holds block m + 1 and takes m + 3
+    auto block = [&](int m, Ahead &next) {
+        T out[8];   // block m - 1, on its way to memory
+#pragma unroll
+        for (int it = 0; it < 8; it++) out[it] = ring[rowAt(rowP(it), rowQ(it)) + (m + 2) % 3 * 8 + e];
+        asm volatile("" ::: "memory");
+        commit(next, m + 1);
+        if (CHAIN && m >= 2) {
+            storesDone();   // those of block m - 2, a block of steps ago
+            publish(m - 1);
+        }
+        if (m < blocks) {
+            if (missing(m)) {
+                do {
+                    fetch(m);
+#pragma unroll
+                    for (int i = 0; i < W; i++) {
+                        readHere(cA.w[i]);
+                        readHere(cB.w[i]);
+                    }
+                } while (missing(m));
+            }
+            T *to = ring + (unsigned)(8 * m + e + SLOTS - 1) % SLOTS;   // the lanes above read them a slot lower
+            const bool in = inRow(8 * m + e - g);
+            if (in & rowA) to[rowAt(-1, g)] = cA.value();
+            if (RANK == 3 && (in & rowB)) to[rowAt(g, -1)] = cB.value();
+        }
+        if (m > 0) {
+            T *x = f.base + f.lo[K] + 8 * (m - 1) + e;
+            auto put = [](T *to, T v) {
+                if (CHAIN) agentStore(to, v);
+                else *to = v;
+            };
+            if (inner(m - 1)) {
+#pragma unroll
+                for (int it = 0; it < 8; it++) put(x + (off[it] - rowP(it) - rowQ(it)), out[it]);
+            } else {
+#pragma unroll
+                for (int it = 0; it < 8; it++) {
+                    const int skew = rowP(it) + rowQ(it);
+                    if ((rowP(it) < na) & (rowQ(it) < nb) & inRow(8 * (m - 1) + e - skew)) put(x + (off[it] - skew), out[it]);
+                }
+            }
+        }
+        fetch(m + 1);   // before the row loads, so that waiting for it leaves those in flight
+        await(m + 3);
+        issue(next, m + 3);
+        if (m < blocks) {
+            asm volatile("" ::: "memory");
+            if (inner(m)) walk(m, std::false_type());
+            else walk(m, std::true_type());
+            // the upper faces' rows: what lanes (PA - 1, .) and (., PB - 1) did in this block
+            const T *done = ring + m % 3 * 8 + e;
+            const int rA = 8 * m + e - (S::PA - 1) - g;
+            if (toA & (g < nb) & inRow(rA)) FlowCell<T>::store(outA + rA * W, done[rowAt(S::PA - 1, gq)], task.tag);
+            if constexpr (RANK == 3) {
+                const int rB = 8 * m + e - (S::PB - 1) - g;
+                if (toB & (g < na) & inRow(rB)) FlowCell<T>::store(outB + rB * W, done[rowAt(g, S::PB - 1)], task.tag);
+            }
+            asm volatile("" ::: "memory");
+        }
+    };
+    for (int m = 0; m < blocks + 1; m += 2) {
+        block(m, odd);
+        block(m + 1, even);   // (one too many of an odd number stores nothing)
+    }
+    if (CHAIN) {
+        storesDone();
+        publish(0x7fffffff);
+    }
 }
 
 // ------------------------------------------------------------------ scheduling
