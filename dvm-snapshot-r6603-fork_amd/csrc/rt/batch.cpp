@@ -13,8 +13,7 @@
 // A loop registered with a chain handler instead joins the last group when
 // that group is a chain of the same handler, whatever arrays they share: the
 // chain's loops stay in program order and the chain handler runs them with
-// their dependencies kept (consecutive ACROSS sweeps of one array, pipelined
-// a few tile-planes apart).  A chain whose loop site the tuner is still
+// their dependencies kept (consecutive ACROSS sweeps of one array, pipelined).  A chain whose loop site the tuner is still
 // exploring runs loop by loop, so that every execution is timed.
 //
 // Two consecutive queued loops of one region whose handlers have a registered

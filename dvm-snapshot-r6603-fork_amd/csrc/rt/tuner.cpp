@@ -177,19 +177,9 @@ std::vector<Candidate> makeCandidates(int kind, int loopRank, int depCount, cons
                 }
             }
     } else if (kind == DVMH_AMD_KIND_CHAIN) {
-        // a chain of sweeps of a tiled-wavefront loop: tile shapes only (the
-        // chain handler runs nothing else); times are per sweep of the chain
+        // a chain of sweeps runs as one dataflow launch of fixed shape (one
+        // configuration: nothing to explore); times are per sweep of the chain
         addCand(v, 256, 1, 1, {{DVMH_AMD_T_VARIANT, 1}, {DVMH_AMD_T_TILE_A, 8}, {DVMH_AMD_T_TILE_B, 8}});
-        const int nts[] = {128, 256, 512};
-        const int tas[] = {8, 12, 16};
-        const int tcs[] = {8, 16, 32};
-        for (int nt : nts)
-            for (int ta : tas)
-                for (int tc : tcs) {
-                    if ((long)(ta + 2) * (ta + 2) * (tc + 2) * 8 > 64512) continue;
-                    if (nt > 4 * ta * ta) continue;
-                    addCand(v, nt, 1, 1, {{DVMH_AMD_T_VARIANT, 1}, {DVMH_AMD_T_TILE_A, ta}, {DVMH_AMD_T_TILE_B, tc}});
-                }
     } else {
         // one launch per hyperplane: threads over the free dependent axes (y only
         // with three or more dependent axes), optional diagonal layout
@@ -204,8 +194,8 @@ std::vector<Candidate> makeCandidates(int kind, int loopRank, int depCount, cons
                 for (int tf = 0; tf <= tfMax; tf++) addCand(v, bx, by, 1, {{DVMH_AMD_T_TRANSFORM, tf}});
             }
         if (loopRank == 3 && depCount == 3) {
-            // tiled variant: TILE_A x TILE_A x TILE_B tiles staged in LDS with a
-            // halo of one, one launch per tile-plane
+            // tiles of TILE_A x TILE_A x TILE_B (handlers that run the sweep as one
+            // dataflow launch take every one of these alike)
             const int nts[] = {64, 128, 256, 512};
             const int tas[] = {4, 8, 12, 16};
             const int tcs[] = {8, 16, 32, 64};

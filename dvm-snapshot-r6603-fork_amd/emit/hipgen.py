@@ -34,9 +34,12 @@ Output, per program:
                        LINE       ACROSS with one dependent axis: one launch,
                                   threads over the independent axes, each
                                   thread walks its line in dependency order.
-                       WAVEFRONT  ACROSS with >= 2 dependent axes: one launch
-                                  per hyperplane of the dependent axes; arrays
-                                  may be in the diagonal layout.
+                       FLOW       ACROSS whose axes all depend (rank 2, 3): one
+                                  dataflow launch per sweep, or per chain of
+                                  sweeps.
+                       WAVEFRONT  other ACROSS with >= 2 dependent axes: one
+                                  launch per hyperplane of the dependent axes;
+                                  arrays may be in the diagonal layout.
 The loop body is inserted verbatim; every schedule respects the dependency
 order, so results are bit-identical to the sequential host order.
 """
@@ -145,40 +148,13 @@ class Loop:
                 hi[a] = d if hi[a] is None else max(hi[a], d)
         return [(l or 0, h or 0) for l, h in zip(lo, hi)]
 
-    def tile_eligible(self):
-        """Rank 3, every loop axis in the ACROSS clause with widths <= 1, and
-        every access of the ACROSS array in the body of the form
-        X[i + d0][j + d1][k + d2] with at most one offset, |offset| <= 1."""
-        if not self.across or self.rank != 3:
-            return False
-        w = self.across['widths']
-        if len(w) != 3 or any(lo > 1 or hi > 1 or (lo == 0 and hi == 0) for lo, hi in w):
-            return False
-        name = self.across['array']
-        if re.search(r'\b' + name + r'\b(?!\s*\[)', self.body):
-            return False
-        for m in re.finditer(r'\b' + name + r'\s*((?:\[[^\[\]]*\]\s*)+)', self.body):
-            idx = re.findall(r'\[([^\[\]]*)\]', m.group(1))
-            if len(idx) != 3:
-                return False
-            moved = 0
-            for (v, _), e in zip(self.vars, idx):
-                mm = re.fullmatch(r'\s*' + v + r'\s*(?:([+-])\s*([01])\s*)?', e)
-                if not mm:
-                    return False
-                if mm.group(2) == '1':
-                    moved += 1
-            if moved > 1:
-                return False
-        return True
-
     def flow_eligible(self):
         """Rank 2 or 3, every loop axis in the ACROSS clause with widths <= 1;
         the body reads the ACROSS array at X[i + d0][j + d1].. with at most one
-        offset, |offset| <= 1, writes it at the loop point only, and writes
-        nothing else but its own variables and reductions: the sweep can then
-        run as one dataflow launch (other arrays and scalars are not passed
-        between the workgroups)."""
+        offset, |offset| <= 1, writes it at the loop point only, touches any
+        other array it writes at the loop point only, and assigns no scalar: the
+        sweep can then run as one dataflow launch (nothing but the ACROSS array
+        passes between its workgroups)."""
         if not self.across or self.rank not in (2, 3):
             return False
         w = self.across['widths']
@@ -186,44 +162,44 @@ class Loop:
             return False
         X = self.across['array']
         arr = [p for p in self.arrays if p[1] == X]
-        if not arr or arr[0][3] != self.rank or arr[0][2] not in ('float', 'double', 'int', 'long'):
+        if not arr or arr[0][3] != self.rank or arr[0][2] not in ('char', 'int', 'long', 'float', 'double'):
             return False
-        if re.search(r'\b' + X + r'\b(?!\s*\[)', self.body) or re.search(r'(\+\+|--|&)\s*' + X + r'\b', self.body):
-            return False
-        written = False
         assign = r'(?:=(?!=)|\+=|-=|\*=|/=|%=|&=|\|=|\^=|<<=|>>=|\+\+|--)'
-        for m in re.finditer(r'\b' + X + r'\s*((?:\[[^\[\]]*\]\s*)+)(' + assign + ')?', self.body):
-            idx = re.findall(r'\[([^\[\]]*)\]', m.group(1))
-            if len(idx) != self.rank:
-                return False
-            moved = 0
-            for (v, _), e in zip(self.vars, idx):
-                mm = re.fullmatch(r'\s*' + v + r'\s*(?:([+-])\s*([01])\s*)?', e)
-                if not mm:
-                    return False
-                moved += mm.group(2) == '1'
-            if moved > (0 if m.group(2) else 1):
-                return False
-            written = written or bool(m.group(2))
-        if not written:
-            return False
+
+        def uses(name):
+            """Per subscripted use: the offsets (None: not of the form v + 0/1), written or not."""
+            out = []
+            for m in re.finditer(r'\b' + name + r'\s*((?:\[[^\[\]]*\]\s*)+)(' + assign + ')?', self.body):
+                idx = re.findall(r'\[([^\[\]]*)\]', m.group(1))
+                mm = [re.fullmatch(r'\s*' + v + r'\s*(?:([+-])\s*([01])\s*)?', e) for (v, _), e in zip(self.vars, idx)]
+                at = [x.group(2) == '1' for x in mm] if len(idx) == self.rank and all(mm) else None
+                out.append((at, bool(m.group(2))))
+            return out
+
         for p in self.params:
-            if p[1] == X:
+            name = p[1]
+            if p[0] not in ('array', 'scalar') or re.search(r'(\+\+|--|&)\s*' + name + r'\b', self.body):
+                return False
+            if p[0] == 'scalar':
+                if re.search(r'(?<![\w.>])' + name + r'\s*' + assign, self.body):
+                    return False
                 continue
-            if p[0] not in ('array', 'scalar') or re.search(r'(\+\+|--|&)\s*' + p[1] + r'\b', self.body):
+            # (an array whose name appears other than subscripted may be passed on and written)
+            if re.search(r'\b' + name + r'\b(?!\s*\[)', self.body):
                 return False
-            if re.search(r'(?<![\w.>])' + p[1] + r'\s*(?:\[[^\]]*\]\s*)*' + assign, self.body):
+            refs = uses(name)
+            if name == X:
+                if any(at is None or sum(at) > (0 if written else 1) for at, written in refs) or not any(wr for _, wr in refs):
+                    return False
+            elif any(wr for _, wr in refs) and any(at is None or sum(at) for at, _ in refs):
                 return False
-            # an array whose name appears other than subscripted may be passed on and written
-            if p[0] == 'array' and re.search(r'\b' + p[1] + r'\b(?!\s*\[)', self.body):
-                return False
-        return all(self.rlen(red) == 1 for red in self.reds)
+        return True
 
     def chain_eligible(self):
         """Consecutive executions (sweeps) of the loop may run pipelined by a
-        chain handler: a tiled-wavefront ACROSS loop marked for batching that
-        writes no array but its ACROSS array and has scalar reductions only."""
-        if not self.batch or not self.tile_eligible():
+        chain handler: a loop marked for batching whose sweeps of three axes are
+        dataflow launches that write no array but the ACROSS array."""
+        if not self.batch or self.rank != 3 or not self.flow_eligible():
             return False
         X = self.across['array']
         for p in self.arrays:
@@ -2433,220 +2409,6 @@ def wave_launch(L, deps):
     return b
 
 
-def tile_kernel(L):
-    """Tiled wavefront for an ACROSS loop whose three axes all depend: tiles of
-    TA x TA x TC iterations are run one tile-plane (a + b + c = const) per
-    launch.  A workgroup stages its tile of the ACROSS array plus a halo of one
-    in LDS (lower halo: final values of earlier tiles; upper halo: values no
-    tile has updated yet), runs the tile's local hyperplanes in order with a
-    workgroup barrier between them, and writes the tile back.  The body reads
-    and writes the ACROSS array through a TileView3 with the usual X[i][j][k]
-    syntax; every dependency is met in the sequential order's sense, so the
-    results are those of the lexicographic sweep.
-
-    The work on one tile is a device function, called by the per-loop kernel
-    (one launch per tile-plane) and by the chain kernel, which runs several
-    consecutive sweeps of the loop in one launch sequence: launch t runs
-    tile-plane t - LAG * s of sweep s for every sweep s that has one, so a
-    sweep stays LAG tile-planes behind the sweep before it."""
-    X = L.across['array']
-    xct = [p for p in L.arrays if p[1] == X][0][2]
-    rng = L.stencil_range(X)   # per axis, the offsets at which the body reads X
-    fp, setup = [], []
-    for p in L.arrays:
-        _, nm, ct, ar = p
-        fp.append(f'{ct} *__restrict__ {nm}_base')
-        fp += [f'IndexT {nm}_s{k}' for k in range(ar)]
-        strides = ', '.join(f'{nm}_s{k}' for k in range(ar))
-        setup.append(f'const IndexT {nm}_str[{ar}] = {{{strides}}};')
-        vn = f'{nm}_g' if nm == X else nm
-        setup.append(f'const auto {vn} = dvmh_dev::makeView<{ct}, IndexT, {ar}, true>({nm}_base, {nm}_str);')
-    for p in L.scalars:
-        fp.append(f'{p[2]} *__restrict__ {p[1]}_ptr')
-        setup.append(scalar_bind(L.body, p))
-    for i in range(3):
-        fp += [f'IndexT lo{i}', f'IndexT cnt{i}', f'IndexT st{i}']
-    call = []
-    for p in L.arrays:
-        call += [f'{p[1]}_base'] + [f'{p[1]}_s{q}' for q in range(p[3])]
-    for p in L.scalars:
-        call.append(f'{p[1]}_ptr')
-    for i in range(3):
-        call += [f'lo{i}', f'cnt{i}', f'st{i}']
-    # ---- the tile: stage, local hyperplanes, write back; reductions by reference
-    tp = list(fp) + ['IndexT dt_TA', 'IndexT dt_TC', 'IndexT dt_ta', 'IndexT dt_tb', 'IndexT dt_tc']
-    for red in L.reds:
-        tp.append(f'{red[2]} &{red[1]}')
-        if len(red) > 3:
-            tp.append(f'{red[4]} &{red[3]}')
-    k = ['template <typename IndexT>',
-         f'__device__ static inline void {L.name}_tile_work({", ".join(tp)}) {{']
-    b = ['extern __shared__ __align__(16) unsigned char dvmh_lds[];']
-    b += setup
-    for v, ct in L.vars:
-        b.append(f'{ct} {v};')
-    for pr in L.privates:
-        b.append(pr + ';')
-    b += ['const IndexT dt_a0 = dt_ta * dt_TA, dt_b0 = dt_tb * dt_TA, dt_c0 = dt_tc * dt_TC;',
-          'const IndexT dt_na = cnt0 - dt_a0 < dt_TA ? cnt0 - dt_a0 : dt_TA;',
-          'const IndexT dt_nb = cnt1 - dt_b0 < dt_TA ? cnt1 - dt_b0 : dt_TA;',
-          'const IndexT dt_nc = cnt2 - dt_c0 < dt_TC ? cnt2 - dt_c0 : dt_TC;',
-          'const IndexT dt_R1 = dt_nb + 2, dt_R2 = dt_nc + 2, dt_R12 = dt_R1 * dt_R2;',
-          'const IndexT dt_elems = (dt_na + 2) * dt_R12;',
-          f'{xct} *dt_tile = ({xct} *)dvmh_lds;',
-          'const IndexT dt_oi = lo0 + dt_a0 - 1, dt_oj = lo1 + dt_b0 - 1, dt_ok = lo2 + dt_c0 - 1;   // array index of tile slot (0, 0, 0)',
-          'const IndexT dt_tid = (IndexT)threadIdx.x, dt_nthr = (IndexT)blockDim.x;',
-          '// stage the tile and its halo, sixteen loads in flight per thread; an index',
-          '// outside those the body reads is clamped into them (its slot is never read)']
-    for a, v in enumerate(('dt_ii', 'dt_jj', 'dt_kk')):
-        b.append(f'const IndexT {v}_lo = lo{a} + ({rng[a][0]}), {v}_hi = lo{a} + cnt{a} - 1 + ({rng[a][1]});')
-    b += ['// slot (p, q, r) of element e = dt_tid + m * dt_nthr, advanced by dt_nthr',
-          '// in the radix (R1, R2) of the tile: two divisions per thread, not per element',
-          'IndexT dt_sp = dt_nthr / dt_R12, dt_sq = (dt_nthr - dt_sp * dt_R12) / dt_R2, dt_sr = dt_nthr - dt_sp * dt_R12 - dt_sq * dt_R2;',
-          'IndexT dt_p = dt_tid / dt_R12, dt_q = (dt_tid - dt_p * dt_R12) / dt_R2, dt_r = dt_tid - dt_p * dt_R12 - dt_q * dt_R2;',
-          'for (IndexT dt_b0 = 0; dt_b0 < dt_elems; dt_b0 += 16 * dt_nthr) {',
-          IND + 'const IndexT dt_e0 = dt_b0 + dt_tid;',
-          IND + f'{xct} dt_v[16];',
-          IND + '#pragma unroll',
-          IND + 'for (int u = 0; u < 16; u++) {',
-          IND * 2 + 'if (dt_b0 + (IndexT)u * dt_nthr >= dt_elems) break;   // (uniform) no element of the workgroup left',
-          IND * 2 + '// (past the last element p runs beyond the tile: the clamp keeps the load in bounds)',
-          IND * 2 + 'IndexT dt_ii = dt_oi + dt_p, dt_jj = dt_oj + dt_q, dt_kk = dt_ok + dt_r;']
-    for v in ('dt_ii', 'dt_jj', 'dt_kk'):
-        b.append(IND * 2 + f'{v} = {v} < {v}_lo ? {v}_lo : ({v} > {v}_hi ? {v}_hi : {v});')
-    b += [IND * 2 + f'dt_v[u] = {X}_g[dt_ii][dt_jj][dt_kk];',
-          IND * 2 + 'dt_r += dt_sr; dt_q += dt_sq; dt_p += dt_sp;',
-          IND * 2 + 'if (dt_r >= dt_R2) { dt_r -= dt_R2; dt_q++; }',
-          IND * 2 + 'if (dt_q >= dt_R1) { dt_q -= dt_R1; dt_p++; }',
-          IND + '}',
-          IND + '#pragma unroll',
-          IND + 'for (int u = 0; u < 16; u++)',
-          IND * 2 + 'if (dt_e0 + (IndexT)u * dt_nthr < dt_elems) dt_tile[dt_e0 + (IndexT)u * dt_nthr] = dt_v[u];',
-          '}',
-          '__syncthreads();',
-          f'const dvmh_dev::TileView3<{xct}, IndexT> {X}{{dt_tile, dt_R1, dt_R2, dt_oi, dt_oj, dt_ok}};',
-          '// local hyperplanes p + q + r = s of the tile, in order; a thread\'s (p, q)',
-          '// columns do not change from one hyperplane to the next: up to four are',
-          '// worked out once (more than four per thread take the generic loop)',
-          'const IndexT dt_nab = dt_na * dt_nb;',
-          'IndexT dt_myp[4], dt_myq[4];',
-          'bool dt_has[4];',
-          '#pragma unroll',
-          'for (int u = 0; u < 4; u++) {',
-          IND + 'const IndexT dt_idx = dt_tid + (IndexT)u * dt_nthr;',
-          IND + 'dt_has[u] = dt_idx < dt_nab;',
-          IND + 'dt_myp[u] = dt_idx / dt_nb;',
-          IND + 'dt_myq[u] = dt_idx - dt_myp[u] * dt_nb;',
-          '}',
-          'const bool dt_few = dt_nab <= 4 * dt_nthr, dt_one = dt_nab <= dt_nthr;',
-          'for (IndexT dt_s = 0; dt_s < dt_na + dt_nb + dt_nc - 2; dt_s++) {',
-          IND + 'if (dt_one) {   // at most one column per thread',
-          IND * 2 + 'const IndexT dt_p = dt_myp[0], dt_q = dt_myq[0];',
-          IND * 2 + 'const IndexT dt_r = dt_s - dt_p - dt_q;',
-          IND * 2 + 'if (dt_has[0] && dt_r >= 0 && dt_r < dt_nc) {',
-          IND * 3 + 'const IndexT t0 = dt_a0 + dt_p, t1 = dt_b0 + dt_q, t2 = dt_c0 + dt_r;',
-          ] + [IND * 3 + var_assign(L, i, f't{i}', f'lo{i}', '(IndexT)1') for i in range(3)] + [indent('{\n' + indent(L.body + '\n', 1) + '}', 3)] + [
-          IND * 2 + '}',
-          IND + '} else if (dt_few) {',
-          IND * 2 + '#pragma unroll',
-          IND * 2 + 'for (int u = 0; u < 4; u++) {',
-          IND * 3 + 'const IndexT dt_p = dt_myp[u], dt_q = dt_myq[u];',
-          IND * 3 + 'const IndexT dt_r = dt_s - dt_p - dt_q;',
-          IND * 3 + 'if (dt_has[u] && dt_r >= 0 && dt_r < dt_nc) {',
-          IND * 4 + 'const IndexT t0 = dt_a0 + dt_p, t1 = dt_b0 + dt_q, t2 = dt_c0 + dt_r;']
-    for i in range(3):
-        b.append(IND * 4 + var_assign(L, i, f't{i}', f'lo{i}', '(IndexT)1'))   # the handlers run unit forward steps only
-    b.append(indent('{\n' + indent(L.body + '\n', 1) + '}', 4))
-    b += [IND * 3 + '}',
-          IND * 2 + '}',
-          IND + '} else {',
-          IND * 2 + 'for (IndexT dt_idx = dt_tid; dt_idx < dt_nab; dt_idx += dt_nthr) {',
-          IND * 3 + 'const IndexT dt_p = dt_idx / dt_nb, dt_q = dt_idx - (dt_idx / dt_nb) * dt_nb;',
-          IND * 3 + 'const IndexT dt_r = dt_s - dt_p - dt_q;',
-          IND * 3 + 'if (dt_r >= 0 && dt_r < dt_nc) {',
-          IND * 4 + 'const IndexT t0 = dt_a0 + dt_p, t1 = dt_b0 + dt_q, t2 = dt_c0 + dt_r;']
-    for i in range(3):
-        b.append(IND * 4 + var_assign(L, i, f't{i}', f'lo{i}', '(IndexT)1'))   # the handlers run unit forward steps only
-    b.append(indent('{\n' + indent(L.body + '\n', 1) + '}', 4))
-    b += [IND * 3 + '}',
-          IND * 2 + '}',
-          IND + '}',
-          IND + '__syncthreads();',
-          '}',
-          '// write back the tile (not the halo); (p, q, r) advanced as in the staging',
-          'const IndexT dt_nbc = dt_nb * dt_nc;',
-          '{',
-          IND + 'const IndexT wp = dt_nthr / dt_nbc, wq = (dt_nthr - wp * dt_nbc) / dt_nc, wr = dt_nthr - wp * dt_nbc - wq * dt_nc;',
-          IND + 'IndexT p = dt_tid / dt_nbc, q = (dt_tid - p * dt_nbc) / dt_nc, r = dt_tid - p * dt_nbc - q * dt_nc;',
-          IND + 'for (IndexT dt_e = dt_tid; dt_e < dt_na * dt_nbc; dt_e += dt_nthr) {',
-          IND * 2 + f'{X}_g[dt_oi + 1 + p][dt_oj + 1 + q][dt_ok + 1 + r] = dt_tile[((p + 1) * dt_R1 + (q + 1)) * dt_R2 + (r + 1)];',
-          IND * 2 + 'r += wr; q += wq; p += wp;',
-          IND * 2 + 'if (r >= dt_nc) { r -= dt_nc; q++; }',
-          IND * 2 + 'if (q >= dt_nb) { q -= dt_nb; p++; }',
-          IND + '}',
-          '}',
-          '__syncthreads();   // the LDS tile is free for the next one']
-    k.append(indent('\n'.join(b) + '\n', 1).rstrip('\n'))
-    k.append('}')
-    redcall = []
-    for red in L.reds:
-        redcall.append(red[1])
-        if len(red) > 3:
-            redcall.append(red[3])
-    # ---- per-loop kernel: one tile-plane per launch
-    kp = list(fp) + ['IndexT dt_TA', 'IndexT dt_TC', 'IndexT dt_ntB', 'IndexT dt_ntC', 'IndexT dt_aLo', 'IndexT dt_tplane']
-    kp += red_kernel_params(L)
-    g = ['template <typename IndexT>',
-         f'__global__ __launch_bounds__(1024) void {L.name}_tile_kernel({", ".join(kp)}) {{']
-    gb = ['const IndexT dt_ta = dt_aLo + (IndexT)blockIdx.x / dt_ntB;',
-          'const IndexT dt_tb = (IndexT)blockIdx.x - ((IndexT)blockIdx.x / dt_ntB) * dt_ntB;',
-          'const IndexT dt_tc = dt_tplane - dt_ta - dt_tb;',
-          'if (dt_tc < 0 || dt_tc >= dt_ntC) return;   // not on this tile-plane (uniform per workgroup)']
-    gb += red_kernel_locals(L)
-    gb.append(f'{L.name}_tile_work<IndexT>({", ".join(call + ["dt_TA", "dt_TC", "dt_ta", "dt_tb", "dt_tc"] + redcall)});')
-    gb += red_kernel_tail(L, '((long)(dt_ta * dt_ntB + dt_tb) * dt_ntC + dt_tc)', accumulate=False)
-    g.append(indent('\n'.join(gb) + '\n', 1).rstrip('\n'))
-    g.append('}')
-    out = '\n'.join(k) + '\n\n' + '\n'.join(g) + '\n'
-    if L.chain_eligible():
-        # ---- chain kernel: sweep s = dt_sLo + blockIdx.y runs tile-plane
-        # dt_launch - dt_lag * s; each sweep folds its reductions into its own
-        # segment of dt_tiles slots, from its own initial value
-        cp = list(fp) + ['IndexT dt_TA', 'IndexT dt_TC', 'IndexT dt_ntA', 'IndexT dt_ntB', 'IndexT dt_ntC',
-                         'IndexT dt_launch', 'IndexT dt_sLo', 'IndexT dt_lag', 'long dt_tiles']
-        for red in L.reds:
-            cp += [f'const {red[2]} *__restrict__ {red[1]}_inits', f'{red[2]} *{red[1]}_grid']
-            if len(red) > 3:
-                cp += [f'const {red[4]} *__restrict__ {red[3]}_inits', f'{red[4]} *{red[3]}_grid']
-        c = ['template <typename IndexT>',
-             f'__global__ __launch_bounds__(1024) void {L.name}_chain_kernel({", ".join(cp)}) {{']
-        cb = ['const IndexT dt_sw = dt_sLo + (IndexT)blockIdx.y;',
-              'const IndexT dt_tplane = dt_launch - dt_lag * dt_sw;',
-              'const IndexT dt_aLo0 = dt_tplane - (dt_ntB - 1) - (dt_ntC - 1);',
-              'const IndexT dt_aLo = dt_aLo0 > 0 ? dt_aLo0 : 0;',
-              'const IndexT dt_aHi = dt_tplane < dt_ntA - 1 ? dt_tplane : dt_ntA - 1;',
-              '// workgroups enumerate (a, j) with j over the shorter of the b and c tile',
-              '// axes; the other follows from a + b + c = tile-plane',
-              'const IndexT dt_nq = dt_ntB < dt_ntC ? dt_ntB : dt_ntC;',
-              'const IndexT dt_ta = dt_aLo + (IndexT)blockIdx.x / dt_nq;',
-              'const IndexT dt_j = (IndexT)blockIdx.x - ((IndexT)blockIdx.x / dt_nq) * dt_nq;',
-              'const IndexT dt_tb = dt_ntB <= dt_ntC ? dt_j : dt_tplane - dt_ta - dt_j;',
-              'const IndexT dt_tc = dt_ntB <= dt_ntC ? dt_tplane - dt_ta - dt_j : dt_j;',
-              '// this sweep has no tile here (before its first or after its last',
-              '// tile-plane, or off the plane): uniform per workgroup',
-              'if (dt_tplane < 0 || dt_ta > dt_aHi || dt_tb < 0 || dt_tb >= dt_ntB || dt_tc < 0 || dt_tc >= dt_ntC) return;']
-        for red in L.reds:
-            cb.append(f'{red[2]} {red[1]} = {red[1]}_inits[dt_sw];')
-            if len(red) > 3:
-                cb.append(f'{red[4]} {red[3]} = {red[3]}_inits[dt_sw];')
-        cb.append(f'{L.name}_tile_work<IndexT>({", ".join(call + ["dt_TA", "dt_TC", "dt_ta", "dt_tb", "dt_tc"] + redcall)});')
-        cb += red_kernel_tail(L, '(long)dt_sw * dt_tiles + ((long)(dt_ta * dt_ntB + dt_tb) * dt_ntC + dt_tc)', accumulate=False)
-        c.append(indent('\n'.join(cb) + '\n', 1).rstrip('\n'))
-        c.append('}')
-        out += '\n' + '\n'.join(c) + '\n'
-    return out
-
-
 def flow_kernel(L):
     """The whole sweep of an ACROSS loop whose axes all depend as one launch
     (dvmh_hip_device.h, dataflow wavefront), and for loops with a chain handler
@@ -2654,16 +2416,16 @@ def flow_kernel(L):
     X = L.across['array']
     r = L.rank
     xct = [p for p in L.arrays if p[1] == X][0][2]
-    fp, setup = [f'dvmh_dev::FlowArgs<{xct}, int, {r}> dvmh_f'], []
+    fp, setup = [f'dvmh_dev::FlowArgs<{xct}, IndexT, {r}> dvmh_f'], []
     for p in L.arrays:
         _, nm, ct, ar = p
         if nm == X:
             continue
         fp.append(f'{ct} *__restrict__ {nm}_base')
-        fp += [f'int {nm}_s{k}' for k in range(ar)]
+        fp += [f'IndexT {nm}_s{k}' for k in range(ar)]
         strides = ', '.join(f'{nm}_s{k}' for k in range(ar))
-        setup.append(f'const int {nm}_str[{ar}] = {{{strides}}};')
-        setup.append(f'const auto {nm} = dvmh_dev::makeView<{ct}, int, {ar}, false>({nm}_base, {nm}_str);')
+        setup.append(f'const IndexT {nm}_str[{ar}] = {{{strides}}};')
+        setup.append(f'const auto {nm} = dvmh_dev::makeView<{ct}, IndexT, {ar}, false>({nm}_base, {nm}_str);')
     for p in L.scalars:
         fp.append(f'{p[2]} *__restrict__ {p[1]}_ptr')
         setup.append(scalar_bind(L.body, p))
@@ -2674,17 +2436,17 @@ def flow_kernel(L):
         body.append(pr + ';')
     for i in range(r):
         body.append(var_assign(L, i, f'dvmh_t{i}', f'dvmh_f.lo[{i}]', '1'))
-    at = ', '.join(f'(int){v}' for v, _ in L.vars)
-    body.append(f'const dvmh_dev::StarView<{xct}, int, {r}> {X}{{dvmh_v, {{{at}}}, 0}};')
+    at = ', '.join(f'(IndexT){v}' for v, _ in L.vars)
+    body.append(f'const dvmh_dev::StarView<{xct}, IndexT, {r}> {X}{{dvmh_v, {{{at}}}, 0}};')
     body.append('{\n' + indent(L.body + '\n', 1) + '}')
 
     def kernel(name, chain, params, init, tail):
-        k = [f'__global__ __launch_bounds__(64) void {name}({", ".join(params)}) {{']
+        k = ['template <typename IndexT>', f'__global__ __launch_bounds__(64) void {name}({", ".join(params)}) {{']
         b = [f'__shared__ {xct} dvmh_ring[dvmh_dev::FlowShape<{r}>::LDS];'] + setup
         b.append('const dvmh_dev::FlowTask dvmh_task = dvmh_dev::flowTake(dvmh_f.ntA, dvmh_f.ntB, dvmh_f.sweeps, dvmh_f.ws);')
         b += init
-        b.append(f'dvmh_dev::flowTile<{xct}, int, {r}, {"true" if chain else "false"}>(dvmh_f, dvmh_task, dvmh_ring, '
-                 f'[&]({xct} *dvmh_v, int dvmh_t0, int dvmh_t1, int dvmh_t2) {{')
+        b.append(f'dvmh_dev::flowTile<{xct}, IndexT, {r}, {"true" if chain else "false"}>(dvmh_f, dvmh_task, dvmh_ring, '
+                 f'[&]({xct} *dvmh_v, IndexT dvmh_t0, IndexT dvmh_t1, IndexT dvmh_t2) {{')
         b += [IND + '(void)dvmh_t2;'] + [IND + ln for ln in '\n'.join(body).split('\n')]
         b.append('});')
         b += tail
@@ -2695,52 +2457,73 @@ def flow_kernel(L):
     tile = '(long)dvmh_task.ta * dvmh_f.ntB + dvmh_task.tb'
     out = kernel(f'{L.name}_flow_kernel', False, fp + red_kernel_params(L) + red_finish_params(L), red_kernel_locals(L),
                  red_kernel_finish(L, tile))
+    if L.chain_eligible():
+        # sweep s folds its reductions into its own segment, from its own initial values
+        cp, init = [], []
+        for red in L.reds:
+            for nm, ct in [(red[1], red[2])] + ([(red[3], red[4])] if len(red) > 3 else []):
+                cp += [f'const {ct} *__restrict__ {nm}_inits', f'{ct} *{nm}_grid']
+                init.append(f'{ct} {nm} = {nm}_inits[dvmh_task.sweep];')
+        out += '\n' + kernel(f'{L.name}_flow_chain_kernel', True, fp + cp, init,
+                             red_kernel_tail(L, f'(long)dvmh_task.sweep * dvmh_f.ntA * dvmh_f.ntB + {tile}', accumulate=False))
     return out
 
 
-def flow_args(L):
-    """Handler lines that set up dvmh_f, and the kernel arguments before the reductions."""
+def flow_check(L, conds, sweeps):
+    """Handler lines: `flow` (the dataflow launch applies: `conds`, unit forward
+    steps, unit stride, room for its workspace dvmh_ws) and its tile counts."""
+    X = L.across['array']
+    r = L.rank
+    xct = [p for p in L.arrays if p[1] == X][0][2]
+    sh = f'dvmh_dev::FlowShape<{r}>'
+    conds = conds + [f'loopSteps[{i}] == 1' for i in range(r)] + [f'{X}_devHdr[{r}] == 1', f'cnt{r - 1} < (1L << 30)',
+                                                                  f'flowTiles * {sweeps} < (1L << 31)']
+    b = [f'DvmType flowA = (cnt0 + {sh}::PA - 1) / {sh}::PA;',
+         f'DvmType flowB = {f"(cnt1 + {sh}::PB - 1) / {sh}::PB" if r == 3 else "1"};',
+         'DvmType flowTiles = flowA * flowB;',
+         'DvmhAmdFlow dvmh_ws;',
+         'bool flow = ' + ' && '.join(conds) + ';',
+         f'if (flow) flow = dvmh_amd_flow_workspace_C(flowTiles * {sweeps}, flowTiles * {r - 1} * dvmh_dev::flowBlocks({r}, cnt{r - 1}) * '
+         '(dvmh_dev::FLOW_CELLS_BYTES / 8), &dvmh_ws) != 0;']
+    return b
+
+
+def flow_launches(L, kernel, sweeps, tail_args):
+    """Handler lines that launch `kernel` for `sweeps` sweeps, by index type."""
     X = L.across['array']
     r = L.rank
     xct = [p for p in L.arrays if p[1] == X][0][2]
     rng = L.stencil_range(X)
-    b = [f'dvmh_dev::FlowArgs<{xct}, int, {r}> dvmh_f;', f'dvmh_f.base = {X};']
-    for a in range(r):
-        b.append(f'dvmh_f.s[{a}] = (int){X}_devHdr[{a + 1}]; dvmh_f.lo[{a}] = (int)boundsLow[{a}]; dvmh_f.cnt[{a}] = (int)cnt{a};')
-        b.append(f'dvmh_f.rlo[{a}] = (int)boundsLow[{a}] + ({rng[a][0]}); dvmh_f.rhi[{a}] = (int)(boundsLow[{a}] + cnt{a} - 1) + ({rng[a][1]});')
-    sh = f'dvmh_dev::FlowShape<{r}>'
-    b.append(f'dvmh_f.ntA = (int)((cnt0 + {sh}::PA - 1) / {sh}::PA);')
-    b.append(f'dvmh_f.ntB = {f"(int)((cnt1 + {sh}::PB - 1) / {sh}::PB)" if r == 3 else "1"};')
-    b.append('DvmType tiles = (DvmType)dvmh_f.ntA * dvmh_f.ntB;')
-    rows = f'({sh}::PA + {sh}::PB)' if r == 3 else f'{sh}::PB'
-    words = f'tiles * {rows} * cnt{r - 1} * dvmh_dev::FlowCell<{xct}>::WORDS'
-    args = ['dvmh_f']
-    for p in L.arrays:
-        if p[1] != X:
-            args += [p[1]] + [f'(int){p[1]}_devHdr[{k + 1}]' for k in range(p[3])]
-    args += [p[1] for p in L.scalars]
-    return b, args, words
+    b = []
+    for it, tag in (('int', 'rt_INT'), ('long long', 'rt_LLONG')):
+        b.append(f'if (kernelIndexT == {tag}) {{')
+        c = [f'dvmh_dev::FlowArgs<{xct}, {it}, {r}> dvmh_f;', f'dvmh_f.base = {X};']
+        for a in range(r):
+            c.append(f'dvmh_f.s[{a}] = ({it}){X}_devHdr[{a + 1}]; dvmh_f.lo[{a}] = ({it})boundsLow[{a}]; dvmh_f.cnt[{a}] = ({it})cnt{a};')
+            c.append(f'dvmh_f.rlo[{a}] = ({it})(boundsLow[{a}] + ({rng[a][0]})); dvmh_f.rhi[{a}] = ({it})(boundsLow[{a}] + cnt{a} - 1 + ({rng[a][1]}));')
+        c += ['dvmh_f.ntA = (int)flowA; dvmh_f.ntB = (int)flowB;', f'dvmh_f.sweeps = (int)({sweeps});', 'dvmh_f.ws = dvmh_ws;']
+        args = ['dvmh_f']
+        for p in L.arrays:
+            if p[1] != X:
+                args += [p[1]] + [f'({it}){p[1]}_devHdr[{k + 1}]' for k in range(p[3])]
+        args += [p[1] for p in L.scalars] + tail_args
+        c.append(f'hipLaunchKernelGGL({kernel}<{it}>, dim3((unsigned)(flowTiles * ({sweeps}))), dim3(64), 0, stream, {", ".join(args)});')
+        b += [IND + ln for ln in c] + ['}']
+    return b
 
 
 def flow_launch(L, otherwise):
     """The dataflow launch where it applies -- unit forward steps, natural
-    layouts, 32-bit indices, room for its workspace -- else `otherwise`.  No
-    size is left to the other kernels: they pay a launch (4-14 us) per
-    hyperplane or tile-plane, this one about 5 us per tile of a diagonal and
-    0.12-0.16 us per step.  One sweep: 2-D 998^2 0.38 against 9.2 ms, 64^2 11
-    against 500 us; 3-D 128^3 0.154 against 0.43 ms, 318^3 0.76 against 1.84."""
-    r = L.rank
-    cond = ['tune[DVMH_AMD_T_VARIANT] == 0', 'kernelIndexT == rt_INT'] + [f'loopSteps[{i}] == 1' for i in range(r)]
-    cond += [f'{p[1]}_tfm == 0' for p in L.arrays] + [f'{L.across["array"]}_devHdr[{r}] == 1']
-    setup, args, words = flow_args(L)
-    b = ['bool flow = ' + ' && '.join(cond) + ';'] + setup
-    b.append(f'if (flow) flow = dvmh_amd_flow_workspace_C(tiles, {words}, &dvmh_f.ws) != 0;')
+    layouts, room for its workspace -- else `otherwise`.  No size is left to
+    the other kernels: they pay a launch (4-14 us) per hyperplane or
+    tile-plane, this one about 5 us per tile of a diagonal and 0.13-0.17 us per
+    step.  One sweep: 2-D 998^2 0.38 against 9.2 ms; 3-D 128^3 0.145 against
+    0.43 ms, 318^3 0.48 against 1.84."""
+    b = flow_check(L, [f'{p[1]}_tfm == 0' for p in L.arrays], '1')
     b.append('if (flow) {')
-    b.append(IND + 'dvmh_f.sweeps = 1;')
-    b += [IND + ln for ln in handler_reds_prepare(L, 'tiles', 0) + red_finish_query(L, 'tiles')]
+    b += [IND + ln for ln in handler_reds_prepare(L, 'flowTiles', 0) + red_finish_query(L, 'flowTiles')]
     b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 0);')
-    b.append(IND + f'hipLaunchKernelGGL({L.name}_flow_kernel, dim3((unsigned)tiles), dim3(64), 0, stream, '
-             f'{", ".join(args + red_fact_args(L) + red_finish_args(L))});')
+    b += [IND + ln for ln in flow_launches(L, f'{L.name}_flow_kernel', '1', red_fact_args(L) + red_finish_args(L))]
     b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 1);')
     b += [IND + ln for ln in handler_reds_finish(L)]
     b.append('} else {')
@@ -3207,71 +2990,37 @@ def line_vec_launch(L):
     return b
 
 
-def tile_launch(L):
-    X = L.across['array']
-    xct = [p for p in L.arrays if p[1] == X][0][2]
-    b = ['DvmType TA = tune[DVMH_AMD_T_TILE_A], TC = tune[DVMH_AMD_T_TILE_B];',
-         'DvmType ntA = (cnt0 + TA - 1) / TA, ntB = (cnt1 + TA - 1) / TA, ntC = (cnt2 + TC - 1) / TC;',
-         f'size_t ldsBytes = (size_t)(TA + 2) * (TA + 2) * (TC + 2) * sizeof({xct});',
-         'DvmType tiles = ntA * ntB * ntC;']
-    b += handler_reds_prepare(L, 'tiles', 0)
-    b.append('dvmh_amd_mark_kernel_C(loop_ref, 0);')
-    b.append('for (DvmType tplane = 0; tplane <= (ntA - 1) + (ntB - 1) + (ntC - 1); tplane++) {')
-    b.append(IND + 'DvmType aLo = tplane - (ntB - 1) - (ntC - 1);')
-    b.append(IND + 'if (aLo < 0) aLo = 0;')
-    b.append(IND + 'DvmType aHi = tplane < ntA - 1 ? tplane : ntA - 1;')
-    b.append(IND + 'DvmType grid = (aHi - aLo + 1) * ntB;')
-    for it in ['int', 'long long']:
-        args = array_fact_args(L, it)
-        for i in range(3):
-            args += [f'({it})boundsLow[{i}]', f'({it})cnt{i}', f'({it})loopSteps[{i}]']
-        args += [f'({it})TA', f'({it})TC', f'({it})ntB', f'({it})ntC', f'({it})aLo', f'({it})tplane']
-        args += red_fact_args(L)
-        cond = f'kernelIndexT == {"rt_INT" if it == "int" else "rt_LLONG"}'
-        b.append(IND + f'if ({cond}) hipLaunchKernelGGL(({L.name}_tile_kernel<{it}>), dim3((unsigned)grid), threads, ldsBytes, '
-                 f'stream, {", ".join(args)});')
-    b.append('}')
-    b.append('dvmh_amd_mark_kernel_C(loop_ref, 1);')
-    b += handler_reds_finish(L)
-    return b
-
-
-# Tile-planes by which a sweep of a chain trails the sweep before it: tile
-# (a, b, c) reads only the tiles one tile-plane below and above it (every
-# access of the ACROSS array moves along one axis by at most one), so sweep s
-# may run tile-plane p once sweep s - 1 has finished tile-plane p + 1; with a
-# lag of two, the tiles two sweeps run in one launch are never neighbours.
-CHAIN_LAG = 2
+# Sweeps per dataflow launch of a chain: a wave finds its task by walking the
+# diagonals of every sweep of the launch.
+CHAIN_SWEEPS = 64
 
 
 def chain_handler(L):
-    """Chain handler of a tiled-wavefront ACROSS loop: the group of
-    consecutive sweeps dvmh_amd_batch_end_C hands over runs as one launch
-    sequence, sweep s CHAIN_LAG tile-planes behind sweep s - 1, each sweep with
-    its own reduction segment.  Sweeps that differ in bounds, arrays, scalars
-    or layout, or a configuration other than the tiled wavefront, run one
-    after another through the ordinary handler."""
+    """Chain handler of an ACROSS loop whose axes all depend: the group of
+    consecutive sweeps dvmh_amd_batch_end_C hands over runs as one dataflow
+    launch, a tile of a sweep as soon as the tiles it reads are far enough in
+    the sweep before it, each sweep with its own reduction segment.  Sweeps that
+    differ in bounds, arrays, scalars or layout run one after another through
+    the ordinary handler.  Measured per sweep (chains of 10 and 30), against a
+    launch per tile-plane of all sweeps: 64^3 53 and 45 us (68, 54), 128^3 73
+    and 56 (101, 77), 318^3 262 and 239 (389, 313)."""
     X = L.across['array']
-    xct = [p for p in L.arrays if p[1] == X][0][2]
     h = [f'extern "C" void {L.name}_cuda_chain(DvmType *pBatchRef) {{']
     b = ['DvmType batchRef = *pBatchRef;',
          'long nl = (long)dvmh_amd_batch_count_C(batchRef);',
          'DvmType loop_ref = dvmh_amd_batch_loop_C(batchRef, 0);',
          'DvmType tune[DVMH_AMD_TUNE_N];',
-         '// the chain has its own tuner site: tile shapes timed per sweep of a chain',
+         '// (the chain has its own site; the launch does not depend on what is chosen)',
          'dvmh_amd_loop_get_tuning_C(loop_ref, DVMH_AMD_KIND_CHAIN, tune);',
          'dim3 threads(0, 0, 0);',
          'hipStream_t stream;',
-         *regs_query(f'{L.name}_chain_kernel<int>'),
+         *regs_query(f'{L.name}_flow_chain_kernel<int>'),
          'DvmType dependency_mask = dvmh_loop_get_dependency_mask_C(loop_ref);',
          'int kernelIndexT = (int)dvmh_loop_guess_index_type_C(loop_ref);',
          'if (kernelIndexT == rt_LONG) kernelIndexT = rt_LLONG;',
          'DvmType boundsLow[3], boundsHigh[3], loopSteps[3];',
          'dvmh_loop_fill_bounds_C(loop_ref, boundsLow, boundsHigh, loopSteps);',
-         'DvmType TA = tune[DVMH_AMD_T_TILE_A], TC = tune[DVMH_AMD_T_TILE_B];',
-         f'size_t ldsBytes = (size_t)(TA + 2) * (TA + 2) * (TC + 2) * sizeof({xct});',
-         'bool chained = tune[DVMH_AMD_T_VARIANT] == 1 && dependency_mask == 7 && TA >= 2 && TC >= 2 && ldsBytes <= 64512 && '
-         'threads.y == 1 && threads.z == 1 && loopSteps[0] == 1 && loopSteps[1] == 1 && loopSteps[2] == 1;']
+         'bool chained = dependency_mask == 7;']
     for pi, p in enumerate(L.params):
         if p[0] == 'array':
             _, nm, ct, ar = p
@@ -3290,7 +3039,10 @@ def chain_handler(L):
     for pi, p in enumerate(L.params):
         b.append(IND + f'if (dvmh_amd_batch_param_C(batchRef, li, {pi}) != dvmh_amd_batch_param_C(batchRef, 0, {pi})) chained = false;')
     b.append('}')
-    b.append('if (!chained) {')
+    b += [f'DvmType cnt{a} = (boundsHigh[{a}] - boundsLow[{a}]) / loopSteps[{a}] + 1;' for a in range(3)]
+    b.append(f'const long most = nl < {CHAIN_SWEEPS} ? nl : {CHAIN_SWEEPS};   // sweeps per launch')
+    b += flow_check(L, ['chained'], 'most')
+    b.append('if (!flow) {')
     b.append(IND + '// one sweep after another through the ordinary handler')
     b.append(IND + 'for (long li = 0; li < nl; li++) {')
     b.append(IND * 2 + 'DvmType lr = dvmh_amd_batch_loop_C(batchRef, li);')
@@ -3302,20 +3054,17 @@ def chain_handler(L):
     b.append(IND + '}')
     b.append(IND + 'return;')
     b.append('}')
-    b += ['DvmType cnt0 = boundsHigh[0] - boundsLow[0] + 1, cnt1 = boundsHigh[1] - boundsLow[1] + 1, cnt2 = boundsHigh[2] - boundsLow[2] + 1;',
-          'DvmType ntA = (cnt0 + TA - 1) / TA, ntB = (cnt1 + TA - 1) / TA, ntC = (cnt2 + TC - 1) / TC;',
-          'DvmType tiles = ntA * ntB * ntC, planes = ntA + ntB + ntC - 2;',
-          'DvmType *segStart = (DvmType *)malloc((size_t)(nl + 1) * sizeof(DvmType));',
-          'for (long li = 0; li <= nl; li++) segStart[li] = li * tiles;']
+    b += ['DvmType *segStart = (DvmType *)malloc((size_t)(nl + 1) * sizeof(DvmType));',
+          'for (long li = 0; li <= nl; li++) segStart[li] = li * flowTiles;']
     ra = []
     for ri, red in enumerate(L.reds):
         ct = red[2]
-        b.append(f'{ct} *{red[1]}_grid = ({ct} *)dvmh_amd_batch_scratch_C(batchRef, nl * tiles * (long)sizeof({ct}));')
+        b.append(f'{ct} *{red[1]}_grid = ({ct} *)dvmh_amd_batch_scratch_C(batchRef, nl * flowTiles * (long)sizeof({ct}));')
         b.append(f'{ct} *{red[1]}_inits = ({ct} *)dvmh_amd_batch_scratch_C(batchRef, nl * (long)sizeof({ct}));')
         b.append(f'{ct} *{red[1]}_ih = ({ct} *)malloc((size_t)nl * sizeof({ct}));')
         if len(red) > 3:
             lt = red[4]
-            b.append(f'{lt} *{red[3]}_grid = ({lt} *)dvmh_amd_batch_scratch_C(batchRef, nl * tiles * (long)sizeof({lt}));')
+            b.append(f'{lt} *{red[3]}_grid = ({lt} *)dvmh_amd_batch_scratch_C(batchRef, nl * flowTiles * (long)sizeof({lt}));')
             b.append(f'{lt} *{red[3]}_inits = ({lt} *)dvmh_amd_batch_scratch_C(batchRef, nl * (long)sizeof({lt}));')
             b.append(f'{lt} *{red[3]}_ih = ({lt} *)malloc((size_t)nl * sizeof({lt}));')
             b.append(f'for (long li = 0; li < nl; li++) dvmh_loop_red_init_C(dvmh_amd_batch_loop_C(batchRef, li), {ri + 1}, &{red[1]}_ih[li], &{red[3]}_ih[li]);')
@@ -3323,31 +3072,12 @@ def chain_handler(L):
         else:
             b.append(f'for (long li = 0; li < nl; li++) dvmh_loop_red_init_C(dvmh_amd_batch_loop_C(batchRef, li), {ri + 1}, &{red[1]}_ih[li], 0);')
         b.append(f'dvmh_amd_batch_upload_C(batchRef, {red[1]}_inits, {red[1]}_ih, nl * (long)sizeof({ct}));')
-        ra += [f'{red[1]}_inits', f'{red[1]}_grid']
-        if len(red) > 3:
-            ra += [f'{red[3]}_inits', f'{red[3]}_grid']
-    b += [f'const DvmType lag = {CHAIN_LAG};',
-          'dvmh_amd_mark_kernel_C(loop_ref, 0);',
-          'for (DvmType t = 0; t < planes + lag * (nl - 1); t++) {',
-          IND + '// sweeps with a tile-plane in this launch: 0 <= t - lag * s < planes',
-          IND + 'DvmType sLo = t - (planes - 1) <= 0 ? 0 : (t - (planes - 1) + lag - 1) / lag;',
-          IND + 'DvmType sHi = t / lag < nl - 1 ? t / lag : nl - 1;',
-          IND + 'if (sLo > sHi) continue;',
-          IND + 'DvmType rows = 0;',
-          IND + 'for (DvmType sw = sLo; sw <= sHi; sw++) {',
-          IND * 2 + 'DvmType p = t - lag * sw, aLo = p - (ntB - 1) - (ntC - 1), aHi = p < ntA - 1 ? p : ntA - 1;',
-          IND * 2 + 'if (aLo < 0) aLo = 0;',
-          IND * 2 + 'if (aHi - aLo + 1 > rows) rows = aHi - aLo + 1;',
-          IND + '}',
-          IND + 'dim3 grid((unsigned)(rows * (ntB < ntC ? ntB : ntC)), (unsigned)(sHi - sLo + 1), 1);']
-    for it in ['int', 'long long']:
-        args = array_fact_args(L, it)
-        for i in range(3):
-            args += [f'({it})boundsLow[{i}]', f'({it})cnt{i}', f'({it})loopSteps[{i}]']
-        args += [f'({it})TA', f'({it})TC', f'({it})ntA', f'({it})ntB', f'({it})ntC', f'({it})t', f'({it})sLo', f'({it})lag',
-                 '(long)tiles'] + ra
-        cond = f'kernelIndexT == {"rt_INT" if it == "int" else "rt_LLONG"}'
-        b.append(IND + f'if ({cond}) hipLaunchKernelGGL(({L.name}_chain_kernel<{it}>), grid, threads, ldsBytes, stream, {", ".join(args)});')
+        for nm in [red[1]] + ([red[3]] if len(red) > 3 else []):
+            ra += [f'{nm}_inits + done', f'{nm}_grid + done * flowTiles']
+    b.append('dvmh_amd_mark_kernel_C(loop_ref, 0);')
+    b.append('for (long done = 0; done < nl; done += most) {')
+    b.append(IND + 'const long sweeps = nl - done < most ? nl - done : most;')
+    b += [IND + ln for ln in flow_launches(L, f'{L.name}_flow_chain_kernel', 'sweeps', ra)]
     b.append('}')
     b.append('dvmh_amd_mark_kernel_C(loop_ref, 1);')
     for ri, red in enumerate(L.reds):
@@ -3437,21 +3167,7 @@ def across_handler(L):
             rest = wave_launch(L, list(deps))
             if m == r and L.flow_eligible():
                 rest = flow_launch(L, rest)
-            if m == 3 and L.tile_eligible():
-                X = L.across['array']
-                xct = [p for p in L.arrays if p[1] == X][0][2]
-                unit = ' && '.join(f'loopSteps[{i}] == 1' for i in range(3))
-                b.append(IND + '// tiled variant: unit forward steps, natural layout, tile fits 64 KB of LDS')
-                b.append(IND + f'bool tiled = tune[DVMH_AMD_T_VARIANT] == 1 && {unit} && {X}_tfm == 0 && threads.y == 1 && '
-                         'threads.z == 1 && tune[DVMH_AMD_T_TILE_A] >= 2 && tune[DVMH_AMD_T_TILE_B] >= 2 && '
-                         f'(tune[DVMH_AMD_T_TILE_A] + 2) * (tune[DVMH_AMD_T_TILE_A] + 2) * (tune[DVMH_AMD_T_TILE_B] + 2) * (DvmType)sizeof({xct}) <= 64512;')
-                b.append(IND + 'if (tiled) {')
-                b += [IND * 2 + s for s in tile_launch(L)]
-                b.append(IND + '} else {')
-                b += [IND * 2 + s for s in rest]
-                b.append(IND + '}')
-            else:
-                b += [IND + s for s in rest]
+            b += [IND + s for s in rest]
     b.append('} else {')
     b.append(IND + f'fprintf(stderr, "{L.name}: unsupported dependency mask %ld\\n", (long)dependency_mask);')
     b.append(IND + 'abort();')
@@ -3512,8 +3228,6 @@ def gpu_loop(L):
                 text.append(wave_kernel(L, list(deps)))
         if L.flow_eligible():
             text.append(flow_kernel(L))
-        if L.tile_eligible():
-            text.append(tile_kernel(L))
         if L.line_tile_eligible():
             text.append(line_tile_kernel(L))
             text.append(line_vec_kernel(L))

@@ -29,12 +29,14 @@ extern "C" {
                                       VARIANT 3, dependent axis innermost and unit stride:
                                       a wave streams 64 lines in aligned 128-byte chunks,
                                       coalesced, transposed through LDS, a lane per line) */
-#define DVMH_AMD_KIND_WAVEFRONT 2  /* ACROSS with >= 2 dependent axes: hyperplane wavefront */
+#define DVMH_AMD_KIND_WAVEFRONT 2  /* ACROSS with >= 2 dependent axes: hyperplane wavefront; a loop whose axes all
+                                      depend runs as one dataflow launch whatever the tiles asked for */
 #define DVMH_AMD_KIND_STENCIL 3    /* PARALLEL whose handler also has the LDS march variant
                                       (VARIANT 1: TILE_A = points per thread on the innermost
                                       axis, CHUNK = planes per workgroup on the outermost) */
 #define DVMH_AMD_KIND_BATCH 4      /* PARALLEL loops of many instances run by one batch kernel */
-#define DVMH_AMD_KIND_CHAIN 5      /* consecutive sweeps of a tiled-wavefront ACROSS loop run by its chain handler */
+#define DVMH_AMD_KIND_CHAIN 5      /* consecutive sweeps of an ACROSS loop run by its chain handler (one dataflow
+                                      launch: a single configuration) */
 #define DVMH_AMD_KIND_PAIR 6       /* a stencil loop and the loop after it run fused by their pair handler
                                       (VARIANT 1, TILE_A and CHUNK as for STENCIL) */
 /* tune[] slots */

@@ -7,12 +7,15 @@
  *   DiagView   the same for a layout whose two fastest storage axes are
  *              diagonalised (planes stored anti-diagonal by anti-diagonal), the
  *              index map of rts/dvmh/include/dvmhlib_device.h:56-98.
- *   MarchView2/3, TileView3, LineView
+ *   MarchView2/3, LineView
  *              the same syntax over copies staged in LDS: a rolling window of
  *              three planes of a read-only stencil array (march variant of
- *              PARALLEL loops), a tile with halo of an ACROSS array (tiled
- *              wavefront), and a chunk of one line of an ACROSS array (tiled
- *              line sweep along the innermost axis).
+ *              PARALLEL loops) and a chunk of one line of an ACROSS array
+ *              (tiled line sweep along the innermost axis).
+ *   StarView, flowTile
+ *              the same syntax over a point and its neighbours in registers,
+ *              and the dataflow wavefront that walks them (ACROSS loops whose
+ *              axes all depend).
  *   reductions wave64 shuffle trees plus one LDS step across the waves of a
  *              workgroup; every thread of the workgroup must call them.
  *   xcdTile    XCD-aware renumbering of workgroups: the hardware deals
@@ -136,31 +139,6 @@ struct MarchView2 {
     int sCur;
     __device__ __forceinline__ MarchRow<T, I> operator[](I i) const {
         return MarchRow<T, I>{lds + (I)marchSlot(sCur, (int)(i - iCur)) * cols, k0};
-    }
-};
-
-// A tile of a rank-3 array staged in LDS (read and written): element (0,0,0)
-// holds array index (i0, j0, k0), planes of rows x cols elements.
-template <typename T, typename I>
-struct TileRow {
-    T *p;
-    I k0;
-    __device__ __forceinline__ T &operator[](I k) const { return p[k - k0]; }
-};
-
-template <typename T, typename I>
-struct TilePlane {
-    T *p;
-    I cols, j0, k0;
-    __device__ __forceinline__ TileRow<T, I> operator[](I j) const { return TileRow<T, I>{p + (j - j0) * cols, k0}; }
-};
-
-template <typename T, typename I>
-struct TileView3 {
-    T *p;
-    I rows, cols, i0, j0, k0;
-    __device__ __forceinline__ TilePlane<T, I> operator[](I i) const {
-        return TilePlane<T, I>{p + (i - i0) * rows * cols, cols, j0, k0};
     }
 };
 
@@ -553,20 +531,23 @@ __device__ __forceinline__ void publishDone(const DvmhAmdRedFinish &f) {
 //
 // The rows of a tile pass through LDS in blocks of eight steps, three of them
 // at a time.  A row is held at the step its elements are walked at (element r
-// of row (p, q) in slot r + p + q), so in every step all lanes use the same
-// slots, at offsets known to the compiler, and a finished block of steps is
-// stored at once.  A block's loads and stores move 64 bytes of eight rows per
-// instruction; two blocks' loads are in flight while one is walked.  Rows a
-// tile needs from its lower neighbours come through cells in device memory: a
-// value in halves, each in an 8-byte word with a 32-bit tag that no earlier
-// launch used, so one load tells whether it is there.
+// of row (p, q) in slot r + p + q and the tile's phase), so in every step all
+// lanes use the same slots, at offsets known to the compiler, and a finished
+// block of steps is stored at once.  A block's loads and stores move eight
+// aligned elements of eight rows per instruction; two blocks' loads are in
+// flight while one is walked.  Rows a tile needs from its lower neighbours come
+// through cells in device memory, 1 KB per face and block of steps, written and
+// read by one instruction: a value in halves, each beside a 32-bit tag that no
+// earlier launch used, so one load tells whether it is there.
 //
-// Bound by the chain of dependent steps: 0.12 us a step for rank 2 (eight
-// dependent FP64 operations and a lane shift), 0.155 for rank 3 (one neighbour
+// Bound by the chain of dependent steps: 0.13 us a step for rank 2 (eight
+// dependent FP64 operations and a lane shift), 0.165 for rank 3 (one neighbour
 // through LDS), and along a diagonal of tiles, per tile, the lanes' skew plus
-// about 4 us until a finished block is seen by the next tile.  Measured, one
-// sweep with reductions: 2-D 998^2 0.38 ms (a launch per hyperplane: 9.2), 3-D
-// 128^3 0.154 ms (a launch per tile-plane: 0.43), 318^3 0.76 ms (1.84).
+// about 4 us until a finished block is seen by the next tile; chains of large
+// grids by memory traffic (26 bytes a point and sweep, 3.5 TB/s).  Measured,
+// one sweep with reductions: 2-D 998^2 0.38 ms (a launch per hyperplane: 9.2),
+// 3-D 128^3 0.145 ms (a launch per tile-plane: 0.43), 318^3 0.48 ms (1.84; 0.76
+// with rows moved unaligned and a cell's halves in two stores).
 template <int RANK> struct FlowShape;
 template <> struct FlowShape<3> {
     // row (p, q), -1 <= p, q <= 8, at (p + 1) * BP + (q + 1) * QP: the 32 lanes
@@ -671,35 +652,38 @@ __device__ __forceinline__ FlowTask flowTake(int ntA, int ntB, int sweeps, const
                     epoch + (unsigned)s + 1};
 }
 
-// A cell: the value's bytes in 32-bit parts, each beside the tag.
+// Cells: 64 values a lane each, the value's halves each beside the tag, moved
+// by one 16-byte access per lane at agent scope (each 8-byte word is written
+// whole; a reader checks both tags).
+typedef unsigned FlowWords __attribute__((ext_vector_type(4)));
+constexpr int FLOW_CELLS_BYTES = 64 * 16;
+
 template <typename T>
-struct FlowCell {
-    static constexpr int WORDS = sizeof(T) > 4 ? 2 : 1;
-    unsigned long long w[WORDS];
-    __device__ __forceinline__ void load(const unsigned long long *p) {
-#pragma unroll
-        for (int i = 0; i < WORDS; i++) w[i] = __hip_atomic_load(p + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+struct FlowCells {
+    FlowWords w;
+    static __device__ __forceinline__ __amdgpu_buffer_rsrc_t at(const void *p, unsigned bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00027000);
     }
-    __device__ __forceinline__ bool holds(unsigned tag) const {
-        bool h = true;
-#pragma unroll
-        for (int i = 0; i < WORDS; i++) h &= (unsigned)(w[i] >> 32) == tag;
-        return h;
+    static constexpr int AGENT = 16;   // cache policy: agent scope (sc1)
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t from, int offset) {
+        w = __builtin_amdgcn_raw_buffer_load_b128(from, threadIdx.x * 16, offset, AGENT);
     }
+    __device__ __forceinline__ bool holds(unsigned tag) const { return (w[1] == tag) & (w[3] == tag); }
     __device__ __forceinline__ T value() const {
-        unsigned x[2] = {(unsigned)w[0], (unsigned)w[WORDS - 1]};
+        const unsigned x[2] = {w[0], w[2]};
         T v;
         __builtin_memcpy(&v, x, sizeof(T));
         return v;
     }
-    static __device__ __forceinline__ void store(unsigned long long *p, T v, unsigned tag) {
+    static __device__ __forceinline__ void store(__amdgpu_buffer_rsrc_t to, int offset, T v, unsigned tag) {
         unsigned x[2] = {0, 0};
         __builtin_memcpy(x, &v, sizeof(T));
-#pragma unroll
-        for (int i = 0; i < WORDS; i++)
-            __hip_atomic_store(p + i, (unsigned long long)tag << 32 | x[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_raw_buffer_store_b128(FlowWords{x[0], tag, x[1], tag}, to, threadIdx.x * 16, offset, AGENT);
     }
 };
+
+// Blocks of a face's cells: one per block of steps of the tile, at most this many.
+__host__ __device__ inline long flowBlocks(int rank, long n) { return (n + (rank == 3 ? 14 : 63) + 7 + 7) >> 3; }
 
 // Lane l gets lane l - 1's x, lane 0 gets `first` (whole wave active).
 template <typename T>
@@ -723,19 +707,22 @@ __device__ __forceinline__ void readHere(T &x) { asm volatile("" : "+v"(x)); }
 // (t0, t1, t2) of the loop (t2 unused for rank 2) with v the star around it.
 // CHAIN: several sweeps of the array in one launch; its elements then pass
 // between workgroups, so they are loaded and stored at agent scope, and a
-// tile's flag says how many blocks of which sweep are in memory.
+// tile's flag says how many chunks of which sweep are in memory.
 template <typename T, typename I, int RANK, bool CHAIN, typename Body>
 __device__ __forceinline__ void flowTile(const FlowArgs<T, I, RANK> &f, const FlowTask &task, T *ring, Body &&body) {
     using S = FlowShape<RANK>;
     constexpr int K = RANK - 1, SKEW = S::PA + S::PB - 2, SLOTS = 24;
-    const int lane = threadIdx.x, g = lane >> 3, e = lane & 7;   // block transfers: eight rows of eight elements
+    const int lane = threadIdx.x, g = lane >> 3, e = lane & 7;   // transfers: eight rows of eight elements
     const int p = RANK == 3 ? g : lane, q = RANK == 3 ? e : 0;   // the lane's own row
     const int ta = task.ta, tb = task.tb;
     const I a0 = (I)ta * S::PA, b0 = (I)tb * S::PB;
     const int na = f.cnt[0] - a0 < S::PA ? (int)(f.cnt[0] - a0) : S::PA;
     const int nb = RANK == 2 ? 1 : (f.cnt[1] - b0 < S::PB ? (int)(f.cnt[1] - b0) : S::PB);
     const int n = (int)f.cnt[K];
-    const int blocks = (n + na + nb - 2 + 7) >> 3;   // blocks of steps
+    // a tile begins up to seven steps late, so that what the next tile needs
+    // in a block of steps is what this one does in a block
+    const int phase = -(ta + tb) & 7;
+    const int blocks = (n + na + nb - 2 + phase + 7) >> 3;   // blocks of steps
     auto clampTo = [](I x, I lo, I hi) { return x < lo ? lo : (x > hi ? hi : x); };
     auto rowOff = [&](int pp, int qq) -> I {
         I o = clampTo(f.lo[0] + a0 + pp, f.rlo[0], f.rhi[0]) * f.s[0];
@@ -743,75 +730,77 @@ __device__ __forceinline__ void flowTile(const FlowArgs<T, I, RANK> &f, const Fl
         return o;
     };
     auto rowAt = [](int pp, int qq) { return (pp + 1) * S::BP + (qq + 1) * S::QP; };
-    // the row a lane moves in transfer `it` of a block
-    auto rowP = [&](int it) { return RANK == 3 ? it : it * 8 + g; };
-    auto rowQ = [&](int) { return RANK == 3 ? g : 0; };
-    // rows moved block by block: the tile's 64, the ones above it and, at the
-    // array's lower edges, the ones below it (elsewhere those come in cells)
+    // Rows a lane moves: transfer it < 8 the tile's own, 8 and 9 the ones above
+    // it, 10 and 11 the ones below (at the array's lower edges; elsewhere those
+    // come in cells).  Row (pp, qq) holds element r in slot r + pp + qq + phase.
+    auto rowP = [&](int it) { return RANK == 2 ? (it < 8 ? it * 8 + g : it == 8 ? S::PA : -1) : it < 8 ? it : it == 8 ? S::PA : it == 10 ? -1 : g; };
+    auto rowQ = [&](int it) { return RANK == 2 ? 0 : it == 9 ? S::PB : it == 11 ? -1 : g; };
     const bool edgeA = ta == 0, edgeB = RANK == 3 && tb == 0;
-    I off[8];
+    auto uses = [&](int it) { return RANK == 3 || it < 9 || it == 10 ? it < 10 || (it == 10 ? edgeA : edgeB) : false; };
+    // A transfer moves eight elements of a row that are aligned in memory (64
+    // bytes of FP64): slots 8 c - 8 + ahead .. + 7 for chunk c, where `ahead`,
+    // 0 .. 7, is the row's own
+    I off[12];      // element index of slot 0
+    int ahead[12];  // plus the lane's element of the chunk
+    auto eachRow = [&](auto &&fn) {
 #pragma unroll
-    for (int it = 0; it < 8; it++) off[it] = rowOff(rowP(it), rowQ(it));
-    const I offA = rowOff(S::PA, g), offB = RANK == 3 ? rowOff(g, S::PB) : 0;
-    const I offLA = rowOff(-1, g), offLB = RANK == 3 ? rowOff(g, -1) : 0;
-    const int gq = RANK == 3 ? g : 0;   // second coordinate of a face row of the first axis
-    // two blocks' loads are in flight while a block is walked (a block of steps
+        for (int it = 0; it < 12; it++)
+            if (RANK == 3 || it < 9 || it == 10) fn(it);
+    };
+    eachRow([&](int it) {
+        off[it] = rowOff(rowP(it), rowQ(it)) + f.lo[K] - (I)(rowP(it) + rowQ(it) + phase);
+        ahead[it] = (int)(-(long)((uintptr_t)f.base / sizeof(T) + off[it]) & 7) + e;
+    });
+    // slot of the ring that a lane's element of chunk c is in
+    auto slotOf = [&](int it, int c8) {
+        const unsigned x = (unsigned)(c8 + ahead[it]);
+        return x < x - SLOTS ? x : x - SLOTS;   // c8 < 24: at most one turn
+    };
+    auto chunk8 = [](int c) { return (unsigned)(c + 2) % 3u * 8u; };   // 8 c - 8, in the ring
+    // two chunks' loads are in flight while a block is walked (a block of steps
     // takes less than a round trip to memory), in two sets of registers
     struct Ahead {
-        T own[8], vA, vB, vLA, vLB;
+        T v[12];
     } even{}, odd{};
-    // (issued on every path, past the row's end from its last element, so that
-    // the waits know how many younger loads may stay in flight)
-    auto issue = [&](Ahead &h, int b) {
-        const I k = f.lo[K] + 8 * b + e;
-        auto ld = [&](I o, int skew) -> T {
-            const T *x = f.base + (o + clampTo(k - skew, f.rlo[K], f.rhi[K]));
-            return CHAIN ? agentLoad(x) : *x;
-        };
-#pragma unroll
-        for (int it = 0; it < 8; it++) h.own[it] = ld(off[it], rowP(it) + rowQ(it));
-        h.vA = ld(offA, S::PA + gq);
-        if constexpr (RANK == 3) h.vB = ld(offB, g + S::PB);
-        if (edgeA) h.vLA = ld(offLA, gq - 1);
-        if constexpr (RANK == 3) if (edgeB) h.vLB = ld(offLB, g - 1);
+    // (issued on every path, past the row's ends from its nearest element, so
+    // that the waits know how many younger loads may stay in flight)
+    auto issue = [&](Ahead &h, int c) {
+        eachRow([&](int it) {
+            if (uses(it)) {
+                const I first = off[it] + (I)(rowP(it) + rowQ(it) + phase) - f.lo[K];
+                const T *x = f.base + (first + clampTo(off[it] - first + 8 * c - 8 + ahead[it], f.rlo[K], f.rhi[K]));
+                h.v[it] = CHAIN ? agentLoad(x) : *x;
+            }
+        });
     };
-    auto commit = [&](const Ahead &h, int b) {
-        T *to = ring + (b % 3) * 8 + e;
-#pragma unroll
-        for (int it = 0; it < 8; it++) to[rowAt(rowP(it), rowQ(it))] = h.own[it];
-        if constexpr (RANK == 3) {
-            to[rowAt(S::PA, g)] = h.vA;
-            to[rowAt(g, S::PB)] = h.vB;
-            if (edgeA) to[rowAt(-1, g)] = h.vLA;
-            if (edgeB) to[rowAt(g, -1)] = h.vLB;
-        } else if (g == 0) {
-            to[rowAt(S::PA, 0)] = h.vA;
-            if (edgeA) to[rowAt(-1, 0)] = h.vLA;
-        }
+    auto commit = [&](const Ahead &h, int c) {
+        const int c8 = chunk8(c);
+        eachRow([&](int it) {
+            if (uses(it) && (RANK == 3 || it < 8 || g == 0)) ring[rowAt(rowP(it), rowQ(it)) + slotOf(it, c8)] = h.v[it];
+        });
     };
-    // cells of a tile's upper faces: PB rows of n towards ta + 1, PA rows towards tb + 1
-    constexpr int W = FlowCell<T>::WORDS;
-    const long tiles = (long)f.ntA * f.ntB, tile = (long)ta * f.ntB + tb;
-    unsigned long long *const cellsA = f.ws.cells, *const cellsB = f.ws.cells + tiles * S::PB * n * W;
+    // cells of a tile's upper faces, 64 per block of steps: lane (g, e) holds what
+    // row g of the face did at step e
+    const long tile = (long)ta * f.ntB + tb;
+    const unsigned faceBytes = (unsigned)flowBlocks(RANK, n) * FLOW_CELLS_BYTES;
+    char *const cells = (char *)f.ws.cells;
+    auto face = [&](long t, int which) { return FlowCells<T>::at(cells + (t * (RANK - 1) + which) * (long)faceBytes, faceBytes); };
     const bool fromA = ta > 0, fromB = RANK == 3 && tb > 0;
     const bool toA = ta + 1 < f.ntA, toB = RANK == 3 && tb + 1 < f.ntB;
-    // lane (g, e) fetches element 8 m + e - g of face row g: what lane (0, g)
-    // (or (g, 0)) needs at step e of block m
-    const bool rowA = fromA && g < nb, rowB = fromB && g < na;
+    const auto inA = face(fromA ? tile - f.ntB : tile, 0), outA = face(tile, 0);
+    const auto inB = face(fromB ? tile - 1 : tile, RANK - 2), outB = face(tile, RANK - 2);
+    const bool rowA = fromA && (RANK == 3 ? g < nb : g == 0), rowB = fromB && g < na;
     auto inRow = [&](int r) { return (unsigned)r < (unsigned)n; };
-    auto cellOf = [&](unsigned long long *c, long t, int rows, int r) { return c + ((t * rows + g) * n + r) * W; };
-    unsigned long long *const inA = cellOf(cellsA, tile - f.ntB, S::PB, 0), *const inB = cellOf(cellsB, tile - 1, S::PA, 0);
-    unsigned long long *const outA = cellOf(cellsA, tile, S::PB, 0), *const outB = cellOf(cellsB, tile, S::PA, 0);
-    // (every lane loads something, some the first cell in vain: a load in a
-    // branch would have to be waited for at the branch's end)
-    FlowCell<T> cA{}, cB{};
+    // block m needs the neighbour's block m + lag (one less where its phase is 0): the
+    // element lane (0, g) or (g, 0) runs above at step e, 8 m + e - g - phase
+    const int lag = S::PA / 8 - (phase == 7 ? 1 : 0);
+    FlowCells<T> cA{}, cB{};
     auto fetch = [&](int m) {
-        const int r = 8 * m + e - g;
-        cA.load(rowA & inRow(r) ? inA + r * W : cellsA);
-        if constexpr (RANK == 3) cB.load(rowB & inRow(r) ? inB + r * W : cellsA);
+        cA.load(inA, (m + lag) * FLOW_CELLS_BYTES);
+        if constexpr (RANK == 3) cB.load(inB, (m + lag) * FLOW_CELLS_BYTES);
     };
     auto missing = [&](int m) {
-        const bool in = inRow(8 * m + e - g);
+        const bool in = inRow(8 * m + e - g - phase);
         bool miss = in & rowA & !cA.holds(task.tag);
         if constexpr (RANK == 3) miss |= in & rowB & !cB.holds(task.tag);
         return __any(miss);
@@ -820,18 +809,18 @@ __device__ __forceinline__ void flowTile(const FlowArgs<T, I, RANK> &f, const Fl
     // and the two above); each sweep has its own, as several sweeps of a tile
     // run at a time
     unsigned long long *const flag = f.ws.flags;
-    const long flagged = task.sweep * tiles + tile;
+    const long tiles = (long)f.ntA * f.ntB, flagged = task.sweep * tiles + tile;
     long watch = -1;
     if constexpr (CHAIN) {
         const long before = flagged - tiles;
         if (task.sweep > 0) watch = lane == 0 ? before : lane == 1 && ta + 1 < f.ntA ? before + f.ntB : lane == 2 && tb + 1 < f.ntB ? before + 1 : -1;
     }
     unsigned long long seen = 0;
-    auto await = [&](int b) {
+    // chunk c may be loaded: the chunk stored at step block c + 1 is in memory
+    auto await = [&](int c) {
         if constexpr (CHAIN) {
             if (task.sweep == 0) return;
-            const int most = (n + SKEW + 7) >> 3;
-            const unsigned long long need = (unsigned long long)(task.tag - 1) << 32 | (unsigned)(b + 1 < most ? b + 1 : most);
+            const unsigned long long need = (unsigned long long)(task.tag - 1) << 32 | (unsigned)(c + 2);
             while (__any(watch >= 0 && seen < need)) {
                 if (watch >= 0 && seen < need) seen = __hip_atomic_load(flag + watch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
@@ -842,35 +831,35 @@ __device__ __forceinline__ void flowTile(const FlowArgs<T, I, RANK> &f, const Fl
         if (lane == 0) __hip_atomic_store(flag + flagged, (unsigned long long)task.tag << 32 | (unsigned)count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
 
-    await(0);
-    issue(even, 0);
-    commit(even, 0);
     await(1);
+    issue(even, 0);
     issue(odd, 1);
-    await(2);
-    issue(even, 2);
-    // the lower edge rows' elements before the first block's
-    if (lane == 0) {
-        if (edgeA) ring[rowAt(-1, 0) + SLOTS - 1] = f.base[rowOff(-1, 0) + f.lo[K]];
-        if (edgeB) ring[rowAt(0, -1) + SLOTS - 1] = f.base[rowOff(0, -1) + f.lo[K]];
-    }
+    commit(even, 0);
+    commit(odd, 1);
     fetch(0);
+    await(3);
+    issue(even, 2);
+    issue(odd, 3);
     const bool mine = p < na && q < nb, whole = na == S::PA && nb == S::PB;
     T *const row = ring + rowAt(p, q);
     T prev = f.base[rowOff(p, q) + clampTo(f.lo[K] - 1, f.rlo[K], f.rhi[K])];   // the element before the first point
     readHere(prev);   // (waited for here, not by every block of steps)
     asm volatile("" ::: "memory");
     // upper neighbours are read two steps ahead (an LDS read takes longer than
-    // what is left of a step once its operands are there)
-    T c = row[0], kp = row[1], ip = row[S::BP + 1], jp{}, kp2 = row[2], ip2 = row[S::BP + 2], jp2{};
-    if constexpr (RANK == 3) {
-        jp = row[S::QP + 1];
-        jp2 = row[S::QP + 2];
-    }
-    // eight steps; GUARD: some lanes are outside the loop in some of them
-    auto walk = [&](int m, auto guard) {
-        const T *before = row + (m + 2) % 3 * 8, *after = row + (m + 1) % 3 * 8;
-        T *now = row + m % 3 * 8;
+    // what is left of a step once its operands are there); slots 1 and 2 of a
+    // row with little ahead come with chunk 2, in block 0
+    T c{}, kp{}, ip{}, jp{}, kp2{}, ip2{}, jp2{};
+    auto first = [&]() {
+        c = row[0], kp = row[1], kp2 = row[2];
+        ip = row[S::BP + 1], ip2 = row[S::BP + 2];
+        if constexpr (RANK == 3) jp = row[S::QP + 1], jp2 = row[S::QP + 2];
+    };
+    // every lane inside the loop at every step of block m
+    auto inner = [&](int m) { return whole && 8 * m >= SKEW + phase && 8 * m + 7 < n + phase; };
+    // eight steps; IN: every lane is inside the loop in all of them
+    auto walk = [&](int m, auto in) {
+        const T *before = row + (unsigned)(m + 2) % 3u * 8, *after = row + (unsigned)(m + 1) % 3u * 8;
+        T *now = row + (unsigned)m % 3u * 8;
         // lower neighbours: what the lanes before did a step ago (their prev),
         // at the tile's edge the row below (there since the block began: read
         // ahead too); along the first axis of a rank 3 tile they are eight
@@ -890,9 +879,9 @@ __device__ __forceinline__ void flowTile(const FlowArgs<T, I, RANK> &f, const Fl
             v[0] = c;
             if constexpr (RANK == 3) {
                 readHere(low);
-                const T beside = laneBelow(prev, prev);
+                const T left = laneBelow(prev, prev);
                 v[1] = low;
-                v[3] = q == 0 ? edge : beside;
+                v[3] = q == 0 ? edge : left;
                 v[4] = jp;
             } else {
                 v[1] = laneBelow(prev, edge);
@@ -900,8 +889,8 @@ __device__ __forceinline__ void flowTile(const FlowArgs<T, I, RANK> &f, const Fl
             v[2] = ip;
             v[1 + 2 * K] = prev;
             v[2 + 2 * K] = kp;
-            const int r = 8 * m + u - p - q;
-            if (!decltype(guard)::value || (mine && r >= 0 && r < n)) {
+            const int r = 8 * m + u - p - q - phase;
+            if (decltype(in)::value || (mine & inRow(r))) {
                 body(v, a0 + p, RANK == 3 ? b0 + q : (I)r, (I)r);
                 now[u] = v[0];
                 prev = v[0];
@@ -918,73 +907,65 @@ __device__ __forceinline__ void flowTile(const FlowArgs<T, I, RANK> &f, const Fl
             edge1 = edge2;
         }
     };
-    // every lane inside the loop at every step of block m
-    auto inner = [&](int m) { return whole && 8 * m >= SKEW && 8 * m + 7 < n; };
-    // next: the set that holds block m + 1 and takes m + 3
+    // next: the set that holds chunk m + 2 and takes m + 4
     auto block = [&](int m, Ahead &next) {
-        T out[8];   // block m - 1, on its way to memory
+        // chunk m - 1 is done: out to memory, its slots take chunk m + 2
+        const int c8 = chunk8(m + 2);
+        T out[8];
 #pragma unroll
-        for (int it = 0; it < 8; it++) out[it] = ring[rowAt(rowP(it), rowQ(it)) + (m + 2) % 3 * 8 + e];
+        for (int it = 0; it < 8; it++) out[it] = ring[rowAt(rowP(it), rowQ(it)) + slotOf(it, c8)];
         asm volatile("" ::: "memory");
-        commit(next, m + 1);
-        if (CHAIN && m >= 2) {
-            storesDone();   // those of block m - 2, a block of steps ago
-            publish(m - 1);
+        commit(next, m + 2);
+        if (CHAIN && m >= 1) {
+            // the stores of the blocks before: at least nine younger loads follow them
+            asm volatile("s_waitcnt vmcnt(9)" ::: "memory");
+            publish(m);
         }
         if (m < blocks) {
             if (missing(m)) {
                 do {
                     fetch(m);
-#pragma unroll
-                    for (int i = 0; i < W; i++) {
-                        readHere(cA.w[i]);
-                        readHere(cB.w[i]);
-                    }
+                    readHere(cA.w);
+                    readHere(cB.w);
+                    asm volatile("" ::: "memory");
                 } while (missing(m));
             }
             T *to = ring + (unsigned)(8 * m + e + SLOTS - 1) % SLOTS;   // the lanes above read them a slot lower
-            const bool in = inRow(8 * m + e - g);
-            if (in & rowA) to[rowAt(-1, g)] = cA.value();
-            if (RANK == 3 && (in & rowB)) to[rowAt(g, -1)] = cB.value();
+            if (rowA) to[rowAt(-1, RANK == 3 ? g : 0)] = cA.value();
+            if (RANK == 3 && rowB) to[rowAt(g, -1)] = cB.value();
         }
-        if (m > 0) {
-            T *x = f.base + f.lo[K] + 8 * (m - 1) + e;
-            auto put = [](T *to, T v) {
-                if (CHAIN) agentStore(to, v);
-                else *to = v;
-            };
-            if (inner(m - 1)) {
+        const int s8 = 8 * m - 16;   // slots s8 + ahead
+        T *const x = f.base + s8;
+        auto put = [](T *to, T v) {
+            if (CHAIN) agentStore(to, v);
+            else *to = v;
+        };
+        if (inner(m - 2) & inner(m - 1)) {
 #pragma unroll
-                for (int it = 0; it < 8; it++) put(x + (off[it] - rowP(it) - rowQ(it)), out[it]);
-            } else {
+            for (int it = 0; it < 8; it++) put(x + (off[it] + ahead[it]), out[it]);
+        } else {
 #pragma unroll
-                for (int it = 0; it < 8; it++) {
-                    const int skew = rowP(it) + rowQ(it);
-                    if ((rowP(it) < na) & (rowQ(it) < nb) & inRow(8 * (m - 1) + e - skew)) put(x + (off[it] - skew), out[it]);
-                }
-            }
+            for (int it = 0; it < 8; it++)
+                if ((rowP(it) < na) & (rowQ(it) < nb) & inRow(s8 + ahead[it] - rowP(it) - rowQ(it) - phase)) put(x + (off[it] + ahead[it]), out[it]);
         }
         fetch(m + 1);   // before the row loads, so that waiting for it leaves those in flight
-        await(m + 3);
-        issue(next, m + 3);
+        await(m + 4);
+        issue(next, m + 4);
         if (m < blocks) {
             asm volatile("" ::: "memory");
-            if (inner(m)) walk(m, std::false_type());
-            else walk(m, std::true_type());
+            if (m == 0) first();
+            if (inner(m)) walk(m, std::true_type());
+            else walk(m, std::false_type());
             // the upper faces' rows: what lanes (PA - 1, .) and (., PB - 1) did in this block
-            const T *done = ring + m % 3 * 8 + e;
-            const int rA = 8 * m + e - (S::PA - 1) - g;
-            if (toA & (g < nb) & inRow(rA)) FlowCell<T>::store(outA + rA * W, done[rowAt(S::PA - 1, gq)], task.tag);
-            if constexpr (RANK == 3) {
-                const int rB = 8 * m + e - (S::PB - 1) - g;
-                if (toB & (g < na) & inRow(rB)) FlowCell<T>::store(outB + rB * W, done[rowAt(g, S::PB - 1)], task.tag);
-            }
+            const T *done = ring + (unsigned)m % 3u * 8 + e;
+            if (toA) FlowCells<T>::store(outA, m * FLOW_CELLS_BYTES, done[rowAt(S::PA - 1, RANK == 3 ? g : 0)], task.tag);
+            if (RANK == 3 && toB) FlowCells<T>::store(outB, m * FLOW_CELLS_BYTES, done[rowAt(g, S::PB - 1)], task.tag);
             asm volatile("" ::: "memory");
         }
     };
-    for (int m = 0; m < blocks + 1; m += 2) {
-        block(m, odd);
-        block(m + 1, even);   // (one too many of an odd number stores nothing)
+    for (int m = 0; m < blocks + 2; m += 2) {
+        block(m, even);
+        block(m + 1, odd);   // (one too many of an odd number stores nothing)
     }
     if (CHAIN) {
         storesDone();
