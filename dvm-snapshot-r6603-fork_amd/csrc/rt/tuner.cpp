@@ -6,7 +6,8 @@
 // configuration (block, iterations per thread, XCD-aware order, kernel variant,
 // LDS window / wavefront tile, layout transform).  Modes:
 //   0  the default configuration (the reference's default blocks,
-//      rts/dvmh/loop.cpp:1464-1485);
+//      rts/dvmh/loop.cpp:1464-1485, unless the handler has a better shape for
+//      the loop's extents: DVMH_AMD_T_OWN);
 //   1  exhaustive: successive executions of a loop site try every candidate,
 //      then the fastest is used; every timing is recorded;
 //   2  cost model: the learned model ranks the candidates, the best few are
@@ -362,6 +363,10 @@ void tunerPick(SpecLoop *sl, long kind, TuneChoice &out) {
     for (int i = 0; i < 3; i++) out.block[i] = c.block[i];
     for (int i = 0; i < DVMH_AMD_TUNE_N; i++) out.tune[i] = c.tune[i];
     out.candidate = chosen;
+    // a loop nobody tuned: its handler may pick a shape from the loop's extents
+    if ((mode == 0 || (mode == 3 && s->measured(chosen) < 0)) &&
+            (kind == DVMH_AMD_KIND_PARALLEL || kind == DVMH_AMD_KIND_STENCIL || kind == DVMH_AMD_KIND_LINE))
+        out.tune[DVMH_AMD_T_OWN] = 1;
     s->lastPicked = chosen;
     sl->candidate = chosen;
     sl->siteKey = s->key;

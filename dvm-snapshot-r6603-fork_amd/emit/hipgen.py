@@ -1035,6 +1035,30 @@ def march_kernel(L, tail=None):
     return '\n'.join(k) + '\n\n' + '\n'.join(g) + '\n'
 
 
+def parallel_own_shape(L):
+    """Handler lines for a loop whose configuration nobody chose
+    (DVMH_AMD_T_OWN): rows at least a wave wide take wider workgroups with four
+    iterations per thread -- fewer workgroups to start and to fold -- than the
+    default blocks (32 x 4 x 2, 32 x 8), and large rank 3 stencils the LDS march.
+    Measured, default -> own shape: 7-point stencil 62^3 20 -> 19 us, 126^3 33 ->
+    26, 190^3 65 -> 43, 254^3 129 -> 76 (march 78), 318^3 247 -> 157 (direct 180),
+    382^3 414 -> 225 (direct 302); MAXLOC over 64^3 21 -> 20, 192^3 72 -> 36;
+    2-D copy and MAX 254^2 17 -> 16, 1022^2 24 -> 19, 4094^2 102 -> 80."""
+    r = L.rank
+    if r not in (2, 3):
+        return []
+    b = [f'if (tune[DVMH_AMD_T_OWN] && cnt{r - 1} >= 64) {{',
+         IND + 'tune[DVMH_AMD_T_DEPTH] = 4;']
+    if r == 3:
+        b.append(IND + 'threads = dim3(64, 4, 1);')
+        if L.stencil:
+            b.append(IND + 'if (cnt2 >= 128 && cnt0 * cnt1 * cnt2 >= 280L * 280 * 280) { tune[DVMH_AMD_T_VARIANT] = 1; tune[DVMH_AMD_T_TILE_A] = 2; tune[DVMH_AMD_T_CHUNK] = 32; }')
+    else:
+        b.append(IND + f'threads = cnt{r - 1} >= 128 ? dim3(128, 4, 1) : dim3(64, 8, 1);')
+    b.append('}')
+    return b
+
+
 def parallel_handler(L):
     r = L.rank
     h = [f'extern "C" void {L.name}_cuda(DvmType *pLoopRef{"".join(", DvmType " + p[1] + "_hdr[]" if p[0] == "array" else ", " + p[2] + " *" + p[1] + "_ptr" for p in L.params)}) {{']
@@ -1042,11 +1066,12 @@ def parallel_handler(L):
                          regs_kernel=f'{L.name}_kernel<int, 1>')
     for p in L.arrays:
         b.append(f'if ({p[1]}_tfm != 0) {{ fprintf(stderr, "{L.name}: array {p[1]} is not in natural layout\\n"); abort(); }}')
-    b.append('int depth = (int)tune[DVMH_AMD_T_DEPTH];')
-    b.append('if (depth != 1 && depth != 2 && depth != 4 && depth != 8) depth = 1;')
     for i in range(r):
         b.append(f'DvmType cnt{i} = (boundsHigh[{i}] - boundsLow[{i}]) / loopSteps[{i}] + 1;')
     ax_x, ax_y, ax_z = r - 1, (r - 2 if r >= 2 else None), (r - 3 if r >= 3 else None)
+    b += parallel_own_shape(L)
+    b.append('int depth = (int)tune[DVMH_AMD_T_DEPTH];')
+    b.append('if (depth != 1 && depth != 2 && depth != 4 && depth != 8) depth = 1;')
     dep_ax = ax_z if ax_z is not None else (ax_y if ax_y is not None else ax_x)
     if L.stencil:
         # LDS march variant: COLS points per thread on x, `march` planes per workgroup
@@ -3129,6 +3154,12 @@ def across_handler(L):
             xct = [p for p in L.arrays if p[1] == X][0][2]
             b.append(IND + '// tiled line sweep: unit steps along the line, natural layout, chunk fits 64 KB of LDS')
             b.append(IND + '// REG (TILE_B = 1): the walk on a register copy, 32-bit indices only (the slot arithmetic must fold)')
+            b.append(IND + '// configuration chosen by nobody: the streamed sweep wherever it applies (64^3 31 -> 9 us, 128^3 58 -> 13,')
+            b.append(IND + '// 256^3 135 -> 50 against the direct sweep in the default 32 x 8 block)')
+            b.append(IND + f'if (tune[DVMH_AMD_T_OWN] && {X}_tfm == 0 && {X}_devHdr[{r}] == 1 && kernelIndexT == rt_INT && (loopSteps[{r - 1}] == 1 || loopSteps[{r - 1}] == -1) && sizeof({xct}) >= 4 && sizeof({xct}) <= 8) {{')
+            b.append(IND * 2 + 'tune[DVMH_AMD_T_VARIANT] = 3;')
+            b.append(IND * 2 + 'threads = dim3(128, 1, 1);')
+            b.append(IND + '}')
             b.append(IND + 'DvmType CK = tune[DVMH_AMD_T_TILE_A], RS = (CK + 2) | 1, REG = tune[DVMH_AMD_T_TILE_B] && kernelIndexT == rt_INT ? 1 : 0;')
             b.append(IND + f'size_t ldsBytes = (((size_t)2 * threads.x * RS * sizeof({xct}) + 15) & ~(size_t)15) + (size_t)threads.x * sizeof(DvmType);')
             cks = ' || '.join(f'CK == {ck}' for ck in LINE_TILE_CK)
@@ -3148,7 +3179,14 @@ def across_handler(L):
         elif dep < r - 1 and L.line_stage_eligible(dep):
             X = L.across['array']
             cks = ' || '.join(f'CK == {ck}' for ck in LINE_REG_CK)
-            b.append(IND + '// register-staged line sweep: unit steps, natural layout, 32-bit indices')
+            b.append(IND + '// register-staged line sweep: unit steps, natural layout, 32-bit indices;')
+            b.append(IND + '// also where nobody chose a configuration (outermost axis 64^3 26 -> 11 us, 128^3 41 -> 20, 256^3 89 -> 51;')
+            b.append(IND + '// middle axis 20 -> 10, 36 -> 16, 90 -> 43, against the direct sweep in the default 32 x 8 block)')
+            b.append(IND + f'if (tune[DVMH_AMD_T_OWN] && {X}_tfm == 0 && kernelIndexT == rt_INT && (loopSteps[{dep}] == 1 || loopSteps[{dep}] == -1)) {{')
+            b.append(IND * 2 + 'tune[DVMH_AMD_T_VARIANT] = 2;')
+            b.append(IND * 2 + 'tune[DVMH_AMD_T_TILE_A] = 16;')
+            b.append(IND * 2 + 'threads = dim3(64, 1, 1);')
+            b.append(IND + '}')
             b.append(IND + 'DvmType CK = tune[DVMH_AMD_T_TILE_A];')
             b.append(IND + f'bool lreg = tune[DVMH_AMD_T_VARIANT] == 2 && (loopSteps[{dep}] == 1 || loopSteps[{dep}] == -1) && '
                      f'{X}_tfm == 0 && kernelIndexT == rt_INT && threads.x * threads.y * threads.z <= 256 && ({cks});')

@@ -47,7 +47,8 @@ extern "C" {
 #define DVMH_AMD_T_TILE_A 4    /* WAVEFRONT: tile extent on the first dependent axis; LINE: chunk steps */
 #define DVMH_AMD_T_TILE_B 5    /* WAVEFRONT: tile extent on the second dependent axis */
 #define DVMH_AMD_T_TRANSFORM 6 /* 1: arrays may be re-laid out for this loop */
-#define DVMH_AMD_T_OWN 7       /* BATCH: 1 = a batch of stencil loops runs its handler's own LDS march shape;
+#define DVMH_AMD_T_OWN 7       /* PARALLEL, STENCIL, LINE: 1 = nobody chose a configuration, the handler may pick one
+                                  from the loop's extents; BATCH: 1 = a batch of stencil loops runs its handler's own LDS march shape;
                                   PAIR: 1 = the pair handler picks its march shape from the pairs' sizes */
 void dvmh_amd_loop_get_tuning_C(DvmType curLoop, DvmType kind, DvmType tune[]);
 
