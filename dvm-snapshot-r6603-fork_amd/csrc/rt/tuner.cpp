@@ -104,6 +104,9 @@ std::vector<Candidate> makeCandidates(int kind, int loopRank, int depCount, cons
                     }
                 }
         }
+        // the shape the handler picks from the extents: a star stencil's register
+        // march where the body is one, else the shape of an untuned loop
+        if (kind != DVMH_AMD_KIND_BATCH && loopRank == 3) addCand(v, 64, 4, 1, {{DVMH_AMD_T_VARIANT, 2}, {DVMH_AMD_T_OWN, 1}});
     } else if (kind == DVMH_AMD_KIND_LINE) {
         // threads over the independent axes, each walks its line
         if (mapped >= 2) addCand(v, 32, 8, 1, {});

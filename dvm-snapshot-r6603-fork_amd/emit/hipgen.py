@@ -148,6 +148,48 @@ class Loop:
                 hi[a] = d if hi[a] is None else max(hi[a], d)
         return [(l or 0, h or 0) for l, h in zip(lo, hi)]
 
+    def star_array(self):
+        """Rank 3: the one array of a plain 4- or 8-byte type that the body only reads,
+        at the loop point and at neighbours along one axis at a time: its planes
+        can live in registers (starMarch).  None if there is no such array, or
+        more than one array is read beside the loop point."""
+        near = [p for p in self.arrays if self.rank == 3 and self._is_stencil(p[1]) and any(lo or hi for lo, hi in self.stencil_range(p[1]))]
+        if len(near) != 1 or len(self.body) > 2000:
+            return None
+        X = near[0][1]
+        if near[0][2] not in ('int', 'long', 'float', 'double'):
+            return None
+        for m in re.finditer(r'\b' + X + r'\s*((?:\[[^\[\]]*\]\s*)+)', self.body):
+            if len(re.findall(r'[+-]\s*1', m.group(1))) > 1:
+                return None
+        return X
+
+    def point_stores(self):
+        """Arrays the body uses at the loop point only and assigns first of all,
+        unconditionally: their element may be kept in a register and stored
+        once, after the body."""
+        if re.search(r'\b(continue|return|goto|break)\b', self.body):
+            return []
+        out = []
+        here = r'\s*' + r'\s*'.join(r'\[\s*' + v + r'\s*\]' for v, _ in self.vars)
+        for p in self.arrays:
+            nm = p[1]
+            if p[3] != self.rank or p[2] not in ('int', 'long', 'float', 'double'):
+                continue
+            uses = list(re.finditer(r'\b' + nm + r'\b', self.body))
+            if not uses or any(not re.match(nm + here + r'(?!\s*\[)', self.body[u.start():]) for u in uses):
+                continue
+            if re.search(r'(&|\+\+|--)\s*' + nm + r'\b', self.body):
+                continue
+            before, rest = self.body[:uses[0].start()], self.body[uses[0].start():]
+            m = re.match(nm + here + r'\s*=(?!=)([^;]*);', rest)
+            if not m or re.search(r'\b' + nm + r'\b', m.group(1)) or not re.search(r'(^|[;{}])\s*$', before):
+                continue
+            if re.search(r'\b(if|for|while|do|switch|else|case|default)\b|\?|:', before):
+                continue
+            out.append(nm)
+        return out
+
     def flow_eligible(self):
         """Rank 2 or 3, every loop axis in the ACROSS clause with widths <= 1;
         the body reads the ACROSS array at X[i + d0][j + d1].. with at most one
@@ -1035,20 +1077,138 @@ def march_kernel(L, tail=None):
     return '\n'.join(k) + '\n\n' + '\n'.join(g) + '\n'
 
 
+STAR_SHAPES = [(1, 1), (2, 1), (2, 2), (4, 1), (4, 2)]   # rows, points per lane and row
+
+
+def star_kernel(L):
+    """Register march of a PARALLEL loop with one star stencil array (VARIANT 2):
+    a workgroup is four waves, which take R rows of its tile each.  NT: arrays stored once per point bypass the
+    caches (their lines are not read again before they would be evicted)."""
+    r = L.rank
+    X = L.star_array()
+    xct = [p for p in L.arrays if p[1] == X][0][2]
+    point = L.point_stores()
+    fp, setup = [], []
+    for p in L.arrays:
+        _, nm, ct, ar = p
+        fp.append(f'{ct} *__restrict__ {nm}_base')
+        fp += [f'IndexT {nm}_s{k}' for k in range(ar)]
+        if nm == X:
+            continue
+        strides = ', '.join(f'{nm}_s{k}' for k in range(ar))
+        setup.append(f'const IndexT {nm}_str[{ar}] = {{{strides}}};')
+        view = f'dvmh_{nm}' if nm in point else nm
+        setup.append(f'const auto {view} = dvmh_dev::makeView<{ct}, IndexT, {ar}, true>({nm}_base, {nm}_str);')
+    for p in L.scalars:
+        fp.append(f'{p[2]} *__restrict__ {p[1]}_ptr')
+        setup.append(scalar_bind(L.body, p))
+    for i in range(r):
+        fp += [f'IndexT lo{i}', f'IndexT cnt{i}', f'IndexT st{i}']
+    fp += ['IndexT nbx', 'IndexT nby', 'IndexT nbz', 'long nblocks', 'int xcd', 'IndexT march', 'IndexT xshift']
+    fp += red_kernel_params(L) + red_finish_params(L)
+    k = ['template <typename IndexT, int R, int C, bool NT>',
+         f'__global__ __launch_bounds__(256) void {L.name}_star_kernel({", ".join(fp)}) {{']
+    b = list(setup) + red_kernel_locals(L)
+    b.append('long tile = dvmh_dev::xcdTile((long)blockIdx.x, nblocks, xcd);')
+    b.append('const IndexT bx = (IndexT)(tile % nbx); tile /= nbx;')
+    b.append('const IndexT by = (IndexT)(tile % nby); tile /= nby;')
+    b.append('const IndexT tz0 = (IndexT)tile * march, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.y);')
+    b.append('const IndexT nMarch = cnt0 - tz0 < march ? cnt0 - tz0 : march;')
+    b.append('const IndexT tx0 = bx * (64 * C) - xshift, ty0 = (by * 4 + wave) * R;')
+    rng = L.stencil_range(X)
+    los, cnts = ', '.join(f'lo{i}' for i in range(r)), ', '.join(f'cnt{i}' for i in range(r))
+    rlo = ', '.join(f'lo{i} + ({rng[i][0]})' for i in range(r))
+    rhi = ', '.join(f'lo{i} + cnt{i} - 1 + ({rng[i][1]})' for i in range(r))
+    b.append(f'const IndexT dvmh_lo[{r}] = {{{los}}}, dvmh_cnt[{r}] = {{{cnts}}}, dvmh_rlo[{r}] = {{{rlo}}}, dvmh_rhi[{r}] = {{{rhi}}};')
+    body = []
+    for v, ct in L.vars:
+        body.append(f'{ct} {v};')
+    for pr in L.privates:
+        body.append(pr + ';')
+    for i in range(r):
+        body.append(var_assign(L, i, f't{i}', f'lo{i}', '1'))   # unit steps only
+    at = ', '.join(f'(IndexT){v}' for v, _ in L.vars)
+    body.append(f'const dvmh_dev::StarView<{xct}, IndexT, {r}> {X}{{dvmh_v, {{{at}}}, 0}};')
+    idx = ''.join(f'[{v}]' for v, _ in L.vars)
+    for p in L.arrays:
+        if p[1] in point:
+            body.append(f'{p[2]} dvmh_{p[1]}_at;')
+            body.append(f'const dvmh_dev::PointView<{p[2]}, {r}> {p[1]}{{&dvmh_{p[1]}_at}};')
+    body.append('{\n' + indent(L.body + '\n', 1) + '}')
+    for nm in point:
+        body.append(f'if (NT) __builtin_nontemporal_store(dvmh_{nm}_at, &dvmh_{nm}{idx});')
+        body.append(f'else dvmh_{nm}{idx} = dvmh_{nm}_at;')
+    b.append('if (tx0 < cnt2 && ty0 < cnt1) {')
+    b.append(IND + f'dvmh_dev::starMarch<{xct}, IndexT, R, C>({X}_base, {X}_s0, {X}_s1, dvmh_lo, dvmh_cnt, dvmh_rlo, dvmh_rhi, '
+             f'tz0, nMarch, ty0, tx0, [&]({xct} (&dvmh_v)[7], IndexT t0, IndexT t1, IndexT t2) {{')
+    b += [IND * 2 + ln for ln in '\n'.join(body).split('\n')]
+    b.append(IND + '});')
+    b.append('}')
+    b += red_kernel_finish(L, 'blockIdx.x')
+    k.append(indent('\n'.join(b) + '\n', 1).rstrip('\n'))
+    k.append('}')
+    return '\n'.join(k) + '\n'
+
+
+def star_shape(L):
+    """Handler lines: the shape of the register march.  TILE_A rows and TILE_B
+    points per lane, CHUNK planes; with DVMH_AMD_T_OWN all are picked here."""
+    r = L.rank
+    arrs = [p for p in L.arrays if p[3] == r]
+    b = [f'bool star = tune[DVMH_AMD_T_VARIANT] == 2 && kernelIndexT == rt_INT && ' + ' && '.join(f'loopSteps[{i}] == 1' for i in range(r)) + ';',
+         'bool starNt = tune[DVMH_AMD_T_DEPTH] == 2;',
+         'DvmType starR = tune[DVMH_AMD_T_TILE_A], starC = tune[DVMH_AMD_T_TILE_B], starMarch = tune[DVMH_AMD_T_CHUNK];',
+         'int starXcd = (int)tune[DVMH_AMD_T_XCD];',
+         'if (star && tune[DVMH_AMD_T_OWN]) {',
+         IND + f'const DvmType cx = cnt{r - 1}, w1 = (cx + 63) / 64, w2 = (cx + 127) / 128;',
+         IND + '// beyond the 256 MB last-level cache stored lines are not found there again (384^3 doubles: 198 -> 175 us;',
+         IND + '// inside it they are: 201 x 187 x 239 24 -> 30, 256^3 37 -> 45)',
+         IND + f'starNt = (double)({" + ".join(f"sizeof({p[2]})" for p in arrs)}) * {" * ".join(f"cnt{i}" for i in range(r))} > 268e6 * 1.02;',
+         IND + 'starXcd = starNt ? 0 : 1;']
+    b += [IND + '// two points per lane unless that leaves lanes of the last tile idle (320: five tiles of 64, 106 us, or three of',
+          IND + '// 128, 112); four rows (1.5 rows loaded per row) while 240 workgroups still march 16 planes, else two, else one',
+          IND + '// (128^3 R = 2 8.9 us, R = 4 9.4, R = 1 9.3; 66^3 R = 1 5.3, R = 2 5.7; 201 x 187 x 239 R = 4 23.5, R = 2 23.8, R = 1 29)',
+          IND + 'starC = 2 * w2 <= w1 + w1 / 16 ? 2 : 1;',
+          IND + 'const DvmType tiles = starC == 2 ? w2 : w1;',
+          IND + 'if (tiles * ((cnt1 + 15) / 16) * cnt0 >= 240 * 16) starR = 4;',
+          IND + 'else if (tiles * ((cnt1 + 7) / 8) * cnt0 >= 240 * 8) starR = 2;',
+          IND + 'else starR = 1, starC = 1;',
+          IND + 'const DvmType perPlane = (starC == 2 ? w2 : w1) * ((cnt1 + 4 * starR - 1) / (4 * starR));',
+          IND + '// one round of workgroups: 256 of the largest tiles (3 waves per SIMD fit; fewer planes are loaded twice),',
+          IND + '// 512 of the others or where memory beyond the cache needs more loads in flight',
+          IND + 'DvmType parts = (starR == 4 && starC == 2 && !starNt ? 256 : 512) / perPlane;']
+    b += [IND + 'if (parts > cnt0 / 4) parts = cnt0 / 4;',
+          IND + 'if (parts < 1) parts = 1;',
+          IND + 'starMarch = (cnt0 + parts - 1) / parts;',
+          '}',
+          'if (star) {',
+          IND + 'threads = dim3(64, 4, 1);',
+          IND + 'tune[DVMH_AMD_T_DEPTH] = 1;',
+          IND + 'star = starMarch >= 1 && (' + ' || '.join(f'(starR == {a} && starC == {c})' for a, c in STAR_SHAPES) + ');',
+          '}']
+    return b
+
+
 def parallel_own_shape(L):
     """Handler lines for a loop whose configuration nobody chose
     (DVMH_AMD_T_OWN): rows at least a wave wide take wider workgroups with four
     iterations per thread -- fewer workgroups to start and to fold -- than the
-    default blocks (32 x 4 x 2, 32 x 8), and large rank 3 stencils the LDS march.
-    Measured, default -> own shape: 7-point stencil 62^3 20 -> 19 us, 126^3 33 ->
-    26, 190^3 65 -> 43, 254^3 129 -> 76 (march 78), 318^3 247 -> 157 (direct 180),
-    382^3 414 -> 225 (direct 302); MAXLOC over 64^3 21 -> 20, 192^3 72 -> 36;
-    2-D copy and MAX 254^2 17 -> 16, 1022^2 24 -> 19, 4094^2 102 -> 80."""
+    default blocks (32 x 4 x 2, 32 x 8); rank 3 star stencils take the register
+    march, other large rank 3 stencils the LDS march.  Measured, default -> own
+    shape: MAXLOC over 64^3 21 -> 20 us, 192^3 72 -> 36; 2-D copy and MAX 254^2
+    17 -> 16, 1022^2 24 -> 19, 4094^2 102 -> 80; 7-point stencil in the default
+    blocks, in wide ones, LDS march and register march: 128^3 33, 26, 35 and 9;
+    201 x 187 x 239 59, 45, 50 and 24; 256^3 129, 76, 78 and 37; 384^3 414, 302,
+    200 and 175."""
     r = L.rank
     if r not in (2, 3):
         return []
-    b = [f'if (tune[DVMH_AMD_T_OWN] && cnt{r - 1} >= 64) {{',
-         IND + 'tune[DVMH_AMD_T_DEPTH] = 4;']
+    b = []
+    if L.star_array():
+        b += ['// a star stencil: the register march, unless most lanes of a row would idle (below 66^3 no difference)',
+              f'if (tune[DVMH_AMD_T_OWN] && cnt{r - 1} >= 32) tune[DVMH_AMD_T_VARIANT] = 2;'] + star_shape(L)
+    b += [f'if (tune[DVMH_AMD_T_OWN] && cnt{r - 1} >= 64' + (' && !star' if L.star_array() else '') + ') {',
+          IND + 'tune[DVMH_AMD_T_DEPTH] = 4;']
     if r == 3:
         b.append(IND + 'threads = dim3(64, 4, 1);')
         if L.stencil:
@@ -1073,6 +1233,16 @@ def parallel_handler(L):
     b.append('int depth = (int)tune[DVMH_AMD_T_DEPTH];')
     b.append('if (depth != 1 && depth != 2 && depth != 4 && depth != 8) depth = 1;')
     dep_ax = ax_z if ax_z is not None else (ax_y if ax_y is not None else ax_x)
+    # tiles after the first start where the rows of the array the body
+    # writes are 128-byte aligned (full cache lines stored)
+    wr = [p for p in L.arrays if p[1] not in L.stencil and p[3] == r and
+          re.search(r'\b' + p[1] + r'\s*(?:\[[^\]]*\]\s*)+(?:=(?!=)|\+=|-=|\*=|/=)', L.body)]
+    if wr:
+        _, wn, wct, _ = wr[0]
+        addr = ' + '.join([wn] + [f'boundsLow[{k}] * {wn}_devHdr[{k + 1}]' for k in range(r)])
+    star = L.star_array()
+    if star:
+        b.append('DvmType xshift = 0;')
     if L.stencil:
         # LDS march variant: COLS points per thread on x, `march` planes per workgroup
         b.append('int variant = (int)tune[DVMH_AMD_T_VARIANT];')
@@ -1099,25 +1269,34 @@ def parallel_handler(L):
         b.append(IND + 'variant = 0;')
         b.append('}')
         b.append('DvmType nbx, nby, nbz;')
-        b.append('DvmType xshift = 0;')
+        if not star:
+            b.append('DvmType xshift = 0;')
         b.append('if (variant == 1) {')
-        # tiles after the first start where the rows of the array the body
-        # writes are 128-byte aligned (full cache lines stored)
-        wr = [p for p in L.arrays if p[1] not in L.stencil and p[3] == r and
-              re.search(r'\b' + p[1] + r'\s*(?:\[[^\]]*\]\s*)+(?:=(?!=)|\+=|-=|\*=|/=)', L.body)]
         if wr:
-            _, wn, wct, _ = wr[0]
-            addr = ' + '.join([wn] + [f'boundsLow[{k}] * {wn}_devHdr[{k + 1}]' for k in range(r)])
             b.append(IND + f'{{ const uintptr_t a = (uintptr_t)({addr});   /* the first point of {wn} */')
             b.append(IND + f'  if ({wn}_devHdr[{r}] == 1 && a % sizeof({wct}) == 0) xshift = (DvmType)((a / sizeof({wct})) % (128 / sizeof({wct}))); }}')
         b.append(IND + f'nbx = (cnt{ax_x} + xshift + (DvmType)threads.x * mcols - 1) / ((DvmType)threads.x * mcols);')
         b.append(IND + (f'nby = (cnt{ax_y} + threads.y - 1) / threads.y;' if r == 3 else 'nby = 1;'))
         b.append(IND + 'nbz = (cnt0 + march - 1) / march;')
-        b.append('} else {')
+        if not star:
+            b.append('} else {')
         pre = IND
     else:
         b.append('DvmType nbx, nby, nbz;')
-        pre = ''
+        pre = IND if star else ''
+    if star:
+        wide = '64 * starC'
+        b.append(('} else ' if L.stencil else '') + 'if (star) {')
+        if wr:
+            b.append(IND + '// where every row is aligned alike and no tile is added')
+            b.append(IND + f'const uintptr_t a = (uintptr_t)({addr});')
+            al = ' && '.join(f'{wn}_devHdr[{q + 1}] * sizeof({wct}) % 128 == 0' for q in range(r - 1))
+            b.append(IND + f'if ({wn}_devHdr[{r}] == 1 && a % sizeof({wct}) == 0 && {al}) xshift = (DvmType)((a / sizeof({wct})) % (128 / sizeof({wct})));')
+            b.append(IND + f'if ((cnt{ax_x} + xshift + {wide} - 1) / ({wide}) > (cnt{ax_x} + {wide} - 1) / ({wide})) xshift = 0;')
+        b.append(IND + f'nbx = (cnt{ax_x} + xshift + {wide} - 1) / ({wide});')
+        b.append(IND + 'nby = (cnt1 + 4 * starR - 1) / (4 * starR);')
+        b.append(IND + 'nbz = (cnt0 + starMarch - 1) / starMarch;')
+        b.append('} else {')
     b.append(pre + f'nbx = (cnt{ax_x} + threads.x - 1) / threads.x;')
     if ax_y is not None:
         dy = ' * depth' if dep_ax == ax_y else ''
@@ -1128,7 +1307,7 @@ def parallel_handler(L):
         b.append(pre + f'nbz = (cnt{ax_z} + threads.z * depth - 1) / (threads.z * depth);')
     else:
         b.append(pre + 'nbz = 1;')
-    if L.stencil:
+    if L.stencil or star:
         b.append('}')
     nb = 'nbx * nby * nbz' + ''.join(f' * cnt{a}' for a in range(0, r - 3))
     b.append(f'DvmType nblocks = {nb};')
@@ -1152,10 +1331,22 @@ def parallel_handler(L):
             for v in sets:
                 b.append(IND * 2 + f'if (mcols == {cols} && npf == {v}) hipLaunchKernelGGL(({L.name}_march_kernel<{it}, {cols}, {v}>), '
                          f'dim3((unsigned)nblocks), threads, ldsBytes, stream, {", ".join(args)});')
+        if not star:
+            b.append(IND + '} else {')
+    ind2 = IND * 2 if L.stencil or star else IND
+    if star:
+        it = 'int'
+        args = array_fact_args(L, it)
+        for i in range(r):
+            args += [f'({it})boundsLow[{i}]', f'({it})cnt{i}', f'({it})loopSteps[{i}]']
+        args += [f'({it})nbx', f'({it})nby', f'({it})nbz', 'nblocks', 'starXcd', f'({it})starMarch', f'({it})xshift']
+        args += red_fact_args(L) + red_finish_args(L)
+        b.append(IND + ('} else ' if L.stencil else '') + 'if (star) {')
+        for rows, c in STAR_SHAPES:
+            for nt in ['false', 'true']:
+                b.append(IND * 2 + f'if (starR == {rows} && starC == {c} && starNt == {nt}) hipLaunchKernelGGL(({L.name}_star_kernel<{it}, {rows}, {c}, {nt}>), '
+                         f'dim3((unsigned)nblocks), threads, 0, stream, {", ".join(args)});')
         b.append(IND + '} else {')
-        ind2 = IND * 2
-    else:
-        ind2 = IND
     for it in ['int', 'long long']:
         args = array_fact_args(L, it)
         for i in range(r):
@@ -1164,7 +1355,7 @@ def parallel_handler(L):
         args += red_fact_args(L) + red_finish_args(L)
         ks = [(c, k) for c, k in kernels if (('rt_INT' in c) == (it == 'int'))]
         b += [ind2 + s for s in launch_dispatch(ks, args, 'dim3((unsigned)nblocks)')]
-    if L.stencil:
+    if L.stencil or star:
         b.append(IND + '}')
     b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 1);')
     b.append('}')
@@ -3279,6 +3470,8 @@ def gpu_loop(L):
         text.append(parallel_kernel(L))
         if L.stencil:
             text.append(march_kernel(L))
+        if L.star_array():
+            text.append(star_kernel(L))
         text.append(parallel_handler(L))
         if L.batch:
             text.append(batch_kernel(L))

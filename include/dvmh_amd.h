@@ -42,7 +42,8 @@ extern "C" {
 /* tune[] slots */
 #define DVMH_AMD_T_DEPTH 0     /* iterations of the slowest mapped axis per thread */
 #define DVMH_AMD_T_XCD 1       /* 1: XCD-aware block-to-tile order */
-#define DVMH_AMD_T_VARIANT 2   /* kernel variant (0 = direct global-memory body) */
+#define DVMH_AMD_T_VARIANT 2   /* kernel variant (0 = direct global-memory body); PARALLEL and STENCIL of rank 3: 2 = register march
+                                  of a star stencil, TILE_A rows x TILE_B points per lane, CHUNK planes, DEPTH 2 = stores past the caches */
 #define DVMH_AMD_T_CHUNK 3     /* LINE: steps per LDS window; WAVEFRONT: tile depth */
 #define DVMH_AMD_T_TILE_A 4    /* WAVEFRONT: tile extent on the first dependent axis; LINE: chunk steps */
 #define DVMH_AMD_T_TILE_B 5    /* WAVEFRONT: tile extent on the second dependent axis */

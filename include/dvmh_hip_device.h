@@ -16,6 +16,8 @@
  *              the same syntax over a point and its neighbours in registers,
  *              and the dataflow wavefront that walks them (ACROSS loops whose
  *              axes all depend).
+ *   starMarch  a march of a read-only star stencil whose planes live in registers
+ *              (PARALLEL loops), read through a StarView.
  *   reductions wave64 shuffle trees plus one LDS step across the waves of a
  *              workgroup; every thread of the workgroup must call them.
  *   xcdTile    XCD-aware renumbering of workgroups: the hardware deals
@@ -581,6 +583,18 @@ struct StarView {
     }
 };
 
+// The element of an array at the loop point, kept in a register: X[i][j][k]
+// with the loop's own indices only.
+template <typename T, int R>
+struct PointView {
+    T *v;
+    template <typename I>
+    __device__ __forceinline__ decltype(auto) operator[](I) const {
+        if constexpr (R == 1) return (*v);
+        else return PointView<T, R - 1>{v};
+    }
+};
+
 template <typename T, typename I, int RANK>
 struct FlowArgs {
     T *base;
@@ -699,9 +713,124 @@ __device__ __forceinline__ T laneBelow(T x, T first) {
     return r;
 }
 
+// Lane l gets lane l + 1's x, lane 63 gets `last` (whole wave active).
+template <typename T>
+__device__ __forceinline__ T laneAbove(T x, T last) {
+    int w[2] = {0, 0}, o[2] = {0, 0};
+    __builtin_memcpy(w, &x, sizeof(T));
+    __builtin_memcpy(o, &last, sizeof(T));
+    constexpr int WAVE_SHL1 = 0x130;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) + 3) / 4; i++) w[i] = __builtin_amdgcn_update_dpp(o[i], w[i], WAVE_SHL1, 0xf, 0xf, false);
+    T r;
+    __builtin_memcpy(&r, w, sizeof(T));
+    return r;
+}
+
+// Lane `lane`'s x in every lane.
+template <typename T>
+__device__ __forceinline__ T laneOf(T x, int lane) {
+    int w[2] = {0, 0};
+    __builtin_memcpy(w, &x, sizeof(T));
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) + 3) / 4; i++) w[i] = __builtin_amdgcn_readlane(w[i], lane);
+    T r;
+    __builtin_memcpy(&r, w, sizeof(T));
+    return r;
+}
+
 // x is in its register here (its load is issued before, not sunk to its use).
 template <typename T>
 __device__ __forceinline__ void readHere(T &x) { asm volatile("" : "+v"(x)); }
+
+// ------------------------------------------------------------------ star march
+// One wave marches nz planes (axis 0) over R rows (axis 1) of 64 * C points of
+// axis 2, point l + 64 c in lane l, and runs body(v, t0, t1, t2) at every loop
+// point; v[0] is the element there, v[1 + 2 a] and v[2 + 2 a] its neighbours
+// below and above along axis a.
+//
+// Every plane a point needs stays in the registers of the lane that owns the
+// point: the planes below, at and above it, and the one being loaded.  The rows
+// beside the R rows and the two columns beside the tile are loaded for the
+// current plane only, neighbours along a row come from the lane beside.  No LDS
+// and no barrier: the loads of the next planes stay in flight across the
+// arithmetic (with planes staged in LDS, two barriers a plane drained them).
+// Bound by memory: 256^3 doubles, 268 MB read and written, 37 us (7.3 TB/s,
+// partly from the last-level cache; planes in LDS 78, direct 76), 201 x 187 x
+// 239 24 us (45), 128^3 9 (26); 384^3, beyond that cache, 175 (200).
+// Loads are clamped into [rlo, rhi], the indices the body may read.
+// (Rank 2 has too little to keep: the same march over rows of 2-D grids is no
+// faster than the direct kernel, 2048^2 23 us both, 1024^2 15 against 14.)
+template <typename T, typename I, int R, int C, typename Body>
+__device__ __forceinline__ void starMarch(const T *__restrict__ base, I s0, I s1, const I (&lo)[3], const I (&cnt)[3],
+        const I (&rlo)[3], const I (&rhi)[3], I tz, I nz, I ty, I tx, Body body) {
+    const int lane = (int)(threadIdx.x & 63);
+    auto clampTo = [&](I x, int a) { return x < rlo[a] ? rlo[a] : (x > rhi[a] ? rhi[a] : x); };
+    I col[C], row[R + 2];
+#pragma unroll
+    for (int c = 0; c < C; c++) col[c] = clampTo(lo[2] + tx + lane + 64 * c, 2);
+    const I side = clampTo(lane < 32 ? lo[2] + tx - 1 : lo[2] + tx + 64 * C, 2);
+#pragma unroll
+    for (int r = 0; r < R + 2; r++) row[r] = clampTo(lo[1] + ty - 1 + r, 1) * s1;
+    T own[4][R][C], beside[2][2][C], edge[2][R];
+    auto loadOwn = [&](int q, I t) {
+        const T *p = base + clampTo(lo[0] + t, 0) * s0;
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int c = 0; c < C; c++) own[q][r][c] = p[row[r + 1] + col[c]];
+    };
+    auto loadBeside = [&](int q, I t) {
+        const T *p = base + clampTo(lo[0] + t, 0) * s0;
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+            beside[q][0][c] = p[row[0] + col[c]];
+            beside[q][1][c] = p[row[R + 1] + col[c]];
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) edge[q][r] = p[row[r + 1] + side];
+    };
+    auto step = [&](I t, int below, int at, int above, int h) {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int c = 0; c < C; c++) {
+                T v[7];
+                const T x = own[at][r][c];
+                v[0] = x;
+                v[1] = own[below][r][c];
+                v[2] = own[above][r][c];
+                v[3] = r == 0 ? beside[h][0][c] : own[at][r == 0 ? 0 : r - 1][c];
+                v[4] = r == R - 1 ? beside[h][1][c] : own[at][r == R - 1 ? r : r + 1][c];
+                v[5] = laneBelow(x, c == 0 ? edge[h][r] : laneOf(own[at][r][c == 0 ? 0 : c - 1], 63));
+                v[6] = laneAbove(x, c == C - 1 ? edge[h][r] : laneOf(own[at][r][c == C - 1 ? c : c + 1], 0));
+                const I tk = tx + lane + 64 * c, tj = ty + r;
+                if (tk >= 0 && tk < cnt[2] && tj < cnt[1]) body(v, t, tj, tk);
+            }
+    };
+    loadOwn(0, tz - 1);
+    loadOwn(1, tz);
+    loadOwn(2, tz + 1);
+    loadBeside(0, tz);
+    const I end = tz + nz;
+    for (I t = tz; t < end; t += 4) {
+        loadOwn(3, t + 2);
+        loadBeside(1, t + 1);
+        step(t, 0, 1, 2, 0);
+        if (t + 1 >= end) break;
+        loadOwn(0, t + 3);
+        loadBeside(0, t + 2);
+        step(t + 1, 1, 2, 3, 1);
+        if (t + 2 >= end) break;
+        loadOwn(1, t + 4);
+        loadBeside(1, t + 3);
+        step(t + 2, 2, 3, 0, 0);
+        if (t + 3 >= end) break;
+        loadOwn(2, t + 5);
+        loadBeside(0, t + 4);
+        step(t + 3, 3, 0, 1, 1);
+    }
+}
 
 // Walks the task's tile.  body(v, t0, t1, t2) runs the loop body at position
 // (t0, t1, t2) of the loop (t2 unused for rank 2) with v the star around it.

@@ -7,6 +7,12 @@ import numpy as np
 import pytest
 
 import helpers as H
+from test_variants import _force
+
+KIND_PARALLEL, KIND_STENCIL = 0, 3
+
+# register march: (rows, points per lane and row, planes, 2 = stores past the caches)
+STARS = [(1, 1, 4, 1), (2, 1, 1, 1), (2, 2, 5, 2), (4, 1, 3, 2), (4, 2, 2, 1), (4, 2, 500, 2), (1, 1, 7, 2)]
 
 
 @pytest.mark.gpu
@@ -30,3 +36,34 @@ def test_lines(n):
     res, ref = H.run_adi3d(n, 2), H.oracle_adi3d(n, 2)
     assert np.array_equal(res['max'], ref['max']) and np.array_equal(res['loc'], ref['loc'])
     assert H.bits_equal(res['A'], ref['A'])
+
+
+def _star(kind, rows, points, planes, nt):
+    _force(kind, (64, 4, 1), [nt, 1, 2, planes, rows, points, 0, 0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('shape', STARS)
+@pytest.mark.parametrize('n', [3, 4, 18, 65, 66, 67, 131])
+def test_star(n, shape):
+    _star(KIND_STENCIL, *shape)
+    try:
+        res = H.run_jac3d(n, 3)
+    finally:
+        _force(KIND_STENCIL, None, None)
+    ref = H.oracle_jac3d(n, 3)
+    assert H.bits_equal(res['A'], ref['A']) and np.array_equal(res['eps'], ref['eps'])
+    assert H.sum_close(res['sum'], ref['sum'])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('n', [40, 66, 100, 131])
+def test_star_float(n):
+    """float, a loop that names no stencil array: every step's maximum as in the direct kernel."""
+    own = H.run_jackat(3, n, 20)
+    _force(KIND_PARALLEL, (32, 4, 2), [1] + [0] * 7)
+    try:
+        ref = H.run_jackat(3, n, 20)
+    finally:
+        _force(KIND_PARALLEL, None, None)
+    assert own[0] == ref[0] and np.array_equal(own[1], ref[1])
