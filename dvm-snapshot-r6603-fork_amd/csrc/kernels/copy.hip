@@ -9,6 +9,7 @@
 
 #include <cstdint>
 
+#include "dvmh_hip_device.h"
 #include "launch.h"
 
 namespace {
@@ -43,7 +44,63 @@ __global__ __launch_bounds__(256) void copyBlockKernel(const T *__restrict__ src
 
 struct B16 { uint64_t a, b; };
 
+// One lane per byte of each variable, the values in the kernel's arguments.
+__global__ __launch_bounds__(DVMH_SMALL_MAX * DVMH_SMALL_BYTES) void setSmallKernel(DvmhSmallSet s) {
+    const int v = (int)threadIdx.x / DVMH_SMALL_BYTES, b = (int)threadIdx.x % DVMH_SMALL_BYTES;
+    if (v < s.count && b < s.bytes[v]) ((unsigned char *)s.dst[v])[b] = s.val[v][b];
+}
+
+// A block of at most DVMH_FETCH_MAX bytes to mapped host memory, one lane per
+// eight bytes of it, and then the completion word.
+__global__ __launch_bounds__(DVMH_FETCH_MAX / 8) void fetchKernel(const unsigned char *__restrict__ src, BlockDesc d, int typeSize, int bytes,
+        unsigned long long *out, unsigned long long *done, unsigned long long seq) {
+    const int first = (int)threadIdx.x * 8;
+    if (first < bytes) {
+        unsigned long long w = 0;
+        for (int b = 0; b < 8 && first + b < bytes;) {
+            int e = (first + b) / typeSize;
+            const int off = first + b - e * typeSize;
+            long at = d.srcBase;
+            for (int a = d.rank - 1; a >= 0; a--) {
+                const int n = (int)d.ext[a], q = e / n;
+                at += (long)(e - q * n) * d.srcStride[a];
+                e = q;
+            }
+            const unsigned char *p = src + at * typeSize + off;
+            if (b == 0 && off + 8 <= typeSize && ((uintptr_t)p & 7) == 0) {
+                w = *(const unsigned long long *)p;
+                break;
+            }
+            for (int q = off; q < typeSize && b < 8 && first + b < bytes; q++, b++) w |= (unsigned long long)*p++ << (8 * b);
+        }
+        dvmh_dev::hostStore(out + threadIdx.x, w);
+    }
+    dvmh_dev::storesDone();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(done, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 }  // namespace
+
+extern "C" void dvmh_hip_set_small(const DvmhSmallSet *set, hipStream_t s) {
+    hipLaunchKernelGGL(setSmallKernel, dim3(1), dim3(DVMH_SMALL_MAX * DVMH_SMALL_BYTES), 0, s, *set);
+}
+
+extern "C" void dvmh_hip_fetch(const void *src, const long *srcSizes, const long *srcOrigin, const long *lo, const long *hi, int rank,
+        long typeSize, void *out, unsigned long long *done, unsigned long long seq, hipStream_t s) {
+    BlockDesc d = {};
+    d.rank = rank;
+    long sc = 1, count = 1;
+    for (int a = rank - 1; a >= 0; a--) {
+        d.ext[a] = hi[a] - lo[a] + 1;
+        d.srcStride[a] = sc;
+        d.srcBase += (lo[a] - srcOrigin[a]) * sc;
+        sc *= srcSizes[a];
+        count *= d.ext[a];
+    }
+    hipLaunchKernelGGL(fetchKernel, dim3(1), dim3(DVMH_FETCH_MAX / 8), 0, s, (const unsigned char *)src, d, (int)typeSize,
+            (int)(count * typeSize), (unsigned long long *)out, done, seq);
+}
 
 extern "C" void dvmh_hip_copy_block(const void *src, const long *srcSizes, const long *srcOrigin, void *dst,
         const long *dstSizes, const long *dstOrigin, const long *lo, const long *hi, int rank, long typeSize,

@@ -14,6 +14,27 @@ extern "C" {
 // (rts/dvmh/cuda_reduction.cu:21-82, performReplicate*).
 void dvmh_hip_fill(void *dst, const void *value, long valueBytes, long count, hipStream_t s);
 
+// Stores up to DVMH_SMALL_MAX variables of up to DVMH_SMALL_BYTES bytes; the
+// values travel in the launch's arguments, so the caller's copies may change
+// as soon as it returns.  In place of a copy from pageable memory and a stream
+// sync for each variable (22 us of host time; one launch 5).
+#define DVMH_SMALL_MAX 8
+#define DVMH_SMALL_BYTES 16
+struct DvmhSmallSet {
+    void *dst[DVMH_SMALL_MAX];
+    int bytes[DVMH_SMALL_MAX];
+    unsigned char val[DVMH_SMALL_MAX][DVMH_SMALL_BYTES];
+    int count;
+};
+void dvmh_hip_set_small(const struct DvmhSmallSet *set, hipStream_t s);
+
+// Packs the block [lo, hi] of an array (at most DVMH_FETCH_MAX bytes, not
+// empty) into `out` (mapped host memory, whole 8-byte words are written), then
+// sets the completion word.
+#define DVMH_FETCH_MAX 2048
+void dvmh_hip_fetch(const void *src, const long *srcSizes, const long *srcOrigin, const long *lo, const long *hi, int rank,
+        long typeSize, void *out, unsigned long long *done, unsigned long long seq, hipStream_t s);
+
 // Fold n partial values (and their loc records) into one result.
 // func: rf_* code; rtType: rt_* element type.  Deterministic: fixed partition,
 // fixed per-thread order and fixed tree; on equal MAX/MIN values the lower

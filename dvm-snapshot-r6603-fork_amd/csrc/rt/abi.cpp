@@ -557,11 +557,14 @@ static void moveBlock(Data *d, const long lo[], const long hi[], bool toHost) {
     if (count <= 0) return;
     if (d->dev.isTransformed(d->rank)) d->setLayout(nullptr, 0);
     size_t nb = (size_t)count * (size_t)d->typeSize;
-    void *stage = gpu.alloc(nb);
-    char *hstage = (char *)gpu.pinnedStaging(nb);
+    const char *fetched = toHost ? gpu.fetchBlock(d->dev.ptr, sizes, origin, lo, hi, d->rank, d->typeSize) : nullptr;
+    void *stage = fetched ? nullptr : gpu.alloc(nb);
+    char *hstage = fetched ? (char *)fetched : (char *)gpu.pinnedStaging(nb);
     if (toHost) {
-        dvmh_hip_copy_block(d->dev.ptr, sizes, origin, stage, bext, lo, lo, hi, d->rank, d->typeSize, gpu.stream);
-        gpu.d2h(hstage, stage, nb);
+        if (!fetched) {
+            dvmh_hip_copy_block(d->dev.ptr, sizes, origin, stage, bext, lo, lo, hi, d->rank, d->typeSize, gpu.stream);
+            gpu.d2h(hstage, stage, nb);
+        }
         // unpack on the host
         long idx[MAX_RANK];
         for (int a = 0; a < d->rank; a++) idx[a] = lo[a];
@@ -884,14 +887,30 @@ extern "C" void dvmh_region_execute_on_targets_C(DvmType curRegion, DvmType devi
         if (ra.part) uploadMissingBox(d, ra.box);
         else uploadMissing(d);
     }
+    DvmhSmallSet set = {};
+    auto send = [&set] {
+        if (set.count == 0) return;
+        dvmh_hip_set_small(&set, gpu.stream);
+        HIP_CHECK(hipGetLastError());
+        set.count = 0;
+    };
     for (auto &rs : r->scalars) {
         Data *d = rs.data;
         d->ensureDev();
         if (!d->devWhole() || d->hostWhole()) {
-            gpu.h2d(d->dev.ptr, d->host, (size_t)d->typeSize);
+            if (d->typeSize <= DVMH_SMALL_BYTES) {
+                set.dst[set.count] = d->dev.ptr;
+                set.bytes[set.count] = (int)d->typeSize;
+                memcpy(set.val[set.count++], d->host, (size_t)d->typeSize);
+                gpu.h2dBytes += d->typeSize;
+                if (set.count == DVMH_SMALL_MAX) send();
+            } else {
+                gpu.h2d(d->dev.ptr, d->host, (size_t)d->typeSize);
+            }
             d->devPieces.add(d->whole());
         }
     }
+    send();
 }
 
 extern "C" void dvmh_region_end_C(DvmType curRegion) {   // :3122

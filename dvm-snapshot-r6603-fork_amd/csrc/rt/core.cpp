@@ -108,10 +108,12 @@ void Gpu::init() {
     HIP_CHECK(hipMalloc((void **)&redCounters, redBytes));
     HIP_CHECK(hipMemset(redCounters, 0, redBytes));
     void *done = nullptr;
-    HIP_CHECK(hipHostMalloc(&done, 64, hipHostMallocMapped));
+    HIP_CHECK(hipHostMalloc(&done, 64 + DVMH_FETCH_MAX, hipHostMallocMapped));
     doneHost = (volatile unsigned long long *)done;
     *doneHost = 0;
     HIP_CHECK(hipHostGetDevicePointer((void **)&doneDev, done, 0));
+    fetchHost = (char *)done + 64;
+    fetchDev = (char *)doneDev + 64;
     HIP_CHECK(hipDeviceSynchronize());
     present = true;
     logMsg(LOG_INFO, "GPU %s (%s): %d CUs, wave%d", props.name, props.arch, props.cuCount, props.waveSize);
@@ -263,7 +265,31 @@ void Gpu::h2d(void *dst, const void *src, size_t bytes) {
     HIP_CHECK(hipStreamSynchronize(stream));
 }
 
+// A few bytes come back faster by a launch that writes them to mapped host
+// memory than by a copy into pageable memory and a stream sync (a region of
+// one small loop, one element read back after it: 36 us with both and the
+// scalars' copies, 17 without).
+const char *Gpu::fetchBlock(const void *src, const long sizes[], const long origin[], const long lo[], const long hi[], int rank,
+        long typeSize) {
+    long count = 1;
+    for (int a = 0; a < rank; a++) count *= hi[a] - lo[a] + 1;
+    if (!settings.pollDone || count <= 0 || typeSize <= 0 || count > DVMH_FETCH_MAX / typeSize) return nullptr;
+    d2hBytes += count * typeSize;
+    const unsigned long long seq = ++doneSeq;
+    dvmh_hip_fetch(src, sizes, origin, lo, hi, rank, typeSize, fetchDev, doneDev, seq, stream);
+    HIP_CHECK(hipGetLastError());
+    waitDone(seq);
+    return fetchHost;
+}
+
 void Gpu::d2h(void *dst, const void *src, size_t bytes) {
+    if (bytes > 0 && bytes <= DVMH_FETCH_MAX) {
+        const long size = (long)bytes, lo = 0, hi = (long)bytes - 1;
+        if (const char *p = fetchBlock(src, &size, &lo, &lo, &hi, 1, 1)) {
+            memcpy(dst, p, bytes);
+            return;
+        }
+    }
     d2hBytes += (long)bytes;
     HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipStreamSynchronize(stream));

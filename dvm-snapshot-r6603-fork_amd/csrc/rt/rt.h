@@ -102,8 +102,14 @@ public:
     void *pinnedStaging(size_t bytes);  // reusable pinned host buffer
     void h2d(void *dst, const void *src, size_t bytes);
     void d2h(void *dst, const void *src, size_t bytes);
+    // A block of at most DVMH_FETCH_MAX bytes through the mapped buffer, waiting
+    // on the completion word; returns the packed bytes (valid until the next
+    // fetch), or 0: too large, or polling is off.
+    const char *fetchBlock(const void *src, const long sizes[], const long origin[], const long lo[], const long hi[], int rank,
+            long typeSize);
     void sync();
 private:
+    char *fetchHost = nullptr, *fetchDev = nullptr;   // DVMH_FETCH_MAX bytes of mapped pinned memory
     std::map<size_t, std::vector<void *>> freeBlocks;
     std::map<void *, size_t> liveBlocks;
     void *staging = nullptr;
