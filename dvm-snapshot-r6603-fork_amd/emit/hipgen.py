@@ -772,12 +772,21 @@ def launch_dispatch(kernels, args, grid, block='threads'):
 
 
 # ----------------------------------------------------------------- GPU: PARALLEL
+def walks(L):
+    """Workgroups of the direct kernel may walk several tiles along the slowest
+    axis: rank 3 loops with a loc reduction, whose fold (value and loc through
+    LDS and two rounds of arrivals) takes a workgroup longer than its tile.
+    256^3 MAXLOC, 8,192 workgroups 35 us, 2,048 25; a plain MAX gains nothing
+    (320^3 floats: 84 and 86)."""
+    return L.rank == 3 and any(len(red) > 3 for red in L.reds)
+
+
 def parallel_kernel(L):
     r = L.rank
     fp, setup = kernel_array_params(L, unit=True)
     for i in range(r):
         fp += [f'IndexT lo{i}', f'IndexT cnt{i}', f'IndexT st{i}']
-    fp += ['IndexT nbx', 'IndexT nby', 'IndexT nbz', 'long nblocks', 'int xcd']
+    fp += ['IndexT nbx', 'IndexT nby', 'IndexT nbz', 'long nblocks', 'int xcd'] + (['IndexT walk'] if walks(L) else [])
     fp += red_kernel_params(L) + red_finish_params(L)
     k = []
     k.append(f'template <typename IndexT, int DEPTH>')
@@ -788,10 +797,10 @@ def parallel_kernel(L):
     for pr in L.privates:
         b.append(pr + ';')
     b += red_kernel_locals(L)
-    b.append('long tile = dvmh_dev::xcdTile((long)blockIdx.x, nblocks, xcd);')
-    b.append('const IndexT bx = (IndexT)(tile % nbx); tile /= nbx;')
-    b.append('const IndexT by = (IndexT)(tile % nby); tile /= nby;')
-    b.append('const IndexT bz = (IndexT)(tile % nbz); tile /= nbz;')
+    b.append('IndexT tile = (IndexT)dvmh_dev::xcdTile((long)blockIdx.x, nblocks, xcd);')
+    b.append('const IndexT bx = tile % nbx; tile /= nbx;')
+    b.append('const IndexT by = tile % nby; tile /= nby;')
+    b.append('const IndexT bz = tile % nbz; tile /= nbz;')
     # thread-mapped axes
     ax_x = r - 1
     ax_y = r - 2 if r >= 2 else None
@@ -799,7 +808,7 @@ def parallel_kernel(L):
     dep_ax = ax_z if ax_z is not None else (ax_y if ax_y is not None else ax_x)
     outer = list(range(0, r - 3)) if r > 3 else []
     for a in reversed(outer):
-        b.append(f'const IndexT t{a} = (IndexT)(tile % cnt{a}); tile /= cnt{a};')
+        b.append(f'const IndexT t{a} = tile % cnt{a}; tile /= cnt{a};')
     b.append(f'const IndexT t{ax_x}_0 = bx * (IndexT)blockDim.x + (IndexT)threadIdx.x;')
     if ax_y is not None:
         b.append(f'const IndexT t{ax_y}_0 = by * (IndexT)blockDim.y + (IndexT)threadIdx.y;')
@@ -810,7 +819,8 @@ def parallel_kernel(L):
         if a is None:
             continue
         if a == dep_ax and r >= 2:
-            b.append(f'const IndexT t{a}_b = t{a}_0 * DEPTH;')
+            if not walks(L):
+                b.append(f'const IndexT t{a}_b = t{a}_0 * DEPTH;')
         else:
             b.append(f'const IndexT t{a} = t{a}_0;')
             conds.append(f't{a} < cnt{a}')
@@ -820,6 +830,14 @@ def parallel_kernel(L):
         # be issued before the first result is stored (iterations of a
         # PARALLEL loop are independent and array pointers are restrict).
         # Threads on the edges take the guarded copy.
+        if walks(L):
+            # `walk` such steps along the slowest axis, in ascending order (a
+            # MAXLOC keeps the first of equal values)
+            b[:] = [ln for ln in b if not ln.startswith('const IndexT t0_0 = ')]
+            b.append('for (IndexT w = 0; w < walk; w++) {')
+            b.append('const IndexT dvmh_z = (bz * walk + w) * (IndexT)blockDim.z;')
+            b.append('if (dvmh_z * DEPTH >= cnt0) break;')
+            b.append('const IndexT t0_b = (dvmh_z + (IndexT)threadIdx.z) * DEPTH;')
         whole = ' && '.join([f't{dep_ax}_b + DEPTH <= cnt{dep_ax}'] + conds)
         b.append(f'if ({whole}) {{')
         fast = [f'const IndexT t{dep_ax} = t{dep_ax}_b + dd;']
@@ -847,6 +865,8 @@ def parallel_kernel(L):
         b += [IND * 2 + ln for ln in '\n'.join(inner).split('\n')]
         b.append(IND + '}')
         b.append('}')
+        if walks(L):
+            b.append('}')
     else:
         b += inner
     b += red_kernel_finish(L, 'blockIdx.x')
@@ -1192,8 +1212,8 @@ def star_shape(L):
 def parallel_own_shape(L):
     """Handler lines for a loop whose configuration nobody chose
     (DVMH_AMD_T_OWN): rows at least a wave wide take wider workgroups with four
-    iterations per thread -- fewer workgroups to start and to fold -- than the
-    default blocks (32 x 4 x 2, 32 x 8); rank 3 star stencils take the register
+    (rank 3: eight) iterations per thread -- fewer workgroups to start and to
+    fold -- than the default blocks (32 x 4 x 2, 32 x 8); rank 3 star stencils take the register
     march, other large rank 3 stencils the LDS march.  Measured, default -> own
     shape: MAXLOC over 64^3 21 -> 20 us, 192^3 72 -> 36; 2-D copy and MAX 254^2
     17 -> 16, 1022^2 24 -> 19, 4094^2 102 -> 80; 7-point stencil in the default
@@ -1208,7 +1228,7 @@ def parallel_own_shape(L):
         b += ['// a star stencil: the register march, unless most lanes of a row would idle (below 66^3 no difference)',
               f'if (tune[DVMH_AMD_T_OWN] && cnt{r - 1} >= 32) tune[DVMH_AMD_T_VARIANT] = 2;'] + star_shape(L)
     b += [f'if (tune[DVMH_AMD_T_OWN] && cnt{r - 1} >= 64' + (' && !star' if L.star_array() else '') + ') {',
-          IND + 'tune[DVMH_AMD_T_DEPTH] = 4;']
+          IND + f'tune[DVMH_AMD_T_DEPTH] = {8 if r == 3 else 4};']
     if r == 3:
         b.append(IND + 'threads = dim3(64, 4, 1);')
         if L.stencil:
@@ -1232,6 +1252,8 @@ def parallel_handler(L):
     b += parallel_own_shape(L)
     b.append('int depth = (int)tune[DVMH_AMD_T_DEPTH];')
     b.append('if (depth != 1 && depth != 2 && depth != 4 && depth != 8) depth = 1;')
+    if walks(L):
+        b.append('DvmType walk = 1;')
     dep_ax = ax_z if ax_z is not None else (ax_y if ax_y is not None else ax_x)
     # tiles after the first start where the rows of the array the body
     # writes are 128-byte aligned (full cache lines stored)
@@ -1307,6 +1329,10 @@ def parallel_handler(L):
         b.append(pre + f'nbz = (cnt{ax_z} + threads.z * depth - 1) / (threads.z * depth);')
     else:
         b.append(pre + 'nbz = 1;')
+    if walks(L):
+        b.append(pre + '// one fold for up to `walk` tiles: 2048 workgroups fill the chip (eight of four waves per CU)')
+        b.append(pre + 'const DvmType fill = 2048 / (nbx * nby) > 1 ? 2048 / (nbx * nby) : 1;')
+        b.append(pre + 'if (tune[DVMH_AMD_T_OWN] && nbz > fill) { walk = (nbz + fill - 1) / fill; nbz = (nbz + walk - 1) / walk; }')
     if L.stencil or star:
         b.append('}')
     nb = 'nbx * nby * nbz' + ''.join(f' * cnt{a}' for a in range(0, r - 3))
@@ -1351,7 +1377,7 @@ def parallel_handler(L):
         args = array_fact_args(L, it)
         for i in range(r):
             args += [f'({it})boundsLow[{i}]', f'({it})cnt{i}', f'({it})loopSteps[{i}]']
-        args += [f'({it})nbx', f'({it})nby', f'({it})nbz', 'nblocks', '(int)tune[DVMH_AMD_T_XCD]']
+        args += [f'({it})nbx', f'({it})nby', f'({it})nbz', 'nblocks', '(int)tune[DVMH_AMD_T_XCD]'] + ([f'({it})walk'] if walks(L) else [])
         args += red_fact_args(L) + red_finish_args(L)
         ks = [(c, k) for c, k in kernels if (('rt_INT' in c) == (it == 'int'))]
         b += [ind2 + s for s in launch_dispatch(ks, args, 'dim3((unsigned)nblocks)')]
