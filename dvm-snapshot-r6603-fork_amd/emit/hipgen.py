@@ -786,7 +786,7 @@ def parallel_kernel(L):
     fp, setup = kernel_array_params(L, unit=True)
     for i in range(r):
         fp += [f'IndexT lo{i}', f'IndexT cnt{i}', f'IndexT st{i}']
-    fp += ['IndexT nbx', 'IndexT nby', 'IndexT nbz', 'long nblocks', 'int xcd'] + (['IndexT walk'] if walks(L) else [])
+    fp += ['IndexT nbx', 'IndexT nby', 'IndexT nbz', 'long nblocks', 'int xcd'] + (['IndexT dvmh_walk'] if walks(L) else [])
     fp += red_kernel_params(L) + red_finish_params(L)
     k = []
     k.append(f'template <typename IndexT, int DEPTH>')
@@ -834,8 +834,8 @@ def parallel_kernel(L):
             # `walk` such steps along the slowest axis, in ascending order (a
             # MAXLOC keeps the first of equal values)
             b[:] = [ln for ln in b if not ln.startswith('const IndexT t0_0 = ')]
-            b.append('for (IndexT w = 0; w < walk; w++) {')
-            b.append('const IndexT dvmh_z = (bz * walk + w) * (IndexT)blockDim.z;')
+            b.append('for (IndexT dvmh_w = 0; dvmh_w < dvmh_walk; dvmh_w++) {')
+            b.append('const IndexT dvmh_z = (bz * dvmh_walk + dvmh_w) * (IndexT)blockDim.z;')
             b.append('if (dvmh_z * DEPTH >= cnt0) break;')
             b.append('const IndexT t0_b = (dvmh_z + (IndexT)threadIdx.z) * DEPTH;')
         whole = ' && '.join([f't{dep_ax}_b + DEPTH <= cnt{dep_ax}'] + conds)
@@ -1102,7 +1102,7 @@ STAR_SHAPES = [(1, 1), (2, 1), (2, 2), (4, 1), (4, 2)]   # rows, points per lane
 
 def star_kernel(L):
     """Register march of a PARALLEL loop with one star stencil array (VARIANT 2):
-    a workgroup is four waves, which take R rows of its tile each.  NT: arrays stored once per point bypass the
+    a workgroup is four waves, which take DVMH_R rows of its tile each.  DVMH_NT: arrays stored once per point bypass the
     caches (their lines are not read again before they would be evicted)."""
     r = L.rank
     X = L.star_array()
@@ -1126,15 +1126,15 @@ def star_kernel(L):
         fp += [f'IndexT lo{i}', f'IndexT cnt{i}', f'IndexT st{i}']
     fp += ['IndexT nbx', 'IndexT nby', 'IndexT nbz', 'long nblocks', 'int xcd', 'IndexT march', 'IndexT xshift']
     fp += red_kernel_params(L) + red_finish_params(L)
-    k = ['template <typename IndexT, int R, int C, bool NT>',
+    k = ['template <typename IndexT, int DVMH_R, int DVMH_C, bool DVMH_NT>',
          f'__global__ __launch_bounds__(256) void {L.name}_star_kernel({", ".join(fp)}) {{']
     b = list(setup) + red_kernel_locals(L)
     b.append('long tile = dvmh_dev::xcdTile((long)blockIdx.x, nblocks, xcd);')
     b.append('const IndexT bx = (IndexT)(tile % nbx); tile /= nbx;')
     b.append('const IndexT by = (IndexT)(tile % nby); tile /= nby;')
-    b.append('const IndexT tz0 = (IndexT)tile * march, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.y);')
+    b.append('const IndexT tz0 = (IndexT)tile * march, dvmh_wave = __builtin_amdgcn_readfirstlane((int)threadIdx.y);')
     b.append('const IndexT nMarch = cnt0 - tz0 < march ? cnt0 - tz0 : march;')
-    b.append('const IndexT tx0 = bx * (64 * C) - xshift, ty0 = (by * 4 + wave) * R;')
+    b.append('const IndexT tx0 = bx * (64 * DVMH_C) - xshift, ty0 = (by * 4 + dvmh_wave) * DVMH_R;')
     rng = L.stencil_range(X)
     los, cnts = ', '.join(f'lo{i}' for i in range(r)), ', '.join(f'cnt{i}' for i in range(r))
     rlo = ', '.join(f'lo{i} + ({rng[i][0]})' for i in range(r))
@@ -1156,10 +1156,10 @@ def star_kernel(L):
             body.append(f'const dvmh_dev::PointView<{p[2]}, {r}> {p[1]}{{&dvmh_{p[1]}_at}};')
     body.append('{\n' + indent(L.body + '\n', 1) + '}')
     for nm in point:
-        body.append(f'if (NT) __builtin_nontemporal_store(dvmh_{nm}_at, &dvmh_{nm}{idx});')
+        body.append(f'if (DVMH_NT) __builtin_nontemporal_store(dvmh_{nm}_at, &dvmh_{nm}{idx});')
         body.append(f'else dvmh_{nm}{idx} = dvmh_{nm}_at;')
     b.append('if (tx0 < cnt2 && ty0 < cnt1) {')
-    b.append(IND + f'dvmh_dev::starMarch<{xct}, IndexT, R, C>({X}_base, {X}_s0, {X}_s1, dvmh_lo, dvmh_cnt, dvmh_rlo, dvmh_rhi, '
+    b.append(IND + f'dvmh_dev::starMarch<{xct}, IndexT, DVMH_R, DVMH_C>({X}_base, {X}_s0, {X}_s1, dvmh_lo, dvmh_cnt, dvmh_rlo, dvmh_rhi, '
              f'tz0, nMarch, ty0, tx0, [&]({xct} (&dvmh_v)[7], IndexT t0, IndexT t1, IndexT t2) {{')
     b += [IND * 2 + ln for ln in '\n'.join(body).split('\n')]
     b.append(IND + '});')
@@ -1175,36 +1175,36 @@ def star_shape(L):
     points per lane, CHUNK planes; with DVMH_AMD_T_OWN all are picked here."""
     r = L.rank
     arrs = [p for p in L.arrays if p[3] == r]
-    b = [f'bool star = tune[DVMH_AMD_T_VARIANT] == 2 && kernelIndexT == rt_INT && ' + ' && '.join(f'loopSteps[{i}] == 1' for i in range(r)) + ';',
-         'bool starNt = tune[DVMH_AMD_T_DEPTH] == 2;',
-         'DvmType starR = tune[DVMH_AMD_T_TILE_A], starC = tune[DVMH_AMD_T_TILE_B], starMarch = tune[DVMH_AMD_T_CHUNK];',
-         'int starXcd = (int)tune[DVMH_AMD_T_XCD];',
-         'if (star && tune[DVMH_AMD_T_OWN]) {',
-         IND + f'const DvmType cx = cnt{r - 1}, w1 = (cx + 63) / 64, w2 = (cx + 127) / 128;',
+    b = [f'bool dvmh_star = tune[DVMH_AMD_T_VARIANT] == 2 && kernelIndexT == rt_INT && ' + ' && '.join(f'loopSteps[{i}] == 1' for i in range(r)) + ';',
+         'bool dvmh_starNt = tune[DVMH_AMD_T_DEPTH] == 2;',
+         'DvmType dvmh_starR = tune[DVMH_AMD_T_TILE_A], dvmh_starC = tune[DVMH_AMD_T_TILE_B], dvmh_starMarch = tune[DVMH_AMD_T_CHUNK];',
+         'int dvmh_starXcd = (int)tune[DVMH_AMD_T_XCD];',
+         'if (dvmh_star && tune[DVMH_AMD_T_OWN]) {',
+         IND + f'const DvmType dvmh_cx = cnt{r - 1}, dvmh_w1 = (dvmh_cx + 63) / 64, dvmh_w2 = (dvmh_cx + 127) / 128;',
          IND + '// beyond the 256 MB last-level cache stored lines are not found there again (384^3 doubles: 198 -> 175 us;',
          IND + '// inside it they are: 201 x 187 x 239 24 -> 30, 256^3 37 -> 45)',
-         IND + f'starNt = (double)({" + ".join(f"sizeof({p[2]})" for p in arrs)}) * {" * ".join(f"cnt{i}" for i in range(r))} > 268e6 * 1.02;',
-         IND + 'starXcd = starNt ? 0 : 1;']
+         IND + f'dvmh_starNt = (double)({" + ".join(f"sizeof({p[2]})" for p in arrs)}) * {" * ".join(f"cnt{i}" for i in range(r))} > 268e6 * 1.02;',
+         IND + 'dvmh_starXcd = dvmh_starNt ? 0 : 1;']
     b += [IND + '// two points per lane unless that leaves lanes of the last tile idle (320: five tiles of 64, 106 us, or three of',
           IND + '// 128, 112); four rows (1.5 rows loaded per row) while 240 workgroups still march 16 planes, else two, else one',
           IND + '// (128^3 R = 2 8.9 us, R = 4 9.4, R = 1 9.3; 66^3 R = 1 5.3, R = 2 5.7; 201 x 187 x 239 R = 4 23.5, R = 2 23.8, R = 1 29)',
-          IND + 'starC = 2 * w2 <= w1 + w1 / 16 ? 2 : 1;',
-          IND + 'const DvmType tiles = starC == 2 ? w2 : w1;',
-          IND + 'if (tiles * ((cnt1 + 15) / 16) * cnt0 >= 240 * 16) starR = 4;',
-          IND + 'else if (tiles * ((cnt1 + 7) / 8) * cnt0 >= 240 * 8) starR = 2;',
-          IND + 'else starR = 1, starC = 1;',
-          IND + 'const DvmType perPlane = (starC == 2 ? w2 : w1) * ((cnt1 + 4 * starR - 1) / (4 * starR));',
+          IND + 'dvmh_starC = 2 * dvmh_w2 <= dvmh_w1 + dvmh_w1 / 16 ? 2 : 1;',
+          IND + 'const DvmType dvmh_tiles = dvmh_starC == 2 ? dvmh_w2 : dvmh_w1;',
+          IND + 'if (dvmh_tiles * ((cnt1 + 15) / 16) * cnt0 >= 240 * 16) dvmh_starR = 4;',
+          IND + 'else if (dvmh_tiles * ((cnt1 + 7) / 8) * cnt0 >= 240 * 8) dvmh_starR = 2;',
+          IND + 'else dvmh_starR = 1, dvmh_starC = 1;',
+          IND + 'const DvmType dvmh_perPlane = (dvmh_starC == 2 ? dvmh_w2 : dvmh_w1) * ((cnt1 + 4 * dvmh_starR - 1) / (4 * dvmh_starR));',
           IND + '// one round of workgroups: 256 of the largest tiles (3 waves per SIMD fit; fewer planes are loaded twice),',
           IND + '// 512 of the others or where memory beyond the cache needs more loads in flight',
-          IND + 'DvmType parts = (starR == 4 && starC == 2 && !starNt ? 256 : 512) / perPlane;']
-    b += [IND + 'if (parts > cnt0 / 4) parts = cnt0 / 4;',
-          IND + 'if (parts < 1) parts = 1;',
-          IND + 'starMarch = (cnt0 + parts - 1) / parts;',
+          IND + 'DvmType dvmh_parts = (dvmh_starR == 4 && dvmh_starC == 2 && !dvmh_starNt ? 256 : 512) / dvmh_perPlane;']
+    b += [IND + 'if (dvmh_parts > cnt0 / 4) dvmh_parts = cnt0 / 4;',
+          IND + 'if (dvmh_parts < 1) dvmh_parts = 1;',
+          IND + 'dvmh_starMarch = (cnt0 + dvmh_parts - 1) / dvmh_parts;',
           '}',
-          'if (star) {',
+          'if (dvmh_star) {',
           IND + 'threads = dim3(64, 4, 1);',
           IND + 'tune[DVMH_AMD_T_DEPTH] = 1;',
-          IND + 'star = starMarch >= 1 && (' + ' || '.join(f'(starR == {a} && starC == {c})' for a, c in STAR_SHAPES) + ');',
+          IND + 'dvmh_star = dvmh_starMarch >= 1 && (' + ' || '.join(f'(dvmh_starR == {a} && dvmh_starC == {c})' for a, c in STAR_SHAPES) + ');',
           '}']
     return b
 
@@ -1227,7 +1227,7 @@ def parallel_own_shape(L):
     if L.star_array():
         b += ['// a star stencil: the register march, unless most lanes of a row would idle (below 66^3 no difference)',
               f'if (tune[DVMH_AMD_T_OWN] && cnt{r - 1} >= 32) tune[DVMH_AMD_T_VARIANT] = 2;'] + star_shape(L)
-    b += [f'if (tune[DVMH_AMD_T_OWN] && cnt{r - 1} >= 64' + (' && !star' if L.star_array() else '') + ') {',
+    b += [f'if (tune[DVMH_AMD_T_OWN] && cnt{r - 1} >= 64' + (' && !dvmh_star' if L.star_array() else '') + ') {',
           IND + f'tune[DVMH_AMD_T_DEPTH] = {8 if r == 3 else 4};']
     if r == 3:
         b.append(IND + 'threads = dim3(64, 4, 1);')
@@ -1253,7 +1253,7 @@ def parallel_handler(L):
     b.append('int depth = (int)tune[DVMH_AMD_T_DEPTH];')
     b.append('if (depth != 1 && depth != 2 && depth != 4 && depth != 8) depth = 1;')
     if walks(L):
-        b.append('DvmType walk = 1;')
+        b.append('DvmType dvmh_walk = 1;')
     dep_ax = ax_z if ax_z is not None else (ax_y if ax_y is not None else ax_x)
     # tiles after the first start where the rows of the array the body
     # writes are 128-byte aligned (full cache lines stored)
@@ -1307,8 +1307,8 @@ def parallel_handler(L):
         b.append('DvmType nbx, nby, nbz;')
         pre = IND if star else ''
     if star:
-        wide = '64 * starC'
-        b.append(('} else ' if L.stencil else '') + 'if (star) {')
+        wide = '64 * dvmh_starC'
+        b.append(('} else ' if L.stencil else '') + 'if (dvmh_star) {')
         if wr:
             b.append(IND + '// where every row is aligned alike and no tile is added')
             b.append(IND + f'const uintptr_t a = (uintptr_t)({addr});')
@@ -1316,8 +1316,8 @@ def parallel_handler(L):
             b.append(IND + f'if ({wn}_devHdr[{r}] == 1 && a % sizeof({wct}) == 0 && {al}) xshift = (DvmType)((a / sizeof({wct})) % (128 / sizeof({wct})));')
             b.append(IND + f'if ((cnt{ax_x} + xshift + {wide} - 1) / ({wide}) > (cnt{ax_x} + {wide} - 1) / ({wide})) xshift = 0;')
         b.append(IND + f'nbx = (cnt{ax_x} + xshift + {wide} - 1) / ({wide});')
-        b.append(IND + 'nby = (cnt1 + 4 * starR - 1) / (4 * starR);')
-        b.append(IND + 'nbz = (cnt0 + starMarch - 1) / starMarch;')
+        b.append(IND + 'nby = (cnt1 + 4 * dvmh_starR - 1) / (4 * dvmh_starR);')
+        b.append(IND + 'nbz = (cnt0 + dvmh_starMarch - 1) / dvmh_starMarch;')
         b.append('} else {')
     b.append(pre + f'nbx = (cnt{ax_x} + threads.x - 1) / threads.x;')
     if ax_y is not None:
@@ -1331,8 +1331,8 @@ def parallel_handler(L):
         b.append(pre + 'nbz = 1;')
     if walks(L):
         b.append(pre + '// one fold for up to `walk` tiles: 2048 workgroups fill the chip (eight of four waves per CU)')
-        b.append(pre + 'const DvmType fill = 2048 / (nbx * nby) > 1 ? 2048 / (nbx * nby) : 1;')
-        b.append(pre + 'if (tune[DVMH_AMD_T_OWN] && nbz > fill) { walk = (nbz + fill - 1) / fill; nbz = (nbz + walk - 1) / walk; }')
+        b.append(pre + 'const DvmType dvmh_fill = 2048 / (nbx * nby) > 1 ? 2048 / (nbx * nby) : 1;')
+        b.append(pre + 'if (tune[DVMH_AMD_T_OWN] && nbz > dvmh_fill) { dvmh_walk = (nbz + dvmh_fill - 1) / dvmh_fill; nbz = (nbz + dvmh_walk - 1) / dvmh_walk; }')
     if L.stencil or star:
         b.append('}')
     nb = 'nbx * nby * nbz' + ''.join(f' * cnt{a}' for a in range(0, r - 3))
@@ -1365,19 +1365,19 @@ def parallel_handler(L):
         args = array_fact_args(L, it)
         for i in range(r):
             args += [f'({it})boundsLow[{i}]', f'({it})cnt{i}', f'({it})loopSteps[{i}]']
-        args += [f'({it})nbx', f'({it})nby', f'({it})nbz', 'nblocks', 'starXcd', f'({it})starMarch', f'({it})xshift']
+        args += [f'({it})nbx', f'({it})nby', f'({it})nbz', 'nblocks', 'dvmh_starXcd', f'({it})dvmh_starMarch', f'({it})xshift']
         args += red_fact_args(L) + red_finish_args(L)
-        b.append(IND + ('} else ' if L.stencil else '') + 'if (star) {')
+        b.append(IND + ('} else ' if L.stencil else '') + 'if (dvmh_star) {')
         for rows, c in STAR_SHAPES:
             for nt in ['false', 'true']:
-                b.append(IND * 2 + f'if (starR == {rows} && starC == {c} && starNt == {nt}) hipLaunchKernelGGL(({L.name}_star_kernel<{it}, {rows}, {c}, {nt}>), '
+                b.append(IND * 2 + f'if (dvmh_starR == {rows} && dvmh_starC == {c} && dvmh_starNt == {nt}) hipLaunchKernelGGL(({L.name}_star_kernel<{it}, {rows}, {c}, {nt}>), '
                          f'dim3((unsigned)nblocks), threads, 0, stream, {", ".join(args)});')
         b.append(IND + '} else {')
     for it in ['int', 'long long']:
         args = array_fact_args(L, it)
         for i in range(r):
             args += [f'({it})boundsLow[{i}]', f'({it})cnt{i}', f'({it})loopSteps[{i}]']
-        args += [f'({it})nbx', f'({it})nby', f'({it})nbz', 'nblocks', '(int)tune[DVMH_AMD_T_XCD]'] + ([f'({it})walk'] if walks(L) else [])
+        args += [f'({it})nbx', f'({it})nby', f'({it})nbz', 'nblocks', '(int)tune[DVMH_AMD_T_XCD]'] + ([f'({it})dvmh_walk'] if walks(L) else [])
         args += red_fact_args(L) + red_finish_args(L)
         ks = [(c, k) for c, k in kernels if (('rt_INT' in c) == (it == 'int'))]
         b += [ind2 + s for s in launch_dispatch(ks, args, 'dim3((unsigned)nblocks)')]
