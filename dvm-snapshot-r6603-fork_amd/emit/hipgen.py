@@ -2423,13 +2423,19 @@ LINE_REG_CK = [8, 16]
 def line_reg_kernel(L, dep):
     """ACROSS with one dependent axis `dep` other than the innermost (threads
     over the independent axes, coalesced along the innermost one): each thread
-    walks its line as in line_kernel, but in chunks of CK steps.  The chunk's
-    elements of the ACROSS array (and the one ahead) are loaded together into
-    a local buffer -- CK + 1 loads in flight instead of one dependent load per
-    step -- the body runs against the buffer (RegLineView), and the chunk is
-    stored back.  The last element of a full chunk is carried into the next.
-    Steps are unrolled, so slot indices are constants and the buffer lives in
-    registers.  Loads are clamped into the indices the body reads."""
+    walks its line as in line_kernel, but in chunks of CK steps: the next
+    chunk's elements of the ACROSS array are loaded while the body runs against
+    the current one's registers (RegLineView) and the chunk is stored back.
+    Steps are unrolled, so slot indices are constants.  Whole chunks need no
+    clamping or guard, and their rows are addressed by a scalar base per chunk,
+    a scalar step and the lane's constant offset (LaneRow): with a thread per
+    line a SIMD holds one wave or none, so what bounds it is the instructions
+    of that wave -- 64-bit lane addresses, clamps and guards were two thirds of
+    them (1,631 -> 1,064 lines of assembly, and no wait for a chunk's own loads).
+    Measured, whole ADI steps of six sweeps (four of these): 65 x 131 x 99
+    96 -> 81 us, 128^3 113 -> 87, 30 x 900 x 200 231 -> 165, 2000 x 20 x 70
+    354 -> 181, 256^3 310 -> 290; chunks of 32 gain nothing more.  The rest of
+    the line runs in short chunks with clamped loads and guarded steps."""
     r = L.rank
     ind = [a for a in range(r) if a != dep]
     X = L.across['array']
@@ -2448,9 +2454,9 @@ def line_reg_kernel(L, dep):
     for pr in L.privates:
         b.append(pr + ';')
     b += red_kernel_locals(L)
-    b.append('long tile = dvmh_dev::xcdTile((long)blockIdx.x, nblocks, xcd);')
-    b.append('const IndexT bx = (IndexT)(tile % nbx); tile /= nbx;')
-    b.append('const IndexT by = (IndexT)(tile % nby); tile /= nby;')
+    b.append('IndexT tile = (IndexT)dvmh_dev::xcdTile((long)blockIdx.x, nblocks, xcd);')
+    b.append('const IndexT bx = tile % nbx; tile /= nbx;')
+    b.append('const IndexT by = tile % nby;')
     ax_x = ind[-1]
     ax_y = ind[-2] if len(ind) >= 2 else None
     conds = []
@@ -2464,32 +2470,84 @@ def line_reg_kernel(L, dep):
     inner = []
     for a in ind:
         inner.append(var_assign(L, a, f't{a}', f'lo{a}', f'st{a}'))
-    inner.append(f'{xct} *const lr_row = {X}_base' + ''.join(f' + (IndexT){L.vars[a][0]} * {X}_s{a}' for a in ind) +
-                 ';   // this thread\'s line')
+    # addresses: a scalar base that moves along the line (one per step, for the
+    # whole wave) and the lane's 32-bit byte offset, the same in every step
+    inner.append(f'const unsigned long lr_a = (unsigned long)({X}_base' + ''.join(f' + (IndexT){L.vars[a][0]} * {X}_s{a}' for a in ind) + ');')
+    low = [f'(st{ax_x} < 0 ? -(long)(blockDim.x - 1) * st{ax_x} * {X}_s{ax_x} : 0)']
+    if ax_y is not None:
+        low.append(f'(st{ax_y} < 0 ? -(long)(blockDim.y - 1) * st{ax_y} * {X}_s{ax_y} : 0)')
+    inner.append(f'char *const lr_u = dvmh_dev::globalPtr<char>((long)(dvmh_dev::firstLane(lr_a) - ({" + ".join(low)}) * (long)sizeof({xct})));')
+    inner.append('const unsigned lr_o = (unsigned)(lr_a - (unsigned long)lr_u);')
+    inner.append(f'const long lr_sb = (long){X}_s{dep} * (long)sizeof({xct});')
+    inner.append(f'auto lr_at = [&](IndexT lr_x) -> {xct} & {{ return *({xct} *)(lr_u + (long)lr_x * lr_sb + lr_o); }};')
     inner.append(f'const IndexT lr_first = lo{dep}, lr_last = lo{dep} + (cnt{dep} - 1) * (IndexT)DIR;')
-    inner.append(f'// indices along the line the body reads (offsets {dmin} .. {dmax}): loads are clamped into them')
+    inner.append(f'// indices along the line the body reads (offsets {dmin} .. {dmax}): loads beyond the loop are clamped into them')
+    inner.append(f'constexpr bool LR_AHEAD = DIR > 0 ? ({dmax}) > 0 : ({dmin}) < 0;')
     inner.append(f'const IndexT lr_rlo = (DIR > 0 ? lr_first : lr_last) + ({dmin}), lr_rhi = (DIR > 0 ? lr_last : lr_first) + ({dmax});')
-    inner.append(f'auto lr_ld = [&](IndexT x) -> {xct} {{ x = x < lr_rlo ? lr_rlo : (x > lr_rhi ? lr_rhi : x); return lr_row[x * {X}_s{dep}]; }};')
-    inner.append(f'{xct} lr_buf[CK + 2];   // slot 1 + s: step s of the chunk; 0: the element behind; CK + 1: ahead')
-    inner.append('lr_buf[0] = lr_ld(lr_first - (IndexT)DIR);')
-    inner.append(f'for (IndexT lr_c0 = 0; lr_c0 < cnt{dep}; lr_c0 += CK) {{')
-    ch = []
-    ch.append(f'const IndexT lr_n = cnt{dep} - lr_c0 < CK ? cnt{dep} - lr_c0 : CK;')
-    ch.append(f'const IndexT lr_x0 = lo{dep} + lr_c0 * (IndexT)DIR;   // array index of slot 1')
-    ch.append('#pragma unroll')
-    ch.append('for (int m = 1; m <= CK + 1; m++) lr_buf[m] = lr_ld(lr_x0 + (IndexT)(m - 1) * (IndexT)DIR);')
-    ch.append(f'const dvmh_dev::RegLineView<{xct}, IndexT, {r}, {dep}, DIR> {X}{{lr_buf, lr_x0, 0}};')
-    ch.append('#pragma unroll')
-    ch.append('for (int lr_s = 0; lr_s < CK; lr_s++) {')
-    ch.append(IND + 'if (lr_s < lr_n) {')
-    ch.append(IND * 2 + f'const IndexT t{dep} = lr_c0 + lr_s;')
-    ch.append(IND * 2 + var_assign(L, dep, f't{dep}', f'lo{dep}', '(IndexT)DIR'))
-    ch.append(indent('{\n' + indent(L.body + '\n', 1) + '}', 2))
-    ch.append(IND + '}')
-    ch.append('}')
-    ch.append('#pragma unroll')
-    ch.append(f'for (int m = 1; m <= CK; m++) if (m <= lr_n) lr_row[(lr_x0 + (IndexT)(m - 1) * (IndexT)DIR) * {X}_s{dep}] = lr_buf[m];')
-    ch.append('lr_buf[0] = lr_buf[CK];   // carried (only a full chunk has a successor)')
+    inner.append(f'auto lr_ld = [&](IndexT lr_x) -> {xct} {{ return lr_at(lr_x < lr_rlo ? lr_rlo : (lr_x > lr_rhi ? lr_rhi : lr_x)); }};')
+    inner.append('// slot 1 + s: step s of the chunk; 0: the element behind; CK + 1: ahead')
+    inner.append(f'{xct} lr_b0[CK + 2], lr_b1[CK + 2];')
+    inner.append('lr_b0[0] = lr_ld(lr_first - (IndexT)DIR);')
+    inner.append(f'const IndexT lr_nf = cnt{dep} / CK;   // whole chunks')
+    inner.append('// the rows of chunk lr_c, from the one lowest in memory')
+    inner.append(f'auto lr_rows = [&](IndexT lr_c) {{ return dvmh_dev::LaneRow<{xct}>(lr_u + (long)(lo{dep} + (DIR > 0 ? lr_c * CK : -(lr_c * CK + CK - 1))) * lr_sb, lr_o); }};')
+    inner.append(f'auto lr_load = [&](IndexT lr_c, {xct} (&lr_to)[CK + 2]) {{')
+    inner.append(IND + f'const dvmh_dev::LaneRow<{xct}> lr_row = lr_rows(lr_c);')
+    inner.append(IND + '#pragma unroll')
+    inner.append(IND + 'for (int lr_m = 0; lr_m < CK; lr_m++) lr_to[1 + lr_m] = lr_row.load((DIR > 0 ? lr_m : CK - 1 - lr_m) * (int)lr_sb);')
+    inner.append('};')
+
+    def walk(buf, x0, first, count, guard):
+        w = [f'const dvmh_dev::RegLineView<{xct}, IndexT, {r}, {dep}, DIR> {X}{{{buf}, {x0}, 0}};',
+             '#pragma unroll',
+             f'for (int lr_s = 0; lr_s < {count}; lr_s++) {{']
+        if guard:
+            w.append(IND + f'if (lr_s < {guard}) {{')
+        w.append(IND + f'const IndexT t{dep} = {first} + lr_s;')
+        w.append(IND + f'(void)t{dep};')
+        w.append(IND + var_assign(L, dep, '(IndexT)lr_s', x0, '(IndexT)DIR'))
+        w.append(indent('{\n' + indent(L.body + '\n', 1) + '}', 1))
+        if guard:
+            w.append(IND + '}')
+        return w + ['}']
+
+    inner.append('// chunk c, in `cur`; the last chunk loads itself again: no branch between loads and waits')
+    inner.append(f'auto lr_chunk = [&](IndexT lr_c, {xct} (&lr_cur)[CK + 2], {xct} (&lr_nxt)[CK + 2]) {{')
+    ch = ['const IndexT lr_x0 = ' + f'lo{dep} + lr_c * CK * (IndexT)DIR;',
+          'lr_load(lr_c + 1 < lr_nf ? lr_c + 1 : lr_c, lr_nxt);',
+          'if constexpr (LR_AHEAD) lr_cur[CK + 1] = lr_ld(lr_x0 + (IndexT)CK * (IndexT)DIR);',
+          '__builtin_amdgcn_sched_barrier(0);']
+    ch += walk('lr_cur', 'lr_x0', 'lr_c * CK', 'CK', None)
+    ch += [f'const dvmh_dev::LaneRow<{xct}> lr_row = lr_rows(lr_c);',
+           '#pragma unroll',
+           'for (int lr_m = 0; lr_m < CK; lr_m++) lr_row.store((DIR > 0 ? lr_m : CK - 1 - lr_m) * (int)lr_sb, lr_cur[1 + lr_m]);',
+           'lr_nxt[0] = lr_cur[CK];']
+    inner += [IND + ln for ln in '\n'.join(ch).split('\n')]
+    inner.append('};')
+    inner += [f'{xct} lr_carry = lr_b0[0];',
+              'if (lr_nf > 0) {',
+              IND + 'lr_load(0, lr_b0);',
+              IND + 'IndexT lr_q = 0;',
+              IND + 'for (; lr_q + 1 < lr_nf; lr_q += 2) {',
+              IND * 2 + 'lr_chunk(lr_q, lr_b0, lr_b1);',
+              IND * 2 + 'lr_chunk(lr_q + 1, lr_b1, lr_b0);',
+              IND + '}',
+              IND + 'lr_carry = lr_b0[0];',
+              IND + 'if (lr_q < lr_nf) { lr_chunk(lr_q, lr_b0, lr_b1); lr_carry = lr_b1[0]; }',
+              '}',
+              '// the rest of the line, in short chunks',
+              'constexpr int LR_T = 8;',
+              f'for (IndexT lr_c0 = lr_nf * CK; lr_c0 < cnt{dep}; lr_c0 += LR_T) {{']
+    ch = [f'const IndexT lr_n = cnt{dep} - lr_c0 < LR_T ? cnt{dep} - lr_c0 : LR_T;',
+          f'const IndexT lr_x0 = lo{dep} + lr_c0 * (IndexT)DIR;',
+          f'{xct} lr_t[LR_T + 2];',
+          'lr_t[0] = lr_carry;',
+          '#pragma unroll',
+          'for (int lr_m = 1; lr_m <= LR_T + 1; lr_m++) lr_t[lr_m] = lr_ld(lr_x0 + (IndexT)(lr_m - 1) * (IndexT)DIR);']
+    ch += walk('lr_t', 'lr_x0', 'lr_c0', 'LR_T', 'lr_n')
+    ch += ['#pragma unroll',
+           'for (int lr_m = 0; lr_m < LR_T; lr_m++) if (lr_m < lr_n) lr_at(lr_x0 + (IndexT)lr_m * (IndexT)DIR) = lr_t[1 + lr_m];',
+           'lr_carry = lr_t[LR_T];   // (only a full chunk has a successor)']
     inner += [IND + ln for ln in '\n'.join(ch).split('\n')]
     inner.append('}')
     b += [IND + ln for ln in '\n'.join(inner).split('\n')]
@@ -3397,8 +3455,8 @@ def across_handler(L):
             X = L.across['array']
             cks = ' || '.join(f'CK == {ck}' for ck in LINE_REG_CK)
             b.append(IND + '// register-staged line sweep: unit steps, natural layout, 32-bit indices;')
-            b.append(IND + '// also where nobody chose a configuration (outermost axis 64^3 26 -> 11 us, 128^3 41 -> 20, 256^3 89 -> 51;')
-            b.append(IND + '// middle axis 20 -> 10, 36 -> 16, 90 -> 43, against the direct sweep in the default 32 x 8 block)')
+            b.append(IND + '// also where nobody chose a configuration (outermost axis 64^3 26 -> 10 us, 128^3 41 -> 15, 256^3 89 -> 44;')
+            b.append(IND + '// middle axis 20 -> 9, 36 -> 12, 90 -> 41, against the direct sweep in the default 32 x 8 block)')
             b.append(IND + f'if (tune[DVMH_AMD_T_OWN] && {X}_tfm == 0 && kernelIndexT == rt_INT && (loopSteps[{dep}] == 1 || loopSteps[{dep}] == -1)) {{')
             b.append(IND * 2 + 'tune[DVMH_AMD_T_VARIANT] = 2;')
             b.append(IND * 2 + 'tune[DVMH_AMD_T_TILE_A] = 16;')
@@ -3407,6 +3465,10 @@ def across_handler(L):
             b.append(IND + 'DvmType CK = tune[DVMH_AMD_T_TILE_A];')
             b.append(IND + f'bool lreg = tune[DVMH_AMD_T_VARIANT] == 2 && (loopSteps[{dep}] == 1 || loopSteps[{dep}] == -1) && '
                      f'{X}_tfm == 0 && kernelIndexT == rt_INT && threads.x * threads.y * threads.z <= 256 && ({cks});')
+            xs = [a for a in range(r) if a != dep]
+            span = f'(DvmType)(threads.x - 1) * labs(loopSteps[{xs[-1]}]) * {X}_devHdr[{xs[-1] + 1}]' + (f' + (DvmType)(threads.y - 1) * labs(loopSteps[{xs[-2]}]) * {X}_devHdr[{xs[-2] + 1}]' if len(xs) > 1 else '')
+            b.append(IND + '// a chunk of rows and a workgroup\'s lanes lie within 2 GB of each other')
+            b.append(IND + f'lreg = lreg && (CK * {X}_devHdr[{dep + 1}] + {span}) * (DvmType)sizeof({[p for p in L.arrays if p[1] == X][0][2]}) < (1L << 31);')
             b.append(IND + 'if (lreg) {')
             b += [IND * 2 + s for s in line_reg_launch(L, dep)]
             b.append(IND + '} else {')

@@ -739,6 +739,50 @@ __device__ __forceinline__ T laneOf(T x, int lane) {
     return r;
 }
 
+// The first active lane's x, as a scalar.
+__device__ __forceinline__ unsigned long firstLane(unsigned long x) {
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)x);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(x >> 32));
+    return (unsigned long)hi << 32 | lo;
+}
+
+// An element per lane at the scalar address `base` + `step` bytes plus the lane's
+// own 32-bit byte offset: the per-step part of the address costs scalar
+// instructions only (4- and 8-byte types).
+template <typename T>
+struct LaneRow {
+    __amdgpu_buffer_rsrc_t rs;
+    char *base;
+    unsigned lane;
+    __device__ __forceinline__ LaneRow(char *b, unsigned l) : rs(__builtin_amdgcn_make_buffer_rsrc(b, 0, -1, 0x00027000)), base(b), lane(l) {}
+    __device__ __forceinline__ T load(int step) const {
+        T v;
+        if constexpr (sizeof(T) == 8) {
+            const auto w = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)lane, step, 0);
+            __builtin_memcpy(&v, &w, 8);
+        } else if constexpr (sizeof(T) == 4) {
+            const auto w = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)lane, step, 0);
+            __builtin_memcpy(&v, &w, 4);
+        } else {
+            v = *(const T *)(base + step + lane);
+        }
+        return v;
+    }
+    __device__ __forceinline__ void store(int step, T v) const {
+        if constexpr (sizeof(T) == 8) {
+            decltype(__builtin_amdgcn_raw_buffer_load_b64(rs, 0, 0, 0)) w;
+            __builtin_memcpy(&w, &v, 8);
+            __builtin_amdgcn_raw_buffer_store_b64(w, rs, (int)lane, step, 0);
+        } else if constexpr (sizeof(T) == 4) {
+            decltype(__builtin_amdgcn_raw_buffer_load_b32(rs, 0, 0, 0)) w;
+            __builtin_memcpy(&w, &v, 4);
+            __builtin_amdgcn_raw_buffer_store_b32(w, rs, (int)lane, step, 0);
+        } else {
+            *(T *)(base + step + lane) = v;
+        }
+    }
+};
+
 // x is in its register here (its load is issued before, not sunk to its use).
 template <typename T>
 __device__ __forceinline__ void readHere(T &x) { asm volatile("" : "+v"(x)); }
