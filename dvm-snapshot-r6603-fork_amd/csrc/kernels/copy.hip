@@ -50,6 +50,11 @@ __global__ __launch_bounds__(DVMH_SMALL_MAX * DVMH_SMALL_BYTES) void setSmallKer
     if (v < s.count && b < s.bytes[v]) ((unsigned char *)s.dst[v])[b] = s.val[v][b];
 }
 
+// Everything before it on the stream is complete.
+__global__ __launch_bounds__(64) void signalKernel(unsigned long long *done, unsigned long long seq) {
+    if (threadIdx.x == 0) __hip_atomic_store(done, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // A block of at most DVMH_FETCH_MAX bytes to mapped host memory, one lane per
 // eight bytes of it, and then the completion word.
 __global__ __launch_bounds__(DVMH_FETCH_MAX / 8) void fetchKernel(const unsigned char *__restrict__ src, BlockDesc d, int typeSize, int bytes,
@@ -84,6 +89,10 @@ __global__ __launch_bounds__(DVMH_FETCH_MAX / 8) void fetchKernel(const unsigned
 
 extern "C" void dvmh_hip_set_small(const DvmhSmallSet *set, hipStream_t s) {
     hipLaunchKernelGGL(setSmallKernel, dim3(1), dim3(DVMH_SMALL_MAX * DVMH_SMALL_BYTES), 0, s, *set);
+}
+
+extern "C" void dvmh_hip_signal(unsigned long long *done, unsigned long long seq, hipStream_t s) {
+    hipLaunchKernelGGL(signalKernel, dim3(1), dim3(64), 0, s, done, seq);
 }
 
 extern "C" void dvmh_hip_fetch(const void *src, const long *srcSizes, const long *srcOrigin, const long *lo, const long *hi, int rank,

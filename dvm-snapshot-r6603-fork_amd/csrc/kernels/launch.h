@@ -28,6 +28,9 @@ struct DvmhSmallSet {
 };
 void dvmh_hip_set_small(const struct DvmhSmallSet *set, hipStream_t s);
 
+// Sets the completion word once everything before it on the stream is done.
+void dvmh_hip_signal(unsigned long long *done, unsigned long long seq, hipStream_t s);
+
 // Packs the block [lo, hi] of an array (at most DVMH_FETCH_MAX bytes, not
 // empty) into `out` (mapped host memory, whole 8-byte words are written), then
 // sets the completion word.

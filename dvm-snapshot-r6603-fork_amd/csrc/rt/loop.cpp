@@ -166,8 +166,17 @@ long pendingPostCount() { return (long)pending.size(); }
 
 void flushDeferredPosts() {
     if (pending.empty()) return;
-    if (pendingDone && settings.pollDone) gpu.waitDone(pendingDone);
-    else gpu.sync();
+    if (settings.pollDone) {
+        // records of batches and replays: a launch behind them sets the word
+        if (!pendingDone) {
+            pendingDone = ++gpu.doneSeq;
+            dvmh_hip_signal(gpu.doneDev, pendingDone, gpu.stream);
+            HIP_CHECK(hipGetLastError());
+        }
+        gpu.waitDone(pendingDone);
+    } else {
+        gpu.sync();
+    }
     pendingDone = 0;
     for (auto &p : pending) {
         p.red->postValues(p.val, p.loc);
