@@ -148,11 +148,25 @@ class Loop:
                 hi[a] = d if hi[a] is None else max(hi[a], d)
         return [(l or 0, h or 0) for l, h in zip(lo, hi)]
 
+    def unconditional(self):
+        """Every iteration makes every access of the body (no branch, loop or
+        short-circuit), so each index of the loop's box moved by the body's
+        offsets lies inside the array and may be loaded ahead.  A guarded access
+        (`if (i > 0) .. A[i - 1]`) may not: its array may end where the loop does."""
+        if re.search(r'\b(if|else|for|while|do|switch|case|goto|continue|break|return)\b|\?|&&|\|\|', self.body):
+            return False
+        # a macro of the program's may choose between its arguments (Max and Min read both)
+        known = {'fabs', 'fabsf', 'sqrt', 'sqrtf', 'exp', 'expf', 'log', 'logf', 'sin', 'cos', 'tan', 'pow', 'fmax', 'fmin', 'fma',
+                 'abs', 'labs', 'Max', 'Min', 'sizeof'}
+        return all(m in known for m in re.findall(r'\b([A-Za-z_]\w*)\s*\(', self.body))
+
     def star_array(self):
         """Rank 3: the one array of a plain 4- or 8-byte type that the body only reads,
         at the loop point and at neighbours along one axis at a time: its planes
         can live in registers (starMarch).  None if there is no such array, or
         more than one array is read beside the loop point."""
+        if not self.unconditional():
+            return None
         near = [p for p in self.arrays if self.rank == 3 and self._is_stencil(p[1]) and any(lo or hi for lo, hi in self.stencil_range(p[1]))]
         if len(near) != 1 or len(self.body) > 2000:
             return None
@@ -194,10 +208,10 @@ class Loop:
         """Rank 2 or 3, every loop axis in the ACROSS clause with widths <= 1;
         the body reads the ACROSS array at X[i + d0][j + d1].. with at most one
         offset, |offset| <= 1, writes it at the loop point only, touches any
-        other array it writes at the loop point only, and assigns no scalar: the
-        sweep can then run as one dataflow launch (nothing but the ACROSS array
+        other array it writes at the loop point only, and assigns no scalar, all
+        of it unconditionally: the sweep can then run as one dataflow launch (nothing but the ACROSS array
         passes between its workgroups)."""
-        if not self.across or self.rank not in (2, 3):
+        if not self.across or self.rank not in (2, 3) or not self.unconditional():
             return False
         w = self.across['widths']
         if len(w) != self.rank or any(lo > 1 or hi > 1 or (lo == 0 and hi == 0) for lo, hi in w):
@@ -1231,7 +1245,7 @@ def parallel_own_shape(L):
           IND + f'tune[DVMH_AMD_T_DEPTH] = {8 if r == 3 else 4};']
     if r == 3:
         b.append(IND + 'threads = dim3(64, 4, 1);')
-        if L.stencil:
+        if L.stencil and L.unconditional():
             b.append(IND + 'if (cnt2 >= 128 && cnt0 * cnt1 * cnt2 >= 280L * 280 * 280) { tune[DVMH_AMD_T_VARIANT] = 1; tune[DVMH_AMD_T_TILE_A] = 2; tune[DVMH_AMD_T_CHUNK] = 32; }')
     else:
         b.append(IND + f'threads = cnt{r - 1} >= 128 ? dim3(128, 4, 1) : dim3(64, 8, 1);')
@@ -3416,6 +3430,8 @@ def across_handler(L):
     for i in range(r):
         b.append(f'DvmType cnt{i} = (boundsHigh[{i}] - boundsLow[{i}]) / loopSteps[{i}] + 1;')
     first = True
+    # (the staged sweeps load ahead: only bodies without guarded accesses take them unasked)
+    own = 'tune[DVMH_AMD_T_OWN]' if L.unconditional() else 'false'
     # one dependent axis: line kernels for each possible axis
     for dep in range(r):
         mask = 1 << (r - 1 - dep)
@@ -3431,7 +3447,7 @@ def across_handler(L):
             b.append(IND + '// REG (TILE_B = 1): the walk on a register copy, 32-bit indices only (the slot arithmetic must fold)')
             b.append(IND + '// configuration chosen by nobody: the streamed sweep wherever it applies (64^3 31 -> 9 us, 128^3 58 -> 13,')
             b.append(IND + '// 256^3 135 -> 50 against the direct sweep in the default 32 x 8 block)')
-            b.append(IND + f'if (tune[DVMH_AMD_T_OWN] && {X}_tfm == 0 && {X}_devHdr[{r}] == 1 && kernelIndexT == rt_INT && (loopSteps[{r - 1}] == 1 || loopSteps[{r - 1}] == -1) && sizeof({xct}) >= 4 && sizeof({xct}) <= 8) {{')
+            b.append(IND + f'if ({own} && {X}_tfm == 0 && {X}_devHdr[{r}] == 1 && kernelIndexT == rt_INT && (loopSteps[{r - 1}] == 1 || loopSteps[{r - 1}] == -1) && sizeof({xct}) >= 4 && sizeof({xct}) <= 8) {{')
             b.append(IND * 2 + 'tune[DVMH_AMD_T_VARIANT] = 3;')
             b.append(IND * 2 + 'threads = dim3(128, 1, 1);')
             b.append(IND + '}')
@@ -3457,7 +3473,7 @@ def across_handler(L):
             b.append(IND + '// register-staged line sweep: unit steps, natural layout, 32-bit indices;')
             b.append(IND + '// also where nobody chose a configuration (outermost axis 64^3 26 -> 10 us, 128^3 41 -> 15, 256^3 89 -> 44;')
             b.append(IND + '// middle axis 20 -> 9, 36 -> 12, 90 -> 41, against the direct sweep in the default 32 x 8 block)')
-            b.append(IND + f'if (tune[DVMH_AMD_T_OWN] && {X}_tfm == 0 && kernelIndexT == rt_INT && (loopSteps[{dep}] == 1 || loopSteps[{dep}] == -1)) {{')
+            b.append(IND + f'if ({own} && {X}_tfm == 0 && kernelIndexT == rt_INT && (loopSteps[{dep}] == 1 || loopSteps[{dep}] == -1)) {{')
             b.append(IND * 2 + 'tune[DVMH_AMD_T_VARIANT] = 2;')
             b.append(IND * 2 + 'tune[DVMH_AMD_T_TILE_A] = 16;')
             b.append(IND * 2 + 'threads = dim3(64, 1, 1);')
