@@ -2783,23 +2783,27 @@ def flow_kernel(L):
     return out
 
 
+def flow_tiles(L):
+    """Handler lines: the tile counts of the dataflow launch."""
+    sh = f'dvmh_dev::FlowShape<{L.rank}>'
+    return [f'DvmType flowA = (cnt0 + {sh}::PA - 1) / {sh}::PA;',
+            f'DvmType flowB = {f"(cnt1 + {sh}::PB - 1) / {sh}::PB" if L.rank == 3 else "1"};',
+            'DvmType flowTiles = flowA * flowB;']
+
+
 def flow_check(L, conds, sweeps):
-    """Handler lines: `flow` (the dataflow launch applies: `conds`, unit forward
-    steps, unit stride, room for its workspace dvmh_ws) and its tile counts."""
+    """Handler lines after flow_tiles: `flow` (the dataflow launch applies:
+    `conds`, unit forward steps, unit stride, no more tasks and no longer rows
+    than it can address, room for its workspace dvmh_ws)."""
     X = L.across['array']
     r = L.rank
-    xct = [p for p in L.arrays if p[1] == X][0][2]
-    sh = f'dvmh_dev::FlowShape<{r}>'
-    conds = conds + [f'loopSteps[{i}] == 1' for i in range(r)] + [f'{X}_devHdr[{r}] == 1', f'cnt{r - 1} < (1L << 30)',
-                                                                  f'flowTiles * {sweeps} < (1L << 31)']
-    b = [f'DvmType flowA = (cnt0 + {sh}::PA - 1) / {sh}::PA;',
-         f'DvmType flowB = {f"(cnt1 + {sh}::PB - 1) / {sh}::PB" if r == 3 else "1"};',
-         'DvmType flowTiles = flowA * flowB;',
-         'DvmhAmdFlow dvmh_ws;',
-         'bool flow = ' + ' && '.join(conds) + ';',
-         f'if (flow) flow = dvmh_amd_flow_workspace_C(flowTiles * {sweeps}, flowTiles * {r - 1} * dvmh_dev::flowBlocks({r}, cnt{r - 1}) * '
-         '(dvmh_dev::FLOW_CELLS_BYTES / 8), &dvmh_ws) != 0;']
-    return b
+    conds = conds + [f'loopSteps[{i}] == 1' for i in range(r)] + [
+        f'{X}_devHdr[{r}] == 1', f'dvmh_dev::flowBlocks({r}, cnt{r - 1}) <= dvmh_dev::FLOW_BLOCKS_MAX',
+        f'flowTiles * {sweeps} <= dvmh_dev::FLOW_TASKS_MAX']
+    return ['DvmhAmdFlow dvmh_ws;',
+            'bool flow = ' + ' && '.join(conds) + ';',
+            f'if (flow) flow = dvmh_amd_flow_workspace_C(flowTiles * {sweeps}, flowTiles * {r - 1} * dvmh_dev::flowBlocks({r}, cnt{r - 1}) * '
+            '(dvmh_dev::FLOW_CELLS_BYTES / 8), &dvmh_ws) != 0;']
 
 
 def flow_launches(L, kernel, sweeps, tail_args):
@@ -2829,11 +2833,11 @@ def flow_launches(L, kernel, sweeps, tail_args):
 def flow_launch(L, otherwise):
     """The dataflow launch where it applies -- unit forward steps, natural
     layouts, room for its workspace -- else `otherwise`.  No size is left to
-    the other kernels: they pay a launch (4-14 us) per hyperplane or
+    the other kernels while its faces and tasks can be addressed: they pay a launch (4-14 us) per hyperplane or
     tile-plane, this one about 5 us per tile of a diagonal and 0.13-0.17 us per
     step.  One sweep: 2-D 998^2 0.38 against 9.2 ms; 3-D 128^3 0.145 against
     0.43 ms, 318^3 0.48 against 1.84."""
-    b = flow_check(L, [f'{p[1]}_tfm == 0' for p in L.arrays], '1')
+    b = flow_tiles(L) + flow_check(L, [f'{p[1]}_tfm == 0' for p in L.arrays], '1')
     b.append('if (flow) {')
     b += [IND + ln for ln in handler_reds_prepare(L, 'flowTiles', 0) + red_finish_query(L, 'flowTiles')]
     b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 0);')
@@ -3354,7 +3358,10 @@ def chain_handler(L):
         b.append(IND + f'if (dvmh_amd_batch_param_C(batchRef, li, {pi}) != dvmh_amd_batch_param_C(batchRef, 0, {pi})) chained = false;')
     b.append('}')
     b += [f'DvmType cnt{a} = (boundsHigh[{a}] - boundsLow[{a}]) / loopSteps[{a}] + 1;' for a in range(3)]
-    b.append(f'const long most = nl < {CHAIN_SWEEPS} ? nl : {CHAIN_SWEEPS};   // sweeps per launch')
+    b += flow_tiles(L)
+    b.append('// sweeps per launch')
+    b.append(f'long most = nl < {CHAIN_SWEEPS} ? nl : {CHAIN_SWEEPS};')
+    b.append('if (flowTiles * most > dvmh_dev::FLOW_TASKS_MAX) most = flowTiles < dvmh_dev::FLOW_TASKS_MAX ? dvmh_dev::FLOW_TASKS_MAX / flowTiles : 1;')
     b += flow_check(L, ['chained'], 'most')
     b.append('if (!flow) {')
     b.append(IND + '// one sweep after another through the ordinary handler')

@@ -699,6 +699,12 @@ struct FlowCells {
 // Blocks of a face's cells: one per block of steps of the tile, at most this many.
 __host__ __device__ inline long flowBlocks(int rank, long n) { return (n + (rank == 3 ? 14 : 63) + 7 + 7) >> 3; }
 
+// A face is addressed by 32-bit byte offsets, up to sixteen blocks past its
+// last (those read as no cell): longer rows take another kernel.
+constexpr long FLOW_BLOCKS_MAX = (1L << 31) / FLOW_CELLS_BYTES - 16;
+// Tiles and sweeps of a launch: a wave each, and a launch has fewer than 2^32 work-items.
+constexpr long FLOW_TASKS_MAX = (1L << 26) - 1;
+
 // Lane l gets lane l - 1's x, lane 0 gets `first` (whole wave active).
 template <typename T>
 __device__ __forceinline__ T laneBelow(T x, T first) {
