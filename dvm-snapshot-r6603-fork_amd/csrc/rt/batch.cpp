@@ -158,7 +158,7 @@ static void runBatchGroup(std::vector<Loop *> &group) {
         ctx.specs.push_back(sl);
     }
     DvmType ref = (DvmType)&ctx;
-    callHandler(group[0]->batchH, &ref);
+    callGpuHandler(group[0]->batchH, &ref);
     for (SpecLoop *sl : ctx.specs) gpuRedFinishFlush(sl);   // finishes requested per loop, if any
     // a configuration the tuner explores on this group (picked through the
     // first loop's reference) is timed from its pick to here, per loop
@@ -209,7 +209,7 @@ void runPairGroup(const std::vector<Loop *> &firsts, const std::vector<Loop *> &
     HandlerDesc h;
     h.func = func;
     DvmType ref = (DvmType)&ctx;
-    callHandler(h, &ref);
+    callGpuHandler(h, &ref);
     if (!ctx.declined) {
         for (SpecLoop *sl : ctx.specs) gpuRedFinishFlush(sl);
         for (SpecLoop *sl : ctx.specs2) gpuRedFinishFlush(sl);

@@ -176,7 +176,7 @@ void Gpu::trimCache() {
     for (auto &kv : freeBlocks)
         for (void *p : kv.second) HIP_CHECK(hipFree(p));
     freeBlocks.clear();
-    if (!graphsExist() && !graphCapturing()) flowRetire(true);
+    if (!graphsExist() && !graphCapturing() && !flowHeld) flowRetire(true);
 }
 
 // Zeroes a dataflow workspace outside the runtime's stream (which may be
@@ -219,7 +219,7 @@ bool Gpu::flowWorkspace(long tiles, long cellWords, DvmhAmdFlow *out) {
         }
         flowSpaces.push_back(FlowSpace{(char *)p, need});
         flowZero(flowSpaces.back());
-        if (!graphCapturing() && !graphsExist()) flowRetire(false);
+        if (!graphCapturing() && !graphsExist() && !flowHeld) flowRetire(false);
     }
     if (!graphCapturing()) flowCheckWrap();
     char *p = flowSpaces.back().p;
@@ -227,6 +227,7 @@ bool Gpu::flowWorkspace(long tiles, long cellWords, DvmhAmdFlow *out) {
     out->flags = (unsigned long long *)(p + head);
     out->cells = (unsigned long long *)(p + head + flags);
     out->wrapped = flowWrappedDev;
+    flowHeld = true;
     return true;
 }
 

@@ -41,6 +41,11 @@ void callHandler(const HandlerDesc &h, DvmType *pLoopRef, const std::vector<void
     table[p.size()]((void *)h.func, pLoopRef, p.data());
 }
 
+void callGpuHandler(const HandlerDesc &h, DvmType *pLoopRef) {
+    callHandler(h, pLoopRef);
+    gpu.flowHeld = false;
+}
+
 // ------------------------------------------------------------ loop helpers
 Loop::~Loop() { magic = 0; }
 
@@ -454,7 +459,7 @@ void performLoopNow(Loop *loop) {
     loop->spec = &sl;
     DvmType ref = (DvmType)&sl;
     if (onGpu) {
-        callHandler(loop->gpuH, &ref);
+        callGpuHandler(loop->gpuH, &ref);
         gpuRedFinishFlush(&sl);
         rt.loopsOnGpu++;
         // executions the tuner explores are timed from its pick to here; settled

@@ -92,6 +92,7 @@ public:
     // workspace of dataflow launches (one at a time on the stream): the current
     // one and, while graphs that use them exist, smaller earlier ones
     bool flowWorkspace(long tiles, long cellWords, DvmhAmdFlow *out);
+    bool flowHeld = false;                   // a running handler holds the current one (and what it allocates after may run short)
     void flowCheckWrap();                    // starts the tags over when a launch has said they run out
     void flowRetire(bool all);               // frees the earlier ones (all: the current one too)
     void waitDone(unsigned long long seq);   // until the word reaches seq (or the stream drains)
@@ -349,6 +350,7 @@ long rtTypeSize(int rtType);
 
 // handler trampoline (rts/dvmh/util.cpp:659-720)
 void callHandler(const HandlerDesc &h, DvmType *pLoopRef, const std::vector<void *> *override = nullptr);
+void callGpuHandler(const HandlerDesc &h, DvmType *pLoopRef);   // what the handler was lent is its own until it returns
 
 // loop execution
 void performLoop(Loop *loop);

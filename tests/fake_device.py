@@ -79,7 +79,7 @@ def loop(r, lib, handler, base, ranges, params, reds=(), across=None, chain=None
     rt.dvmh_loop_map_C(l, base, L(len(ranges)), *[L(rt.dvmh_alignment_linear_C(L(a + 1), L(1), L(0))) for a in range(len(ranges))])
     if across:
         rt.dvmh_loop_across_C(l, L(0), base, L(len(ranges)), *[L(w) for w in across])
-    for func, v in reds:
+    for func, v in reds:   # (values: double)
         rt.dvmh_loop_reduction_C(l, L(func), ctypes.byref(v), L(INT_DOUBLE), L(1), None, L(0))
     fn = getattr(D.load(lib), handler) if isinstance(handler, str) else handler
     refs = [p if isinstance(p, ctypes.Array) else ctypes.byref(p) for p in params]

@@ -80,3 +80,39 @@ tiles = 1024 * 1024
 assert sum(g for _, g in got) == 130 * tiles and all(g % tiles == 0 and g * 64 < 1 << 32 for _, g in got), got
 assert all('chain' in n for n, _ in got)
 ''')
+
+
+def test_workspace_outlives_an_allocation_that_runs_short():
+    """A handler is handed the workspace, then allocates its partials; where
+    the device has no room left for them, what is freed to make some must not
+    be the workspace.  After the handler it may be."""
+    fake_device.run(LOOPS + '''
+class Flow(ctypes.Structure):
+    _fields_ = [('control', ctypes.c_void_p), ('flags', ctypes.c_void_p), ('cells', ctypes.c_void_p), ('wrapped', ctypes.c_void_p)]
+A = T.array(16, 16, 16)
+seen = []
+@ctypes.CFUNCTYPE(None, ctypes.POINTER(T.L))
+def handler(ref):
+    ws, part = Flow(), ctypes.c_void_p()
+    assert T.rt.dvmh_amd_flow_workspace_C(T.L(100), T.L(1 << 20), ctypes.byref(ws))
+    assert F.fake_live(ws.control) and F.fake_live(ws.cells)
+    # (a block the cache can give back, so that the retry finds room)
+    F.fake_capacity(F.fake_used())
+    refused = F.fake_refused()
+    T.rt.dvmh_loop_cuda_register_red_C(T.L(ref[0]), T.L(1), ctypes.byref(part), None)
+    T.rt.dvmh_loop_cuda_red_prepare_C(T.L(ref[0]), T.L(1), T.L(1 << 17), T.L(0))
+    assert F.fake_refused() > refused and F.fake_live(part.value)
+    assert F.fake_live(ws.control) and F.fake_live(ws.cells)
+    seen.append(ws.cells)
+r = T.region(A)
+spare = T.array(1 << 18)
+T.rt.dvmh_region_end_C(T.region(spare))
+T.rt.dvmh_delete_object_(spare)
+T.loop(r, None, handler, A, [(1, 14)] * 3, [], reds=[(3, e)])
+T.rt.dvmh_region_end_C(r)
+assert seen and F.fake_live(seen[0])
+F.fake_capacity(F.fake_used())
+B = T.array(1 << 17)
+T.rt.dvmh_region_end_C(T.region(B))
+assert not F.fake_live(seen[0])
+''')
