@@ -56,6 +56,7 @@ RED_FUNC = {'sum': 'rf_SUM', 'prod': 'rf_PROD', 'max': 'rf_MAX', 'min': 'rf_MIN'
 RED_OP = {'sum': 'OpSum', 'prod': 'OpProd', 'max': 'OpMax', 'min': 'OpMin', 'and': 'OpAnd', 'or': 'OpOr', 'xor': 'OpXor'}
 OMP_RED = {'sum': '+', 'prod': '*', 'max': 'max', 'min': 'min', 'and': '&', 'or': '|', 'xor': '^'}
 IND = '    '
+FLOW_TYPES = ('char', 'int', 'long', 'float', 'double')   # element types of the dataflow launch
 
 
 def indent(text, n):
@@ -218,7 +219,7 @@ class Loop:
             return False
         X = self.across['array']
         arr = [p for p in self.arrays if p[1] == X]
-        if not arr or arr[0][3] != self.rank or arr[0][2] not in ('char', 'int', 'long', 'float', 'double'):
+        if not arr or arr[0][3] != self.rank or arr[0][2] not in FLOW_TYPES:
             return False
         assign = r'(?:=(?!=)|\+=|-=|\*=|/=|%=|&=|\|=|\^=|<<=|>>=|\+\+|--)'
 

@@ -791,7 +791,15 @@ struct LaneRow {
 
 // x is in its register here (its load is issued before, not sunk to its use).
 template <typename T>
-__device__ __forceinline__ void readHere(T &x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ void readHere(T &x) {
+    if constexpr (sizeof(T) < 4) {   // (no register of its own width)
+        int w = x;
+        asm volatile("" : "+v"(w));
+        x = (T)w;
+    } else {
+        asm volatile("" : "+v"(x));
+    }
+}
 
 // ------------------------------------------------------------------ star march
 // One wave marches nz planes (axis 0) over R rows (axis 1) of 64 * C points of
