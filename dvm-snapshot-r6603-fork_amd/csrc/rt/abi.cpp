@@ -424,6 +424,7 @@ extern "C" void *dvmh_get_natural_base_C(DvmType deviceNum, const DvmType dvmDes
     DVMH_CHECK(deviceNum == 0 || deviceNum == 1, "Illegal device number %ld passed to dvmh_get_natural_base_C", deviceNum);
     Data *d = asData(dvmDesc, "dvmh_get_natural_base_C");
     if (deviceNum == 0) return d->hostNaturalBase();
+    gpu.closeLaunch();
     return d->hasDev ? d->devNaturalBase() : nullptr;
 }
 
@@ -431,6 +432,7 @@ extern "C" void *dvmh_get_device_addr_C(DvmType deviceNum, const void *addr) {  
     if (deviceNum == 0) return (void *)addr;
     Data *d = regularVarOf(addr);
     DVMH_CHECK(d != nullptr, "Can not get device address of unknown variable %p", addr);
+    gpu.closeLaunch();
     return d->hasDev ? d->dev.ptr : nullptr;
 }
 
@@ -440,6 +442,7 @@ extern "C" DvmType dvmh_fill_header_C(DvmType deviceNum, const void *baseAddr, c
     Data *d = asData(dvmDesc, "dvmh_fill_header_C");
     DVMH_CHECK(devHeader != nullptr, "NULL header passed to dvmh_fill_header_C");
     if (deviceNum == 1 && d->hasDev) {
+        gpu.closeLaunch();
         d->fillDevHeader(baseAddr, devHeader, extendedParams);
         return (d->dev.isTransformed(d->rank) ? 1 : 0) + (d->dev.isDiagonalized() ? 1 : 0);
     }

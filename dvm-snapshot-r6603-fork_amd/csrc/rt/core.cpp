@@ -138,6 +138,12 @@ void Gpu::waitDone(unsigned long long seq) {
     }
 }
 
+void Gpu::closeLaunch() {
+    if (!launchOpen || inHandler) return;
+    sync();
+    launchOpen = false;
+}
+
 void *Gpu::alloc(size_t bytes) {
     if (bytes == 0) bytes = 8;
     size_t rounded = (bytes + 255) & ~(size_t)255;
@@ -280,6 +286,7 @@ const char *Gpu::fetchBlock(const void *src, const long sizes[], const long orig
     dvmh_hip_fetch(src, sizes, origin, lo, hi, rank, typeSize, fetchDev, doneDev, seq, stream);
     HIP_CHECK(hipGetLastError());
     waitDone(seq);
+    launchOpen = false;   // (a launch of its own, behind every loop)
     return fetchHost;
 }
 

@@ -42,7 +42,9 @@ void callHandler(const HandlerDesc &h, DvmType *pLoopRef, const std::vector<void
 }
 
 void callGpuHandler(const HandlerDesc &h, DvmType *pLoopRef) {
+    gpu.inHandler++;
     callHandler(h, pLoopRef);
+    gpu.inHandler--;
     gpu.flowHeld = false;
 }
 
@@ -154,10 +156,11 @@ char *mappedDevicePtr(char *h) {
     return (char *)d;
 }
 
-// Completion word value that covers every pending post, 0 when one of them
-// came from a path without it (batches, graph replays): then the stream is
-// synchronised.
+// Completion word value that covers every pending post, 0 when the last came
+// from a path without it (batches, graph replays): a launch behind them sets it
+// then.  pendingOwn: the loop whose reductions they are sets it itself.
 static unsigned long long pendingDone = 0;
+static bool pendingOwn = false;
 
 void flushPostsFor(const void *addr) {
     for (auto &p : pending)
@@ -177,10 +180,13 @@ void flushDeferredPosts() {
             pendingDone = ++gpu.doneSeq;
             dvmh_hip_signal(gpu.doneDev, pendingDone, gpu.stream);
             HIP_CHECK(hipGetLastError());
+            pendingOwn = false;
         }
         gpu.waitDone(pendingDone);
+        gpu.launchOpen = pendingOwn;
     } else {
         gpu.sync();
+        gpu.launchOpen = false;
     }
     pendingDone = 0;
     for (auto &p : pending) {
@@ -313,6 +319,7 @@ void gpuRedFinishFlush(SpecLoop *sl) {
             r->resVal = r->resLoc = nullptr;
         }
         pendingDone = sl->redSeq;
+        pendingOwn = true;
         releasePartials();
         return;
     }
@@ -370,7 +377,10 @@ void gpuRedFinishFlush(SpecLoop *sl) {
         const unsigned long long seq = signal ? ++gpu.doneSeq : 0;
         dvmh_hip_reduce_finish_multi(group[0]->r->rtType, (int)group.size(), d, gpu.finishCounters, signal ? gpu.doneDev : nullptr,
                 seq, sl->stream);
-        if (signal) pendingDone = seq;
+        if (signal) {
+            pendingDone = seq;
+            pendingOwn = false;
+        }
         for (void *p : slots) gpu.release(p);
     }
     releasePartials();

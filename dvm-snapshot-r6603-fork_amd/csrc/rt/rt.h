@@ -96,6 +96,13 @@ public:
     void flowCheckWrap();                    // starts the tags over when a launch has said they run out
     void flowRetire(bool all);               // frees the earlier ones (all: the current one too)
     void waitDone(unsigned long long seq);   // until the word reaches seq (or the stream drains)
+    // A loop that folds its own reductions sets the word from its last
+    // workgroup: its launch, and with it what it stored to arrays, may end
+    // later.  Work on the runtime's stream comes after it anyway; a reader
+    // elsewhere must not get a device address before it has ended.
+    bool launchOpen = false;
+    int inHandler = 0;                       // GPU handlers running (their launches are on the stream)
+    void closeLaunch();                      // device addresses are about to leave the runtime
     void init();
     void *alloc(size_t bytes);          // size-keyed cache in front of hipMalloc
     void release(void *p);              // back to the cache
