@@ -64,6 +64,98 @@ def indent(text, n):
     return ''.join(pad + ln if ln.strip() else ln for ln in text.splitlines(True))
 
 
+# Calls that evaluate their arguments and return (a macro of another name may
+# choose between its arguments, or jump).
+PLAIN_CALLS = {'fabs', 'fabsf', 'sqrt', 'sqrtf', 'exp', 'expf', 'log', 'logf', 'sin', 'sinf', 'cos', 'cosf', 'tan', 'tanf', 'pow', 'powf',
+               'fmax', 'fmaxf', 'fmin', 'fminf', 'fma', 'fmaf', 'abs', 'labs', 'Max', 'Min', 'MAX', 'MIN', 'max', 'min'}
+
+
+def reached(body):
+    """Per character of a loop body, whether every iteration evaluates what
+    stands there: not under if, else, a loop or a switch, not to the right of ?:, &&
+    or || in its expression, not in or behind a call that is none of PLAIN_CALLS,
+    and not behind a jump or a label.  Where in doubt, False."""
+    text = re.sub(r'/\*.*?\*/|//[^\n]*|"(?:\\.|[^"\\])*"|\'(?:\\.|[^\'\\])*\'', lambda m: ' ' * len(m.group()), body, flags=re.S)
+    out = [False] * len(text)
+    if '#' in text:
+        return out
+    ended = False   # behind a jump or a call that may hide one
+
+    def closing(i):
+        """Behind the bracket that closes the one at i."""
+        depth = 0
+        for k in range(i, len(text)):
+            depth += (text[k] in '([{') - (text[k] in ')]}')
+            if depth == 0:
+                return k + 1
+        raise ValueError
+
+    def expression(a, b, sure):
+        nonlocal ended
+        stop = b
+        for m in re.finditer(r'\?|&&|\|\||\b([A-Za-z_]\w*)\s*\(', text[a:b]):
+            if m.group(1) in PLAIN_CALLS:
+                continue
+            stop = min(stop, a + m.start())
+            if m.group(1):
+                break
+        for k in range(a, stop):
+            out[k] = sure and not ended
+        ended = ended or any(c not in PLAIN_CALLS for c in re.findall(r'\b([A-Za-z_]\w*)\s*\(', text[a:b]))
+
+    def blank(i):
+        while i < len(text) and text[i].isspace():
+            i += 1
+        return i
+
+    def statement(i, sure):
+        """Marks the statement at i; returns the position behind it."""
+        nonlocal ended
+        i = blank(i)
+        if text[i] == '{':
+            end = closing(i) - 1
+            i = blank(i + 1)
+            while i < end:
+                i = blank(statement(i, sure))
+            return end + 1
+        word = re.match(r'[A-Za-z_]\w*', text[i:])
+        word = word.group() if word else ''
+        if word in ('if', 'for', 'while', 'switch'):
+            a = blank(i + len(word))
+            b = closing(a)
+            if word == 'for':
+                parts = [a + 1 + m.start() for m in re.finditer(';', text[a + 1:b - 1])]
+                expression(a + 1, parts[0], sure)
+                expression(parts[0], parts[1], sure)
+                expression(parts[1], b - 1, False)
+            else:
+                expression(a + 1, b - 1, sure)
+            i = statement(b, False)
+            if word == 'if' and re.match(r'else\b', text[blank(i):]):
+                i = statement(blank(i) + 4, False)
+            return i
+        if word == 'do':
+            i = blank(statement(i + 2, False))
+            return text.index(';', i) + 1
+        if word in ('break', 'continue', 'return', 'goto', 'case', 'default', 'asm') or re.match(r'[A-Za-z_]\w*\s*:', text[i:]):
+            ended = True
+        depth = 0
+        for k in range(i, len(text)):
+            depth += (text[k] in '([{') - (text[k] in ')]}')
+            if depth == 0 and text[k] == ';':
+                expression(i, k, sure)
+                return k + 1
+        raise ValueError
+
+    try:
+        i = blank(0)
+        while i < len(text):
+            i = blank(statement(i, True))
+    except (ValueError, IndexError):
+        return [False] * len(text)
+    return out
+
+
 class Loop:
     def __init__(self, d, prog):
         self.prog = prog
@@ -135,41 +227,46 @@ class Loop:
 
     def stencil_range(self, name):
         """Per loop axis, the (lowest, highest) offset at which the body reads
-        `name` (each in -1..1).  Every index of [lo + lowest, last + highest]
-        on an axis is read by some iteration, so a load clamped into that range
-        stays inside the array."""
-        lo = [None] * self.rank
-        hi = [None] * self.rank
-        for m in re.finditer(r'\b' + name + r'\s*((?:\[[^\[\]]*\]\s*)+)', self.body):
-            idx = re.findall(r'\[([^\[\]]*)\]', m.group(1))
-            for a, ((v, _), e) in enumerate(zip(self.vars, idx)):
-                mm = re.fullmatch(r'\s*' + v + r'\s*(?:([+-])\s*([01])\s*)?', e)
-                d = 0 if not mm.group(1) else (int(mm.group(2)) if mm.group(1) == '+' else -int(mm.group(2)))
-                lo[a] = d if lo[a] is None else min(lo[a], d)
-                hi[a] = d if hi[a] is None else max(hi[a], d)
-        return [(l or 0, h or 0) for l, h in zip(lo, hi)]
+        `name` (each in -1..1): a load ahead is clamped into
+        [lo + lowest, last + highest] on each axis."""
+        offs = [off for _, off in self.accesses(name)] or [[0] * self.rank]
+        return [(min(o[a] for o in offs), max(o[a] for o in offs)) for a in range(self.rank)]
 
-    def unconditional(self):
-        """Every iteration makes every access of the body (no branch, loop or
-        short-circuit), so each index of the loop's box moved by the body's
-        offsets lies inside the array and may be loaded ahead.  A guarded access
-        (`if (i > 0) .. A[i - 1]`) may not: its array may end where the loop does."""
-        if re.search(r'\b(if|else|for|while|do|switch|case|goto|continue|break|return)\b|\?|&&|\|\|', self.body):
-            return False
-        # a macro of the program's may choose between its arguments (Max and Min read both)
-        known = {'fabs', 'fabsf', 'sqrt', 'sqrtf', 'exp', 'expf', 'log', 'logf', 'sin', 'cos', 'tan', 'pow', 'fmax', 'fmin', 'fma',
-                 'abs', 'labs', 'Max', 'Min', 'sizeof'}
-        return all(m in known for m in re.findall(r'\b([A-Za-z_]\w*)\s*\(', self.body))
+    def accesses(self, name):
+        """(position in the body, offset per axis) of each access
+        name[v0 +- 0/1][v1 +- 0/1].. ."""
+        out = []
+        for m in re.finditer(r'\b' + name + r'\s*((?:\[[^\[\]]*\]\s*)+)', self.body):
+            off = []
+            for (v, _), e in zip(self.vars, re.findall(r'\[([^\[\]]*)\]', m.group(1))):
+                mm = re.fullmatch(r'\s*' + v + r'\s*(?:([+-])\s*([01])\s*)?', e)
+                off.append(0 if not mm.group(1) else (int(mm.group(2)) if mm.group(1) == '+' else -int(mm.group(2))))
+            out.append((m.start(), off))
+        return out
+
+    def loads_ahead(self, name):
+        """Every index of the loop's box moved by the offsets at which the body
+        accesses `name` lies inside the array, so that it may be loaded ahead of
+        the body: every iteration reaches the lowest and the highest offset of
+        each axis.  Where a condition guards such an access
+        (`if (i > 0) .. A[i - 1]`) the array may end where the loop does; other
+        conditions (`if (d > eps) eps = d;`) do not matter."""
+        always = reached(self.body)
+        every, sure = self.accesses(name), [off for at, off in self.accesses(name) if always[at]]
+        return bool(sure) and all(min(o[a] for o in sure) == min(o[a] for _, o in every) and
+                                  max(o[a] for o in sure) == max(o[a] for _, o in every) for a in range(self.rank))
+
+    def leaves(self):
+        """The body may end an iteration early: it cannot be a function's body."""
+        return bool(re.search(r'\b(continue|return|goto)\b', self.body))
 
     def star_array(self):
         """Rank 3: the one array of a plain 4- or 8-byte type that the body only reads,
         at the loop point and at neighbours along one axis at a time: its planes
         can live in registers (starMarch).  None if there is no such array, or
         more than one array is read beside the loop point."""
-        if not self.unconditional():
-            return None
         near = [p for p in self.arrays if self.rank == 3 and self._is_stencil(p[1]) and any(lo or hi for lo, hi in self.stencil_range(p[1]))]
-        if len(near) != 1 or len(self.body) > 2000:
+        if len(near) != 1 or len(self.body) > 2000 or self.leaves() or not self.loads_ahead(near[0][1]):
             return None
         X = near[0][1]
         if near[0][2] not in ('int', 'long', 'float', 'double'):
@@ -209,10 +306,10 @@ class Loop:
         """Rank 2 or 3, every loop axis in the ACROSS clause with widths <= 1;
         the body reads the ACROSS array at X[i + d0][j + d1].. with at most one
         offset, |offset| <= 1, writes it at the loop point only, touches any
-        other array it writes at the loop point only, and assigns no scalar, all
-        of it unconditionally: the sweep can then run as one dataflow launch (nothing but the ACROSS array
-        passes between its workgroups)."""
-        if not self.across or self.rank not in (2, 3) or not self.unconditional():
+        other array it writes at the loop point only, and assigns no scalar, and
+        the ACROSS array may be loaded ahead: the sweep can then run as one
+        dataflow launch (nothing but that array passes between its workgroups)."""
+        if not self.across or self.rank not in (2, 3) or self.leaves():
             return False
         w = self.across['widths']
         if len(w) != self.rank or any(lo > 1 or hi > 1 or (lo == 0 and hi == 0) for lo, hi in w):
@@ -250,7 +347,7 @@ class Loop:
                     return False
             elif any(wr for _, wr in refs) and any(at is None or sum(at) for at, _ in refs):
                 return False
-        return True
+        return self.loads_ahead(X)
 
     def chain_eligible(self):
         """Consecutive executions (sweeps) of the loop may run pipelined by a
@@ -1246,7 +1343,7 @@ def parallel_own_shape(L):
           IND + f'tune[DVMH_AMD_T_DEPTH] = {8 if r == 3 else 4};']
     if r == 3:
         b.append(IND + 'threads = dim3(64, 4, 1);')
-        if L.stencil and L.unconditional():
+        if L.stencil and all(L.loads_ahead(nm) for nm in L.stencil):
             b.append(IND + 'if (cnt2 >= 128 && cnt0 * cnt1 * cnt2 >= 280L * 280 * 280) { tune[DVMH_AMD_T_VARIANT] = 1; tune[DVMH_AMD_T_TILE_A] = 2; tune[DVMH_AMD_T_CHUNK] = 32; }')
     else:
         b.append(IND + f'threads = cnt{r - 1} >= 128 ? dim3(128, 4, 1) : dim3(64, 8, 1);')
@@ -3439,7 +3536,9 @@ def across_handler(L):
         b.append(f'DvmType cnt{i} = (boundsHigh[{i}] - boundsLow[{i}]) / loopSteps[{i}] + 1;')
     first = True
     # (the staged sweeps load ahead: only bodies without guarded accesses take them unasked)
-    own = 'tune[DVMH_AMD_T_OWN]' if L.unconditional() else 'false'
+    own = 'false'
+    if any(L.line_stage_eligible(a) for a in range(r)) and L.loads_ahead(L.across['array']):
+        own = 'tune[DVMH_AMD_T_OWN]'
     # one dependent axis: line kernels for each possible axis
     for dep in range(r):
         mask = 1 << (r - 1 - dep)

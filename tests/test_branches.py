@@ -1,0 +1,156 @@
+"""Loops with branches (programs/branches.cdv).  A condition that stands beside
+the accesses to neighbours keeps the kernels that load ahead; one that guards
+them does not.  Results must equal a sequential evaluation bit for bit."""
+import ctypes
+import os
+import sys
+
+import numpy as np
+import pytest
+
+import dvmh_amd as D
+import helpers as H
+from test_cdvmh import _u01
+
+sys.path.insert(0, os.path.join(H.REPO, 'dvm-snapshot-r6603-fork_amd', 'emit'))
+import hipgen  # noqa: E402
+
+_dp = ctypes.POINTER(ctypes.c_double)
+SEED = D.SEED_BASE + 11
+
+T = 'double t = X[i - 1][j] + X[i + 1][j] + X[i][j - 1] + X[i][j + 1];\n'
+FORMS = [   # body, every neighbour is reached in every iteration
+    (T + 'X[i][j] = t;', True),
+    (T + 'if (t > r) r = t;\nX[i][j] = t;', True),
+    (T + 'r = MAX(r, t);\nX[i][j] = t > 1 ? t : X[i][j];', True),
+    (T + 'r = r > t && t > 0 ? r : t;\nif (t > 0) X[i][j] = t; else { X[i][j] = -t; }', True),
+    (T + 'for (int q = 0; q < 3; q++) t *= 0.5;\nwhile (t > 4) { t -= 1; if (t < 0) break; }\nX[i][j] = t;', True),
+    (T + 'switch ((int)t) { case 0: t = 1; break; default: t = 2; }\nX[i][j] = t;', True),
+    (T + 'X[i][j] = weight(t);', True),
+    ('/* if (i) */ ' + T + 'X[i][j] = t;   // && so on', True),
+    (T + 'if (i > 1) t += X[i - 1][j];\nX[i][j] = t;', True),          # reached anyway
+    ('if (i > 0) { ' + T + ' X[i][j] = t; }', False),
+    ('double t = X[i + 1][j] + X[i][j + 1];\nif (i > 0) t += X[i - 1][j];\nX[i][j] = t + X[i][j - 1];', False),
+    ('double t = i > 0 ? X[i - 1][j] : 0;\nX[i][j] = t + X[i + 1][j] + X[i][j - 1] + X[i][j + 1];', False),
+    ('double t = X[i + 1][j] + X[i][j - 1] + X[i][j + 1];\nX[i][j] = t * (i > 0 && X[i - 1][j] > 0);', False),
+    ('for (int q = 0; q < i; q++) X[i][j] += X[i - 1][j] + X[i][j - 1] + X[i + 1][j] + X[i][j + 1];', False),
+    ('do { if (i < 1) break; X[i][j] += X[i - 1][j]; } while (0);', False),
+    ('SELECT(i > 0, X[i][j]);\n' + T + 'X[i][j] = t;', False),           # may jump
+    ('X[i][j] = weight(X[i - 1][j]);', False),                           # may be a macro that picks
+    ('X[i][j] = X[i][j] > 0 || X[i - 1][j] > 0;', False),
+    ('if (j == 3) goto out;\n' + T + 'X[i][j] = t;\nout: ;', False),
+    ('switch (j) { case 1: X[i][j] = X[i - 1][j]; }', False),
+    ('{ { ' + T + ' } if (r > 0) r = 0; }\nX[i][j] = r;', True),
+    (T + 'X[i][j] = t', False),                                          # no statement: in doubt
+]
+
+
+@pytest.mark.parametrize('body,ahead', FORMS)
+def test_what_may_be_loaded_ahead(body, ahead):
+    L = hipgen.Loop({'name': 'l', 'vars': [('i', 'int'), ('j', 'int')], 'params': [('array', 'X', 'double', 2)],
+                     'reductions': [('max', 'r', 'double')], 'across': {'array': 'X', 'widths': [(1, 1), (1, 1)]}, 'body': body}, 't')
+    assert L.loads_ahead('X') == ahead
+    assert L.flow_eligible() == ahead
+
+
+def test_early_end_keeps_other_kernels():
+    """(a kernel whose body is a function's)"""
+    L = hipgen.Loop({'name': 'l', 'vars': [('i', 'int'), ('j', 'int')], 'params': [('array', 'X', 'double', 2)],
+                     'across': {'array': 'X', 'widths': [(1, 1), (1, 1)]}, 'body': T + 'if (t < 0) continue;\nX[i][j] = t;'}, 't')
+    assert L.loads_ahead('X') and not L.flow_eligible()
+
+
+def _grid(n):
+    return _u01(SEED, np.arange(n ** 3, dtype=np.uint64)).reshape(n, n, n)
+
+
+def sor_reference(n, iters, w):
+    a = _grid(n).tolist()
+    hist = []
+    for _ in range(iters):
+        eps = 0.0
+        for i in range(1, n - 1):
+            for j in range(1, n - 1):
+                row, up, down, left, right = a[i][j], a[i - 1][j], a[i + 1][j], a[i][j - 1], a[i][j + 1]
+                for k in range(1, n - 1):
+                    s = row[k]
+                    t = (up[k] + down[k] + left[k] + right[k] + row[k - 1] + row[k + 1]) / 6.0
+                    d = abs(t - s)
+                    if d > eps:
+                        eps = d
+                    if s > 0.05 and d > 0.001:
+                        row[k] = s + (0.5 * w if d > 0.5 else w) * (t - s)
+        hist.append(eps)
+    return np.array(hist), np.array(a).ravel()
+
+
+def edge_reference(n, iters, w):
+    a = _grid(n).tolist()
+    for _ in range(iters):
+        for i in range(n):
+            for j in range(n):
+                for k in range(n):
+                    t = 0.0
+                    if i > 0:
+                        t += a[i - 1][j][k]
+                    if j > 0:
+                        t += a[i][j - 1][k]
+                    t += a[i][j][k - 1] if k > 0 else 0.5
+                    if i < n - 1:
+                        t += a[i + 1][j][k]
+                    a[i][j][k] = (1 - w) * a[i][j][k] + w * t
+    return None, np.array(a).ravel()
+
+
+def jac_reference(n, iters, c):
+    A = _grid(n)
+    hist = []
+    for _ in range(iters):
+        m = A[1:-1, 1:-1, 1:-1]
+        t = A[:-2, 1:-1, 1:-1] + A[2:, 1:-1, 1:-1] + A[1:-1, :-2, 1:-1] + A[1:-1, 2:, 1:-1] + A[1:-1, 1:-1, :-2] + A[1:-1, 1:-1, 2:]
+        d = np.abs(t / 6.0 - m)
+        hist.append(max(0.0, d.max()))
+        A[1:-1, 1:-1, 1:-1] = np.where(d > 0.3, t / 6.0, m)
+        for i in range(1, n):
+            t = A[i] + c * A[i - 1]
+            A[i] = np.where(t < 2.0, t, A[i])
+        for k in range(1, n):
+            A[:, :, k] = A[:, :, k] + c * A[:, :, k - 1]
+    return np.array(hist), A.ravel()
+
+
+REFERENCE = {'sor3d': sor_reference, 'edge3d': edge_reference, 'jac3d': jac_reference}
+
+
+def run(which, n, iters, factor):
+    f = getattr(D.load('libcdv_branches.so'), 'branch_' + which)
+    f.restype = None
+    hist, out = np.zeros(iters), np.zeros(n ** 3)
+    args = [ctypes.c_long(n), ctypes.c_int(iters), ctypes.c_double(factor), ctypes.c_ulonglong(SEED)]
+    D.runtime()
+    f(*args, *([] if which == 'edge3d' else [H.dp(hist)]), H.dp(out))
+    return (None if which == 'edge3d' else hist), out
+
+
+def check(which, n, iters):
+    factor = 0.2 if which != 'sor3d' else 1.25
+    hist, out = run(which, n, iters, factor)
+    rh, ro = REFERENCE[which](n, iters, factor)
+    assert H.bits_equal(out, ro)
+    assert hist is None or np.array_equal(hist, rh)
+
+
+@pytest.mark.parametrize('which', sorted(REFERENCE))
+def test_host_path(which):
+    if D.stats()['gpu_present']:
+        pytest.skip('the host path runs where no GPU is present; the GPU tests cover this case')
+    check(which, 9, 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('which', sorted(REFERENCE))
+@pytest.mark.parametrize('n', [3, 5, 10, 19, 34, 67])
+def test_gpu(which, n):
+    before = D.stats()['loops_gpu']
+    check(which, n, 2)
+    assert D.stats()['loops_gpu'] > before
