@@ -56,7 +56,8 @@ RED_FUNC = {'sum': 'rf_SUM', 'prod': 'rf_PROD', 'max': 'rf_MAX', 'min': 'rf_MIN'
 RED_OP = {'sum': 'OpSum', 'prod': 'OpProd', 'max': 'OpMax', 'min': 'OpMin', 'and': 'OpAnd', 'or': 'OpOr', 'xor': 'OpXor'}
 OMP_RED = {'sum': '+', 'prod': '*', 'max': 'max', 'min': 'min', 'and': '&', 'or': '|', 'xor': '^'}
 IND = '    '
-FLOW_TYPES = ('char', 'int', 'long', 'float', 'double')   # element types of the dataflow launch
+# element types of the dataflow launch
+FLOW_TYPES = ('char', 'unsigned char', 'int', 'unsigned', 'unsigned int', 'long', 'unsigned long', 'long long', 'unsigned long long', 'float', 'double')
 
 
 def indent(text, n):
