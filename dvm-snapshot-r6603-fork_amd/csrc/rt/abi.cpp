@@ -1145,6 +1145,17 @@ extern "C" void dvmh_loop_fill_bounds_C(DvmType curLoop, DvmType boundsLow[], Dv
     }
 }
 
+extern "C" DvmType dvmh_amd_loop_reads_inside_C(DvmType curLoop, const DvmType dvmDesc[], const DvmType offLow[], const DvmType offHigh[]) {
+    const Loop *l = loopOf(curLoop, "dvmh_amd_loop_reads_inside_C");
+    const Data *d = asData(dvmDesc, "dvmh_amd_loop_reads_inside_C");
+    if (d->rank != l->rank) return 0;
+    for (int i = 0; i < l->rank; i++) {
+        const long first = std::min(l->lo[i], l->hi[i]), last = std::max(l->lo[i], l->hi[i]);
+        if (first + offLow[i] < d->space[i].lo || last + offHigh[i] > d->space[i].hi) return 0;
+    }
+    return 1;
+}
+
 extern "C" DvmType dvmh_loop_get_slot_count_C(DvmType curLoop) {
     Object *o = asObject(curLoop);
     if (o->kind == Kind::SpecLoop && ((SpecLoop *)o)->device == 1) return 1;

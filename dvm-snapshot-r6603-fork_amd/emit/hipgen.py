@@ -257,6 +257,15 @@ class Loop:
         return bool(sure) and all(min(o[a] for o in sure) == min(o[a] for _, o in every) and
                                   max(o[a] for o in sure) == max(o[a] for _, o in every) for a in range(self.rank))
 
+    def inside(self, name, loop='loop_ref', header=None):
+        """Handler lines and an expression: the kernels that load `name` ahead
+        may run.  A guarded access leaves that to where the array ends."""
+        if self.loads_ahead(name):
+            return [], 'true'
+        off = ', '.join(str(min(lo, 0)) for lo, _ in self.stencil_range(name)) + ', ' + ', '.join(str(max(hi, 0)) for _, hi in self.stencil_range(name))
+        return [f'static const DvmType dvmh_{name}_off[{2 * self.rank}] = {{{off}}};'], \
+            f'dvmh_amd_loop_reads_inside_C({loop}, {header or name + "_hdr"}, dvmh_{name}_off, dvmh_{name}_off + {self.rank}) != 0'
+
     def leaves(self):
         """The body may end an iteration early: it cannot be a function's body."""
         return bool(re.search(r'\b(continue|return|goto)\b', self.body))
@@ -1387,6 +1396,10 @@ def parallel_handler(L):
         b.append('int npf = 0;')
         unit = ' && '.join(f'loopSteps[{i}] == 1' for i in range(r))
         shape_ok = 'threads.z == 1' + (' && threads.y == 1' if r == 2 else '')
+        for nm in L.stencil:
+            lines, cond = L.inside(nm)
+            if lines:
+                b += lines + [f'if (variant == 1 && !({cond})) variant = 0;']
         b.append(f'if (variant == 1 && ({unit}) && {shape_ok} && mcols >= 1 && mcols <= 4 && march >= 1) {{')
         rows = '((size_t)threads.y + 2)' if r == 3 else '(size_t)1'
         b.append(IND + f'size_t mplane = {rows} * ((size_t)threads.x * mcols + 2);')
@@ -1753,7 +1766,8 @@ def batch_handler(L):
               '} else {',
               IND + 'bvariant = 0;',
               '}']
-    b += ['int nonunit = 0;',
+    guarded = bm and not all(L.loads_ahead(nm) for nm in L.stencil)
+    b += ['int nonunit = 0;'] + (['int outside = 0;'] if guarded else []) + [
           f'long *desc = (long *)calloc((size_t)nl * {dlen}, sizeof(long));',
          'DvmType *tstart = (DvmType *)calloc((size_t)nl + 1, sizeof(DvmType));',
          'long tiles = 0;',
@@ -1772,6 +1786,10 @@ def batch_handler(L):
             lb.append(f'  d[{lay[("base", nm)]}] = (long)base;')
             for q in range(ar):
                 lb.append(f'  d[{lay[("str", nm)] + q}] = devHdr[{q + 1}];')
+            if nm in L.stencil and bm:
+                lines, cond = L.inside(nm, 'lr', 'hdr')
+                if lines:
+                    lb += ['  ' + ln for ln in lines] + [f'  if (bvariant == 1 && !({cond})) outside = 1;']
             lb.append(f'  for (int q = 0; q < {ar}; q++) if (labs(devHdr[q + 1]) > maxStride) maxStride = labs(devHdr[q + 1]); }}')
         else:
             lb.append(f'd[{lay[("sc", p[1])]}] = (long)dvmh_get_device_addr_C(1, dvmh_amd_batch_param_C(batchRef, li, {pi}));')
@@ -1817,8 +1835,9 @@ def batch_handler(L):
     b.append('}')
     b.append('tstart[nl] = tiles;')
     if bm:
-        # a loop with non-unit steps, or 64-bit indices: every loop of the batch runs the direct tiles
-        b.append('if (bvariant == 1 && (nonunit || wide)) {')
+        # a loop with non-unit steps, 64-bit indices, or loads ahead that could leave its array: every loop of the
+        # batch runs the direct tiles
+        b.append(f'if (bvariant == 1 && (nonunit || wide{" || outside" if guarded else ""})) {{')
         b.append(IND + 'bvariant = 0;')
         b.append(IND + 'tiles = 0;')
         b.append(IND + 'for (long li = 0; li < nl; li++) {')
@@ -2349,6 +2368,10 @@ def pair_handler(L1, L2):
                 lb.append(f'  d[{lay[("base", nm)]}] = (long)base;')
                 for q in range(ar):
                     lb.append(f'  d[{lay[("str", nm)] + q}] = devHdr[{q + 1}];')
+                if mem == 0 and nm in L1.stencil:
+                    lines, cond = L1.inside(nm, 'lr1', 'hdr')
+                    if lines:
+                        lb += ['  ' + ln for ln in lines] + [f'  if (!({cond})) fused = false;']
                 lb.append(f'  for (int q = 0; q < {ar}; q++) if (labs(devHdr[q + 1]) > maxStride) maxStride = labs(devHdr[q + 1]); }}')
             else:
                 lb.append(f'd[{lay[("sc", p[1])]}] = (long)dvmh_get_device_addr_C(1, dvmh_amd_pair_param_C(batchRef, {mem}, li, {pi}));')
@@ -3562,6 +3585,10 @@ def across_handler(L):
             b.append(IND + 'DvmType CK = tune[DVMH_AMD_T_TILE_A], RS = (CK + 2) | 1, REG = tune[DVMH_AMD_T_TILE_B] && kernelIndexT == rt_INT ? 1 : 0;')
             b.append(IND + f'size_t ldsBytes = (((size_t)2 * threads.x * RS * sizeof({xct}) + 15) & ~(size_t)15) + (size_t)threads.x * sizeof(DvmType);')
             cks = ' || '.join(f'CK == {ck}' for ck in LINE_TILE_CK)
+            lines, cond = L.inside(X)
+            b += [IND + ln for ln in lines]
+            if lines:
+                b.append(IND + f'if ((tune[DVMH_AMD_T_VARIANT] == 1 || tune[DVMH_AMD_T_VARIANT] == 3) && !({cond})) tune[DVMH_AMD_T_VARIANT] = 0;')
             b.append(IND + f'bool ltile = tune[DVMH_AMD_T_VARIANT] == 1 && (loopSteps[{r - 1}] == 1 || loopSteps[{r - 1}] == -1) && '
                      f'{X}_tfm == 0 && threads.x <= 256 && threads.y == 1 && threads.z == 1 && ({cks}) && ldsBytes <= 64512;')
             b.append(IND + '// streamed line sweep (variant 3): unit stride along the line, 32-bit indices, whole waves, no dynamic LDS')
@@ -3592,6 +3619,9 @@ def across_handler(L):
             xs = [a for a in range(r) if a != dep]
             span = f'(DvmType)(threads.x - 1) * labs(loopSteps[{xs[-1]}]) * {X}_devHdr[{xs[-1] + 1}]' + (f' + (DvmType)(threads.y - 1) * labs(loopSteps[{xs[-2]}]) * {X}_devHdr[{xs[-2] + 1}]' if len(xs) > 1 else '')
             b.append(IND + '// a chunk of rows and a workgroup\'s lanes lie within 2 GB of each other')
+            lines, cond = L.inside(X)
+            if lines:
+                b += [IND + ln for ln in lines] + [IND + f'if (lreg && !({cond})) lreg = false;']
             b.append(IND + f'lreg = lreg && (CK * {X}_devHdr[{dep + 1}] + {span}) * (DvmType)sizeof({[p for p in L.arrays if p[1] == X][0][2]}) < (1L << 31);')
             b.append(IND + 'if (lreg) {')
             b += [IND * 2 + s for s in line_reg_launch(L, dep)]

@@ -53,6 +53,11 @@ extern "C" {
                                   PAIR: 1 = the pair handler picks its march shape from the pairs' sizes */
 void dvmh_amd_loop_get_tuning_C(DvmType curLoop, DvmType kind, DvmType tune[]);
 
+/* 1 when every index of the loop's box moved by an offset between offLow[i] and
+ * offHigh[i] lies inside the array, axis by axis (loop axis i is array axis i):
+ * a kernel may then load the array ahead of a body that guards its accesses. */
+DvmType dvmh_amd_loop_reads_inside_C(DvmType curLoop, const DvmType dvmDesc[], const DvmType offLow[], const DvmType offHigh[]);
+
 /* ---- in-kernel reduction finish --------------------------------------------------
  * A handler whose loop is one launch may let the launch fold its scalar
  * reductions itself (see dvmh_hip_device.h): after dvmh_loop_cuda_red_prepare_C

@@ -11,6 +11,7 @@ import pytest
 import dvmh_amd as D
 import helpers as H
 from test_cdvmh import _u01
+from test_variants import _force
 
 sys.path.insert(0, os.path.join(H.REPO, 'dvm-snapshot-r6603-fork_amd', 'emit'))
 import hipgen  # noqa: E402
@@ -119,17 +120,30 @@ def jac_reference(n, iters, c):
     return np.array(hist), A.ravel()
 
 
-REFERENCE = {'sor3d': sor_reference, 'edge3d': edge_reference, 'jac3d': jac_reference}
+def edge2d_reference(n, iters, _):
+    A = _u01(SEED, np.arange(n ** 2, dtype=np.uint64)).reshape(n, n)
+    for _ in range(iters):
+        t = A.copy()
+        t[1:] += A[:-1]
+        t[:-1] += A[1:]
+        t += np.concatenate([np.full((n, 1), 0.25), A[:, :-1]], axis=1)
+        t += np.concatenate([A[:, 1:], np.full((n, 1), 0.75)], axis=1)
+        A = 0.2 * t
+    return None, A.ravel()
+
+
+REFERENCE = {'edge2d': edge2d_reference, 'sor3d': sor_reference, 'edge3d': edge_reference, 'jac3d': jac_reference}
 
 
 def run(which, n, iters, factor):
     f = getattr(D.load('libcdv_branches.so'), 'branch_' + which)
     f.restype = None
-    hist, out = np.zeros(iters), np.zeros(n ** 3)
-    args = [ctypes.c_long(n), ctypes.c_int(iters), ctypes.c_double(factor), ctypes.c_ulonglong(SEED)]
+    hist = None if which.startswith('edge') else np.zeros(iters)
+    out = np.zeros(n ** int(which[-2]))
     D.runtime()
-    f(*args, *([] if which == 'edge3d' else [H.dp(hist)]), H.dp(out))
-    return (None if which == 'edge3d' else hist), out
+    f(ctypes.c_long(n), ctypes.c_int(iters), *([] if which == 'edge2d' else [ctypes.c_double(factor)]), ctypes.c_ulonglong(SEED),
+      *([] if hist is None else [H.dp(hist)]), H.dp(out))
+    return hist, out
 
 
 def check(which, n, iters):
@@ -154,3 +168,18 @@ def test_gpu(which, n):
     before = D.stats()['loops_gpu']
     check(which, n, 2)
     assert D.stats()['loops_gpu'] > before
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('kind,block,tune', [(1, (64, 1, 1), [1, 0, 2, 0, 16, 0, 0, 0]), (1, (128, 1, 1), [1, 0, 3, 0, 0, 0, 0, 0]),
+                                             (1, (64, 1, 1), [1, 0, 1, 0, 16, 1, 0, 0]), (3, (64, 4, 1), [1, 0, 1, 16, 2, 0, 0, 0]),
+                                             (3, (64, 4, 1), [1, 1, 2, 8, 2, 1, 0, 0]), (3, (256, 1, 1), [1, 0, 1, 8, 4, 0, 0, 0])])
+def test_variants_gpu(kind, block, tune):
+    """Staged variants asked for: taken where no load leaves the array, the
+    direct kernel elsewhere."""
+    _force(kind, block, tune)
+    try:
+        check('jac3d', 34, 2)
+        check('edge2d', 131, 2)
+    finally:
+        _force(kind, None, None)
