@@ -39,7 +39,9 @@ Output, per program:
                                   sweeps.
                        WAVEFRONT  other ACROSS with >= 2 dependent axes: one
                                   launch per hyperplane of the dependent axes;
-                                  arrays may be in the diagonal layout.
+                                  arrays may be in the diagonal layout; with three
+                                  axes, also tiles staged in LDS, one launch per
+                                  plane of tiles.
 The loop body is inserted verbatim; every schedule respects the dependency
 order, so results are bit-identical to the sequential host order.
 """
@@ -312,6 +314,18 @@ class Loop:
             out.append(nm)
         return out
 
+    ASSIGN = r'(?:=(?!=)|\+=|-=|\*=|/=|%=|&=|\|=|\^=|<<=|>>=|\+\+|--)'
+
+    def uses(self, name):
+        """Per subscripted use: the axes moved (None: not of the form v + 0/1), written or not."""
+        out = []
+        for m in re.finditer(r'\b' + name + r'\s*((?:\[[^\[\]]*\]\s*)+)(' + self.ASSIGN + ')?', self.body):
+            idx = re.findall(r'\[([^\[\]]*)\]', m.group(1))
+            mm = [re.fullmatch(r'\s*' + v + r'\s*(?:([+-])\s*([01])\s*)?', e) for (v, _), e in zip(self.vars, idx)]
+            at = [x.group(2) == '1' for x in mm] if len(idx) == self.rank and all(mm) else None
+            out.append((at, bool(m.group(2))))
+        return out
+
     def flow_eligible(self):
         """Rank 2 or 3, every loop axis in the ACROSS clause with widths <= 1;
         the body reads the ACROSS array at X[i + d0][j + d1].. with at most one
@@ -328,36 +342,41 @@ class Loop:
         arr = [p for p in self.arrays if p[1] == X]
         if not arr or arr[0][3] != self.rank or arr[0][2] not in FLOW_TYPES:
             return False
-        assign = r'(?:=(?!=)|\+=|-=|\*=|/=|%=|&=|\|=|\^=|<<=|>>=|\+\+|--)'
-
-        def uses(name):
-            """Per subscripted use: the offsets (None: not of the form v + 0/1), written or not."""
-            out = []
-            for m in re.finditer(r'\b' + name + r'\s*((?:\[[^\[\]]*\]\s*)+)(' + assign + ')?', self.body):
-                idx = re.findall(r'\[([^\[\]]*)\]', m.group(1))
-                mm = [re.fullmatch(r'\s*' + v + r'\s*(?:([+-])\s*([01])\s*)?', e) for (v, _), e in zip(self.vars, idx)]
-                at = [x.group(2) == '1' for x in mm] if len(idx) == self.rank and all(mm) else None
-                out.append((at, bool(m.group(2))))
-            return out
-
         for p in self.params:
             name = p[1]
             if p[0] not in ('array', 'scalar') or re.search(r'(\+\+|--|&)\s*' + name + r'\b', self.body):
                 return False
             if p[0] == 'scalar':
-                if re.search(r'(?<![\w.>])' + name + r'\s*' + assign, self.body):
+                if re.search(r'(?<![\w.>])' + name + r'\s*' + self.ASSIGN, self.body):
                     return False
                 continue
             # (an array whose name appears other than subscripted may be passed on and written)
             if re.search(r'\b' + name + r'\b(?!\s*\[)', self.body):
                 return False
-            refs = uses(name)
+            refs = self.uses(name)
             if name == X:
                 if any(at is None or sum(at) > (0 if written else 1) for at, written in refs) or not any(wr for _, wr in refs):
                     return False
             elif any(wr for _, wr in refs) and any(at is None or sum(at) for at, _ in refs):
                 return False
         return self.loads_ahead(X)
+
+    def tile_eligible(self):
+        """The tiled wavefront may run the loop: rank 3, every loop axis in the
+        ACROSS clause with widths <= 1, every access of the ACROSS array
+        X[i + d0][j + d1][k + d2] with at most one offset, |offset| <= 1, and none
+        where it is written; and the dataflow launch does not (a guarded access, values
+        that pass through a second array, an assigned scalar)."""
+        if not self.across or self.rank != 3 or self.flow_eligible() or self.leaves():   # (a barrier follows each step)
+            return False
+        w = self.across['widths']
+        name = self.across['array']
+        arr = [p for p in self.arrays if p[1] == name]
+        if len(w) != 3 or any(lo > 1 or hi > 1 or (lo == 0 and hi == 0) for lo, hi in w) or not arr or arr[0][3] != 3:
+            return False
+        if re.search(r'\b' + name + r'\b(?!\s*\[)', self.body) or re.search(r'(\+\+|--|&)\s*' + name + r'\b', self.body):
+            return False
+        return all(at is not None and sum(at) <= (0 if written else 1) for at, written in self.uses(name))
 
     def chain_eligible(self):
         """Consecutive executions (sweeps) of the loop may run pipelined by a
@@ -2972,6 +2991,200 @@ def flow_launch(L, otherwise):
     return b
 
 
+def tile_kernel(L):
+    """Tiled wavefront for an ACROSS loop whose three axes all depend and that the
+    dataflow launch does not take (tile_eligible; a configuration of the tuner,
+    318^3 1.84 ms a sweep against 6.7 with a launch per hyperplane): tiles of
+    TA x TA x TC iterations are run one tile-plane (a + b + c = const) per
+    launch.  A workgroup stages its tile of the ACROSS array plus a halo of one
+    in LDS (lower halo: final values of earlier tiles; upper halo: values no
+    tile has updated yet), runs the tile's local hyperplanes in order with a
+    workgroup barrier between them, and writes the tile back.  The body reads
+    and writes the ACROSS array through a TileView3 with the usual X[i][j][k]
+    syntax; every dependency is met in the sequential order's sense, so the
+    results are those of the lexicographic sweep."""
+    X = L.across['array']
+    xct = [p for p in L.arrays if p[1] == X][0][2]
+    rng = L.stencil_range(X)   # per axis, the offsets at which the body reads X
+    fp, setup = [], []
+    for p in L.arrays:
+        _, nm, ct, ar = p
+        fp.append(f'{ct} *__restrict__ {nm}_base')
+        fp += [f'IndexT {nm}_s{k}' for k in range(ar)]
+        strides = ', '.join(f'{nm}_s{k}' for k in range(ar))
+        setup.append(f'const IndexT {nm}_str[{ar}] = {{{strides}}};')
+        vn = f'dvmh_{nm}' if nm == X else nm
+        setup.append(f'const auto {vn} = dvmh_dev::makeView<{ct}, IndexT, {ar}, true>({nm}_base, {nm}_str);')
+    for p in L.scalars:
+        fp.append(f'{p[2]} *__restrict__ {p[1]}_ptr')
+        setup.append(scalar_bind(L.body, p))
+    for i in range(3):
+        fp += [f'IndexT lo{i}', f'IndexT cnt{i}', f'IndexT st{i}']
+    fp += ['IndexT dt_TA', 'IndexT dt_TC', 'IndexT dt_ntB', 'IndexT dt_ntC', 'IndexT dt_aLo', 'IndexT dt_tplane'] + red_kernel_params(L)
+    k = ['template <typename IndexT>', f'__global__ __launch_bounds__(1024) void {L.name}_tile_kernel({", ".join(fp)}) {{']
+    b = ['const IndexT dt_ta = dt_aLo + (IndexT)blockIdx.x / dt_ntB;',
+         'const IndexT dt_tb = (IndexT)blockIdx.x - ((IndexT)blockIdx.x / dt_ntB) * dt_ntB;',
+         'const IndexT dt_tc = dt_tplane - dt_ta - dt_tb;',
+         'if (dt_tc < 0 || dt_tc >= dt_ntC) return;   // not on this tile-plane (uniform per workgroup)']
+    b += red_kernel_locals(L)
+    b += ['extern __shared__ __align__(16) unsigned char dvmh_lds[];']
+    b += setup
+    for v, ct in L.vars:
+        b.append(f'{ct} {v};')
+    for pr in L.privates:
+        b.append(pr + ';')
+    b += ['const IndexT dt_a0 = dt_ta * dt_TA, dt_b0 = dt_tb * dt_TA, dt_c0 = dt_tc * dt_TC;',
+          'const IndexT dt_na = cnt0 - dt_a0 < dt_TA ? cnt0 - dt_a0 : dt_TA;',
+          'const IndexT dt_nb = cnt1 - dt_b0 < dt_TA ? cnt1 - dt_b0 : dt_TA;',
+          'const IndexT dt_nc = cnt2 - dt_c0 < dt_TC ? cnt2 - dt_c0 : dt_TC;',
+          'const IndexT dt_R1 = dt_nb + 2, dt_R2 = dt_nc + 2, dt_R12 = dt_R1 * dt_R2;',
+          'const IndexT dt_elems = (dt_na + 2) * dt_R12;',
+          f'{xct} *dt_tile = ({xct} *)dvmh_lds;',
+          'const IndexT dt_oi = lo0 + dt_a0 - 1, dt_oj = lo1 + dt_b0 - 1, dt_ok = lo2 + dt_c0 - 1;   // array index of tile slot (0, 0, 0)',
+          'const IndexT dt_tid = (IndexT)threadIdx.x, dt_nthr = (IndexT)blockDim.x;',
+          '// stage the tile and its halo, sixteen loads in flight per thread; an index',
+          '// outside those the body reads is clamped into them (its slot is never read)']
+    for a, v in enumerate(('dt_ii', 'dt_jj', 'dt_kk')):
+        b.append(f'const IndexT {v}_lo = lo{a} + ({rng[a][0]}), {v}_hi = lo{a} + cnt{a} - 1 + ({rng[a][1]});')
+    b += ['// slot (p, q, r) of element e = dt_tid + m * dt_nthr, advanced by dt_nthr',
+          '// in the radix (R1, R2) of the tile: two divisions per thread, not per element',
+          'IndexT dt_sp = dt_nthr / dt_R12, dt_sq = (dt_nthr - dt_sp * dt_R12) / dt_R2, dt_sr = dt_nthr - dt_sp * dt_R12 - dt_sq * dt_R2;',
+          'IndexT dt_p = dt_tid / dt_R12, dt_q = (dt_tid - dt_p * dt_R12) / dt_R2, dt_r = dt_tid - dt_p * dt_R12 - dt_q * dt_R2;',
+          'for (IndexT dt_b0 = 0; dt_b0 < dt_elems; dt_b0 += 16 * dt_nthr) {',
+          IND + 'const IndexT dt_e0 = dt_b0 + dt_tid;',
+          IND + f'{xct} dt_v[16];',
+          IND + '#pragma unroll',
+          IND + 'for (int dt_u = 0; dt_u < 16; dt_u++) {',
+          IND * 2 + 'if (dt_b0 + (IndexT)dt_u * dt_nthr >= dt_elems) break;   // (uniform) no element of the workgroup left',
+          IND * 2 + '// (past the last element p runs beyond the tile: the clamp keeps the load in bounds)',
+          IND * 2 + 'IndexT dt_ii = dt_oi + dt_p, dt_jj = dt_oj + dt_q, dt_kk = dt_ok + dt_r;']
+    for v in ('dt_ii', 'dt_jj', 'dt_kk'):
+        b.append(IND * 2 + f'{v} = {v} < {v}_lo ? {v}_lo : ({v} > {v}_hi ? {v}_hi : {v});')
+    b += [IND * 2 + f'dt_v[dt_u] = dvmh_{X}[dt_ii][dt_jj][dt_kk];',
+          IND * 2 + 'dt_r += dt_sr; dt_q += dt_sq; dt_p += dt_sp;',
+          IND * 2 + 'if (dt_r >= dt_R2) { dt_r -= dt_R2; dt_q++; }',
+          IND * 2 + 'if (dt_q >= dt_R1) { dt_q -= dt_R1; dt_p++; }',
+          IND + '}',
+          IND + '#pragma unroll',
+          IND + 'for (int dt_u = 0; dt_u < 16; dt_u++)',
+          IND * 2 + 'if (dt_e0 + (IndexT)dt_u * dt_nthr < dt_elems) dt_tile[dt_e0 + (IndexT)dt_u * dt_nthr] = dt_v[dt_u];',
+          '}',
+          '__syncthreads();',
+          f'const dvmh_dev::TileView3<{xct}, IndexT> {X}{{dt_tile, dt_R1, dt_R2, dt_oi, dt_oj, dt_ok}};',
+          '// local hyperplanes p + q + r = s of the tile, in order; a thread\'s (p, q)',
+          '// columns do not change from one hyperplane to the next: up to four are',
+          '// worked out once (more than four per thread take the generic loop)',
+          'const IndexT dt_nab = dt_na * dt_nb;',
+          'IndexT dt_myp[4], dt_myq[4];',
+          'bool dt_has[4];',
+          '#pragma unroll',
+          'for (int dt_u = 0; dt_u < 4; dt_u++) {',
+          IND + 'const IndexT dt_idx = dt_tid + (IndexT)dt_u * dt_nthr;',
+          IND + 'dt_has[dt_u] = dt_idx < dt_nab;',
+          IND + 'dt_myp[dt_u] = dt_idx / dt_nb;',
+          IND + 'dt_myq[dt_u] = dt_idx - dt_myp[dt_u] * dt_nb;',
+          '}',
+          'const bool dt_few = dt_nab <= 4 * dt_nthr, dt_one = dt_nab <= dt_nthr;',
+          'for (IndexT dt_s = 0; dt_s < dt_na + dt_nb + dt_nc - 2; dt_s++) {',
+          IND + 'if (dt_one) {   // at most one column per thread',
+          IND * 2 + 'const IndexT dt_p = dt_myp[0], dt_q = dt_myq[0];',
+          IND * 2 + 'const IndexT dt_r = dt_s - dt_p - dt_q;',
+          IND * 2 + 'if (dt_has[0] && dt_r >= 0 && dt_r < dt_nc) {',
+          IND * 3 + 'const IndexT t0 = dt_a0 + dt_p, t1 = dt_b0 + dt_q, t2 = dt_c0 + dt_r;',
+          ] + [IND * 3 + var_assign(L, i, f't{i}', f'lo{i}', '(IndexT)1') for i in range(3)] + [indent('{\n' + indent(L.body + '\n', 1) + '}', 3)] + [
+          IND * 2 + '}',
+          IND + '} else if (dt_few) {',
+          IND * 2 + '#pragma unroll',
+          IND * 2 + 'for (int dt_u = 0; dt_u < 4; dt_u++) {',
+          IND * 3 + 'const IndexT dt_p = dt_myp[dt_u], dt_q = dt_myq[dt_u];',
+          IND * 3 + 'const IndexT dt_r = dt_s - dt_p - dt_q;',
+          IND * 3 + 'if (dt_has[dt_u] && dt_r >= 0 && dt_r < dt_nc) {',
+          IND * 4 + 'const IndexT t0 = dt_a0 + dt_p, t1 = dt_b0 + dt_q, t2 = dt_c0 + dt_r;']
+    for i in range(3):
+        b.append(IND * 4 + var_assign(L, i, f't{i}', f'lo{i}', '(IndexT)1'))   # the handlers run unit forward steps only
+    b.append(indent('{\n' + indent(L.body + '\n', 1) + '}', 4))
+    b += [IND * 3 + '}',
+          IND * 2 + '}',
+          IND + '} else {',
+          IND * 2 + 'for (IndexT dt_idx = dt_tid; dt_idx < dt_nab; dt_idx += dt_nthr) {',
+          IND * 3 + 'const IndexT dt_p = dt_idx / dt_nb, dt_q = dt_idx - (dt_idx / dt_nb) * dt_nb;',
+          IND * 3 + 'const IndexT dt_r = dt_s - dt_p - dt_q;',
+          IND * 3 + 'if (dt_r >= 0 && dt_r < dt_nc) {',
+          IND * 4 + 'const IndexT t0 = dt_a0 + dt_p, t1 = dt_b0 + dt_q, t2 = dt_c0 + dt_r;']
+    for i in range(3):
+        b.append(IND * 4 + var_assign(L, i, f't{i}', f'lo{i}', '(IndexT)1'))   # the handlers run unit forward steps only
+    b.append(indent('{\n' + indent(L.body + '\n', 1) + '}', 4))
+    b += [IND * 3 + '}',
+          IND * 2 + '}',
+          IND + '}',
+          IND + '__syncthreads();',
+          '}',
+          '// write back the tile (not the halo); (p, q, r) advanced as in the staging',
+          'const IndexT dt_nbc = dt_nb * dt_nc;',
+          '{',
+          IND + 'const IndexT wp = dt_nthr / dt_nbc, wq = (dt_nthr - wp * dt_nbc) / dt_nc, wr = dt_nthr - wp * dt_nbc - wq * dt_nc;',
+          IND + 'IndexT p = dt_tid / dt_nbc, q = (dt_tid - p * dt_nbc) / dt_nc, r = dt_tid - p * dt_nbc - q * dt_nc;',
+          IND + 'for (IndexT dt_e = dt_tid; dt_e < dt_na * dt_nbc; dt_e += dt_nthr) {',
+          IND * 2 + f'dvmh_{X}[dt_oi + 1 + p][dt_oj + 1 + q][dt_ok + 1 + r] = dt_tile[((p + 1) * dt_R1 + (q + 1)) * dt_R2 + (r + 1)];',
+          IND * 2 + 'r += wr; q += wq; p += wp;',
+          IND * 2 + 'if (r >= dt_nc) { r -= dt_nc; q++; }',
+          IND * 2 + 'if (q >= dt_nb) { q -= dt_nb; p++; }',
+          IND + '}',
+          '}',
+          '__syncthreads();   // the LDS tile is free for the next one']
+    b += red_kernel_tail(L, '((long)(dt_ta * dt_ntB + dt_tb) * dt_ntC + dt_tc)', accumulate=False)
+    k.append(indent('\n'.join(b) + '\n', 1).rstrip('\n'))
+    k.append('}')
+    return '\n'.join(k) + '\n'
+
+
+def tile_launch(L):
+    X = L.across['array']
+    xct = [p for p in L.arrays if p[1] == X][0][2]
+    b = ['DvmType TA = tune[DVMH_AMD_T_TILE_A], TC = tune[DVMH_AMD_T_TILE_B];',
+         'DvmType ntA = (cnt0 + TA - 1) / TA, ntB = (cnt1 + TA - 1) / TA, ntC = (cnt2 + TC - 1) / TC;',
+         f'size_t ldsBytes = (size_t)(TA + 2) * (TA + 2) * (TC + 2) * sizeof({xct});',
+         'DvmType tiles = ntA * ntB * ntC;']
+    b += handler_reds_prepare(L, 'tiles', 0)
+    b.append('dvmh_amd_mark_kernel_C(loop_ref, 0);')
+    b.append('for (DvmType tplane = 0; tplane <= (ntA - 1) + (ntB - 1) + (ntC - 1); tplane++) {')
+    b.append(IND + 'DvmType aLo = tplane - (ntB - 1) - (ntC - 1);')
+    b.append(IND + 'if (aLo < 0) aLo = 0;')
+    b.append(IND + 'DvmType aHi = tplane < ntA - 1 ? tplane : ntA - 1;')
+    b.append(IND + 'DvmType grid = (aHi - aLo + 1) * ntB;')
+    for it in ['int', 'long long']:
+        args = array_fact_args(L, it)
+        for i in range(3):
+            args += [f'({it})boundsLow[{i}]', f'({it})cnt{i}', f'({it})loopSteps[{i}]']
+        args += [f'({it})TA', f'({it})TC', f'({it})ntB', f'({it})ntC', f'({it})aLo', f'({it})tplane']
+        args += red_fact_args(L)
+        cond = f'kernelIndexT == {"rt_INT" if it == "int" else "rt_LLONG"}'
+        b.append(IND + f'if ({cond}) hipLaunchKernelGGL(({L.name}_tile_kernel<{it}>), dim3((unsigned)grid), threads, ldsBytes, '
+                 f'stream, {", ".join(args)});')
+    b.append('}')
+    b.append('dvmh_amd_mark_kernel_C(loop_ref, 1);')
+    b += handler_reds_finish(L)
+    return b
+
+
+def tile_or(L, otherwise):
+    """The tiled wavefront where the tuner asks for it: unit forward steps, natural
+    layout, a tile that fits 64 KB of LDS, no load outside the array."""
+    X = L.across['array']
+    xct = [p for p in L.arrays if p[1] == X][0][2]
+    b, ahead = L.inside(X)
+    unit = ' && '.join(f'loopSteps[{i}] == 1' for i in range(3))
+    b = list(b) + [f'bool tiled = tune[DVMH_AMD_T_VARIANT] == 1 && {unit} && {X}_tfm == 0 && threads.y == 1 && threads.z == 1 && '
+                   'tune[DVMH_AMD_T_TILE_A] >= 2 && tune[DVMH_AMD_T_TILE_B] >= 2 && '
+                   f'(tune[DVMH_AMD_T_TILE_A] + 2) * (tune[DVMH_AMD_T_TILE_A] + 2) * (tune[DVMH_AMD_T_TILE_B] + 2) * (DvmType)sizeof({xct}) <= 64512 && '
+                   f'{ahead};', 'if (tiled) {']
+    b += [IND + ln for ln in tile_launch(L)]
+    b.append('} else {')
+    b += [IND + ln for ln in otherwise]
+    b.append('}')
+    return b
+
+
 # Chunk lengths (iterations per staged chunk) the tiled line sweep is
 # instantiated for; a thread keeps its share of the next chunk, CK + 1
 # elements, in registers while the current one is computed.
@@ -3638,6 +3851,8 @@ def across_handler(L):
             rest = wave_launch(L, list(deps))
             if m == r and L.flow_eligible():
                 rest = flow_launch(L, rest)
+            elif m == 3 and L.tile_eligible():
+                rest = tile_or(L, rest)
             b += [IND + s for s in rest]
     b.append('} else {')
     b.append(IND + f'fprintf(stderr, "{L.name}: unsupported dependency mask %ld\\n", (long)dependency_mask);')
@@ -3699,6 +3914,8 @@ def gpu_loop(L):
                 text.append(wave_kernel(L, list(deps)))
         if L.flow_eligible():
             text.append(flow_kernel(L))
+        if L.tile_eligible():
+            text.append(tile_kernel(L))
         if L.line_tile_eligible():
             text.append(line_tile_kernel(L))
             text.append(line_vec_kernel(L))

@@ -7,11 +7,12 @@
  *   DiagView   the same for a layout whose two fastest storage axes are
  *              diagonalised (planes stored anti-diagonal by anti-diagonal), the
  *              index map of rts/dvmh/include/dvmhlib_device.h:56-98.
- *   MarchView2/3, LineView
+ *   MarchView2/3, TileView3, LineView
  *              the same syntax over copies staged in LDS: a rolling window of
  *              three planes of a read-only stencil array (march variant of
- *              PARALLEL loops) and a chunk of one line of an ACROSS array
- *              (tiled line sweep along the innermost axis).
+ *              PARALLEL loops), a tile with halo of an ACROSS array (tiled
+ *              wavefront), and a chunk of one line of an ACROSS array (tiled
+ *              line sweep along the innermost axis).
  *   StarView, flowTile
  *              the same syntax over a point and its neighbours in registers,
  *              and the dataflow wavefront that walks them (ACROSS loops whose
@@ -141,6 +142,31 @@ struct MarchView2 {
     int sCur;
     __device__ __forceinline__ MarchRow<T, I> operator[](I i) const {
         return MarchRow<T, I>{lds + (I)marchSlot(sCur, (int)(i - iCur)) * cols, k0};
+    }
+};
+
+// A tile of a rank-3 array staged in LDS (read and written): element (0,0,0)
+// holds array index (i0, j0, k0), planes of rows x cols elements.
+template <typename T, typename I>
+struct TileRow {
+    T *p;
+    I k0;
+    __device__ __forceinline__ T &operator[](I k) const { return p[k - k0]; }
+};
+
+template <typename T, typename I>
+struct TilePlane {
+    T *p;
+    I cols, j0, k0;
+    __device__ __forceinline__ TileRow<T, I> operator[](I j) const { return TileRow<T, I>{p + (j - j0) * cols, k0}; }
+};
+
+template <typename T, typename I>
+struct TileView3 {
+    T *p;
+    I rows, cols, i0, j0, k0;
+    __device__ __forceinline__ TilePlane<T, I> operator[](I i) const {
+        return TilePlane<T, I>{p + (i - i0) * rows * cols, cols, j0, k0};
     }
 };
 

@@ -132,7 +132,28 @@ def edge2d_reference(n, iters, _):
     return None, A.ravel()
 
 
-REFERENCE = {'edge2d': edge2d_reference, 'sor3d': sor_reference, 'edge3d': edge_reference, 'jac3d': jac_reference}
+def two3d_reference(n, iters, w):
+    a, b = _grid(n).tolist(), np.full((n, n, n), 0.5).tolist()
+    hist = []
+    for _ in range(iters):
+        eps = 0.0
+        for i in range(1, n - 1):
+            for j in range(1, n - 1):
+                for k in range(1, n - 1):
+                    t = (a[i - 1][j][k] + a[i + 1][j][k] + a[i][j - 1][k] + a[i][j + 1][k] + a[i][j][k - 1] + a[i][j][k + 1]) / 6.0
+                    b[i][j][k] = 0.5 * b[i - 1][j][k] + 0.25 * b[i][j][k - 1] + 0.125 * t
+                    a[i][j][k] = (1 - w) * a[i][j][k] + w * (t - 0.125 * b[i][j - 1][k])
+                    if t > eps:
+                        eps = t
+        for i in range(1, n - 1):
+            for j in range(1, n - 1):
+                for k in range(1, n - 1):
+                    a[i][j][k] = 0.25 * (a[i - 1][j][k] + a[i][j + 1][k] + a[i][j][k - 1] + a[i][j][k])
+        hist.append(eps)
+    return np.array(hist), np.array(a).ravel()
+
+
+REFERENCE = {'two3d': two3d_reference, 'edge2d': edge2d_reference, 'sor3d': sor_reference, 'edge3d': edge_reference, 'jac3d': jac_reference}
 
 
 def run(which, n, iters, factor):
@@ -147,7 +168,7 @@ def run(which, n, iters, factor):
 
 
 def check(which, n, iters):
-    factor = 0.2 if which != 'sor3d' else 1.25
+    factor = {'sor3d': 1.25, 'two3d': 0.8}.get(which, 0.2)
     hist, out = run(which, n, iters, factor)
     rh, ro = REFERENCE[which](n, iters, factor)
     assert H.bits_equal(out, ro)
@@ -183,3 +204,17 @@ def test_variants_gpu(kind, block, tune):
         check('edge2d', 131, 2)
     finally:
         _force(kind, None, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('nt,ta,tc', [(64, 4, 8), (256, 8, 16), (256, 12, 16), (32, 16, 8)])
+@pytest.mark.parametrize('n', [3, 9, 20, 35])
+def test_tiles_gpu(nt, ta, tc, n):
+    """The tiled wavefront, which such sweeps keep, with one column per thread,
+    up to four and more; edge3d's guards close, so it runs hyperplanes."""
+    _force(2, (nt, 1, 1), [1, 0, 1, 0, ta, tc, 0, 0])
+    try:
+        check('two3d', n, 2)
+        check('edge3d', n, 2)
+    finally:
+        _force(2, None, None)

@@ -85,3 +85,28 @@ def test_batch_and_register_sweep(tmp_path, guard):
     sweep = 'if (i > 0) A[i][j] = A[i][j] + A[i - 1][j];' if guard else 'A[i][j] = A[i][j] + A[i - 1][j];'
     text = _emit(tmp_path, sweep, across={'array': 'A', 'widths': [(1, 0), (0, 0)]})
     assert ('if (lreg && !(dvmh_amd_loop_reads_inside_C(loop_ref, A_hdr, ' in text) == guard
+
+
+def test_tiled_wavefront():
+    """Three dependent axes: what the dataflow launch does not take (values that
+    pass through a second array, guarded accesses) keeps the tiles of a tuned loop."""
+    fake_device.run(CODE + '''
+w, e, n = ctypes.c_double(0.5), ctypes.c_double(), T.L(40)
+A, B = T.array(40, 40, 40), T.array(40, 40, 40)
+def kernels(text, lo, hi, params, reds=()):
+    r = T.region(A, B, scalars=[w, n])
+    F.fake_clear()
+    T.loop(r, lib, named(text) + '_cuda', A, [(lo, hi)] * 3, params, reds=reds, across=[1] * 6)
+    T.rt.dvmh_region_end_C(r)
+    return {k for k in ('flow', 'tile', 'wave012') for x, _, _ in T.launches() if k + '_kernel' in x}
+two = 'B[i][j][k] = 0.5 * B[i - 1][j][k]'
+for tuned in (False, True):
+    if tuned:
+        force(2, (256, 1, 1), variant=1, a=8, b=8)
+    other = {'tile' if tuned else 'wave012'}
+    assert kernels(two, 1, 38, [A, B, w], [(3, e)]) == other
+    assert kernels('if (i > 0 && j > 0 && k > 0)', 1, 38, [A]) == other
+    assert kernels('if (i > 0 && j > 0 && k > 0)', 0, 38, [A]) == {'wave012'}
+    assert kernels('if (i < n - 1)', 0, 39, [A, n, w]) == {'wave012'}
+    assert kernels('double d = fabs(t - s);', 1, 38, [A, w], [(3, e)]) == {'flow'}
+''')
