@@ -59,6 +59,7 @@ void Settings::load() {
     allowAsync = envLong("DVMH_ALLOW_ASYNC", 0) != 0;   // rts/dvmh/settings.cpp:361
     pollDone = envLong("DVMH_AMD_POLL", 1) != 0;
     flowTag = envLong("DVMH_AMD_FLOW_TAG", 0);
+    flowMb = envLong("DVMH_AMD_FLOW_MB", -1);
     graph = envLong("DVMH_AMD_GRAPH", 0) != 0;
     graphMinNodes = envLong("DVMH_AMD_GRAPH_MIN_NODES", 6);
     tuneRepeats = (int)envLong("DVMH_AMD_TUNE_REPEATS", 1);
@@ -157,6 +158,16 @@ void *Gpu::alloc(size_t bytes) {
         if (e != hipSuccess) {
             (void)hipGetLastError();
             trimCache();
+            e = hipMalloc(&p, rounded);
+        }
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            // captured graphs hold the workspace of the dataflow launches in
+            // them, and blocks of their own
+            if (graphsExist() && !graphCapturing()) {
+                graphsForget();
+                trimCache();
+            }
             HIP_CHECK(hipMalloc(&p, rounded));
         }
     }
@@ -210,7 +221,9 @@ bool Gpu::flowWorkspace(long tiles, long cellWords, DvmhAmdFlow *out) {
         *flowWrapped = 0;
         HIP_CHECK(hipHostGetDevicePointer((void **)&flowWrappedDev, h, 0));
     }
+    if (settings.flowMb >= 0 && need > (size_t)settings.flowMb << 20) return false;
     if (flowSpaces.empty() || flowSpaces.back().bytes < need) {
+        if (flowRefused && need >= flowRefused) return false;
         // earlier launches (and graphs) may still use the smaller one: it stays
         // until no graph does
         void *p = nullptr;
@@ -220,8 +233,17 @@ bool Gpu::flowWorkspace(long tiles, long cellWords, DvmhAmdFlow *out) {
             trimCache();
             if (hipMalloc(&p, need) != hipSuccess) {
                 (void)hipGetLastError();
+                flowRefused = need;
                 return false;
             }
+        }
+        // what the handler allocates next must find room as well
+        size_t left = 0, all = 0;
+        HIP_CHECK(hipMemGetInfo(&left, &all));
+        if (left < need / 8 + ((size_t)64 << 20)) {
+            HIP_CHECK(hipFree(p));
+            flowRefused = need;
+            return false;
         }
         flowSpaces.push_back(FlowSpace{(char *)p, need});
         flowZero(flowSpaces.back());
@@ -355,7 +377,10 @@ long rtTypeSize(int t) {
 
 // ---------------------------------------------------------------- Data
 Data::~Data() {
-    if (hasDev && dev.ptr) gpu.release(dev.ptr);
+    if (hasDev && dev.ptr) {
+        gpu.release(dev.ptr);
+        gpu.flowRefused = 0;
+    }
     if (ownsHost) free(host);
     magic = 0;
 }

@@ -422,6 +422,29 @@ bool graphsExist() {
     return false;
 }
 
+// Where memory runs short, in the middle of a run: entries stay (a caller may
+// hold one) and count as never seen.
+static std::vector<char *> retiredPinned;
+
+void graphsForget() {
+    gpu.sync();
+    auto forget = [](GraphEntry &g) {
+        retiredPinned.insert(retiredPinned.end(), g.pinned.begin(), g.pinned.end());   // pending posts read these
+        g.pinned.clear();
+        destroyEntry(g);
+    };
+    for (auto &kv : graphs) forget(kv.second);
+    for (auto &kv : batchGraphs) {
+        forget(kv.second.g);
+        kv.second.postAt.clear();
+    }
+}
+
+void graphFreeRetired() {
+    for (char *p : retiredPinned) HIP_CHECK(hipHostFree(p));
+    retiredPinned.clear();
+}
+
 void graphReleaseAll() {
     gpu.sync();
     for (auto &kv : graphs) destroyEntry(kv.second);

@@ -195,6 +195,7 @@ void flushDeferredPosts() {
     }
     pending.clear();
     pinnedPool.reset();
+    graphFreeRetired();
 }
 
 void addPendingPost(const std::shared_ptr<Reduction> &r, char *val, char *loc, bool addInitial) {

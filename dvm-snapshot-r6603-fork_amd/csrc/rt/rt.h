@@ -61,6 +61,7 @@ struct Settings {
     bool fuse = true;              // DVMH_AMD_FUSE (default 1): registered loop pairs held back together run fused
     bool index64 = false;          // DVMH_AMD_INDEX64: every loop's kernels take 64-bit index arithmetic
     long flowTag = 0;              // DVMH_AMD_FLOW_TAG: launch tag dataflow workspaces start from
+    long flowMb = -1;              // DVMH_AMD_FLOW_MB: the largest dataflow workspace (megabytes; -1: what the device has room for)
     std::string tuneDb;         // DVMH_AMD_TUNEDB: file of recorded timings
     std::string modelFile;      // DVMH_AMD_MODEL: trained cost-model weights
     void load();
@@ -92,6 +93,7 @@ public:
     // workspace of dataflow launches (one at a time on the stream): the current
     // one and, while graphs that use them exist, smaller earlier ones
     bool flowWorkspace(long tiles, long cellWords, DvmhAmdFlow *out);
+    size_t flowRefused = 0;                  // there was no room for so much, and no array has been freed since (0: there was)
     bool flowHeld = false;                   // a running handler holds the current one (and what it allocates after may run short)
     void flowCheckWrap();                    // starts the tags over when a launch has said they run out
     void flowRetire(bool all);               // frees the earlier ones (all: the current one too)
@@ -406,6 +408,8 @@ long layoutChanges();
 // lazy regions and graphs (graph.cpp)
 bool regionIsLazy(const Region *r);
 bool graphsExist();                 // some captured graph may be replayed
+void graphsForget();                // frees every captured graph (they are captured again when they recur)
+void graphFreeRetired();            // what pending posts of forgotten graphs read
 bool graphCapturing();
 void graphNoteAlloc(void *p);
 char *graphPinnedSlot(size_t bytes);

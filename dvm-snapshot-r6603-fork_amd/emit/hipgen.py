@@ -2909,7 +2909,7 @@ def flow_kernel(L):
         k.append('}')
         return '\n'.join(k) + '\n'
 
-    tile = '(long)dvmh_task.ta * dvmh_f.ntB + dvmh_task.tb'
+    tile = 'dvmh_f.first + (long)dvmh_task.ta * dvmh_f.ntB + dvmh_task.tb'
     out = kernel(f'{L.name}_flow_kernel', False, fp + red_kernel_params(L) + red_finish_params(L), red_kernel_locals(L),
                  red_kernel_finish(L, tile))
     if L.chain_eligible():
@@ -2924,6 +2924,17 @@ def flow_kernel(L):
     return out
 
 
+def flow_conditions(L, conds):
+    """The dataflow launch applies: `conds`, unit forward steps, unit stride."""
+    X = L.across['array']
+    return ' && '.join(conds + [f'loopSteps[{i}] == 1' for i in range(L.rank)] + [f'{X}_devHdr[{L.rank}] == 1'])
+
+
+def flow_words(L, tiles, points):
+    """Words of the cells of `tiles` tiles whose rows have `points` points."""
+    return f'{tiles} * {L.rank - 1} * dvmh_dev::flowBlocks({L.rank}, {points}) * (dvmh_dev::FLOW_CELLS_BYTES / 8)'
+
+
 def flow_tiles(L):
     """Handler lines: the tile counts of the dataflow launch."""
     sh = f'dvmh_dev::FlowShape<{L.rank}>'
@@ -2932,57 +2943,73 @@ def flow_tiles(L):
             'DvmType flowTiles = flowA * flowB;']
 
 
-def flow_check(L, conds, sweeps):
-    """Handler lines after flow_tiles: `flow` (the dataflow launch applies:
-    `conds`, unit forward steps, unit stride, no more tasks and no longer rows
-    than it can address, room for its workspace dvmh_ws)."""
-    X = L.across['array']
-    r = L.rank
-    conds = conds + [f'loopSteps[{i}] == 1' for i in range(r)] + [
-        f'{X}_devHdr[{r}] == 1', f'dvmh_dev::flowBlocks({r}, cnt{r - 1}) <= dvmh_dev::FLOW_BLOCKS_MAX',
-        f'flowTiles * {sweeps} <= dvmh_dev::FLOW_TASKS_MAX']
-    return ['DvmhAmdFlow dvmh_ws;',
-            'bool flow = ' + ' && '.join(conds) + ';',
-            f'if (flow) flow = dvmh_amd_flow_workspace_C(flowTiles * {sweeps}, flowTiles * {r - 1} * dvmh_dev::flowBlocks({r}, cnt{r - 1}) * '
-            '(dvmh_dev::FLOW_CELLS_BYTES / 8), &dvmh_ws) != 0;']
-
-
-def flow_launches(L, kernel, sweeps, tail_args):
-    """Handler lines that launch `kernel` for `sweeps` sweeps, by index type."""
+def flow_launches(L, kernel, tiles, sweeps, tail_args, part=None):
+    """Handler lines that launch `kernel` for `sweeps` sweeps of `tiles` tiles, by
+    index type; `part`: per axis, the offset and extent of the part of the loop
+    it walks, else all of it."""
     X = L.across['array']
     r = L.rank
     xct = [p for p in L.arrays if p[1] == X][0][2]
     rng = L.stencil_range(X)
+    part = part or {}
     b = []
     for it, tag in (('int', 'rt_INT'), ('long long', 'rt_LLONG')):
         b.append(f'if (kernelIndexT == {tag}) {{')
         c = [f'dvmh_dev::FlowArgs<{xct}, {it}, {r}> dvmh_f;', f'dvmh_f.base = {X};']
         for a in range(r):
-            c.append(f'dvmh_f.s[{a}] = ({it}){X}_devHdr[{a + 1}]; dvmh_f.lo[{a}] = ({it})boundsLow[{a}]; dvmh_f.cnt[{a}] = ({it})cnt{a};')
-            c.append(f'dvmh_f.rlo[{a}] = ({it})(boundsLow[{a}] + ({rng[a][0]})); dvmh_f.rhi[{a}] = ({it})(boundsLow[{a}] + cnt{a} - 1 + ({rng[a][1]}));')
-        c += ['dvmh_f.ntA = (int)flowA; dvmh_f.ntB = (int)flowB;', f'dvmh_f.sweeps = (int)({sweeps});', 'dvmh_f.ws = dvmh_ws;']
+            at, n = part.get(a, (None, f'cnt{a}'))
+            lo = f'boundsLow[{a}]' + (f' + {at}' if at else '')
+            c.append(f'dvmh_f.s[{a}] = ({it}){X}_devHdr[{a + 1}]; dvmh_f.lo[{a}] = ({it})({lo}); dvmh_f.cnt[{a}] = ({it}){n};')
+            c.append(f'dvmh_f.rlo[{a}] = ({it})({lo} + ({rng[a][0]})); dvmh_f.rhi[{a}] = ({it})({lo} + {n} - 1 + ({rng[a][1]}));')
+        c += [f'dvmh_f.ntA = (int){"dvmh_a" if 0 in part else "flowA"}; dvmh_f.ntB = (int)flowB;', f'dvmh_f.sweeps = (int)({sweeps});',
+              f'dvmh_f.first = {"dvmh_first" if 0 in part else "0"};', 'dvmh_f.ws = dvmh_ws;']
         args = ['dvmh_f']
         for p in L.arrays:
             if p[1] != X:
                 args += [p[1]] + [f'({it}){p[1]}_devHdr[{k + 1}]' for k in range(p[3])]
         args += [p[1] for p in L.scalars] + tail_args
-        c.append(f'hipLaunchKernelGGL({kernel}<{it}>, dim3((unsigned)(flowTiles * ({sweeps}))), dim3(64), 0, stream, {", ".join(args)});')
+        c.append(f'hipLaunchKernelGGL({kernel}<{it}>, dim3((unsigned)({tiles} * ({sweeps}))), dim3(64), 0, stream, {", ".join(args)});')
         b += [IND + ln for ln in c] + ['}']
     return b
 
 
 def flow_launch(L, otherwise):
     """The dataflow launch where it applies -- unit forward steps, natural
-    layouts, room for its workspace -- else `otherwise`.  No size is left to
-    the other kernels while its faces and tasks can be addressed: they pay a launch (4-14 us) per hyperplane or
-    tile-plane, this one about 5 us per tile of a diagonal and 0.13-0.17 us per
-    step.  One sweep: 2-D 998^2 0.38 against 9.2 ms; 3-D 128^3 0.145 against
-    0.43 ms, 318^3 0.48 against 1.84."""
-    b = flow_tiles(L) + flow_check(L, [f'{p[1]}_tfm == 0' for p in L.arrays], '1')
+    layouts -- else `otherwise`.  No size is left to the other kernels: they pay
+    a launch (4-14 us) per hyperplane or tile-plane, this one about 5 us per tile
+    of a diagonal and 0.13-0.17 us per step.  One sweep: 2-D 998^2 0.38 against
+    9.2 ms; 3-D 128^3 0.145 against 0.43 ms, 318^3 0.48 against 1.84.
+
+    The sweep is one launch unless its rows or tiles are too many for one or
+    there is no room for the cells of all of them: then parts of it, along the
+    first and the innermost axis, run one after another (every point a part
+    reads below it is final, every one above it is old)."""
+    r = L.rank
+    k = r - 1
+    sh = f'dvmh_dev::FlowShape<{r}>'
+    b = flow_tiles(L)
+    b += ['DvmhAmdFlow dvmh_ws;',
+          f'bool flow = {flow_conditions(L, [f"{p[1]}_tfm == 0" for p in L.arrays])};',
+          f'const DvmType flowRow = cnt{k} < dvmh_dev::FLOW_ROW_MAX ? cnt{k} : dvmh_dev::FLOW_ROW_MAX, '
+          f'flowRows = (cnt{k} + flowRow - 1) / flowRow;',
+          'DvmType flowPart = flowA;   // tiles along the first axis in a launch',
+          'while (flow && !(flowPart * flowB <= dvmh_dev::FLOW_TASKS_MAX && '
+          f'dvmh_amd_flow_workspace_C(flowPart * flowB, {flow_words(L, "flowPart * flowB", "flowRow")}, &dvmh_ws))) {{',
+          IND + 'flow = flowPart > 1;',
+          IND + 'flowPart = (flowPart + 1) / 2;',
+          '}']
     b.append('if (flow) {')
-    b += [IND + ln for ln in handler_reds_prepare(L, 'flowTiles', 0) + red_finish_query(L, 'flowTiles')]
+    b += [IND + ln for ln in handler_reds_prepare(L, 'flowTiles * flowRows', 0) + red_finish_query(L, 'flowTiles * flowRows')]
     b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 0);')
-    b += [IND + ln for ln in flow_launches(L, f'{L.name}_flow_kernel', '1', red_fact_args(L) + red_finish_args(L))]
+    b += [IND + 'DvmType dvmh_first = 0;',
+          IND + 'for (DvmType dvmh_at = 0; dvmh_at < flowA; dvmh_at += flowPart) {',
+          IND * 2 + 'const DvmType dvmh_a = flowA - dvmh_at < flowPart ? flowA - dvmh_at : flowPart;',
+          IND * 2 + f'const DvmType dvmh_lo0 = dvmh_at * {sh}::PA, dvmh_n0 = cnt0 - dvmh_lo0 < dvmh_a * {sh}::PA ? cnt0 - dvmh_lo0 : dvmh_a * {sh}::PA;',
+          IND * 2 + f'for (DvmType dvmh_lo{k} = 0; dvmh_lo{k} < cnt{k}; dvmh_lo{k} += flowRow) {{',
+          IND * 3 + f'const DvmType dvmh_n{k} = cnt{k} - dvmh_lo{k} < flowRow ? cnt{k} - dvmh_lo{k} : flowRow;']
+    b += [IND * 3 + ln for ln in flow_launches(L, f'{L.name}_flow_kernel', 'dvmh_a * flowB', '1', red_fact_args(L) + red_finish_args(L),
+                                               {0: ('dvmh_lo0', 'dvmh_n0'), k: (f'dvmh_lo{k}', f'dvmh_n{k}')})]
+    b += [IND * 3 + 'dvmh_first += dvmh_a * flowB;', IND * 2 + '}', IND + '}']
     b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 1);')
     b += [IND + ln for ln in handler_reds_finish(L)]
     b.append('} else {')
@@ -3697,7 +3724,9 @@ def chain_handler(L):
     b.append('// sweeps per launch')
     b.append(f'long most = nl < {CHAIN_SWEEPS} ? nl : {CHAIN_SWEEPS};')
     b.append('if (flowTiles * most > dvmh_dev::FLOW_TASKS_MAX) most = flowTiles < dvmh_dev::FLOW_TASKS_MAX ? dvmh_dev::FLOW_TASKS_MAX / flowTiles : 1;')
-    b += flow_check(L, ['chained'], 'most')
+    b += ['DvmhAmdFlow dvmh_ws;',
+          f'bool flow = {flow_conditions(L, ["chained"])} && cnt{L.rank - 1} <= dvmh_dev::FLOW_ROW_MAX && flowTiles * most <= dvmh_dev::FLOW_TASKS_MAX;',
+          f'if (flow) flow = dvmh_amd_flow_workspace_C(flowTiles * most, {flow_words(L, "flowTiles", f"cnt{L.rank - 1}")}, &dvmh_ws) != 0;']
     b.append('if (!flow) {')
     b.append(IND + '// one sweep after another through the ordinary handler')
     b.append(IND + 'for (long li = 0; li < nl; li++) {')
@@ -3733,7 +3762,7 @@ def chain_handler(L):
     b.append('dvmh_amd_mark_kernel_C(loop_ref, 0);')
     b.append('for (long done = 0; done < nl; done += most) {')
     b.append(IND + 'const long sweeps = nl - done < most ? nl - done : most;')
-    b += [IND + ln for ln in flow_launches(L, f'{L.name}_flow_chain_kernel', 'sweeps', ra)]
+    b += [IND + ln for ln in flow_launches(L, f'{L.name}_flow_chain_kernel', 'flowTiles', 'sweeps', ra)]
     b.append('}')
     b.append('dvmh_amd_mark_kernel_C(loop_ref, 1);')
     for ri, red in enumerate(L.reds):

@@ -628,6 +628,7 @@ struct FlowArgs {
     I lo[RANK], cnt[RANK];  // the loop
     I rlo[RANK], rhi[RANK]; // array indices the body may read: loads are clamped into them
     int ntA, ntB, sweeps;
+    long first;             // tiles of the loop in launches before this one
     DvmhAmdFlow ws;
 };
 
@@ -726,8 +727,9 @@ struct FlowCells {
 __host__ __device__ inline long flowBlocks(int rank, long n) { return (n + (rank == 3 ? 14 : 63) + 7 + 7) >> 3; }
 
 // A face is addressed by 32-bit byte offsets, up to sixteen blocks past its
-// last (those read as no cell): longer rows take another kernel.
+// last (those read as no cell); the points of a row that are walked in one launch.
 constexpr long FLOW_BLOCKS_MAX = (1L << 31) / FLOW_CELLS_BYTES - 16;
+constexpr long FLOW_ROW_MAX = FLOW_BLOCKS_MAX * 8 - 128;
 // Tiles and sweeps of a launch: a wave each, and a launch has fewer than 2^32 work-items.
 constexpr long FLOW_TASKS_MAX = (1L << 26) - 1;
 

@@ -2,7 +2,7 @@
 tests/fake_hip.cpp: what the runtime and the emitted handlers decide on the
 host (which kernels, which shapes, which memory) without a GPU.  In the child,
 `import fake_device as T` gives the counters of the fake (T.F) and small
-wrappers of the DVMH C interface."""
+wrappers of the DVMH C interface (which work on a real device as well)."""
 import ctypes
 import functools
 import os
@@ -13,6 +13,8 @@ import tempfile
 HERE = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(HERE)
 PKG = os.path.join(REPO, 'dvm-snapshot-r6603-fork_amd')
+if PKG not in sys.path:
+    sys.path.insert(0, PKG)
 L = ctypes.c_long
 INOUT, CUDA, INT_DOUBLE = L(3), L(2), 4
 
@@ -37,16 +39,18 @@ def run(code, timeout=120, **env):
 if 'FAKE_HIP' in os.environ:
     F = ctypes.CDLL(os.environ['FAKE_HIP'], mode=ctypes.RTLD_GLOBAL)
     F.fake_launch_name.restype = ctypes.c_char_p
-    for _n in ('capacity', 'used', 'refused', 'syncs', 'graphs', 'launches', 'launch_grid', 'launch_block'):
+    for _n in ('capacity', 'used', 'refused', 'asked', 'syncs', 'graphs', 'launches', 'launch_grid', 'launch_block'):
         getattr(F, 'fake_' + _n).restype = L
     F.fake_capacity.argtypes = F.fake_launch_name.argtypes = F.fake_launch_grid.argtypes = F.fake_launch_block.argtypes = [L]
     F.fake_live.argtypes = [ctypes.c_void_p]
-    import dvmh_amd as D
-    rt = D.runtime()
-    for _n in ('dvmh_region_create_C', 'dvmh_loop_create_C', 'dvmh_handler_func_C', 'dvmh_alignment_linear_C', 'dvmh_distribution_block_C'):
-        getattr(rt, _n).restype = L
-    rt.dvmh_get_natural_base_C.restype = rt.dvmh_get_device_addr_C.restype = ctypes.c_void_p
-    rt.dvmh_init_lib_C(0)
+
+import dvmh_amd as D  # noqa: E402  (behind the fake)
+
+rt = D.runtime()
+for _n in ('dvmh_region_create_C', 'dvmh_loop_create_C', 'dvmh_handler_func_C', 'dvmh_alignment_linear_C', 'dvmh_distribution_block_C'):
+    getattr(rt, _n).restype = L
+rt.dvmh_get_natural_base_C.restype = rt.dvmh_get_device_addr_C.restype = ctypes.c_void_p
+rt.dvmh_init_lib_C(0)
 
 
 def array(*dims, rt_type=INT_DOUBLE):

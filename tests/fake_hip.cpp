@@ -27,7 +27,7 @@ constexpr size_t KEPT = 4096;
 long launched = 0;
 std::map<char *, size_t> blocks, pinned;
 size_t capacity = (size_t)288 << 30, used = 0;
-long syncs = 0, refused = 0, graphs = 0;
+long syncs = 0, asked = 0, refused = 0, graphs = 0;
 bool capturing = false;
 dim3 configGrid, configBlock;
 
@@ -44,6 +44,7 @@ extern "C" {
 void fake_capacity(long bytes) { capacity = (size_t)bytes; }
 long fake_used() { return (long)used; }
 long fake_refused() { return refused; }
+long fake_asked() { return asked; }   // hipMalloc calls
 long fake_syncs() { return syncs; }
 long fake_graphs() { return graphs; }
 // p lies in memory the device has handed out and not taken back
@@ -60,6 +61,7 @@ long fake_launch_grid(long i) { return launches[(size_t)i].grid; }
 long fake_launch_block(long i) { return launches[(size_t)i].block; }
 
 hipError_t hipMalloc(void **p, size_t bytes) {
+    asked++;
     if (used + bytes > capacity) {
         refused++;
         *p = nullptr;
