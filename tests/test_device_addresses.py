@@ -1,7 +1,9 @@
 """A loop that folds its own reductions hands them to the host before its
 launch has ended.  A device address that leaves the runtime after that must not
-be used before the end: asking for one waits for the stream, once, and not in a
+be used before the end: asking for one waits for the launch, once, and not in a
 handler, whose launches come after the loop anyway.  (HIP calls faked.)"""
+import pytest
+
 import fake_device
 
 CODE = '''
@@ -15,15 +17,18 @@ def sweep(handler='loop_sor3d_32_cuda'):
 asks = [lambda: T.rt.dvmh_get_natural_base_C(T.L(1), A), lambda: T.rt.dvmh_get_device_addr_C(T.L(1), ctypes.byref(w)),
         lambda: T.rt.dvmh_fill_header_C(T.L(1), ctypes.c_void_p(0), A, (T.L * 64)(), None)]
 def waits(ask):
+    """Stream syncs, or launches that only set the completion word."""
+    F.fake_clear()
     before = F.fake_syncs()
     ask()
-    return F.fake_syncs() - before
+    return F.fake_syncs() - before + sum(1 for n, g, b in T.launches() if (g, b) == (1, 64) and 'loop' not in n)
 sweep()
 '''
 
 
-def test_address_waits_for_the_launch():
-    fake_device.run(CODE + '''
+@pytest.mark.parametrize('poll', ['1', '0'])
+def test_address_waits_for_the_launch(poll):
+    polled = '''
 for ask in asks:
     sweep()
     assert waits(ask) == 1
@@ -32,7 +37,13 @@ for ask in asks:
     sweep()
     assert waits(ask) == 1
 assert T.rt.dvmh_get_natural_base_C(T.L(0), A)
-''')
+'''
+    synced = '''   # (the results came by a stream sync)
+for ask in asks:
+    sweep()
+    assert [waits(a) for a in asks] == [0, 0, 0]
+'''
+    fake_device.run(CODE + (polled if poll == '1' else synced), DVMH_AMD_POLL=poll)
 
 
 def test_not_where_the_launch_has_ended():
