@@ -83,14 +83,21 @@ def loop(r, lib, handler, base, ranges, params, reds=(), across=None, chain=None
     rt.dvmh_loop_map_C(l, base, L(len(ranges)), *[L(rt.dvmh_alignment_linear_C(L(a + 1), L(1), L(0))) for a in range(len(ranges))])
     if across:
         rt.dvmh_loop_across_C(l, L(0), base, L(len(ranges)), *[L(w) for w in across])
-    for func, v in reds:   # (values: double)
-        rt.dvmh_loop_reduction_C(l, L(func), ctypes.byref(v), L(INT_DOUBLE), L(1), None, L(0))
+    for func, v, *loc in reds:   # (values: double)
+        rt.dvmh_loop_reduction_C(l, L(func), ctypes.byref(v), L(INT_DOUBLE), L(1), ctypes.byref(loc[0]) if loc else None,
+                                 L(ctypes.sizeof(loc[0]) if loc else 0))
     fn = getattr(D.load(lib), handler) if isinstance(handler, str) else handler
     refs = [p if isinstance(p, ctypes.Array) else ctypes.byref(p) for p in params]
     rt.dvmh_loop_register_handler_C(l, CUDA, L(0), L(rt.dvmh_handler_func_C(fn, L(len(refs)), *refs)))
     if chain:
         rt.dvmh_amd_loop_register_chain_handler_C(l, L(rt.dvmh_handler_func_C(getattr(D.load(lib), chain), L(0))))
     rt.dvmh_loop_perform_C(l)
+
+
+def host(a, shape, ctype=ctypes.c_double):
+    """The host copy of array `a`, as numpy sees it."""
+    import numpy as np
+    return np.ctypeslib.as_array(ctypes.cast(rt.dvmh_get_natural_base_C(L(0), a), ctypes.POINTER(ctype)), shape=shape)
 
 
 def launches():

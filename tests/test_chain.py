@@ -1,16 +1,17 @@
 """Chains of ACROSS sweeps: consecutive executions of the SOR sweep loop
 queued in one batch (programs/sor3d.c sor3d_iterate_chain) run through the
-loop's chain handler, every sweep two tile-planes behind the one before it in
-one launch sequence, each with its own REDUCTION(MAX) segment.  Results must
-equal the sequential sweeps bit for bit, whatever the group size, tile shape
-and grid size; configurations other than the tiled wavefront fall back to one
-sweep after another."""
+loop's chain handler as one dataflow launch, each with its own REDUCTION(MAX)
+segment.  Results must equal the sequential sweeps bit for bit, whatever the
+group size and grid size, and whatever configuration is asked for (the launch
+has one); sweeps that differ, and those there is no workspace for
+(test_flow_limits.py), run one after another."""
 import ctypes
 
 import numpy as np
 import pytest
 
 import dvmh_amd as D
+import fake_device as T
 import helpers as H
 
 KIND_WAVEFRONT = 2
@@ -55,8 +56,8 @@ def test_chain_host_path():
 @pytest.mark.parametrize('n,iters,group', [(5, 3, 3), (23, 7, 3), (23, 6, 6), (41, 9, 4), (70, 5, 5)])
 def test_chain_bit_exact(cfg, n, iters, group):
     """Tiles overhanging the loop, tiles larger than it (n = 5), groups that
-    divide the sweeps and groups that leave a shorter last group; tiles with at
-    most one column per thread, up to four (128 x 16 x 16) and more (32 x 16 x 8)."""
+    divide the sweeps and groups that leave a shorter last group; the forced
+    configurations must not matter."""
     block, tune = _tile(*cfg)
     _force(block, tune)
     before = D.stats()
@@ -73,8 +74,7 @@ def test_chain_bit_exact(cfg, n, iters, group):
 
 @pytest.mark.gpu
 def test_chain_falls_back_without_tiles():
-    """Hyperplane configuration (not the tiled wavefront): the chain handler
-    runs the group's sweeps one after another."""
+    """A hyperplane configuration does not matter to a chain either."""
     _force((64, 1, 1), [1, 0, 0, 0, 0, 0, 0, 0])
     try:
         res = H.run_sor3d_chain(19, 5, 5)
@@ -87,9 +87,7 @@ def test_chain_falls_back_without_tiles():
 @pytest.mark.gpu
 @pytest.mark.parametrize('cfg', [(256, 8, 8), (256, 12, 16)])
 def test_chain_full_size(cfg):
-    """320^3 (the SOR workload's size), 6 sweeps in one chain: 8^3 tiles, and
-    12 x 12 x 16 tiles on 256 threads (one column per thread, the shape the
-    tuner keeps)."""
+    """320^3 (the SOR workload's size), 6 sweeps in one chain."""
     block, tune = _tile(*cfg)
     _force(block, tune)
     try:
@@ -101,11 +99,46 @@ def test_chain_full_size(cfg):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('what', ['bounds', 'scalar', 'array'])
+def test_sweeps_that_differ(what):
+    """One queue of sweeps that differ in their bounds, their scalar or their
+    array: no chain of them is one launch.  Equal to the sweeps without a queue."""
+    n = 19
+    got = []
+    for queued in (True, False):
+        w = [ctypes.c_double(1.5), ctypes.c_double(1.5 if what != 'scalar' else 1.1)]
+        nn, seed = ctypes.c_long(n), ctypes.c_ulonglong(5)
+        X = [T.array(n, n, n), T.array(n, n, n)]
+        r = T.region(*X, scalars=[nn, seed])
+        for x in X:
+            T.loop(r, 'libprog_sor3d.so', 'loop_sor3d_18_cuda', x, [(0, n - 1)] * 3, [x, nn, seed])
+        T.rt.dvmh_region_end_C(r)
+        eps = [ctypes.c_double() for _ in range(5)]
+        if queued:
+            T.rt.dvmh_amd_batch_begin_C()
+        for q in range(5):
+            x = X[q % 2 if what == 'array' else 0]
+            v = w[q % 2 if what == 'scalar' else 0]
+            hi = n - 2 - (q % 2 if what == 'bounds' else 0)
+            r = T.region(*X, scalars=w)
+            T.loop(r, 'libprog_sor3d.so', 'loop_sor3d_32_cuda', x, [(1, hi), (1, n - 2), (1, hi)], [x, v], reds=[(3, eps[q])], across=[1] * 6,
+                   chain='loop_sor3d_32_cuda_chain', line=32)
+            T.rt.dvmh_region_end_C(r)
+        if queued:
+            T.rt.dvmh_amd_batch_end_C()
+        for x in X:
+            T.rt.dvmh_get_actual_array2_(x)
+        got.append([T.host(x, (n ** 3,)).copy() for x in X] + [np.array([e.value for e in eps])])
+        for x in X:
+            T.rt.dvmh_delete_object_(x)
+    assert all(H.bits_equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.gpu
 def test_chain_tuned_bit_exact():
     """Cost-model mode: the per-loop site is explored sweep by sweep inside the
-    first groups, then the chain's own site times its tile shapes group by
-    group (exhaustively: no records of chains train the model).  Every run is
-    bit-exact and the chain site ends settled with a recorded best shape."""
+    first groups, then the chain's own site times its one configuration.  Every
+    run is bit-exact and the chain site ends settled."""
     from dvmh_amd import costmodel as CM
     r = CM.rt()
     if r.dvmh_amd_model_load_C(CM.MODEL.encode()) < 0:

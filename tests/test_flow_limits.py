@@ -1,6 +1,7 @@
 """Host decisions about the dataflow launch of ACROSS loops, with the HIP calls
 faked (no GPU, nothing runs): the longest rows and the most tiles it is used
 for, chains cut to what one launch can hold, and the workspace it is handed."""
+import ctypes
 import os
 import subprocess
 import sys
@@ -228,11 +229,7 @@ def test_in_parts_gpu(mb):
 @pytest.mark.parametrize('cut', [1, 8, 9, 30])
 def test_rows_in_parts_gpu(cut):
     """A sweep cut along its innermost axis, the parts one after another."""
-    import ctypes
-    T = fake_device
-    n = 40
-    P = D.Program('sor3d')
-    P.fn('setup', [ctypes.c_long, ctypes.c_ulonglong])
+    T, n = fake_device, 40
     w, e, nn, seed = ctypes.c_double(1.5), ctypes.c_double(0), ctypes.c_long(n), ctypes.c_ulonglong(D.SEED_BASE + 3)
     A = T.array(n, n, n)
     r = T.region(A, scalars=[w, nn, seed])
@@ -241,7 +238,7 @@ def test_rows_in_parts_gpu(cut):
         T.loop(r, 'libprog_sor3d.so', 'loop_sor3d_32_cuda', A, [(1, n - 2), (1, n - 2), part], [A, w], reds=[(3, e)], across=[1] * 6)
     T.rt.dvmh_region_end_C(r)
     T.rt.dvmh_get_actual_array2_(A)
-    got = np.ctypeslib.as_array(ctypes.cast(T.rt.dvmh_get_natural_base_C(T.L(0), A), ctypes.POINTER(ctypes.c_double)), shape=(n ** 3,)).copy()
+    got = T.host(A, (n ** 3,)).copy()
     T.rt.dvmh_delete_object_(A)
     ref = H.oracle_sor3d(n, 1)
     assert H.bits_equal(got, ref['A']) and e.value == ref['eps'][0]
