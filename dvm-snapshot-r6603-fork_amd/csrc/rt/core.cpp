@@ -245,9 +245,10 @@ bool Gpu::flowWorkspace(long tiles, long cellWords, DvmhAmdFlow *out) {
                 return false;
             }
         }
-        // what the handler allocates next must find room as well
-        size_t left = 0, all = 0;
-        HIP_CHECK(hipMemGetInfo(&left, &all));
+        // what the handler allocates next must find room as well (small ones
+        // hardly matter to it, and asking takes 0.2 ms)
+        size_t left = ~(size_t)0, all = 0;
+        if (need > (size_t)32 << 20) HIP_CHECK(hipMemGetInfo(&left, &all));
         if (left < need / 8 + ((size_t)64 << 20)) {
             HIP_CHECK(hipFree(p));
             flowRefused = need;

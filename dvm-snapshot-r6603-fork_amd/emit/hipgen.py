@@ -1322,8 +1322,9 @@ def star_shape(L):
          'int dvmh_starXcd = (int)tune[DVMH_AMD_T_XCD];',
          'if (dvmh_star && tune[DVMH_AMD_T_OWN]) {',
          IND + f'const DvmType dvmh_cx = cnt{r - 1}, dvmh_w1 = (dvmh_cx + 63) / 64, dvmh_w2 = (dvmh_cx + 127) / 128;',
-         IND + '// beyond the 256 MB last-level cache stored lines are not found there again (384^3 doubles: 198 -> 175 us;',
-         IND + '// inside it they are: 201 x 187 x 239 24 -> 30, 256^3 37 -> 45)',
+         IND + '// beyond the 256 MB last-level cache stored lines are not found there again, inside it they are.  An iteration',
+         IND + '// with its folds, stores through the caches and past them: 216 MB 49 and 61 us, 268 MB 68 and 80, 288 MB 102 and',
+         IND + '// 102, 315 MB 102 and 85, 515 MB 130 and 119, 618 MB 182 and 171',
          IND + f'dvmh_starNt = (double)({" + ".join(f"sizeof({p[2]})" for p in arrs)}) * {" * ".join(f"cnt{i}" for i in range(r))} > 268e6 * 1.02;',
          IND + 'dvmh_starXcd = dvmh_starNt ? 0 : 1;']
     b += [IND + '// two points per lane unless that leaves lanes of the last tile idle (320: five tiles of 64, 106 us, or three of',
@@ -2909,9 +2910,12 @@ def flow_kernel(L):
         k.append('}')
         return '\n'.join(k) + '\n'
 
-    tile = 'dvmh_f.first + (long)dvmh_task.ta * dvmh_f.ntB + dvmh_task.tb'
-    out = kernel(f'{L.name}_flow_kernel', False, fp + red_kernel_params(L) + red_finish_params(L), red_kernel_locals(L),
-                 red_kernel_finish(L, tile))
+    tile = '(long)dvmh_task.ta * dvmh_f.ntB + dvmh_task.tb'
+    # dvmh_before: tiles of the loop in launches before this one (as the last
+    # argument: in FlowArgs it moved the others, and the walk's schedule with
+    # them, 318^3 483 -> 500 us)
+    out = kernel(f'{L.name}_flow_kernel', False, fp + red_kernel_params(L) + red_finish_params(L) + ['long dvmh_before'], red_kernel_locals(L),
+                 red_kernel_finish(L, f'dvmh_before + {tile}') if L.reds else [])
     if L.chain_eligible():
         # sweep s folds its reductions into its own segment, from its own initial values
         cp, init = [], []
@@ -2962,7 +2966,7 @@ def flow_launches(L, kernel, tiles, sweeps, tail_args, part=None):
             c.append(f'dvmh_f.s[{a}] = ({it}){X}_devHdr[{a + 1}]; dvmh_f.lo[{a}] = ({it})({lo}); dvmh_f.cnt[{a}] = ({it}){n};')
             c.append(f'dvmh_f.rlo[{a}] = ({it})({lo} + ({rng[a][0]})); dvmh_f.rhi[{a}] = ({it})({lo} + {n} - 1 + ({rng[a][1]}));')
         c += [f'dvmh_f.ntA = (int){"dvmh_a" if 0 in part else "flowA"}; dvmh_f.ntB = (int)flowB;', f'dvmh_f.sweeps = (int)({sweeps});',
-              f'dvmh_f.first = {"dvmh_first" if 0 in part else "0"};', 'dvmh_f.ws = dvmh_ws;']
+              'dvmh_f.ws = dvmh_ws;']
         args = ['dvmh_f']
         for p in L.arrays:
             if p[1] != X:
@@ -3001,15 +3005,15 @@ def flow_launch(L, otherwise):
     b.append('if (flow) {')
     b += [IND + ln for ln in handler_reds_prepare(L, 'flowTiles * flowRows', 0) + red_finish_query(L, 'flowTiles * flowRows')]
     b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 0);')
-    b += [IND + 'DvmType dvmh_first = 0;',
+    b += [IND + 'long dvmh_before = 0;',
           IND + 'for (DvmType dvmh_at = 0; dvmh_at < flowA; dvmh_at += flowPart) {',
           IND * 2 + 'const DvmType dvmh_a = flowA - dvmh_at < flowPart ? flowA - dvmh_at : flowPart;',
           IND * 2 + f'const DvmType dvmh_lo0 = dvmh_at * {sh}::PA, dvmh_n0 = cnt0 - dvmh_lo0 < dvmh_a * {sh}::PA ? cnt0 - dvmh_lo0 : dvmh_a * {sh}::PA;',
           IND * 2 + f'for (DvmType dvmh_lo{k} = 0; dvmh_lo{k} < cnt{k}; dvmh_lo{k} += flowRow) {{',
           IND * 3 + f'const DvmType dvmh_n{k} = cnt{k} - dvmh_lo{k} < flowRow ? cnt{k} - dvmh_lo{k} : flowRow;']
-    b += [IND * 3 + ln for ln in flow_launches(L, f'{L.name}_flow_kernel', 'dvmh_a * flowB', '1', red_fact_args(L) + red_finish_args(L),
+    b += [IND * 3 + ln for ln in flow_launches(L, f'{L.name}_flow_kernel', 'dvmh_a * flowB', '1', red_fact_args(L) + red_finish_args(L) + ['dvmh_before'],
                                                {0: ('dvmh_lo0', 'dvmh_n0'), k: (f'dvmh_lo{k}', f'dvmh_n{k}')})]
-    b += [IND * 3 + 'dvmh_first += dvmh_a * flowB;', IND * 2 + '}', IND + '}']
+    b += [IND * 3 + 'dvmh_before += dvmh_a * flowB;   // tiles of the loop in launches before the next', IND * 2 + '}', IND + '}']
     b.append(IND + 'dvmh_amd_mark_kernel_C(loop_ref, 1);')
     b += [IND + ln for ln in handler_reds_finish(L)]
     b.append('} else {')

@@ -29,8 +29,9 @@ extern "C" {
                                       VARIANT 3, dependent axis innermost and unit stride:
                                       a wave streams 64 lines in aligned 128-byte chunks,
                                       coalesced, transposed through LDS, a lane per line) */
-#define DVMH_AMD_KIND_WAVEFRONT 2  /* ACROSS with >= 2 dependent axes: hyperplane wavefront; a loop whose axes all
-                                      depend runs as one dataflow launch whatever the tiles asked for */
+#define DVMH_AMD_KIND_WAVEFRONT 2  /* ACROSS with >= 2 dependent axes: hyperplane wavefront (VARIANT 1, three axes:
+                                      tiles staged in LDS); a loop whose axes all depend and whose body allows it
+                                      runs as one dataflow launch whatever is asked for */
 #define DVMH_AMD_KIND_STENCIL 3    /* PARALLEL whose handler also has the LDS march variant
                                       (VARIANT 1: TILE_A = points per thread on the innermost
                                       axis, CHUNK = planes per workgroup on the outermost) */

@@ -572,7 +572,8 @@ __device__ __forceinline__ void publishDone(const DvmhAmdRedFinish &f) {
 // dependent FP64 operations and a lane shift), 0.165 for rank 3 (one neighbour
 // through LDS), and along a diagonal of tiles, per tile, the lanes' skew plus
 // about 4 us until a finished block is seen by the next tile; chains of large
-// grids by memory traffic (26 bytes a point and sweep, 3.5 TB/s).  Measured,
+// grids by the same with several sweeps in flight (they move 26 bytes a point
+// and sweep, 3.5 TB/s of the 6.3 a copy reaches).  Measured,
 // one sweep with reductions: 2-D 998^2 0.38 ms (a launch per hyperplane: 9.2),
 // 3-D 128^3 0.145 ms (a launch per tile-plane: 0.43), 318^3 0.48 ms (1.84; 0.76
 // with rows moved unaligned and a cell's halves in two stores).
@@ -628,7 +629,6 @@ struct FlowArgs {
     I lo[RANK], cnt[RANK];  // the loop
     I rlo[RANK], rhi[RANK]; // array indices the body may read: loads are clamped into them
     int ntA, ntB, sweeps;
-    long first;             // tiles of the loop in launches before this one
     DvmhAmdFlow ws;
 };
 
@@ -841,9 +841,10 @@ __device__ __forceinline__ void readHere(T &x) {
 // current plane only, neighbours along a row come from the lane beside.  No LDS
 // and no barrier: the loads of the next planes stay in flight across the
 // arithmetic (with planes staged in LDS, two barriers a plane drained them).
-// Bound by memory: 256^3 doubles, 268 MB read and written, 37 us (7.3 TB/s,
-// partly from the last-level cache; planes in LDS 78, direct 76), 201 x 187 x
-// 239 24 us (45), 128^3 9 (26); 384^3, beyond that cache, 175 (200).
+// Bound by memory.  Without a reduction: 256^3 doubles, 268 MB read and written,
+// 37 us (7.3 TB/s, partly from the last-level cache; planes in LDS 78, direct
+// 76), 201 x 187 x 239 24 us (45), 128^3 9 (26); 384^3, beyond that cache, 175
+// (200).  With MAX and SUM folded in the launch: 201 x 187 x 239 30 us, 384^3 182.
 // Loads are clamped into [rlo, rhi], the indices the body may read.
 // (Rank 2 has too little to keep: the same march over rows of 2-D grids is no
 // faster than the direct kernel, 2048^2 23 us both, 1024^2 15 against 14.)
