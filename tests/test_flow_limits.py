@@ -212,6 +212,12 @@ for n in (20, 67, 131):
         assert H.bits_equal(res['A'], ref['A']) and np.array_equal(res['eps'], ref['eps']), n
 for n in (66, 200, 331):
     _check_relax2d(n, 2)
+rt = H.D.runtime()
+rt.dvmh_amd_set_graph_C(1)
+rt.dvmh_amd_set_graph_min_nodes_C(1)
+before = H.D.stats()['graph_replays']
+res, ref = H.run_sor3d(67, 8, flags=H.D.REGION_AMD_GRAPH), H.oracle_sor3d(67, 8)
+assert H.bits_equal(res['A'], ref['A']) and np.array_equal(res['eps'], ref['eps']) and H.D.stats()['graph_replays'] > before + 4
 print('equal')
 '''
 
@@ -219,8 +225,8 @@ print('equal')
 @pytest.mark.gpu
 @pytest.mark.parametrize('mb', [0, 1, 3])
 def test_in_parts_gpu(mb):
-    """No workspace, one for a row of tiles or so, one for some: sweeps in parts,
-    chains sweep by sweep."""
+    """No workspace, one for a row of tiles or so, one for some: sweeps in parts
+    (replayed from a graph too), chains sweep by sweep."""
     p = subprocess.run([sys.executable, '-c', CHILD], env=dict(os.environ, DVMH_AMD_FLOW_MB=str(mb)), capture_output=True, text=True, timeout=100)
     assert p.returncode == 0 and p.stdout.strip().endswith('equal'), p.stderr[-2000:]
 
