@@ -68,9 +68,9 @@ def indent(text, n):
 
 
 # Calls that evaluate their arguments and return (a macro of another name may
-# choose between its arguments, or jump).
-PLAIN_CALLS = {'fabs', 'fabsf', 'sqrt', 'sqrtf', 'exp', 'expf', 'log', 'logf', 'sin', 'sinf', 'cos', 'cosf', 'tan', 'tanf', 'pow', 'powf',
-               'fmax', 'fmaxf', 'fmin', 'fminf', 'fma', 'fmaf', 'abs', 'labs', 'Max', 'Min', 'MAX', 'MIN', 'max', 'min'}
+# choose between its arguments, or jump); the short ones are a few instructions.
+SHORT_CALLS = {'fabs', 'fabsf', 'fmax', 'fmaxf', 'fmin', 'fminf', 'fma', 'fmaf', 'abs', 'labs', 'Max', 'Min', 'MAX', 'MIN', 'max', 'min'}
+PLAIN_CALLS = SHORT_CALLS | {'sqrt', 'sqrtf', 'exp', 'expf', 'log', 'logf', 'sin', 'sinf', 'cos', 'cosf', 'tan', 'tanf', 'pow', 'powf'}
 
 
 def reached(body):
@@ -268,6 +268,17 @@ class Loop:
         return [f'static const DvmType dvmh_{name}_off[{2 * self.rank}] = {{{off}}};'], \
             f'dvmh_amd_loop_reads_inside_C({loop}, {header or name + "_hdr"}, dvmh_{name}_off, dvmh_{name}_off + {self.rank}) != 0'
 
+    def marches(self):
+        """A wave's points may take the body one after another, as the marches
+        have them: no loop, no call of unknown length, and no branch beside a long
+        one.  200^3, register march and direct: a residual kept by an if 25 and 35
+        us, exp unconditionally 38 and 38, exp or sin by a branch 67 and 47, a while
+        57 and 37."""
+        calls = set(re.findall(r'\b([A-Za-z_]\w*)\s*\(', self.body)) - {'if', 'sizeof', 'return'}
+        if re.search(r'\b(for|while|do|switch)\b', self.body):
+            return False
+        return calls <= (SHORT_CALLS if re.search(r'\bif\b|\?|&&|\|\|', self.body) else PLAIN_CALLS)
+
     def leaves(self):
         """The body may end an iteration early: it cannot be a function's body."""
         return bool(re.search(r'\b(continue|return|goto)\b', self.body))
@@ -278,7 +289,7 @@ class Loop:
         can live in registers (starMarch).  None if there is no such array, or
         more than one array is read beside the loop point."""
         near = [p for p in self.arrays if self.rank == 3 and self._is_stencil(p[1]) and any(lo or hi for lo, hi in self.stencil_range(p[1]))]
-        if len(near) != 1 or len(self.body) > 2000 or self.leaves() or not self.loads_ahead(near[0][1]):
+        if len(near) != 1 or len(self.body) > 2000 or self.leaves() or not self.marches() or not self.loads_ahead(near[0][1]):
             return None
         X = near[0][1]
         if near[0][2] not in ('int', 'long', 'float', 'double'):
@@ -1373,7 +1384,7 @@ def parallel_own_shape(L):
           IND + f'tune[DVMH_AMD_T_DEPTH] = {8 if r == 3 else 4};']
     if r == 3:
         b.append(IND + 'threads = dim3(64, 4, 1);')
-        if L.stencil and all(L.loads_ahead(nm) for nm in L.stencil):
+        if L.stencil and L.marches() and all(L.loads_ahead(nm) for nm in L.stencil):
             b.append(IND + 'if (cnt2 >= 128 && cnt0 * cnt1 * cnt2 >= 280L * 280 * 280) { tune[DVMH_AMD_T_VARIANT] = 1; tune[DVMH_AMD_T_TILE_A] = 2; tune[DVMH_AMD_T_CHUNK] = 32; }')
     else:
         b.append(IND + f'threads = cnt{r - 1} >= 128 ? dim3(128, 4, 1) : dim3(64, 8, 1);')

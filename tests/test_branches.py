@@ -54,6 +54,19 @@ def test_what_may_be_loaded_ahead(body, ahead):
     assert L.flow_eligible() == ahead
 
 
+@pytest.mark.parametrize('tail,march', [
+    ('B[i][j][k] = t;', True), ('B[i][j][k] = exp(t) + sqrt(t);', True), ('if (t > r) r = t;\nB[i][j][k] = fabs(t);', True),
+    ('B[i][j][k] = t > 1 ? MAX(t, 2.0) : t;', True), ('B[i][j][k] = t > 0 ? sqrt(t) : 0;', False), ('if (t > 1) t = sin(t);\nB[i][j][k] = t;', False),
+    ('while (t > 1) t *= 0.5;\nB[i][j][k] = t;', False), ('for (int q = 0; q < 4; q++) t *= t;\nB[i][j][k] = t;', False),
+    ('B[i][j][k] = weight(t);', False)])
+def test_which_bodies_march(tail, march):
+    """The register march where nobody tuned: not for bodies that take lanes apart for long."""
+    L = hipgen.Loop({'name': 'l', 'vars': [(v, 'int') for v in 'ijk'], 'params': [('array', 'A', 'double', 3), ('array', 'B', 'double', 3)],
+                     'reductions': [('max', 'r', 'double')],
+                     'body': 'double t = A[i - 1][j][k] + A[i + 1][j][k] + A[i][j - 1][k] + A[i][j][k + 1];\n' + tail}, 't')
+    assert (L.star_array() == 'A') == march
+
+
 def test_early_end_keeps_other_kernels():
     """(a kernel whose body is a function's)"""
     L = hipgen.Loop({'name': 'l', 'vars': [('i', 'int'), ('j', 'int')], 'params': [('array', 'X', 'double', 2)],
